@@ -613,6 +613,21 @@ hg_status build_range(hg_ctx c, const BinMap &map, int kb, int ob, uint64_t n, u
                       const void *d_keys, void *d_off, void *d_csr, uint64_t *d_csr_index = nullptr,
                       bool pack_in = false) {
   if (n == 0) return fill_offsets(c, d_off, ob, R + 1, 0);
+  if (!pack_in && !d_csr_index && build_one_takes(n, R, kb)) {
+    LaunchBuildOne b{};
+    b.key_bytes = kb;
+    b.off_bytes = ob;
+    b.keys = d_keys;
+    b.csr = d_csr;
+    b.off = d_off;
+    b.n = (uint32_t)n;
+    b.bin_lo = (uint32_t)lo;
+    b.nbins = (uint32_t)R;
+    b.map = map;
+    Prof pf(c, "final");
+    HG_HIP(launch_build_one(b, c->stream));
+    return HG_OK;
+  }
   const uint32_t W = choose_width(n, R, kb, build_fill());
   const uint64_t F = (R + W - 1) / W;
   const uint64_t k = level1_group(F);

@@ -1,0 +1,65 @@
+"""Small and mid-sized tables, which take shorter kernel sequences than large
+ones: edges of every size class against the CPU oracle."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+from hashgraph_amd import workloads as wl
+from oracle import oracle as o
+
+
+def _to_dev(a, dev):
+    import torch
+    return torch.from_numpy(a.view(np.int32 if a.dtype == np.uint32 else np.int64).copy()).to(dev)
+
+
+def _same(off, csr, keys, M, ob):
+    goff = off.cpu().numpy().view(np.uint32 if ob == 4 else np.uint64).astype(np.uint64)
+    gcsr = csr.cpu().numpy().view(keys.dtype).copy()
+    eoff, ecsr = o.build_csr(keys, M)
+    assert np.array_equal(goff, eoff), "offsets differ"
+    o.canon(goff, gcsr)
+    o.canon(eoff, ecsr)
+    assert np.array_equal(gcsr, ecsr), "bin contents differ"
+
+
+@pytest.mark.parametrize("kb,ob", [(4, 4), (8, 8)])
+@pytest.mark.parametrize("n,M", [(1, 1), (1, 65535), (1024, 4096), (1024, 4097), (1025, 1000), (4096, 65535),
+                                 (4097, 3), (16384, 16384), (16384, 65536), (16385, 16385)])
+def test_one_workgroup_build(n, M, kb, ob, dev):
+    import hashgraph_amd as hg
+    print(f"one-workgroup build n={n} M={M} kb={kb} ob={ob}", flush=True)
+    keys = wl.uniform_keys(n + M, n, kb)
+    off, csr = hg.build(_to_dev(keys, dev), M, offset_bytes=ob)
+    _same(off, csr, keys, M, ob)
+
+
+@pytest.mark.parametrize("kb", [4, 8])
+def test_one_workgroup_build_in_place_and_hot_key(kb, dev):
+    """The CSR written over the input keys; a table of one repeated key."""
+    import torch
+    import hashgraph_amd as hg
+    n, M = 16384, 5000
+    for keys in (wl.uniform_keys(9, n, kb), np.full(n, 12345, dtype=np.uint32 if kb == 4 else np.uint64)):
+        dk = _to_dev(keys, dev)
+        off = torch.empty(M + 1, dtype=torch.int32, device=dev)
+        hg.build(dk, M, out=(off, dk))
+        _same(off, dk, keys, M, 4)
+
+
+def test_one_workgroup_build_learned(dev):
+    """A learned table of one workgroup: every key in the bin its hash gives."""
+    import torch
+    import hashgraph_amd as hg
+    keys = wl.lognormal_keys(3, 16000)
+    dk = _to_dev(keys, dev)
+    M = 12000
+    model, _ = hg.rmi_train(dk, M, n_sample=4000, seed=1, n_leaves=1024)
+    off, csr = hg.build(dk, M, hash_kind=hg.HG_HASH_RMI, rmi_model=model)
+    bins = hg.table_bins(dk, M, hash_kind=hg.HG_HASH_RMI, rmi_model=model).to(torch.int64)
+    deg = torch.bincount(bins, minlength=M)
+    assert torch.equal(off[1:].to(torch.int64), torch.cumsum(deg, 0)) and int(off[0]) == 0
+    cb = hg.table_bins(csr, M, hash_kind=hg.HG_HASH_RMI, rmi_model=model).to(torch.int64)
+    assert torch.equal(cb, torch.repeat_interleave(torch.arange(M, device=dev), deg))
+    assert torch.equal(torch.sort(csr).values, torch.sort(dk).values)
