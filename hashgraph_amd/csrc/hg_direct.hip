@@ -31,7 +31,126 @@ __global__ __launch_bounds__(BLOCK) void k_build_one(const K *keys, K *csr, OFF 
   final_bucket<K, OFF, BLOCK, KPT, HK>(keys, csr, off, it, mp, smem32, lds_bytes, nullptr);
 }
 
+// ---------------------------------------------------------------------------
+// Direct probe: every thread hashes U probe keys, reads their bins' offsets
+// and walks the bins in global memory; the probe keys are not partitioned.
+// Bound by the latency of three dependent reads per key (probe key, offsets,
+// bin), so the U reads of a step are all issued before the first is used, and
+// from about 10^5 keys on by the lines those reads bring in: 2^20 uint32 keys
+// against 2^20 take 49 us (124 us partitioned), about 22 keys/ns beyond.
+// Matches: one block scan and one reservation per workgroup.  A key of a bin
+// longer than PROBE_BIN_LIMIT goes to the `heavy` list for the caller.
+//
+// `st` (a DirectState, zero between calls) collects the counts; the last
+// workgroup to finish stores them to `res` in pinned host memory and zeroes
+// the state again, so a call needs no fill and no copy back.
+// ---------------------------------------------------------------------------
+struct DirectState {
+  unsigned long long cursor;  // matches
+  unsigned int heavy;         // keys listed
+  unsigned int ticket;        // workgroups done
+};
+static_assert(sizeof(DirectState) <= DIRECT_STATE_BYTES, "DirectState");
+
+template <typename OFF>
+__device__ __forceinline__ void load_pair(const OFF *p, OFF &a, OFF &b) {
+  OFF v[2];
+  __builtin_memcpy(v, p, sizeof(v));  // one load (element alignment is enough on gfx950)
+  a = v[0];
+  b = v[1];
+}
+
+template <typename K, typename OFF, int BLOCK, int U, int HK>
+__global__ __launch_bounds__(BLOCK) void k_probe_direct(const K *__restrict__ probe, uint32_t n, BinMap mp,
+                                                        const OFF *__restrict__ offA, const K *__restrict__ keysA,
+                                                        K *__restrict__ out, uint64_t capacity, K *__restrict__ heavy,
+                                                        DirectState *__restrict__ st,
+                                                        unsigned long long *__restrict__ res) {
+  __shared__ uint32_t s_tmp[BLOCK / 64 + 1];
+  __shared__ unsigned long long s_base;
+  const uint32_t k0 = blockIdx.x * (BLOCK * U);
+  const uint32_t cnt = min((uint32_t)(BLOCK * U), n - k0);
+  const __amdgpu_buffer_rsrc_t rs = make_rsrc(probe + k0, cnt * (uint32_t)sizeof(K));
+  K kr[U];
+  OFF b0[U], b1[U];
+  uint32_t m[U];
+#pragma unroll
+  for (int j = 0; j < U; j++) kr[j] = buf_load<K>(rs, threadIdx.x * (uint32_t)sizeof(K), j * BLOCK * (uint32_t)sizeof(K));
+#pragma unroll
+  for (int j = 0; j < U; j++) {
+    const uint32_t l = bin_of<K, HK>(kr[j], mp);  // slots past cnt hold key 0: a valid bin
+    load_pair(offA + l, b0[j], b1[j]);
+  }
+  uint32_t longest = 0;
+#pragma unroll
+  for (int j = 0; j < U; j++) {
+    m[j] = 0;
+    if (j * BLOCK + threadIdx.x >= cnt) b1[j] = b0[j];
+    if (b1[j] - b0[j] > PROBE_BIN_LIMIT) {
+      heavy[atomicAdd(&st->heavy, 1u)] = kr[j];
+      b1[j] = b0[j];
+    }
+    longest = max(longest, (uint32_t)(b1[j] - b0[j]));
+  }
+  // the U walks advance together, two keys of each bin per step
+  for (uint32_t q = 0; q < longest; q += 2) {
+    K v[U][2];
+#pragma unroll
+    for (int j = 0; j < U; j++)
+#pragma unroll
+      for (int i = 0; i < 2; i++) v[j][i] = b0[j] + q + i < b1[j] ? keysA[b0[j] + q + i] : (K)~kr[j];
+#pragma unroll
+    for (int j = 0; j < U; j++)
+#pragma unroll
+      for (int i = 0; i < 2; i++) m[j] += v[j][i] == kr[j] ? 1u : 0u;
+  }
+  uint32_t mine = 0;
+#pragma unroll
+  for (int j = 0; j < U; j++) mine += m[j];
+  uint32_t tot;
+  const uint32_t ex = block_exclusive_sum<BLOCK, uint32_t>(mine, s_tmp, tot);
+  if (threadIdx.x == 0) s_base = tot ? atomicAdd(&st->cursor, (unsigned long long)tot) : 0ull;
+  __syncthreads();
+  if (out != nullptr && mine) {
+    unsigned long long w = s_base + ex;
+#pragma unroll
+    for (int j = 0; j < U; j++)
+      for (uint32_t r = 0; r < m[j]; r++, w++)
+        if (w < capacity) out[w] = kr[j];
+  }
+  if (threadIdx.x == 0) {
+    __threadfence();  // this workgroup's adds before its ticket (the barrier above ordered the others' list adds)
+    if (atomicAdd(&st->ticket, 1u) == gridDim.x - 1) {
+      __threadfence();
+      res[0] = atomicExch(&st->cursor, 0ull);
+      res[1] = atomicExch(&st->heavy, 0u);
+      atomicExch(&st->ticket, 0u);
+      __threadfence_system();
+    }
+  }
+}
+
 namespace {
+
+template <typename K, typename OFF, int HK>
+hipError_t launch_direct_u(const LaunchProbeDirect &p, hipStream_t st) {
+  auto go = [&](auto kern, uint32_t block, uint32_t per) {
+    hipLaunchKernelGGL(kern, dim3((p.n + per - 1) / per), dim3(block), 0, st, (const K *)p.probe, p.n, p.map,
+                       (const OFF *)p.offA, (const K *)p.keysA, (K *)p.out, p.capacity, (K *)p.heavy,
+                       (DirectState *)p.state, p.res);
+    return hipGetLastError();
+  };
+  // few keys are spread over more, smaller workgroups; many take fewer
+  // reservations of the shared cursor (one address: about 80 a microsecond)
+  if (p.n <= 65536) return go(&k_probe_direct<K, OFF, 256, 1, HK>, 256, 256);
+  if (p.n <= (1u << 18)) return go(&k_probe_direct<K, OFF, 256, 4, HK>, 256, 1024);
+  return go(&k_probe_direct<K, OFF, 1024, 4, HK>, 1024, 4096);
+}
+
+template <typename K, typename OFF>
+hipError_t launch_direct_hk(const LaunchProbeDirect &p, hipStream_t st) {
+  return p.map.kind == 0 ? launch_direct_u<K, OFF, HK_MURMUR>(p, st) : launch_direct_u<K, OFF, HK_RMI>(p, st);
+}
 
 template <typename K, typename OFF, int BLOCK, int KPT, int HK>
 hipError_t launch_one(const LaunchBuildOne &b, hipStream_t st) {
@@ -78,6 +197,13 @@ hipError_t launch_build_one(const LaunchBuildOne &b, hipStream_t st) {
   if (b.key_bytes == 4)
     return b.off_bytes == 4 ? launch_one_hk<uint32_t, uint32_t>(b, st) : launch_one_hk<uint32_t, uint64_t>(b, st);
   return b.off_bytes == 4 ? launch_one_hk<uint64_t, uint32_t>(b, st) : launch_one_hk<uint64_t, uint64_t>(b, st);
+}
+
+hipError_t launch_probe_direct(const LaunchProbeDirect &p, hipStream_t st) {
+  if (!p.n || p.map.kind > 1) return hipErrorInvalidValue;
+  if (p.key_bytes == 4)
+    return p.off_bytes == 4 ? launch_direct_hk<uint32_t, uint32_t>(p, st) : launch_direct_hk<uint32_t, uint64_t>(p, st);
+  return p.off_bytes == 4 ? launch_direct_hk<uint64_t, uint32_t>(p, st) : launch_direct_hk<uint64_t, uint64_t>(p, st);
 }
 
 hipError_t set_direct_kernel_attributes() {

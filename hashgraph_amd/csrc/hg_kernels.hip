@@ -18,10 +18,6 @@
 
 namespace hg {
 
-// Bins longer than this are not walked by the probe kernels but answered from
-// a value table by k_probe_heavy (duplicates: a walk would cost
-// |A_bin| x |B_bin| comparisons).
-constexpr uint64_t PROBE_BIN_LIMIT = 32;
 // A join bin pair with more key pairs than this is answered from a value
 // table (k_join_heavy) instead of the nested loop.
 constexpr uint64_t JOIN_PAIR_LIMIT = 4096;

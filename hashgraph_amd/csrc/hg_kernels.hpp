@@ -114,6 +114,25 @@ struct LaunchBuildOne {
   BinMap map;
 };
 
+// Bins longer than this are not walked by the probe kernels but answered from
+// a value table by k_probe_heavy (duplicates: a walk would cost
+// |A_bin| x |B_bin| comparisons).
+constexpr uint64_t PROBE_BIN_LIMIT = 32;
+
+// Probe without a partition of the probe keys.
+constexpr uint32_t DIRECT_STATE_BYTES = 64;
+struct LaunchProbeDirect {
+  int key_bytes, off_bytes;
+  BinMap map;
+  const void *probe, *offA, *keysA;
+  uint32_t n;
+  void *out;
+  uint64_t capacity;
+  void *heavy;              // n keys: the probe keys whose bin is longer than PROBE_BIN_LIMIT
+  void *state;              // DIRECT_STATE_BYTES of device memory, zero before and after every launch
+  unsigned long long *res;  // pinned host memory: matches, keys listed in heavy
+};
+
 // The listed bins of a row-id join, compared pair by pair in tiles.
 struct LaunchJoinPairs {
   int key_bytes, off_bytes;
@@ -259,6 +278,7 @@ hipError_t set_direct_kernel_attributes();
 constexpr uint32_t BUILD_ONE_KEYS = 16384;
 bool build_one_takes(uint64_t n, uint64_t nbins, int key_bytes);
 hipError_t launch_build_one(const LaunchBuildOne &b, hipStream_t st);
+hipError_t launch_probe_direct(const LaunchProbeDirect &p, hipStream_t st);
 // maps[t].kind and each segment's map kind from use[] (learned when set)
 hipError_t launch_set_kinds(const uint32_t *use, SegDesc *segs, uint32_t nsegs, BinMap *maps, uint32_t nmaps,
                             hipStream_t st);

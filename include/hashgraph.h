@@ -131,8 +131,8 @@ hg_status hg_intersect(hg_ctx ctx, const hg_table_desc *descA, const void *d_off
 /* ---- probe: raw keys against a built table -------------------------------
  * Same result as building d_probe into a table B over A's bins and calling
  * hg_intersect(A, B) (same count, same multiset of emitted keys: each probe
- * key x is emitted cA(x) times), without materialising B's CSR.  Output order
- * is grouped by buckets of A's bins.  Any table hg_build accepts can be
+ * key x is emitted cA(x) times), without materialising B's CSR.  The output
+ * order is unspecified.  Any table hg_build accepts can be
  * probed (B is partitioned in two levels for tables beyond ~2^28 bins).    */
 hg_status hg_probe(hg_ctx ctx, const hg_table_desc *descA, const void *d_offA, const void *d_keysA,
                    const void *d_probe, uint64_t n_probe, void *d_out, uint64_t capacity, uint64_t *h_count);

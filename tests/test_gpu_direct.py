@@ -63,3 +63,53 @@ def test_one_workgroup_build_learned(dev):
     cb = hg.table_bins(csr, M, hash_kind=hg.HG_HASH_RMI, rmi_model=model).to(torch.int64)
     assert torch.equal(cb, torch.repeat_interleave(torch.arange(M, device=dev), deg))
     assert torch.equal(torch.sort(csr).values, torch.sort(dk).values)
+
+
+def _probe_equal(hg, off, csr, M, A, B, dev, ob=4):
+    dB = _to_dev(B, dev)
+    eo, ek = o.build_csr(A, M)
+    bo, bk = o.build_csr(B, M)
+    ecnt, elst = o.intersect(eo, ek, bo, bk)
+    assert hg.probe(off, csr, M, dB, emit=False)[0] == ecnt
+    cnt, out = hg.probe(off, csr, M, dB)
+    assert cnt == ecnt
+    assert np.array_equal(np.sort(out.cpu().numpy().view(A.dtype)), np.sort(elst))
+    return ecnt
+
+
+@pytest.mark.parametrize("kb,ob", [(4, 4), (8, 8)])
+@pytest.mark.parametrize("nB", [1, 255, 257, 65536, 65537, (1 << 18) + 1, (1 << 21) - 1])
+def test_direct_probe_sizes(nB, kb, ob, dev):
+    """Every workgroup size of the direct probe, with a remainder."""
+    import hashgraph_amd as hg
+    print(f"direct probe nB={nB} kb={kb} ob={ob}", flush=True)
+    A = wl.uniform_keys(5, 100003, kb)
+    M = 65537
+    off, csr = hg.build(_to_dev(A, dev), M, offset_bytes=ob)
+    _probe_equal(hg, off, csr, M, A, wl.probe_keys(A, 6, nB, 0.5, kb), dev, ob)
+
+
+@pytest.mark.parametrize("kb", [4, 8])
+def test_direct_probe_long_bins_short_output_and_overlap(kb, dev):
+    """Keys of long bins (answered by the partitioned probe) beside keys of
+    short ones; a buffer one match short; matches written over the probe keys."""
+    import torch
+    import hashgraph_amd as hg
+    A = wl.uniform_keys(11, 50000, kb)
+    A[:700] = A[0]
+    A[1000:1033] = A[1000]
+    M = 50000
+    B = wl.probe_keys(A, 12, 20000, 0.6, kb)
+    B[:40] = A[0]
+    B[50:60] = A[1000]
+    off, csr = hg.build(_to_dev(A, dev), M)
+    n = _probe_equal(hg, off, csr, M, A, B, dev)
+    dB = _to_dev(B, dev)
+    short = torch.zeros(n - 1, dtype=dB.dtype, device=dev)
+    with pytest.raises(hg.HGError):
+        hg.probe(off, csr, M, dB, out=short)
+    full = hg.probe(off, csr, M, dB)[1]
+    both = torch.zeros(n + len(B), dtype=dB.dtype, device=dev)
+    both[100:100 + len(B)] = dB
+    cnt, _ = hg.probe(off, csr, M, both[100:100 + len(B)], out=both)
+    assert cnt == n and torch.equal(torch.sort(both[:n]).values, torch.sort(full).values)
