@@ -109,6 +109,31 @@ def _check_dev(*ts):
             raise ValueError("tensors must be contiguous device tensors")
 
 
+def _emit(call, guess: int, alloc, cnt, where: str):
+    """Matches of a call whose caller named no capacity: one pass into buffers
+    of `guess` matches instead of a counting pass before it (at 10^8 joined
+    keys each pass takes about a millisecond).  More matches than that, or too
+    little memory for the guess, give buffers of the exact size and the pass
+    again.  call(bufs, capacity) -> status, alloc(n) -> list of n-match
+    buffers; returns the buffers, exactly cnt long."""
+    bufs = None
+    if guess:
+        try:
+            bufs = alloc(guess)
+        except _torch().OutOfMemoryError:
+            pass
+    st = call(bufs, guess if bufs else 0)
+    if st == _lib.HG_OK and bufs:
+        # the spare room goes back to the allocator
+        return bufs if cnt.value == guess else [b[: cnt.value].clone() for b in bufs]
+    if st != _lib.HG_OK and (st != _lib.HG_ERR_CAPACITY or not bufs):
+        check(st, where)
+    del bufs
+    bufs = alloc(max(cnt.value, 1))
+    check(call(bufs, cnt.value), where)
+    return [b[: cnt.value] for b in bufs]
+
+
 def build(keys, n_bins: int, offset_bytes: int = 4, hash_kind: int = HG_HASH_MURMUR3, rmi_model=None, out=None):
     """Build the CSR of `keys` over n_bins bins.  Returns (offsets, csr_keys):
     offsets int32/int64[n_bins+1], csr_keys like keys."""
@@ -142,9 +167,13 @@ def probe(offsets, csr_keys, n_bins: int, probe_keys, emit: bool = True, capacit
         return cnt.value, None
     if out is None:
         if capacity is None:
-            check(c.lib.hg_probe(c.bind_stream(), ctypes.byref(d), _p(offsets), _p(csr_keys), _p(probe_keys),
-                                 probe_keys.numel(), None, 0, ctypes.byref(cnt)), "hg_probe")
-            capacity = cnt.value
+            def call(bufs, cap):
+                return c.lib.hg_probe(c.bind_stream(), ctypes.byref(d), _p(offsets), _p(csr_keys), _p(probe_keys),
+                                      probe_keys.numel(), _p(bufs[0]) if bufs else None, cap, ctypes.byref(cnt))
+
+            m = _emit(call, probe_keys.numel(),
+                      lambda n: [torch.empty(n, dtype=csr_keys.dtype, device=csr_keys.device)], cnt, "hg_probe")
+            return cnt.value, m[0]
         out = torch.empty(max(capacity, 1), dtype=csr_keys.dtype, device=csr_keys.device)
     else:
         capacity = out.numel()
@@ -165,14 +194,17 @@ def intersect(offA, keysA, offB, keysB, n_bins: int, emit: bool = True, hash_kin
     dA = _desc(keysA.numel(), n_bins, kb, ob, hash_kind, rmi_model)
     dB = _desc(keysB.numel(), n_bins, kb, ob, hash_kind, rmi_model)
     cnt = ctypes.c_uint64(0)
-    check(c.lib.hg_intersect(c.bind_stream(), ctypes.byref(dA), _p(offA), _p(keysA), ctypes.byref(dB), _p(offB),
-                             _p(keysB), None, 0, ctypes.byref(cnt)), "hg_intersect")
+
+    def call(bufs, cap):
+        return c.lib.hg_intersect(c.bind_stream(), ctypes.byref(dA), _p(offA), _p(keysA), ctypes.byref(dB), _p(offB),
+                                  _p(keysB), _p(bufs[0]) if bufs else None, cap, ctypes.byref(cnt))
+
     if not emit:
+        check(call(None, 0), "hg_intersect")
         return cnt.value, None
-    out = torch.empty(max(cnt.value, 1), dtype=keysA.dtype, device=keysA.device)
-    check(c.lib.hg_intersect(c.bind_stream(), ctypes.byref(dA), _p(offA), _p(keysA), ctypes.byref(dB), _p(offB),
-                             _p(keysB), _p(out), cnt.value, ctypes.byref(cnt)), "hg_intersect")
-    return cnt.value, out[: cnt.value]
+    m = _emit(call, min(keysA.numel(), keysB.numel()),
+              lambda n: [torch.empty(n, dtype=keysA.dtype, device=keysA.device)], cnt, "hg_intersect")
+    return cnt.value, m[0]
 
 
 def intersect_rle(offA, keysA, offB, keysB, n_bins: int, hash_kind: int = HG_HASH_MURMUR3, rmi_model=None,
@@ -229,19 +261,25 @@ def intersect_indexed(offA, keysA, indA, offB, keysB, indB, n_bins: int, emit: b
     dA = _desc(keysA.numel(), n_bins, kb, ob)
     dB = _desc(keysB.numel(), n_bins, kb, ob)
     cnt = ctypes.c_uint64(0)
-    if capacity is None:
-        check(c.lib.hg_intersect_indexed(c.bind_stream(), ctypes.byref(dA), _p(offA), _p(keysA), _p(indA),
-                                         ctypes.byref(dB), _p(offB), _p(keysB), _p(indB), None, None, 0,
-                                         ctypes.byref(cnt)), "hg_intersect_indexed")
-        if not emit:
-            return cnt.value, None, None
-        capacity = cnt.value
-    pa = torch.empty(max(capacity, 1), dtype=torch.int64, device=keysA.device)
-    pb = torch.empty(max(capacity, 1), dtype=torch.int64, device=keysA.device)
-    check(c.lib.hg_intersect_indexed(c.bind_stream(), ctypes.byref(dA), _p(offA), _p(keysA), _p(indA),
-                                     ctypes.byref(dB), _p(offB), _p(keysB), _p(indB), _p(pa), _p(pb), capacity,
-                                     ctypes.byref(cnt)), "hg_intersect_indexed")
-    return cnt.value, pa[: cnt.value], pb[: cnt.value]
+
+    def call(bufs, cap):
+        pa, pb = bufs if bufs else (None, None)
+        return c.lib.hg_intersect_indexed(c.bind_stream(), ctypes.byref(dA), _p(offA), _p(keysA), _p(indA),
+                                          ctypes.byref(dB), _p(offB), _p(keysB), _p(indB), _p(pa), _p(pb), cap,
+                                          ctypes.byref(cnt))
+
+    def alloc(n):
+        return [torch.empty(n, dtype=torch.int64, device=keysA.device) for _ in range(2)]
+
+    if capacity is not None:
+        pa, pb = alloc(max(capacity, 1))
+        check(call((pa, pb), capacity), "hg_intersect_indexed")
+        return cnt.value, pa[: cnt.value], pb[: cnt.value]
+    if not emit:
+        check(call(None, 0), "hg_intersect_indexed")
+        return cnt.value, None, None
+    pa, pb = _emit(call, min(keysA.numel(), keysB.numel()), alloc, cnt, "hg_intersect_indexed")
+    return cnt.value, pa, pb
 
 
 def exclusive_scan(x):

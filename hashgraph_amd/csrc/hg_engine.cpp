@@ -900,7 +900,8 @@ bool probe_direct_takes(const hg_table_desc *A, const void *d_probe, uint64_t n_
   if (n_probe > std::max(kDirectProbe, A->n_keys / kDirectProbeShare) || A->n_keys > 8 * A->n_bins) return false;
   // matches are written while other workgroups still read the probe keys
   const uintptr_t o = (uintptr_t)d_out, q = (uintptr_t)d_probe;
-  return !d_out || o + capacity * A->key_bytes <= q || q + n_probe * A->key_bytes <= o;
+  const uint64_t room = std::min<uint64_t>(capacity, 1ull << 40) * A->key_bytes;
+  return !d_out || o + room <= q || q + n_probe * A->key_bytes <= o;
 }
 
 extern "C" {
@@ -1617,6 +1618,22 @@ hg_status hg_intersect_indexed(hg_ctx c, const hg_table_desc *descA, const void 
       return fail(HG_ERR_UNSUPPORTED, "bins with more than 4096 key pairs hold " + std::to_string(pairs) +
                                           " key pairs together; the row-id join compares them one by one and "
                                           "takes at most 2^36");
+    }
+    if (pairs > capacity) {
+      // the listed bins may not fit: their matches are counted first (value
+      // tables, far below the compares), so a short buffer is refused before
+      // every pair is compared for nothing
+      LaunchJoin h = j;
+      h.pa = h.pb = nullptr;
+      h.capacity = 0;
+      h.cursor = small + 3;
+      HG_HIP(launch_join_heavy(h, c->stream));
+      unsigned long long heavy = 0;
+      HG_TRY(sync_read(c, &heavy, small + 3, 8));
+      if (res[0] + heavy > capacity) {
+        *h_count = res[0] + heavy;
+        return fail(HG_ERR_CAPACITY, "output capacity smaller than the match count");
+      }
     }
     LaunchJoinPairs p{};
     p.key_bytes = j.key_bytes;

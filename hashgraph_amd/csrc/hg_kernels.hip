@@ -2970,6 +2970,16 @@ hipError_t launch_join_pairs_heavy(const LaunchJoinPairs &p, hipStream_t st) {
                           : launch_join_pairs_heavy_t<uint64_t, uint64_t>(p, st);
 }
 
+// The bins k_join listed (a grid that returns at once when there are none).
+template <typename K, typename OFF>
+static hipError_t launch_join_heavy_t(const LaunchJoin &j, hipStream_t st) {
+  const uint32_t gh = (uint32_t)std::min<uint64_t>(std::max<uint64_t>(j.hlist_cap, 1), 1024);
+  hipLaunchKernelGGL((k_join_heavy<K, OFF, 1024>), dim3(gh), dim3(1024), 0, st, (const OFF *)j.offA, (const K *)j.keysA,
+                     (const OFF *)j.offB, (const K *)j.keysB, (K *)j.out, j.capacity, j.cursor,
+                     (const uint32_t *)j.hlist, (const unsigned int *)j.hlist_n, j.hlist_cap);
+  return hipGetLastError();
+}
+
 template <typename K, typename OFF>
 static hipError_t launch_join_t(const LaunchJoin &j, hipStream_t st) {
   constexpr int JB = JOIN_BINS;
@@ -2982,12 +2992,7 @@ static hipError_t launch_join_t(const LaunchJoin &j, hipStream_t st) {
                      (const OFF *)j.offB, (const K *)j.keysB, j.M, (K *)j.out, j.capacity, j.cursor, j.key_cap, j.hlist,
                      j.hlist_n, j.hlist_cap, j.indA, j.indB, j.pa, j.pb);
   if (j.pa) return hipGetLastError();  // the row-id join answers its listed bins itself
-  // the heavy bins (a grid that returns at once when k_join listed none)
-  const uint32_t gh = (uint32_t)std::min<uint64_t>(std::max<uint64_t>(j.hlist_cap, 1), 1024);
-  hipLaunchKernelGGL((k_join_heavy<K, OFF, 1024>), dim3(gh), dim3(1024), 0, st, (const OFF *)j.offA, (const K *)j.keysA,
-                     (const OFF *)j.offB, (const K *)j.keysB, (K *)j.out, j.capacity, j.cursor,
-                     (const uint32_t *)j.hlist, (const unsigned int *)j.hlist_n, j.hlist_cap);
-  return hipGetLastError();
+  return launch_join_heavy_t<K, OFF>(j, st);
 }
 
 hipError_t launch_join(const LaunchJoin &j, hipStream_t st) {
@@ -2995,6 +3000,14 @@ hipError_t launch_join(const LaunchJoin &j, hipStream_t st) {
   if (j.key_bytes == 4)
     return j.off_bytes == 4 ? launch_join_t<uint32_t, uint32_t>(j, st) : launch_join_t<uint32_t, uint64_t>(j, st);
   return j.off_bytes == 4 ? launch_join_t<uint64_t, uint32_t>(j, st) : launch_join_t<uint64_t, uint64_t>(j, st);
+}
+
+hipError_t launch_join_heavy(const LaunchJoin &j, hipStream_t st) {
+  if (j.key_bytes == 4)
+    return j.off_bytes == 4 ? launch_join_heavy_t<uint32_t, uint32_t>(j, st)
+                            : launch_join_heavy_t<uint32_t, uint64_t>(j, st);
+  return j.off_bytes == 4 ? launch_join_heavy_t<uint64_t, uint32_t>(j, st)
+                          : launch_join_heavy_t<uint64_t, uint64_t>(j, st);
 }
 
 uint32_t join_key_cap(int key_bytes, int off_bytes, bool emit, bool with_index) {

@@ -307,6 +307,7 @@ hipError_t launch_colscan(const LaunchCol &lc, hipStream_t st);
 hipError_t launch_final(const LaunchFinal &lf, hipStream_t st);
 hipError_t launch_probe(const LaunchProbe &p, hipStream_t st);
 hipError_t launch_join(const LaunchJoin &j, hipStream_t st);
+hipError_t launch_join_heavy(const LaunchJoin &j, hipStream_t st);  // the listed bins of a launch_join alone
 // tiles (1024 x 1024 entries) and key pairs (summed, each capped at 2^37) of listed bins
 hipError_t launch_pair_tiles(const void *offA, const void *offB, int off_bytes, const uint32_t *hlist, uint32_t n,
                              unsigned long long *tiles, unsigned long long *pairs, hipStream_t st);

@@ -113,3 +113,28 @@ def test_direct_probe_long_bins_short_output_and_overlap(kb, dev):
     both[100:100 + len(B)] = dB
     cnt, _ = hg.probe(off, csr, M, both[100:100 + len(B)], out=both)
     assert cnt == n and torch.equal(torch.sort(both[:n]).values, torch.sort(full).values)
+
+
+@pytest.mark.parametrize("kb", [4, 8])
+def test_matches_beyond_the_first_buffers(kb, dev):
+    """Calls that name no capacity and match more often than either side has
+    keys: short bins, then one value in thousands of copies on both sides."""
+    import torch
+    import hashgraph_amd as hg
+    for reps, one in ((3, 0), (1, 3000)):
+        base = wl.uniform_keys(21, 4000, kb)
+        A = np.concatenate([np.repeat(base, reps), np.full(one, base[0], dtype=base.dtype)])
+        B = A[::-1].copy()
+        M = 5000
+        ta, tb = hg.build_indexed(_to_dev(A, dev), M), hg.build_indexed(_to_dev(B, dev), M)
+        eo, ek = o.build_csr(A, M)
+        bo, bk = o.build_csr(B, M)
+        ecnt, elst = o.intersect(eo, ek, bo, bk)
+        assert ecnt > len(A)
+        _probe_equal(hg, ta[0], ta[1], M, A, B, dev)
+        cnt, out = hg.intersect(ta[0], ta[1], tb[0], tb[1], M)
+        assert cnt == ecnt and np.array_equal(np.sort(out.cpu().numpy().view(A.dtype)), np.sort(elst))
+        cnt, pa, pb = hg.intersect_indexed(*ta, *tb, M)
+        assert cnt == ecnt == pa.numel() == pb.numel()
+        assert np.array_equal(A[pa.cpu().numpy()], B[pb.cpu().numpy()])
+        assert torch.unique((pa << 32) | pb).numel() == cnt
