@@ -77,7 +77,8 @@ Div32 make_div(uint32_t d) {
 uint32_t final_cap(int kb) { return std::min<uint32_t>(1024u * (uint32_t)final_kpt(kb), 65535u); }
 
 // Bucket fill of the build (HG_BUILD_FILL overrides it for tuning: above 1
-// buckets exceed the final stage's VGPR capacity and take k_final_big).
+// buckets exceed the final stage's VGPR capacity and take the oversized-bucket
+// kernels).
 double build_fill() {
   if (const char *e = getenv("HG_BUILD_FILL")) {
     const double v = atof(e);
@@ -538,7 +539,8 @@ SegDesc range_seg(uint64_t kbeg, uint64_t kend, uint64_t bin_lo, uint64_t nbins,
 // Final stage over the columns of a level.
 hg_status run_final(hg_ctx c, const Level &L, const LevelDev &d, int kb, int ob, const void *part, void *csr, void *off,
                     uint64_t *csr_index = nullptr) {
-  HG_HIP(launch_make_items(d.segs, (uint32_t)L.segs.size(), d.bstart, d.coltot, d.fin, L.ncols_total, c->stream));
+  HG_HIP(launch_make_items(d.segs, (uint32_t)L.segs.size(), d.bstart, d.coltot, d.fin, L.ncols_total, d.big_ctl,
+                           ProbeZero{}, c->stream));
   LaunchFinal f{};
   f.key_bytes = kb;
   f.off_bytes = ob;
@@ -1137,7 +1139,7 @@ hg_status hg_build_noalloc(hg_ctx c, const hg_table_desc *desc, const void *d_ke
   lc.bstart = d.bstart;
   HG_HIP(launch_colscan(lc, c->stream));
   HG_HIP(launch_part_scatter(p, c->stream));
-  HG_HIP(launch_make_items(d.segs, 1, d.bstart, d.coltot, d.fin, (uint32_t)F, c->stream));
+  HG_HIP(launch_make_items(d.segs, 1, d.bstart, d.coltot, d.fin, (uint32_t)F, d.big_ctl, ProbeZero{}, c->stream));
   LaunchFinal f{};
   f.key_bytes = kb;
   f.off_bytes = ob;
@@ -1464,10 +1466,13 @@ hg_status hg_probe(hg_ctx c, const hg_table_desc *descA, const void *d_offA, con
     HG_TRY(run_level(c, L, d, kb, part, part2));
     part = part2;
   }
-  HG_HIP(launch_fill_u64(small, 0ull, 4, c->stream));
-  if (done) HG_HIP(launch_fill_u64(small, done, 1, c->stream));
-  HG_HIP(launch_fill_u32(hmark, 0u, L.ncols_total, c->stream));
-  HG_HIP(launch_make_items(d.segs, (uint32_t)L.segs.size(), d.bstart, d.coltot, d.fin, L.ncols_total, c->stream));
+  ProbeZero z;
+  z.hmark = hmark;
+  z.gate = (unsigned int *)(small + 1);
+  z.cursor = small;
+  z.count = done;
+  HG_HIP(launch_make_items(d.segs, (uint32_t)L.segs.size(), d.bstart, d.coltot, d.fin, L.ncols_total, d.big_ctl, z,
+                           c->stream));
   LaunchProbe pr{};
   pr.key_bytes = kb;
   pr.off_bytes = ob;
@@ -1482,16 +1487,24 @@ hg_status hg_probe(hg_ctx c, const hg_table_desc *descA, const void *d_offA, con
   pr.out = d_out;
   pr.capacity = d_out ? capacity : 0;
   pr.cursor = small;
-  pr.gate = (unsigned int *)(small + 2);
+  pr.gate = z.gate;
   pr.hmark = hmark;
   pr.big_slot = d.big_slot;
   pr.big_ctl = d.big_ctl;
   {
     Prof pf(c, "probe");
-    HG_HIP(launch_probe(pr, c->stream));
+    HG_HIP(launch_probe_one(pr, c->stream));
   }
-  unsigned long long cnt = 0;
-  HG_TRY(sync_read(c, &cnt, small, 8));
+  unsigned long long res[2] = {0, 0};  // matches, both gates
+  HG_TRY(sync_read(c, res, small, 16));
+  if (res[1]) {  // items or bins left (skewed keys)
+    {
+      Prof pf(c, "probe");
+      HG_HIP(launch_probe_rest(pr, c->stream));
+    }
+    HG_TRY(sync_read(c, res, small, 8));
+  }
+  const unsigned long long cnt = res[0];
   *h_count = cnt;
   if (d_out && cnt > capacity) return fail(HG_ERR_CAPACITY, "output capacity smaller than the match count");
   return HG_OK;
@@ -2729,11 +2742,12 @@ hg_status batch_launch_probe(hg_ctx c, const hg_batch_desc *bd, BatchSide &S, co
                              const uint32_t *d_offsets, const void *d_csr, uint64_t *d_counts, void *d_out = nullptr,
                              const uint64_t *d_out_off = nullptr) {
   HG_HIP(launch_fill_u64((unsigned long long *)d_counts, 0ull, bd->n_tables, c->stream));
-  HG_HIP(launch_fill_u32(S.flag, 0u, 3, c->stream));  // [1], [2]: the probe gates
-  HG_HIP(launch_fill_u32(S.hmark, 0u, S.L.ncols_total, c->stream));
   HG_TRY(run_level(c, S.L, S.d, (int)bd->key_bytes, d_probe, S.part));
+  ProbeZero z;
+  z.hmark = S.hmark;
+  z.gate = S.flag + 1;
   HG_HIP(launch_make_items(S.d.segs, (uint32_t)S.L.segs.size(), S.d.bstart, S.d.coltot, S.d.fin, S.L.ncols_total,
-                           c->stream));
+                           S.d.big_ctl, z, c->stream));
   LaunchProbe pr{};
   pr.key_bytes = (int)bd->key_bytes;
   pr.off_bytes = 4;
@@ -2754,7 +2768,8 @@ hg_status batch_launch_probe(hg_ctx c, const hg_batch_desc *bd, BatchSide &S, co
   pr.big_slot = S.d.big_slot;
   pr.big_ctl = S.d.big_ctl;
   Prof pf(c, "probe");
-  HG_HIP(launch_probe(pr, c->stream));
+  HG_HIP(launch_probe_one(pr, c->stream));
+  HG_HIP(launch_probe_rest(pr, c->stream));
   return HG_OK;
 }
 

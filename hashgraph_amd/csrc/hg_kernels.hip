@@ -52,6 +52,9 @@ constexpr size_t PROBE_LDS = HG_PROBE_LDS;
 constexpr uint32_t BIG_CAP = 16384;
 constexpr uint32_t BIG_CHUNK = 65536;
 constexpr uint32_t BIG_BINS = 32768;
+constexpr uint32_t BIG_GRID = 512;  // workgroups of the oversized-bucket kernels
+constexpr uint32_t PROBE_BIG_CHUNK = 32768;  // keys of an oversized probe bucket per workgroup task
+constexpr uint32_t PROBE_BIG_GRID = 1024;
 constexpr int BIG_UB = 8;  // keys per thread whose loads the oversized-bucket kernels keep in flight
 
 // Workgroup b of a partition pass runs on XCD b % 8 (round-robin dispatch).
@@ -349,73 +352,88 @@ __global__ __launch_bounds__(BLOCK) void k_part_scatter(const K *__restrict__ ke
 
 
 // ---------------------------------------------------------------------------
+// Oversized buckets (skewed keys: a hot key's bin can hold 10^8 keys).  Up to
+// BIG_CAP of them are split into chunks and spread over the whole grid: the
+// workgroup that meets an oversized item lists it (big_register: slot and
+// chunks from one packed atomic, so chunk_start rises with the slot), then
+// per-chunk LDS bin counts are added into global per-bin counters, one
+// workgroup per bucket scans them into the offsets, and each chunk reserves
+// its places bin by bin (one global atomic per chunk and non-empty bin) and
+// writes its keys.  A wave whose keys all fall into one bin adds them with one
+// LDS atomic.  Bins are handled in passes of BIG_BINS.  Buckets that do not fit
+// the list are streamed by single workgroups after the listed ones.
+// ---------------------------------------------------------------------------
+struct BigCtl {
+  unsigned long long packed;  // listed slots << 40 | chunks
+  unsigned long long bins;    // per-bin counters asked for
+  uint32_t unlisted;          // some item did not fit
+  uint32_t item[BIG_CAP];
+  uint32_t chunk_start[BIG_CAP];
+  uint32_t bin_base[BIG_CAP];
+};
+
+__device__ void big_clear(BigCtl *ctl) {
+  ctl->packed = 0;
+  ctl->bins = 0;
+  ctl->unlisted = 0;
+}
+
+// One thread: lists item i (count keys, nbins per-bin counters from *bin0 on)
+// and returns its slot, ~0 when the list or the counters are full; big_slot[i]
+// keeps it.
+__device__ __forceinline__ uint32_t big_register(BigCtl *ctl, uint32_t *big_slot, uint32_t i, uint32_t count,
+                                                 uint32_t nbins, uint32_t big_cap, uint32_t chunk_keys,
+                                                 uint32_t *bin0) {
+  uint32_t slot = ~0u;
+  const unsigned long long b0 = atomicAdd(&ctl->bins, (unsigned long long)nbins);
+  if (b0 + nbins <= big_cap) {
+    const uint32_t nch = (count + chunk_keys - 1) / chunk_keys;
+    const unsigned long long p = atomicAdd(&ctl->packed, (1ull << 40) | nch);
+    if ((p >> 40) < BIG_CAP) {
+      slot = (uint32_t)(p >> 40);
+      ctl->item[slot] = i;
+      ctl->chunk_start[slot] = (uint32_t)p;
+      ctl->bin_base[slot] = (uint32_t)b0;
+      *bin0 = (uint32_t)b0;
+    }
+  }
+  if (slot == ~0u) ctl->unlisted = 1u;
+  big_slot[i] = slot;
+  return slot;
+}
+
+__device__ __forceinline__ uint32_t big_listed(const BigCtl *ctl) {
+  return (uint32_t)min(ctl->packed >> 40, (unsigned long long)BIG_CAP);
+}
+// chunks of the listed items
+__device__ __forceinline__ uint32_t big_chunks(const BigCtl *ctl, const FinItem *items, uint32_t chunk_keys) {
+  const uint32_t n = big_listed(ctl);
+  if (n == 0) return 0;
+  return ctl->chunk_start[n - 1] + (items[ctl->item[n - 1]].count + chunk_keys - 1) / chunk_keys;
+}
+
+// ---------------------------------------------------------------------------
 // Final stage: one workgroup per bucket (final_bucket).
 // ---------------------------------------------------------------------------
 template <typename K, typename OFF, int BLOCK, int KPT, int HK, bool SPLIT = false>
 __global__ __launch_bounds__(BLOCK) void k_final(const K *__restrict__ part, K *__restrict__ csr, OFF *__restrict__ off,
                                                  const FinItem *__restrict__ items, const BinMap *__restrict__ maps,
-                                                 uint32_t lds_bytes, unsigned int *__restrict__ big_seen,
-                                                 uint64_t *__restrict__ csr_index) {
+                                                 uint32_t lds_bytes, BigCtl *__restrict__ ctl,
+                                                 uint32_t *__restrict__ big_slot, uint32_t *__restrict__ big_cnt,
+                                                 uint32_t big_cap, uint64_t *__restrict__ csr_index) {
   extern __shared__ __align__(16) uint32_t smem32[];
   const FinItem it = items[blockIdx.x];
-  if (it.count > BLOCK * KPT || it.count > 65535u) {  // the oversized-bucket kernels' item: they run
-    if (threadIdx.x == 0) atomicOr(big_seen, 1u);
+  if (it.count > BLOCK * KPT || it.count > 65535u) {  // the oversized-bucket kernels' item: listed, its counters cleared
+    if (threadIdx.x == 0)
+      smem32[0] = big_register(ctl, big_slot, blockIdx.x, it.count, it.nbins, big_cap, BIG_CHUNK, &smem32[1]);
+    __syncthreads();
+    if (smem32[0] == ~0u) return;
+    uint32_t *c = big_cnt + smem32[1];
+    for (uint32_t i = threadIdx.x; i < it.nbins; i += BLOCK) c[i] = 0;
     return;
   }
   const BinMap mp = maps[it.table];
   final_bucket<K, OFF, BLOCK, KPT, HK, SPLIT>(part, csr, off, it, mp, smem32, lds_bytes, csr_index);
-}
-
-// ---------------------------------------------------------------------------
-// Final stage for buckets too large for k_final (skewed keys).  One
-// workgroup streams the bucket: per sub-range of SUB bins, count in LDS,
-// scan, write offsets, stream again placing keys with LDS atomics.
-// ---------------------------------------------------------------------------
-template <typename K, typename OFF, int BLOCK, int SUB, bool SPLIT = false>
-__global__ __launch_bounds__(BLOCK) void k_final_big(const K *__restrict__ part, K *__restrict__ csr, OFF *__restrict__ off,
-                                                     const FinItem *__restrict__ items, const BinMap *__restrict__ maps,
-                                                     uint32_t small_cap, const uint32_t *__restrict__ big_slot,
-                                                     const unsigned int *__restrict__ big_seen,
-                                                     uint64_t *__restrict__ csr_index) {
-  __shared__ uint32_t s_cnt[SUB];
-  __shared__ uint32_t s_tmp[BLOCK / 64 + 1];
-  if (*big_seen == 0) return;  // no oversized item
-  const FinItem it = items[blockIdx.x];
-  if (it.count <= small_cap) return;               // k_final's item
-  if (big_slot[blockIdx.x] != ~0u) return;         // the multi-workgroup path's item
-  const BinMap mp = maps[it.table];
-  const uint64_t cnt = it.count;
-  const K *kp = part + it.key_start;
-  K *dst = csr + it.key_start;
-  const uint64_t obase = it.key_start - it.key_rel;
-  uint64_t done = 0;
-  for (uint32_t s0 = 0; s0 < it.nbins; s0 += SUB) {
-    const uint32_t n = min((uint32_t)SUB, it.nbins - s0);
-    for (uint32_t i = threadIdx.x; i < n; i += BLOCK) s_cnt[i] = 0;
-    __syncthreads();
-    for (uint64_t i = threadIdx.x; i < cnt; i += BLOCK) {
-      const uint32_t l = bin_of<K>(kp[i], mp) - it.bin_lo - s0;
-      if (l < n) atomicAdd(&s_cnt[l], 1u);
-    }
-    __syncthreads();
-    const uint32_t tot = lds_exclusive_scan<BLOCK>(s_cnt, n, s_tmp);
-    for (uint32_t l = threadIdx.x; l < n; l += BLOCK) off[it.off_pos + s0 + l] = (OFF)(obase + done + s_cnt[l]);
-    __syncthreads();
-    for (uint64_t i = threadIdx.x; i < cnt; i += BLOCK) {
-      const K k = kp[i];
-      const uint32_t l = bin_of<K>(k, mp) - it.bin_lo - s0;
-      if (l < n) {
-        const uint64_t w = done + atomicAdd(&s_cnt[l], 1u);
-        if constexpr (SPLIT)
-          split_store((uint32_t *)csr + it.key_start, csr_index + it.key_start, w, k);
-        else
-          dst[w] = k;
-      }
-    }
-    __syncthreads();
-    done += tot;
-  }
-  if (it.end_pos != ~0ull && threadIdx.x == 0) off[it.end_pos] = (OFF)(obase + cnt);
 }
 
 // ---------------------------------------------------------------------------
@@ -456,7 +474,8 @@ __global__ __launch_bounds__(BLOCK) void k_probe1(const K *__restrict__ bpart, c
                                                   const K *__restrict__ keysA, K *__restrict__ out, uint64_t capacity,
                                                   unsigned long long *__restrict__ cursor, uint32_t lds_bytes,
                                                   unsigned int *__restrict__ hmark, unsigned int *__restrict__ gate,
-                                                  const uint64_t *__restrict__ out_off) {
+                                                  const uint64_t *__restrict__ out_off, uint32_t small_cap,
+                                                  BigCtl *__restrict__ ctl, uint32_t *__restrict__ big_slot) {
   extern __shared__ __align__(16) uint8_t smem[];
   __shared__ uint32_t s_tmp[BLOCK / 64 + 1];
   __shared__ unsigned long long s_base;
@@ -465,7 +484,10 @@ __global__ __launch_bounds__(BLOCK) void k_probe1(const K *__restrict__ bpart, c
   const OFF *ob = offA + it.off_pos;
   const uint64_t a_lo = (uint64_t)ob[0], a_hi = (uint64_t)ob[W];
   if (!probe1_takes(it.count, a_hi - a_lo, W, (uint32_t)sizeof(K), BLOCK * KPT, lds_bytes)) {
-    if (threadIdx.x == 0) atomicOr(&gate[0], 1u);  // k_probe's or k_probe_big's item: they run
+    if (threadIdx.x == 0) {  // k_probe's or (listed here) k_probe_big's item: they run
+      atomicOr(&gate[0], 1u);
+      if (it.count > small_cap) big_register(ctl, big_slot, blockIdx.x, it.count, 0, 0, PROBE_BIG_CHUNK, s_tmp);
+    }
     return;
   }
   const uint32_t na = (uint32_t)(a_hi - a_lo);
@@ -2109,10 +2131,19 @@ hipError_t launch_level_setup(const SegDesc &sd, const BinMap &map, uint32_t til
 // Work items of the final stage / probe from the partition pass results: one
 // item per column (bucket) of every segment.
 // ---------------------------------------------------------------------------
+// Also clears what the next kernels count into: the list of oversized buckets
+// and (probe) the marks of heavy items, the gates and the match cursor.
 __global__ void k_make_items(const SegDesc *__restrict__ segs, uint32_t nsegs, const uint32_t *__restrict__ bstart,
-                             const uint32_t *__restrict__ coltot, FinItem *__restrict__ items, uint32_t ncols_total) {
+                             const uint32_t *__restrict__ coltot, FinItem *__restrict__ items, uint32_t ncols_total,
+                             BigCtl *__restrict__ ctl, ProbeZero z) {
   const uint32_t g = blockIdx.x * blockDim.x + threadIdx.x;
+  if (g == 0) {
+    big_clear(ctl);
+    if (z.gate) z.gate[0] = z.gate[1] = 0;
+    if (z.cursor) *z.cursor = z.count;
+  }
   if (g >= ncols_total) return;
+  if (z.hmark) z.hmark[g] = 0;
   uint32_t lo = 0, hi = nsegs;  // last segment with bucket_base <= g
   while (hi - lo > 1) {
     const uint32_t mid = (lo + hi) >> 1;
@@ -2137,95 +2168,9 @@ __global__ void k_make_items(const SegDesc *__restrict__ segs, uint32_t nsegs, c
   items[g] = it;
 }
 
-// ---------------------------------------------------------------------------
-// Oversized buckets (skewed keys: a hot key's bin can hold 10^8 keys).  Up to
-// BIG_CAP of them are split into chunks of BIG_CHUNK keys and spread over the
-// whole grid: per-chunk LDS bin counts are added into global per-bin
-// counters, one workgroup per bucket scans them into the offsets, and each
-// chunk then reserves its places bin by bin (one global atomic per chunk and
-// non-empty bin) and writes its keys.  A wave whose keys all fall into one
-// bin adds them with one LDS atomic.  Bins are handled in passes of
-// BIG_BINS.  Buckets beyond BIG_CAP take k_final_big.
-// ---------------------------------------------------------------------------
-struct BigCtl {
-  uint32_t nbig, total_chunks, total_bins;
-  uint32_t seen;  // k_final left an oversized item (zeroed before k_final)
-  uint32_t item[BIG_CAP];
-  uint32_t chunk_start[BIG_CAP + 1];
-  uint32_t bin_base[BIG_CAP + 1];
-};
-
-// Takes the oversized items (count > small_cap) in order while their bins
-// fit big_cap counters (and at most BIG_CAP of them); prefix sums give chunk
-// (chunk_keys keys each) and bin bases.  *seen == 0: no oversized item.
-__global__ __launch_bounds__(1024) void k_big_list(const FinItem *__restrict__ items, uint32_t nitems, uint32_t small_cap,
-                                                   uint32_t big_cap, uint32_t chunk_keys, const unsigned int *seen,
-                                                   uint32_t *__restrict__ big_slot, BigCtl *__restrict__ ctl) {
-  __shared__ uint32_t s_tmp[1024 / 64 + 1];
-  __shared__ uint32_t s_slot, s_ch, s_bin, s_nacc, s_acc_ch, s_acc_bin;
-  if (*seen == 0) {  // no oversized item: empty lists (the big-item kernels read no big_slot)
-    if (threadIdx.x == 0) {
-      ctl->chunk_start[0] = 0;
-      ctl->bin_base[0] = 0;
-      ctl->nbig = 0;
-      ctl->total_chunks = 0;
-      ctl->total_bins = 0;
-    }
-    return;
-  }
-  if (threadIdx.x == 0) s_slot = s_ch = s_bin = s_nacc = s_acc_ch = s_acc_bin = 0;
-  __syncthreads();
-  for (uint32_t i0 = 0; i0 < nitems; i0 += 1024) {
-    const uint32_t i = i0 + threadIdx.x;
-    FinItem it{};
-    if (i < nitems) it = items[i];
-    const bool big = i < nitems && it.count > small_cap;
-    const uint32_t nch = big ? (uint32_t)((it.count + chunk_keys - 1) / chunk_keys) : 0u;
-    const uint32_t nbn = big ? it.nbins : 0u;
-    uint32_t t_slot, t_ch, t_bin;
-    const uint32_t e_slot = block_exclusive_sum<1024, uint32_t>(big ? 1u : 0u, s_tmp, t_slot);
-    const uint32_t e_ch = block_exclusive_sum<1024, uint32_t>(nch, s_tmp, t_ch);
-    const uint32_t e_bin = block_exclusive_sum<1024, uint32_t>(nbn, s_tmp, t_bin);
-    const uint32_t slot = s_slot + e_slot, cb = s_ch + e_ch, bb = s_bin + e_bin;
-    const bool acc = big && slot < BIG_CAP && (uint64_t)bb + nbn <= big_cap;
-    if (i < nitems) big_slot[i] = acc ? slot : ~0u;
-    if (acc) {
-      ctl->item[slot] = i;
-      ctl->chunk_start[slot] = cb;
-      ctl->bin_base[slot] = bb;
-    }
-    uint32_t a_tot, c_tot, b_tot;
-    (void)block_exclusive_sum<1024, uint32_t>(acc ? 1u : 0u, s_tmp, a_tot);
-    (void)block_exclusive_sum<1024, uint32_t>(acc ? nch : 0u, s_tmp, c_tot);
-    (void)block_exclusive_sum<1024, uint32_t>(acc ? nbn : 0u, s_tmp, b_tot);
-    if (threadIdx.x == 0) {
-      s_slot += t_slot;
-      s_ch += t_ch;
-      s_bin += t_bin;
-      s_nacc += a_tot;
-      s_acc_ch += c_tot;
-      s_acc_bin += b_tot;
-    }
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) {
-    const uint32_t nbig = s_nacc;
-    ctl->chunk_start[nbig] = s_acc_ch;
-    ctl->bin_base[nbig] = s_acc_bin;
-    ctl->nbig = nbig;
-    ctl->total_chunks = s_acc_ch;
-    ctl->total_bins = s_acc_bin;
-  }
-}
-
-__global__ __launch_bounds__(256) void k_big_zero(const BigCtl *__restrict__ ctl, uint32_t *__restrict__ gcnt) {
-  const uint32_t n = ctl->total_bins;
-  for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) gcnt[i] = 0;
-}
-
 // slot of chunk g: last s with chunk_start[s] <= g
 __device__ __forceinline__ uint32_t big_slot_of(const BigCtl *ctl, uint32_t g) {
-  uint32_t lo = 0, hi = ctl->nbig;
+  uint32_t lo = 0, hi = big_listed(ctl);
   while (hi - lo > 1) {
     const uint32_t mid = (lo + hi) >> 1;
     if (ctl->chunk_start[mid] <= g) lo = mid;
@@ -2262,7 +2207,7 @@ __global__ __launch_bounds__(BLOCK) void k_big_count(const K *__restrict__ part,
                                                      const BinMap *__restrict__ maps, const BigCtl *__restrict__ ctl,
                                                      uint32_t *__restrict__ gcnt) {
   __shared__ uint32_t s_cnt[BIG_BINS];
-  const uint32_t total = ctl->total_chunks;
+  const uint32_t total = big_chunks(ctl, items, BIG_CHUNK);
   for (uint32_t g = blockIdx.x; g < total; g += gridDim.x) {
     const uint32_t slot = big_slot_of(ctl, g);
     const FinItem it = items[ctl->item[slot]];
@@ -2304,7 +2249,8 @@ template <typename OFF>
 __global__ __launch_bounds__(1024) void k_big_scan(const FinItem *__restrict__ items, const BigCtl *__restrict__ ctl,
                                                    uint32_t *__restrict__ gcnt, OFF *__restrict__ off) {
   __shared__ uint32_t s_tmp[1024 / 64 + 1];
-  for (uint32_t slot = blockIdx.x; slot < ctl->nbig; slot += gridDim.x) {
+  const uint32_t nbig = big_listed(ctl);
+  for (uint32_t slot = blockIdx.x; slot < nbig; slot += gridDim.x) {
     const FinItem it = items[ctl->item[slot]];
     uint32_t *g = gcnt + ctl->bin_base[slot];
     const uint64_t obase = it.key_start - it.key_rel;
@@ -2325,13 +2271,56 @@ __global__ __launch_bounds__(1024) void k_big_scan(const FinItem *__restrict__ i
   }
 }
 
-template <typename K, int BLOCK, bool SPLIT = false>
-__global__ __launch_bounds__(BLOCK) void k_big_place(const K *__restrict__ part, K *__restrict__ csr,
-                                                     const FinItem *__restrict__ items, const BinMap *__restrict__ maps,
-                                                     const BigCtl *__restrict__ ctl, uint32_t *__restrict__ gcur,
-                                                     uint64_t *__restrict__ csr_index) {
+// ---------------------------------------------------------------------------
+// Final stage of an oversized bucket that is not listed.  One workgroup
+// streams the bucket: per sub-range of SUB bins, count in LDS, scan, write
+// offsets, stream again placing keys with LDS atomics.
+// ---------------------------------------------------------------------------
+template <typename K, typename OFF, int BLOCK, int SUB, bool SPLIT = false>
+__device__ void final_big(const K *__restrict__ part, K *__restrict__ csr, OFF *__restrict__ off, const FinItem &it,
+                          const BinMap &mp, uint32_t *s_cnt, uint32_t *s_tmp, uint64_t *__restrict__ csr_index) {
+  const uint64_t cnt = it.count;
+  const K *kp = part + it.key_start;
+  K *dst = csr + it.key_start;
+  const uint64_t obase = it.key_start - it.key_rel;
+  uint64_t done = 0;
+  for (uint32_t s0 = 0; s0 < it.nbins; s0 += SUB) {
+    const uint32_t n = min((uint32_t)SUB, it.nbins - s0);
+    for (uint32_t i = threadIdx.x; i < n; i += BLOCK) s_cnt[i] = 0;
+    __syncthreads();
+    for (uint64_t i = threadIdx.x; i < cnt; i += BLOCK) {
+      const uint32_t l = bin_of<K>(kp[i], mp) - it.bin_lo - s0;
+      if (l < n) atomicAdd(&s_cnt[l], 1u);
+    }
+    __syncthreads();
+    const uint32_t tot = lds_exclusive_scan<BLOCK>(s_cnt, n, s_tmp);
+    for (uint32_t l = threadIdx.x; l < n; l += BLOCK) off[it.off_pos + s0 + l] = (OFF)(obase + done + s_cnt[l]);
+    __syncthreads();
+    for (uint64_t i = threadIdx.x; i < cnt; i += BLOCK) {
+      const K k = kp[i];
+      const uint32_t l = bin_of<K>(k, mp) - it.bin_lo - s0;
+      if (l < n) {
+        const uint64_t w = done + atomicAdd(&s_cnt[l], 1u);
+        if constexpr (SPLIT)
+          split_store((uint32_t *)csr + it.key_start, csr_index + it.key_start, w, k);
+        else
+          dst[w] = k;
+      }
+    }
+    __syncthreads();
+    done += tot;
+  }
+  if (it.end_pos != ~0ull && threadIdx.x == 0) off[it.end_pos] = (OFF)(obase + cnt);
+}
+
+template <typename K, typename OFF, int BLOCK, bool SPLIT = false>
+__global__ __launch_bounds__(BLOCK) void k_big_place(const K *__restrict__ part, K *__restrict__ csr, OFF *__restrict__ off,
+                                                     const FinItem *__restrict__ items, uint32_t nitems,
+                                                     uint32_t small_cap, const BinMap *__restrict__ maps,
+                                                     const BigCtl *__restrict__ ctl, const uint32_t *__restrict__ big_slot,
+                                                     uint32_t *__restrict__ gcur, uint64_t *__restrict__ csr_index) {
   __shared__ uint32_t s_cnt[BIG_BINS];
-  const uint32_t total = ctl->total_chunks;
+  const uint32_t total = big_chunks(ctl, items, BIG_CHUNK);
   for (uint32_t g = blockIdx.x; g < total; g += gridDim.x) {
     const uint32_t slot = big_slot_of(ctl, g);
     const FinItem it = items[ctl->item[slot]];
@@ -2405,13 +2394,20 @@ __global__ __launch_bounds__(BLOCK) void k_big_place(const K *__restrict__ part,
       __syncthreads();
     }
   }
+  // items that did not fit the list: one workgroup each
+  if (ctl->unlisted == 0) return;
+  __shared__ uint32_t s_tmp[BLOCK / 64 + 1];
+  for (uint32_t i = blockIdx.x; i < nitems; i += gridDim.x) {
+    const FinItem it = items[i];
+    if (it.count <= small_cap || big_slot[i] != ~0u) continue;
+    final_big<K, OFF, BLOCK, 16384, SPLIT>(part, csr, off, it, maps[it.table], s_cnt, s_tmp, csr_index);
+    __syncthreads();
+  }
 }
 
 // Probe of buckets too large for k_probe: B's keys of the bucket are
 // streamed and each walks its bin of A in global memory.  probe_big_range
 // handles keys [k0, k1) of item `ii` (a workgroup-uniform range).
-constexpr uint32_t PROBE_BIG_CHUNK = 32768;  // keys of an oversized bucket per workgroup task
-constexpr uint32_t PROBE_BIG_GRID = 1024;
 template <typename K, typename OFF, int BLOCK>
 __device__ void probe_big_range(const K *__restrict__ bpart, const FinItem &it, uint32_t ii, const BinMap &mp,
                                 const OFF *__restrict__ offA, const K *__restrict__ keysA, K *__restrict__ out,
@@ -2496,43 +2492,23 @@ __device__ void probe_big_range(const K *__restrict__ bpart, const FinItem &it, 
   }
 }
 
-// Oversized buckets that k_big_list did not list (big_slot ~0: beyond
-// BIG_CAP of them): one workgroup per bucket.
-template <typename K, typename OFF, int BLOCK>
-__global__ __launch_bounds__(BLOCK) void k_probe_big(const K *__restrict__ bpart, const FinItem *__restrict__ items,
-                                                     const BinMap *__restrict__ maps, const OFF *__restrict__ offA,
-                                                     const K *__restrict__ keysA, K *__restrict__ out, uint64_t capacity,
-                                                     unsigned long long *__restrict__ cursor, uint32_t small_cap,
-                                                     const uint32_t *__restrict__ big_slot,
-                                                     unsigned int *__restrict__ hmark,
-                                                     unsigned int *__restrict__ gate,
-                                                     const uint64_t *__restrict__ out_off) {
-  __shared__ unsigned long long s_t64[BLOCK / 64 + 1];
-  __shared__ unsigned long long s_base;
-  if (gate[0] == 0) return;  // k_probe1 took every item
-  const FinItem it = items[blockIdx.x];
-  if (it.count <= small_cap || big_slot[blockIdx.x] != ~0u) return;
-  const BinMap mp = maps[it.table];
-  probe_big_range<K, OFF, BLOCK>(bpart, it, blockIdx.x, mp, offA, keysA, out, capacity, cursor, hmark, gate, 0,
-                                 it.count, s_t64, &s_base, out_off);
-}
-
 // The listed oversized buckets, cut into tasks of PROBE_BIG_CHUNK keys that
 // the grid shares (a bucket of a hot or out-of-distribution range of B keys
-// no longer runs on one workgroup).
+// no longer runs on one workgroup), then the unlisted ones, one workgroup each.
 template <typename K, typename OFF, int BLOCK>
-__global__ __launch_bounds__(BLOCK) void k_probe_big_chunks(const K *__restrict__ bpart, const FinItem *__restrict__ items,
+__global__ __launch_bounds__(BLOCK) void k_probe_big(const K *__restrict__ bpart, const FinItem *__restrict__ items,
                                                             const BinMap *__restrict__ maps, const OFF *__restrict__ offA,
                                                             const K *__restrict__ keysA, K *__restrict__ out,
                                                             uint64_t capacity, unsigned long long *__restrict__ cursor,
                                                             const BigCtl *__restrict__ ctl,
-                                                            unsigned int *__restrict__ hmark,
+                                                            const uint32_t *__restrict__ big_slot, uint32_t nitems,
+                                                            uint32_t small_cap, unsigned int *__restrict__ hmark,
                                                             unsigned int *__restrict__ gate,
                                                             const uint64_t *__restrict__ out_off) {
   __shared__ unsigned long long s_t64[BLOCK / 64 + 1];
   __shared__ unsigned long long s_base;
-  if (gate[0] == 0) return;  // k_probe1 took every item (the list was not written)
-  const uint32_t total = ctl->total_chunks;
+  if (gate[0] == 0) return;  // k_probe1 took every item
+  const uint32_t total = big_chunks(ctl, items, PROBE_BIG_CHUNK);
   for (uint32_t g = blockIdx.x; g < total; g += gridDim.x) {
     const uint32_t slot = big_slot_of(ctl, g);
     const uint32_t ii = ctl->item[slot];
@@ -2542,6 +2518,13 @@ __global__ __launch_bounds__(BLOCK) void k_probe_big_chunks(const K *__restrict_
     const uint64_t k1 = min((uint64_t)it.count, k0 + PROBE_BIG_CHUNK);
     probe_big_range<K, OFF, BLOCK>(bpart, it, ii, mp, offA, keysA, out, capacity, cursor, hmark, gate, k0, k1, s_t64,
                                    &s_base, out_off);
+  }
+  if (ctl->unlisted == 0) return;
+  for (uint32_t i = blockIdx.x; i < nitems; i += gridDim.x) {
+    const FinItem it = items[i];
+    if (it.count <= small_cap || big_slot[i] != ~0u) continue;
+    probe_big_range<K, OFF, BLOCK>(bpart, it, i, maps[it.table], offA, keysA, out, capacity, cursor, hmark, gate, 0,
+                                   it.count, s_t64, &s_base, out_off);
   }
 }
 
@@ -2761,37 +2744,31 @@ hipError_t launch_colscan(const LaunchCol &lc, hipStream_t st) {
 
 template <typename K, typename OFF, bool SPLIT>
 static hipError_t launch_final_t(const LaunchFinal &lf, hipStream_t st) {
-  if (lf.nitems) hipLaunchKernelGGL(k_fill<uint32_t>, dim3(1), dim3(64), 0, st, &((BigCtl *)lf.big_ctl)->seen, 0u, (uint64_t)1);
-  if (lf.nitems) {
-    constexpr int KPT = sizeof(K) == 4 ? KPT_U32 : 32;
-    const hipError_t e = dispatch_hk(lf.hk, [&](auto h) {
-      constexpr int H = decltype(h)::value;
-      // the split store exists for murmur3 tables only (launch_final checks)
-      auto kern = &k_final<K, OFF, 1024, KPT, H>;
-      if constexpr (SPLIT && H == HK_MURMUR) kern = &k_final<K, OFF, 1024, KPT, H, true>;
-      hipLaunchKernelGGL(kern, dim3(lf.nitems), dim3(1024), lf.lds_bytes, st, (const K *)lf.part, (K *)lf.csr,
-                         (OFF *)lf.off, lf.items, lf.maps, lf.lds_bytes, &((BigCtl *)lf.big_ctl)->seen, lf.csr_index);
-      return hipGetLastError();
-    });
-    if (e != hipSuccess) return e;
-  }
-  if (lf.nitems) {
-    constexpr int KPT = sizeof(K) == 4 ? KPT_U32 : 32;
-    const uint32_t small_cap = std::min(1024u * KPT, 65535u);
-    BigCtl *ctl = (BigCtl *)lf.big_ctl;
-    hipLaunchKernelGGL(k_big_list, dim3(1), dim3(1024), 0, st, lf.items, lf.nitems, small_cap, lf.big_cap, BIG_CHUNK,
-                       (const unsigned int *)&ctl->seen, lf.big_slot, ctl);
-    hipLaunchKernelGGL(k_big_zero, dim3(256), dim3(256), 0, st, (const BigCtl *)ctl, lf.big_cnt);
-    hipLaunchKernelGGL((k_big_count<K, 1024>), dim3(2048), dim3(1024), 0, st, (const K *)lf.part, lf.items, lf.maps,
-                       (const BigCtl *)ctl, lf.big_cnt);
-    hipLaunchKernelGGL((k_big_scan<OFF>), dim3(256), dim3(1024), 0, st, lf.items, (const BigCtl *)ctl, lf.big_cnt,
-                       (OFF *)lf.off);
-    hipLaunchKernelGGL((k_big_place<K, 1024, SPLIT>), dim3(2048), dim3(1024), 0, st, (const K *)lf.part, (K *)lf.csr,
-                       lf.items, lf.maps, (const BigCtl *)ctl, lf.big_cnt, lf.csr_index);
-    hipLaunchKernelGGL((k_final_big<K, OFF, 1024, 16384, SPLIT>), dim3(lf.nitems), dim3(1024), 0, st, (const K *)lf.part,
-                       (K *)lf.csr, (OFF *)lf.off, lf.items, lf.maps, small_cap, (const uint32_t *)lf.big_slot,
-                       (const unsigned int *)&ctl->seen, lf.csr_index);
-  }
+  if (!lf.nitems) return hipSuccess;
+  constexpr int KPT = sizeof(K) == 4 ? KPT_U32 : 32;
+  BigCtl *ctl = (BigCtl *)lf.big_ctl;
+  const hipError_t e = dispatch_hk(lf.hk, [&](auto h) {
+    constexpr int H = decltype(h)::value;
+    // the split store exists for murmur3 tables only (launch_final checks)
+    auto kern = &k_final<K, OFF, 1024, KPT, H>;
+    if constexpr (SPLIT && H == HK_MURMUR) kern = &k_final<K, OFF, 1024, KPT, H, true>;
+    hipLaunchKernelGGL(kern, dim3(lf.nitems), dim3(1024), lf.lds_bytes, st, (const K *)lf.part, (K *)lf.csr,
+                       (OFF *)lf.off, lf.items, lf.maps, lf.lds_bytes, ctl, lf.big_slot, lf.big_cnt, lf.big_cap,
+                       lf.csr_index);
+    return hipGetLastError();
+  });
+  if (e != hipSuccess) return e;
+  // three kernels that return at once when no item was oversized: two
+  // workgroups per CU (their 128 KB of LDS admit one at a time) dispatch in
+  // under 2 us, the 2048 they had took 4.5 us
+  const uint32_t small_cap = std::min(1024u * KPT, 65535u);
+  hipLaunchKernelGGL((k_big_count<K, 1024>), dim3(BIG_GRID), dim3(1024), 0, st, (const K *)lf.part, lf.items, lf.maps,
+                     (const BigCtl *)ctl, lf.big_cnt);
+  hipLaunchKernelGGL((k_big_scan<OFF>), dim3(256), dim3(1024), 0, st, lf.items, (const BigCtl *)ctl, lf.big_cnt,
+                     (OFF *)lf.off);
+  hipLaunchKernelGGL((k_big_place<K, OFF, 1024, SPLIT>), dim3(BIG_GRID), dim3(1024), 0, st, (const K *)lf.part,
+                     (K *)lf.csr, (OFF *)lf.off, lf.items, lf.nitems, small_cap, lf.maps, (const BigCtl *)ctl,
+                     (const uint32_t *)lf.big_slot, lf.big_cnt, lf.csr_index);
   return hipGetLastError();
 }
 
@@ -2809,7 +2786,6 @@ hipError_t launch_final(const LaunchFinal &lf, hipStream_t st) {
 }
 
 int final_kpt(int key_bytes) { return key_bytes == 4 ? KPT_U32 : 32; }
-uint32_t final_big_items() { return BIG_CAP; }
 size_t final_big_ctl_bytes() { return sizeof(BigCtl); }
 
 // One-pass probe's bucket limits: keys of B per workgroup, keys of A in LDS.
@@ -2817,46 +2793,56 @@ template <typename K> constexpr int probe1_kpt() { return sizeof(K) == 4 ? 32 : 
 constexpr uint32_t PROBE1_LDS = 156 * 1024;  // keys of A + 16-bit offsets
 
 template <typename K, typename OFF>
-static hipError_t launch_probe_t(const LaunchProbe &p, hipStream_t st) {
+static hipError_t launch_probe_one_t(const LaunchProbe &p, hipStream_t st) {
   constexpr int KPT = sizeof(K) == 4 ? KPT_U32 : 32;
-  constexpr int KPT1 = probe1_kpt<K>();
+  return dispatch_hk(p.hk, [&](auto h) {
+    hipLaunchKernelGGL((k_probe1<K, OFF, 1024, probe1_kpt<K>(), decltype(h)::value>), dim3(p.nitems), dim3(1024),
+                       (size_t)PROBE1_LDS, st, (const K *)p.bpart, p.items, p.maps, (const OFF *)p.offA,
+                       (const K *)p.keysA, (K *)p.out, p.capacity, p.cursor, PROBE1_LDS, p.hmark, p.gate, p.out_off,
+                       std::min(1024u * KPT, 65535u), (BigCtl *)p.big_ctl, p.big_slot);
+    return hipGetLastError();
+  });
+}
+
+template <typename K, typename OFF>
+static hipError_t launch_probe_rest_t(const LaunchProbe &p, hipStream_t st) {
+  constexpr int KPT = sizeof(K) == 4 ? KPT_U32 : 32;
   constexpr int SUB = probe_sub<OFF>();
   if (p.akey_cap < PROBE_BIN_LIMIT) return hipErrorInvalidValue;  // a walkable bin must fit in LDS
   const size_t lds = ((SUB + 2) * sizeof(OFF) + 15) / 16 * 16 + (size_t)p.akey_cap * sizeof(K);
   const hipError_t e = dispatch_hk(p.hk, [&](auto h) {
-    hipLaunchKernelGGL((k_probe1<K, OFF, 1024, KPT1, decltype(h)::value>), dim3(p.nitems), dim3(1024),
-                       (size_t)PROBE1_LDS, st, (const K *)p.bpart, p.items, p.maps, (const OFF *)p.offA,
-                       (const K *)p.keysA, (K *)p.out, p.capacity, p.cursor, PROBE1_LDS, p.hmark, p.gate, p.out_off);
     hipLaunchKernelGGL((k_probe<K, OFF, 1024, KPT, SUB, decltype(h)::value>), dim3(p.nitems), dim3(1024), lds, st,
                        (const K *)p.bpart, p.items, p.maps, (const OFF *)p.offA, (const K *)p.keysA, (K *)p.out,
-                       p.capacity, p.cursor, p.akey_cap, p.hmark, (uint32_t)(1024 * KPT1), PROBE1_LDS, p.gate,
-                       p.out_off);
+                       p.capacity, p.cursor, p.akey_cap, p.hmark, (uint32_t)(1024 * probe1_kpt<K>()), PROBE1_LDS,
+                       p.gate, p.out_off);
     return hipGetLastError();
   });
   if (e != hipSuccess) return e;
-  const uint32_t small_cap = std::min(1024u * KPT, 65535u);
-  // oversized buckets: up to BIG_CAP of them listed and cut into tasks of
-  // PROBE_BIG_CHUNK keys for the whole grid, the rest one workgroup each
-  BigCtl *ctl = (BigCtl *)p.big_ctl;
-  hipLaunchKernelGGL(k_big_list, dim3(1), dim3(1024), 0, st, p.items, p.nitems, small_cap, 0xFFFFFFFFu, PROBE_BIG_CHUNK,
-                     (const unsigned int *)p.gate, p.big_slot, ctl);
-  hipLaunchKernelGGL((k_probe_big<K, OFF, 1024>), dim3(p.nitems), dim3(1024), 0, st, (const K *)p.bpart, p.items, p.maps,
-                     (const OFF *)p.offA, (const K *)p.keysA, (K *)p.out, p.capacity, p.cursor, small_cap,
-                     (const uint32_t *)p.big_slot, p.hmark, p.gate, p.out_off);
-  hipLaunchKernelGGL((k_probe_big_chunks<K, OFF, 1024>), dim3(PROBE_BIG_GRID), dim3(1024), 0, st, (const K *)p.bpart,
+  hipLaunchKernelGGL((k_probe_big<K, OFF, 1024>), dim3(PROBE_BIG_GRID), dim3(1024), 0, st, (const K *)p.bpart,
                      p.items, p.maps, (const OFF *)p.offA, (const K *)p.keysA, (K *)p.out, p.capacity, p.cursor,
-                     (const BigCtl *)ctl, p.hmark, p.gate, p.out_off);
+                     (const BigCtl *)p.big_ctl, (const uint32_t *)p.big_slot, p.nitems, std::min(1024u * KPT, 65535u),
+                     p.hmark, p.gate, p.out_off);
   hipLaunchKernelGGL((k_probe_heavy<K, OFF, 1024>), dim3(p.nitems), dim3(1024), 0, st, (const K *)p.bpart, p.items,
                      (const OFF *)p.offA, (const K *)p.keysA, (K *)p.out, p.capacity, p.cursor,
                      (const unsigned int *)p.hmark, (const unsigned int *)p.gate, p.out_off);
   return hipGetLastError();
 }
 
-hipError_t launch_probe(const LaunchProbe &p, hipStream_t st) {
+hipError_t launch_probe_one(const LaunchProbe &p, hipStream_t st) {
   if (!p.nitems) return hipSuccess;
   if (p.key_bytes == 4)
-    return p.off_bytes == 4 ? launch_probe_t<uint32_t, uint32_t>(p, st) : launch_probe_t<uint32_t, uint64_t>(p, st);
-  return p.off_bytes == 4 ? launch_probe_t<uint64_t, uint32_t>(p, st) : launch_probe_t<uint64_t, uint64_t>(p, st);
+    return p.off_bytes == 4 ? launch_probe_one_t<uint32_t, uint32_t>(p, st)
+                            : launch_probe_one_t<uint32_t, uint64_t>(p, st);
+  return p.off_bytes == 4 ? launch_probe_one_t<uint64_t, uint32_t>(p, st)
+                          : launch_probe_one_t<uint64_t, uint64_t>(p, st);
+}
+hipError_t launch_probe_rest(const LaunchProbe &p, hipStream_t st) {
+  if (!p.nitems) return hipSuccess;
+  if (p.key_bytes == 4)
+    return p.off_bytes == 4 ? launch_probe_rest_t<uint32_t, uint32_t>(p, st)
+                            : launch_probe_rest_t<uint32_t, uint64_t>(p, st);
+  return p.off_bytes == 4 ? launch_probe_rest_t<uint64_t, uint32_t>(p, st)
+                          : launch_probe_rest_t<uint64_t, uint64_t>(p, st);
 }
 
 uint32_t probe_akey_cap(int key_bytes, int off_bytes) {
@@ -3215,10 +3201,10 @@ size_t rle_giant_bytes(int key_bytes) { return sizeof(GiantCtl) + rle_giant_slot
 uint64_t rle_chunks(uint64_t M) { return (M + RLE_CHUNK - 1) / RLE_CHUNK; }
 
 hipError_t launch_make_items(const SegDesc *segs, uint32_t nsegs, const uint32_t *bstart, const uint32_t *coltot,
-                             FinItem *items, uint32_t ncols_total, hipStream_t st) {
+                             FinItem *items, uint32_t ncols_total, void *big_ctl, const ProbeZero &z, hipStream_t st) {
   if (!ncols_total) return hipSuccess;
   hipLaunchKernelGGL(k_make_items, dim3((ncols_total + 255) / 256), dim3(256), 0, st, segs, nsegs, bstart, coltot, items,
-                     ncols_total);
+                     ncols_total, (BigCtl *)big_ctl, z);
   return hipGetLastError();
 }
 

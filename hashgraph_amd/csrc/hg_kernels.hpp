@@ -79,8 +79,8 @@ struct LaunchProbe {
   unsigned long long *cursor;  // match counters, one per table (FinItem.table)
   unsigned int *hmark;         // nitems, zeroed: items with a bin beyond the walk limit
   unsigned int *gate;          // 2 zeroed words: [0] k_probe1 left items, [1] a bin was marked heavy
-  uint32_t *big_slot;          // nitems words and a final_big_ctl_bytes() area: the list of the
-  void *big_ctl;               // oversized buckets (written by the probe itself)
+  uint32_t *big_slot;          // nitems words and a final_big_ctl_bytes() area (cleared by
+  void *big_ctl;               // launch_make_items): the list of the oversized buckets
   const uint64_t *out_off;     // null: out[0 .. capacity) for every table; else table t's
                                // matches go to out[out_off[t] .. out_off[t+1]) (device array)
 };
@@ -305,7 +305,10 @@ hipError_t launch_part_hist(const LaunchPart &lp, hipStream_t st);
 hipError_t launch_part_scatter(const LaunchPart &lp, hipStream_t st);
 hipError_t launch_colscan(const LaunchCol &lc, hipStream_t st);
 hipError_t launch_final(const LaunchFinal &lf, hipStream_t st);
-hipError_t launch_probe(const LaunchProbe &p, hipStream_t st);
+// The one-pass kernel, then the kernels of the items and bins it left: they
+// need not run when both gates are still 0 (and return at once if they do).
+hipError_t launch_probe_one(const LaunchProbe &p, hipStream_t st);
+hipError_t launch_probe_rest(const LaunchProbe &p, hipStream_t st);
 hipError_t launch_join(const LaunchJoin &j, hipStream_t st);
 hipError_t launch_join_heavy(const LaunchJoin &j, hipStream_t st);  // the listed bins of a launch_join alone
 // tiles (1024 x 1024 entries) and key pairs (summed, each capped at 2^37) of listed bins
@@ -333,11 +336,18 @@ hipError_t launch_gen_uniform(void *out, uint64_t n, int key_bytes, uint64_t s0,
 hipError_t launch_level_setup(const SegDesc &sd, const BinMap &map, uint32_t tile_keys, uint32_t chunk, TileDesc *tiles,
                               SegDesc *segs, ColItem *items, ColItem *items2, uint64_t *psum_base, uint32_t *nchunks,
                               BinMap *maps, hipStream_t st);
+// and the state of what runs on the items cleared: the list of oversized
+// buckets (big_ctl) and z's words (null members: not there)
+struct ProbeZero {
+  unsigned int *hmark = nullptr;         // one per item
+  unsigned int *gate = nullptr;          // two words
+  unsigned long long *cursor = nullptr;  // set to count
+  unsigned long long count = 0;
+};
 hipError_t launch_make_items(const SegDesc *segs, uint32_t nsegs, const uint32_t *bstart, const uint32_t *coltot,
-                             FinItem *items, uint32_t ncols_total, hipStream_t st);
+                             FinItem *items, uint32_t ncols_total, void *big_ctl, const ProbeZero &z, hipStream_t st);
 
 int final_kpt(int key_bytes);
-uint32_t final_big_items();
 size_t final_big_ctl_bytes();
 // keys staged per LDS round of the scatter for a level whose widest segment
 // has max_cols columns (0: the columns do not leave room for staging)
