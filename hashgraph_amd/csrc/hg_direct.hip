@@ -38,8 +38,8 @@ __global__ __launch_bounds__(BLOCK) void k_build_one(const K *keys, K *csr, OFF 
 // bin), so the U reads of a step are all issued before the first is used, and
 // from about 10^5 keys on by the lines those reads bring in: 2^20 uint32 keys
 // against 2^20 take 49 us (124 us partitioned), about 22 keys/ns beyond.
-// Matches: one block scan and one reservation per workgroup.  A key of a bin
-// longer than PROBE_BIN_LIMIT goes to the `heavy` list for the caller.
+// Matches, and the keys of bins longer than PROBE_BIN_LIMIT (listed in `heavy`
+// for the caller): one block scan and one reservation of each per workgroup.
 //
 // `st` (a DirectState, zero between calls) collects the counts; the last
 // workgroup to finish stores them to `res` in pinned host memory and zeroes
@@ -68,6 +68,7 @@ __global__ __launch_bounds__(BLOCK) void k_probe_direct(const K *__restrict__ pr
                                                         unsigned long long *__restrict__ res) {
   __shared__ uint32_t s_tmp[BLOCK / 64 + 1];
   __shared__ unsigned long long s_base;
+  __shared__ uint32_t s_heavy;
   const uint32_t k0 = blockIdx.x * (BLOCK * U);
   const uint32_t cnt = min((uint32_t)(BLOCK * U), n - k0);
   const __amdgpu_buffer_rsrc_t rs = make_rsrc(probe + k0, cnt * (uint32_t)sizeof(K));
@@ -81,13 +82,13 @@ __global__ __launch_bounds__(BLOCK) void k_probe_direct(const K *__restrict__ pr
     const uint32_t l = bin_of<K, HK>(kr[j], mp);  // slots past cnt hold key 0: a valid bin
     load_pair(offA + l, b0[j], b1[j]);
   }
-  uint32_t longest = 0;
+  uint32_t longest = 0, hm = 0;  // hm: slots whose key goes to the heavy list
 #pragma unroll
   for (int j = 0; j < U; j++) {
     m[j] = 0;
     if (j * BLOCK + threadIdx.x >= cnt) b1[j] = b0[j];
     if (b1[j] - b0[j] > PROBE_BIN_LIMIT) {
-      heavy[atomicAdd(&st->heavy, 1u)] = kr[j];
+      hm |= 1u << j;
       b1[j] = b0[j];
     }
     longest = max(longest, (uint32_t)(b1[j] - b0[j]));
@@ -107,19 +108,31 @@ __global__ __launch_bounds__(BLOCK) void k_probe_direct(const K *__restrict__ pr
   uint32_t mine = 0;
 #pragma unroll
   for (int j = 0; j < U; j++) mine += m[j];
+  // one scan of both counts: at most 2^17 matches and 2^12 listed keys a workgroup
+  static_assert(BLOCK * U * PROBE_BIN_LIMIT <= (1u << 17) && BLOCK * U < (1 << 14), "packed scan");
   uint32_t tot;
-  const uint32_t ex = block_exclusive_sum<BLOCK, uint32_t>(mine, s_tmp, tot);
-  if (threadIdx.x == 0) s_base = tot ? atomicAdd(&st->cursor, (unsigned long long)tot) : 0ull;
+  const uint32_t ex = block_exclusive_sum<BLOCK, uint32_t>(mine | ((uint32_t)__popc(hm) << 18), s_tmp, tot);
+  if (threadIdx.x == 0) {
+    const uint32_t tm = tot & 0x3FFFFu, th = tot >> 18;
+    s_base = tm ? atomicAdd(&st->cursor, (unsigned long long)tm) : 0ull;
+    s_heavy = th ? atomicAdd(&st->heavy, th) : 0u;
+  }
   __syncthreads();
+  if (hm) {
+    uint32_t w = s_heavy + (ex >> 18);
+#pragma unroll
+    for (int j = 0; j < U; j++)
+      if ((hm >> j) & 1u) heavy[w++] = kr[j];
+  }
   if (out != nullptr && mine) {
-    unsigned long long w = s_base + ex;
+    unsigned long long w = s_base + (ex & 0x3FFFFu);
 #pragma unroll
     for (int j = 0; j < U; j++)
       for (uint32_t r = 0; r < m[j]; r++, w++)
         if (w < capacity) out[w] = kr[j];
   }
   if (threadIdx.x == 0) {
-    __threadfence();  // this workgroup's adds before its ticket (the barrier above ordered the others' list adds)
+    __threadfence();  // this workgroup's adds before its ticket
     if (atomicAdd(&st->ticket, 1u) == gridDim.x - 1) {
       __threadfence();
       res[0] = atomicExch(&st->cursor, 0ull);

@@ -1374,6 +1374,7 @@ hg_status hg_probe(hg_ctx c, const hg_table_desc *descA, const void *d_offA, con
   const int kb = (int)descA->key_bytes, ob = (int)descA->offset_bytes;
   const BinMap map = make_map(M, descA->hash_kind, descA->d_rmi_model);
   uint64_t done = 0;  // matches already counted (and emitted) by the direct probe
+  bool done_direct = false;
   if (probe_direct_takes(descA, d_probe, n_probe, d_out, capacity)) {
     HG_TRY(arena_ensure(c, 2, n_probe * kb));
     LaunchProbeDirect p{};
@@ -1402,6 +1403,7 @@ hg_status hg_probe(hg_ctx c, const hg_table_desc *descA, const void *d_offA, con
       if (d_out && done > capacity) return fail(HG_ERR_CAPACITY, "output capacity smaller than the match count");
       return HG_OK;
     }
+    done_direct = true;
     // the keys of long bins go through the partitioned probe, whose value
     // tables answer them
   }
@@ -1491,13 +1493,17 @@ hg_status hg_probe(hg_ctx c, const hg_table_desc *descA, const void *d_offA, con
   pr.hmark = hmark;
   pr.big_slot = d.big_slot;
   pr.big_ctl = d.big_ctl;
+  // long bins are known of (listed keys) or likely (long on average): the
+  // kernels that answer them follow at once, else only if a gate asks for them
+  const bool rest = done_direct || descA->n_keys > 8 * M;
   {
     Prof pf(c, "probe");
     HG_HIP(launch_probe_one(pr, c->stream));
+    if (rest) HG_HIP(launch_probe_rest(pr, c->stream));
   }
   unsigned long long res[2] = {0, 0};  // matches, both gates
   HG_TRY(sync_read(c, res, small, 16));
-  if (res[1]) {  // items or bins left (skewed keys)
+  if (res[1] && !rest) {  // items or bins left (skewed keys)
     {
       Prof pf(c, "probe");
       HG_HIP(launch_probe_rest(pr, c->stream));
