@@ -364,9 +364,10 @@ __global__ __launch_bounds__(BLOCK) void k_part_scatter(const K *__restrict__ ke
 // the list are streamed by single workgroups after the listed ones.
 // ---------------------------------------------------------------------------
 struct BigCtl {
-  unsigned long long packed;  // listed slots << 40 | chunks
-  unsigned long long bins;    // per-bin counters asked for
-  uint32_t unlisted;          // some item did not fit
+  // the first BIG_CTL_ZERO words of 8 bytes are cleared before the list is used
+  unsigned long long packed;    // listed slots << 40 | chunks
+  unsigned long long bins;      // per-bin counters asked for
+  unsigned long long unlisted;  // some item did not fit
   uint32_t item[BIG_CAP];
   uint32_t chunk_start[BIG_CAP];
   uint32_t bin_base[BIG_CAP];
@@ -2750,18 +2751,26 @@ static hipError_t launch_final_t(const LaunchFinal &lf, hipStream_t st) {
   const hipError_t e = dispatch_hk(lf.hk, [&](auto h) {
     constexpr int H = decltype(h)::value;
     // the split store exists for murmur3 tables only (launch_final checks)
-    auto kern = &k_final<K, OFF, 1024, KPT, H>;
-    if constexpr (SPLIT && H == HK_MURMUR) kern = &k_final<K, OFF, 1024, KPT, H, true>;
-    hipLaunchKernelGGL(kern, dim3(lf.nitems), dim3(1024), lf.lds_bytes, st, (const K *)lf.part, (K *)lf.csr,
-                       (OFF *)lf.off, lf.items, lf.maps, lf.lds_bytes, ctl, lf.big_slot, lf.big_cnt, lf.big_cap,
-                       lf.csr_index);
-    return hipGetLastError();
+    constexpr bool S = SPLIT && H == HK_MURMUR;
+    auto go = [&](auto kern, uint32_t block) {
+      hipLaunchKernelGGL(kern, dim3(lf.nitems), dim3(block), lf.lds_bytes, st, (const K *)lf.part, (K *)lf.csr,
+                         (OFF *)lf.off, lf.items, lf.maps, lf.lds_bytes, ctl, lf.big_slot, lf.big_cnt, lf.big_cap,
+                         lf.csr_index);
+      return hipGetLastError();
+    };
+    // the small classes serve one table, murmur3 or learned
+    if constexpr (H != HK_ANY) {
+      if (lf.cls == 0) return go(&k_final<K, OFF, 256, 16, H, S>, 256);
+      if (lf.cls == 1) return go(&k_final<K, OFF, 512, 16, H, S>, 512);
+      if (lf.cls == 2) return go(&k_final<K, OFF, 1024, 16, H, S>, 1024);
+    }
+    return go(&k_final<K, OFF, 1024, KPT, H, S>, 1024);
   });
   if (e != hipSuccess) return e;
   // three kernels that return at once when no item was oversized: two
   // workgroups per CU (their 128 KB of LDS admit one at a time) dispatch in
   // under 2 us, the 2048 they had took 4.5 us
-  const uint32_t small_cap = std::min(1024u * KPT, 65535u);
+  const uint32_t small_cap = std::min(final_class_keys(lf.cls), 65535u);
   hipLaunchKernelGGL((k_big_count<K, 1024>), dim3(BIG_GRID), dim3(1024), 0, st, (const K *)lf.part, lf.items, lf.maps,
                      (const BigCtl *)ctl, lf.big_cnt);
   hipLaunchKernelGGL((k_big_scan<OFF>), dim3(256), dim3(1024), 0, st, lf.items, (const BigCtl *)ctl, lf.big_cnt,
@@ -2772,7 +2781,9 @@ static hipError_t launch_final_t(const LaunchFinal &lf, hipStream_t st) {
   return hipGetLastError();
 }
 
+static_assert(final_class_keys(FINAL_CLASSES - 1) == 1024u * KPT_U32, "largest final-stage class");
 hipError_t launch_final(const LaunchFinal &lf, hipStream_t st) {
+  if (lf.cls < 0 || lf.cls >= FINAL_CLASSES || (lf.cls != FINAL_CLASSES - 1 && lf.hk == HK_ANY)) return hipErrorInvalidValue;
   if (lf.csr_index) {  // index-carrying build of 32-bit keys: 8-byte murmur3 records split on store
     if (lf.key_bytes != 8 || lf.hk != HK_MURMUR) return hipErrorInvalidValue;
     return lf.off_bytes == 4 ? launch_final_t<uint64_t, uint32_t, true>(lf, st)
@@ -3234,6 +3245,14 @@ static hipError_t join_set_lds() {
   return r;
 }
 
+template <typename K, typename OFF, int H, bool S>
+static hipError_t set_final_classes() {
+  hipError_t r = set_lds(&k_final<K, OFF, 256, 16, H, S>);
+  if (r == hipSuccess) r = set_lds(&k_final<K, OFF, 512, 16, H, S>);
+  if (r == hipSuccess) r = set_lds(&k_final<K, OFF, 1024, 16, H, S>);
+  return r;
+}
+
 hipError_t set_kernel_attributes() {
   hipError_t e = hipSuccess;
 #define HG_SET(...) do { hipError_t e_ = set_lds(__VA_ARGS__); if (e_ != hipSuccess) e = e_; } while (0)
@@ -3262,6 +3281,14 @@ hipError_t set_kernel_attributes() {
       if constexpr (H == HK_MURMUR) {
         if (r == hipSuccess) r = set_lds(&k_final<uint64_t, uint32_t, 1024, 32, H, true>);
         if (r == hipSuccess) r = set_lds(&k_final<uint64_t, uint64_t, 1024, 32, H, true>);
+        if (r == hipSuccess) r = set_final_classes<uint64_t, uint32_t, H, true>();
+        if (r == hipSuccess) r = set_final_classes<uint64_t, uint64_t, H, true>();
+      }
+      if constexpr (H != HK_ANY) {
+        if (r == hipSuccess) r = set_final_classes<uint32_t, uint32_t, H, false>();
+        if (r == hipSuccess) r = set_final_classes<uint32_t, uint64_t, H, false>();
+        if (r == hipSuccess) r = set_final_classes<uint64_t, uint32_t, H, false>();
+        if (r == hipSuccess) r = set_final_classes<uint64_t, uint64_t, H, false>();
       }
       if (r == hipSuccess) r = set_lds(&k_probe1<uint32_t, uint32_t, 1024, probe1_kpt<uint32_t>(), H>);
       if (r == hipSuccess) r = set_lds(&k_probe1<uint32_t, uint64_t, 1024, probe1_kpt<uint32_t>(), H>);

@@ -42,11 +42,16 @@ struct LaunchCol {
   uint32_t *bstart;
 };
 
+// Bucket size classes of the final stage: keys a workgroup holds.  Small
+// tables take small buckets, so that there are workgroups for every CU.
+constexpr int FINAL_CLASSES = 4;
+constexpr uint32_t final_class_keys(int cls) { return 4096u << cls; }
 struct LaunchFinal {
   int key_bytes, off_bytes;
   int hk;
   uint32_t nitems;
   uint32_t lds_bytes;
+  int cls = FINAL_CLASSES - 1;  // bucket size class (final_class_keys)
   const void *part;
   void *csr;
   void *off;
@@ -112,6 +117,29 @@ struct LaunchBuildOne {
   void *csr, *off;
   uint32_t n, bin_lo, nbins;  // keys, all with a bin in [bin_lo, bin_lo + nbins)
   BinMap map;
+};
+
+// Narrow partition pass: keys whose bins lie in [bin_lo, bin_lo + nbins) into
+// ncols buckets of div.d bins, range r of per keys counted in row r.
+constexpr uint32_t NARROW_COLS = 512, NARROW_ROWS = 512;
+struct NarrowGeom {
+  uint64_t n, nbins;
+  uint32_t per, ncols, bin_lo;
+  Div32 div;
+  BinMap map;
+};
+struct LaunchNarrow {
+  int key_bytes;
+  bool pack;          // 32-bit keys made into 8-byte records (key_bytes 8)
+  uint32_t rows;
+  NarrowGeom geom;
+  const void *keys;
+  void *out;
+  uint32_t *cmat, *tot;        // rows * ncols, ncols
+  FinItem *items;              // ncols, for the final stage
+  BinMap *maps;                // one
+  unsigned long long *zero;    // nzero words cleared for the final stage
+  uint32_t nzero;
 };
 
 // Bins longer than this are not walked by the probe kernels but answered from
@@ -303,6 +331,7 @@ uint32_t rle_heavy_grid();
 size_t rle_giant_ctl_bytes();
 hipError_t launch_part_hist(const LaunchPart &lp, hipStream_t st);
 hipError_t launch_part_scatter(const LaunchPart &lp, hipStream_t st);
+hipError_t launch_narrow(const LaunchNarrow &p, hipStream_t st);
 hipError_t launch_colscan(const LaunchCol &lc, hipStream_t st);
 hipError_t launch_final(const LaunchFinal &lf, hipStream_t st);
 // The one-pass kernel, then the kernels of the items and bins it left: they
@@ -348,6 +377,8 @@ hipError_t launch_make_items(const SegDesc *segs, uint32_t nsegs, const uint32_t
                              FinItem *items, uint32_t ncols_total, void *big_ctl, const ProbeZero &z, hipStream_t st);
 
 int final_kpt(int key_bytes);
+// words of a final_big_ctl_bytes() area that are zero when no item is listed
+constexpr uint32_t BIG_CTL_ZERO = 3;
 size_t final_big_ctl_bytes();
 // keys staged per LDS round of the scatter for a level whose widest segment
 // has max_cols columns (0: the columns do not leave room for staging)

@@ -138,3 +138,57 @@ def test_matches_beyond_the_first_buffers(kb, dev):
         assert cnt == ecnt == pa.numel() == pb.numel()
         assert np.array_equal(A[pa.cpu().numpy()], B[pb.cpu().numpy()])
         assert torch.unique((pa << 32) | pb).numel() == cnt
+
+
+# keys at the edges of the final stage's size classes (0.875 of the class times
+# the 512 buckets of a narrow pass), ragged ranges, sparse and dense tables
+@pytest.mark.parametrize("kb,ob", [(4, 4), (8, 8)])
+@pytest.mark.parametrize("n,M", [(16385, 65537), (20011, 3000017), (70001, 70001), (300007, 40009), (1835007, 1835009),
+                                 (1835009, 1835007), (3670021, 3670013), (7340041, 7340033)])
+def test_narrow_build(n, M, kb, ob, dev):
+    import hashgraph_amd as hg
+    print(f"narrow build n={n} M={M} kb={kb} ob={ob}", flush=True)
+    keys = wl.uniform_keys(n + M, n, kb)
+    off, csr = hg.build(_to_dev(keys, dev), M, offset_bytes=ob)
+    _same(off, csr, keys, M, ob)
+
+
+@pytest.mark.parametrize("kb", [4, 8])
+def test_narrow_build_oversized_buckets(kb, dev):
+    """Hot keys: buckets beyond every size class, beside ordinary ones."""
+    import hashgraph_amd as hg
+    dt = np.uint32 if kb == 4 else np.uint64
+    keys = wl.uniform_keys(31, 900000, kb)
+    keys[100:300000] = keys[0]
+    keys[400000:420000] = keys[1]
+    for M in (900000, 65537):
+        off, csr = hg.build(_to_dev(keys.astype(dt), dev), M)
+        _same(off, csr, keys, M, 4)
+
+
+@pytest.mark.parametrize("kb", [4, 8])
+@pytest.mark.parametrize("n", [20011, 1835009])
+def test_narrow_indexed_build(n, kb, dev):
+    import torch
+    import hashgraph_amd as hg
+    keys = wl.uniform_keys(n, n, kb)
+    keys[5:4000] = keys[5]
+    dk = _to_dev(keys, dev)
+    off, csr, ind = hg.build_indexed(dk, n)
+    _same(off, csr, keys, n, 4)
+    assert torch.equal(dk[ind], csr) and torch.equal(torch.sort(ind).values, torch.arange(n, device=dev))
+
+
+def test_narrow_learned_build(dev):
+    import torch
+    import hashgraph_amd as hg
+    n, M = 1000003, 900001
+    dk = wl.lognormal_keys(8, n, device=dev)
+    model, _ = hg.rmi_train(dk, M, seed=2)
+    kw = {"hash_kind": hg.HG_HASH_RMI, "rmi_model": model}
+    off, csr = hg.build(dk, M, **kw)
+    deg = torch.bincount(hg.table_bins(dk, M, **kw).to(torch.int64), minlength=M)
+    assert torch.equal(off[1:].to(torch.int64), torch.cumsum(deg, 0)) and int(off[0]) == 0
+    assert torch.equal(hg.table_bins(csr, M, **kw).to(torch.int64),
+                       torch.repeat_interleave(torch.arange(M, device=dev), deg))
+    assert torch.equal(torch.sort(csr).values, torch.sort(dk).values)
