@@ -37,7 +37,8 @@ __global__ __launch_bounds__(BLOCK) void k_build_one(const K *keys, K *csr, OFF 
 // Bound by the latency of three dependent reads per key (probe key, offsets,
 // bin), so the U reads of a step are all issued before the first is used, and
 // from about 10^5 keys on by the lines those reads bring in: 2^20 uint32 keys
-// against 2^20 take 49 us (124 us partitioned), about 22 keys/ns beyond.
+// against 2^20 take 49 us (105 us through the wide partition pass), about 22
+// keys/ns beyond.
 // Matches, and the keys of bins longer than PROBE_BIN_LIMIT (listed in `heavy`
 // for the caller): one block scan and one reservation of each per workgroup.
 //

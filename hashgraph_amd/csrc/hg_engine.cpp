@@ -631,8 +631,8 @@ int narrow_class(uint64_t n, uint64_t R, uint32_t &W) {
   return -1;
 }
 
-hg_status build_narrow(hg_ctx c, const BinMap &map, int kb, int ob, uint64_t n, uint64_t lo, uint64_t R, int cls,
-                       uint32_t W, const void *d_keys, void *d_off, void *d_csr, uint64_t *d_csr_index, bool pack_in) {
+// Key ranges and buckets (W bins each) of a narrow pass.
+LaunchNarrow narrow_launch(const BinMap &map, int kb, uint64_t n, uint64_t lo, uint64_t R, uint32_t W) {
   LaunchNarrow p{};
   NarrowGeom &g = p.geom;
   g.n = n;
@@ -643,8 +643,15 @@ hg_status build_narrow(hg_ctx c, const BinMap &map, int kb, int ob, uint64_t n, 
   g.div = make_div(W);
   g.map = map;
   p.key_bytes = kb;
-  p.pack = pack_in;
   p.rows = (uint32_t)((n + g.per - 1) / g.per);
+  return p;
+}
+
+hg_status build_narrow(hg_ctx c, const BinMap &map, int kb, int ob, uint64_t n, uint64_t lo, uint64_t R, int cls,
+                       uint32_t W, const void *d_keys, void *d_off, void *d_csr, uint64_t *d_csr_index, bool pack_in) {
+  LaunchNarrow p = narrow_launch(map, kb, n, lo, R, W);
+  const NarrowGeom &g = p.geom;
+  p.pack = pack_in;
   const uint64_t big_cap = std::max<uint64_t>(1, std::min<uint64_t>(R, 1ull << 28));
   Plan P0, P1;
   const size_t i_part = P0.add(n * kb);
@@ -689,6 +696,33 @@ hg_status build_narrow(hg_ctx c, const BinMap &map, int kb, int ob, uint64_t n, 
   Prof pf(c, "final");
   HG_HIP(launch_final(f, c->stream));
   return HG_OK;
+}
+
+// Geometry of a narrow probe: keys of B per workgroup and its LDS, the
+// smallest class whose buckets (W bins) are at most NARROW_COLS.  A bucket
+// should fill at most 0.8 of the class, and its keys of A with its offsets the
+// class's share of a CU's LDS, eight standard deviations above the mean (what
+// exceeds it takes k_probe).  Returns 0 when no class does: the wide pass.
+// Narrow against wide, as many uint32 probe keys as table keys: 60 against
+// 113 us at 2^21, 80 against 121 us at 2^22, 153 against 200 us at 12 M.
+uint32_t narrow_probe(uint64_t nb, uint64_t na, uint64_t M, int kb, uint32_t &W, uint32_t &lds) {
+  const double r = (double)na / (double)M;
+  for (int cls = 0; cls < 4; cls++) {
+    // the last two classes: 16 K keys with the whole LDS, then what the wide probe holds
+    const uint32_t keys = cls < 3 ? 4096u << cls : probe_one_keys(kb);
+    const uint32_t room = cls == 0 ? 52 * 1024 : cls < 3 ? 78 * 1024 : PROBE1_LDS;
+    double w = std::min(0.8 * keys * (double)M / (double)nb, 65535.0);
+    w = std::min(w, std::max(2.0 * keys, std::ceil((double)M / NARROW_COLS)));
+    for (; w >= 1; w *= 0.97) {
+      const double mean = w * r;
+      lds = probe_one_lds((uint32_t)w, (uint64_t)(mean + 8 * std::sqrt(mean) + 64), kb);
+      if (lds <= room) break;
+    }
+    if (w < 1) continue;
+    W = (uint32_t)w;
+    if ((M + W - 1) / W <= NARROW_COLS) return keys;
+  }
+  return 0;
 }
 
 // CSR of n keys whose bins all lie in [lo, lo + R): d_off[0..R] with values
@@ -972,16 +1006,111 @@ std::vector<LaunchRmiBatch> rmi_launches(std::vector<RmiBatchItem> &items, int k
 // ===========================================================================
 // C ABI
 // ===========================================================================
+// Wide pass of hg_probe: the probe keys partitioned by buckets of the table's
+// bins (one or two levels) and pr's items, their state and the one-pass
+// kernel's class filled in.
+static hg_status probe_wide(hg_ctx c, const BinMap &map, int kb, uint64_t n_keys, uint64_t M, const void *d_probe,
+                     uint64_t n_probe, uint64_t done, LaunchProbe &pr) {
+  const uint32_t W = choose_width(std::max<uint64_t>(n_probe, n_keys), M, kb, probe_fill(kb));
+  const uint64_t F = (M + W - 1) / W;
+  // Beyond kFMax buckets, B is partitioned twice: into super-buckets of k
+  // buckets, whose sizes are read back, then each super-bucket into its
+  // buckets (as the build's second level).
+  const uint64_t k = level1_group(F);
+  const bool two = k > 1;
+  if ((uint64_t)W * k >= (1ull << 32)) return fail(HG_ERR_UNSUPPORTED, "probe geometry too large");
+  Plan P0;
+  const size_t i_part = P0.add(n_probe * kb);
+  const size_t i_part2 = P0.add(two ? n_probe * kb : 1);
+  const size_t i_small = P0.add(256);
+  const size_t i_mark = P0.add((size_t)(F + kFMax + 1) * 4);  // >= the buckets of the last level
+  HG_TRY(arena_ensure(c, 0, P0.total()));
+  Carve cv0;
+  cv0.init(c, 0, P0);
+  void *part = cv0.get<void>(i_part);
+  unsigned long long *small = cv0.get<unsigned long long>(i_small);
+  unsigned int *hmark = cv0.get<unsigned int>(i_mark);
+  Level L;
+  LevelDev d;
+  if (!two) {
+    SegDesc s = range_seg(0, n_probe, 0, M, W, map);
+    s.fin_off_base = 0;
+    s.fin_key_rel = 0;
+    s.table = 0;
+    L.segs.push_back(s);
+    L.maps.push_back(map);
+    L.auto_tile(n_probe);
+    L.prepare();
+    HG_TRY(setup_level(c, L, d));
+    HG_TRY(run_level(c, L, d, kb, d_probe, part));
+  } else {
+    const uint64_t W1 = (uint64_t)W * k;
+    Level L1;
+    L1.segs.push_back(range_seg(0, n_probe, 0, M, (uint32_t)W1, map));
+    L1.maps.push_back(map);
+    L1.auto_tile(n_probe);
+    L1.prepare();
+    LevelDev d1;
+    HG_TRY(setup_level(c, L1, d1));
+    HG_TRY(run_level(c, L1, d1, kb, d_probe, part));
+    std::vector<uint32_t> cnt(L1.ncols_total), st(L1.ncols_total);
+    HG_TRY(sync_read(c, cnt.data(), d1.coltot, cnt.size() * 4));
+    HG_TRY(sync_read(c, st.data(), d1.bstart, st.size() * 4));
+    for (uint32_t g = 0; g < L1.ncols_total; g++) {
+      const uint64_t lo = (uint64_t)g * W1, nb = std::min<uint64_t>(W1, M - lo);
+      SegDesc s = range_seg(st[g], (uint64_t)st[g] + cnt[g], lo, nb, W, map);
+      s.fin_off_base = lo;
+      s.fin_key_rel = 0;
+      s.table = 0;
+      L.segs.push_back(s);
+    }
+    L.maps.push_back(map);
+    L.auto_tile(n_probe);
+    L.prepare();
+    HG_TRY(setup_level(c, L, d));
+    void *part2 = cv0.get<void>(i_part2);
+    HG_TRY(run_level(c, L, d, kb, part, part2));
+    part = part2;
+  }
+  ProbeZero z;
+  z.hmark = hmark;
+  z.gate = (unsigned int *)(small + 1);
+  z.cursor = small;
+  z.count = done;
+  HG_HIP(launch_make_items(d.segs, (uint32_t)L.segs.size(), d.bstart, d.coltot, d.fin, L.ncols_total, d.big_ctl, z,
+                           c->stream));
+  pr.hk = L.hash_kind();
+  pr.nitems = L.ncols_total;
+  pr.bpart = part;
+  pr.items = d.fin;
+  pr.maps = d.maps;
+  pr.cursor = small;
+  pr.gate = z.gate;
+  pr.hmark = hmark;
+  pr.big_slot = d.big_slot;
+  pr.big_ctl = d.big_ctl;
+  pr.one_keys = probe_one_keys(kb);
+  pr.one_lds = PROBE1_LDS;
+  return HG_OK;
+}
+
 // Whether hg_probe walks the table without partitioning the probe keys.  A
-// direct probe moves two cache lines a key but takes one launch (49 us at 2^20
-// uint32 keys a side against 124 us partitioned, 97 against 123 us at 2^21,
-// 190 against 130 us at 2^22); a partitioned one reads the whole table,
-// whatever the number of probe keys (2^23 keys against a table of 2^27: 475 us
-// either way).  Tables of long bins go to the partitioned probe at once.
-constexpr uint64_t kDirectProbe = 1ull << 21, kDirectProbeShare = 32;
-bool probe_direct_takes(const hg_table_desc *A, const void *d_probe, uint64_t n_probe, const void *d_out,
+// direct probe moves two cache lines a key but takes one launch; a narrow pass
+// takes four (uint32 keys against as many: 49 us direct and 55 us narrow at
+// 2^20, 73 and 59 us at 1.5 M; uint64: 55 and 67 us, 78 and 72 us).  The wide
+// pass reads the whole table, whatever the number of probe keys (2^21 keys
+// against a table of 2^27: 136 us direct, 434 us wide; 2^23 keys: 475 us either
+// way).  Tables of long bins go to the partitioned probe at once.
+constexpr uint64_t kDirectProbe = 1ull << 21, kDirectProbeShare = 32;       // where the other way is the wide pass
+constexpr uint64_t kDirectNarrow4 = 1ull << 20, kDirectNarrow8 = 5ull << 18;  // where it is the narrow one
+static bool probe_direct_takes(const hg_table_desc *A, const void *d_probe, uint64_t n_probe, const void *d_out,
                         uint64_t capacity) {
-  if (n_probe > std::max(kDirectProbe, A->n_keys / kDirectProbeShare) || A->n_keys > 8 * A->n_bins) return false;
+  if (A->n_keys > 8 * A->n_bins) return false;
+  uint32_t W, lds;
+  const bool narrow = narrow_probe(n_probe, A->n_keys, A->n_bins, (int)A->key_bytes, W, lds) != 0;
+  const uint64_t most = !narrow ? std::max(kDirectProbe, A->n_keys / kDirectProbeShare)
+                                : A->key_bytes == 4 ? kDirectNarrow4 : kDirectNarrow8;
+  if (n_probe > most) return false;
   // matches are written while other workgroups still read the probe keys
   const uintptr_t o = (uintptr_t)d_out, q = (uintptr_t)d_probe;
   const uint64_t room = std::min<uint64_t>(capacity, 1ull << 40) * A->key_bytes;
@@ -1489,92 +1618,58 @@ hg_status hg_probe(hg_ctx c, const hg_table_desc *descA, const void *d_offA, con
     // the keys of long bins go through the partitioned probe, whose value
     // tables answer them
   }
-  const uint32_t W = choose_width(std::max<uint64_t>(n_probe, descA->n_keys), M, kb, probe_fill(kb));
-  const uint64_t F = (M + W - 1) / W;
-  // Beyond kFMax buckets, B is partitioned twice: into super-buckets of k
-  // buckets, whose sizes are read back, then each super-bucket into its
-  // buckets (as the build's second level).
-  const uint64_t k = level1_group(F);
-  const bool two = k > 1;
-  if ((uint64_t)W * k >= (1ull << 32)) return fail(HG_ERR_UNSUPPORTED, "probe geometry too large");
-  Plan P0;
-  const size_t i_part = P0.add(n_probe * kb);
-  const size_t i_part2 = P0.add(two ? n_probe * kb : 1);
-  const size_t i_small = P0.add(256);
-  const size_t i_mark = P0.add((size_t)(F + kFMax + 1) * 4);  // >= the buckets of the last level
-  HG_TRY(arena_ensure(c, 0, P0.total()));
-  Carve cv0;
-  cv0.init(c, 0, P0);
-  void *part = cv0.get<void>(i_part);
-  unsigned long long *small = cv0.get<unsigned long long>(i_small);
-  unsigned int *hmark = cv0.get<unsigned int>(i_mark);
-  Level L;
-  LevelDev d;
-  if (!two) {
-    SegDesc s = range_seg(0, n_probe, 0, M, W, map);
-    s.fin_off_base = 0;
-    s.fin_key_rel = 0;
-    s.table = 0;
-    L.segs.push_back(s);
-    L.maps.push_back(map);
-    L.auto_tile(n_probe);
-    L.prepare();
-    HG_TRY(setup_level(c, L, d));
-    HG_TRY(run_level(c, L, d, kb, d_probe, part));
-  } else {
-    const uint64_t W1 = (uint64_t)W * k;
-    Level L1;
-    L1.segs.push_back(range_seg(0, n_probe, 0, M, (uint32_t)W1, map));
-    L1.maps.push_back(map);
-    L1.auto_tile(n_probe);
-    L1.prepare();
-    LevelDev d1;
-    HG_TRY(setup_level(c, L1, d1));
-    HG_TRY(run_level(c, L1, d1, kb, d_probe, part));
-    std::vector<uint32_t> cnt(L1.ncols_total), st(L1.ncols_total);
-    HG_TRY(sync_read(c, cnt.data(), d1.coltot, cnt.size() * 4));
-    HG_TRY(sync_read(c, st.data(), d1.bstart, st.size() * 4));
-    for (uint32_t g = 0; g < L1.ncols_total; g++) {
-      const uint64_t lo = (uint64_t)g * W1, nb = std::min<uint64_t>(W1, M - lo);
-      SegDesc s = range_seg(st[g], (uint64_t)st[g] + cnt[g], lo, nb, W, map);
-      s.fin_off_base = lo;
-      s.fin_key_rel = 0;
-      s.table = 0;
-      L.segs.push_back(s);
-    }
-    L.maps.push_back(map);
-    L.auto_tile(n_probe);
-    L.prepare();
-    HG_TRY(setup_level(c, L, d));
-    void *part2 = cv0.get<void>(i_part2);
-    HG_TRY(run_level(c, L, d, kb, part, part2));
-    part = part2;
-  }
-  ProbeZero z;
-  z.hmark = hmark;
-  z.gate = (unsigned int *)(small + 1);
-  z.cursor = small;
-  z.count = done;
-  HG_HIP(launch_make_items(d.segs, (uint32_t)L.segs.size(), d.bstart, d.coltot, d.fin, L.ncols_total, d.big_ctl, z,
-                           c->stream));
   LaunchProbe pr{};
+  uint32_t Wn, lds = 0;
+  if (const uint32_t one = narrow_probe(n_probe, descA->n_keys, M, kb, Wn, lds); one) {
+    LaunchNarrow p = narrow_launch(map, kb, n_probe, 0, M, Wn);
+    Plan P0, P1;
+    const size_t i_part = P0.add(n_probe * kb);
+    const size_t i_cmat = P1.add((size_t)p.rows * p.geom.ncols * 4), i_tot = P1.add(NARROW_COLS * 4),
+                 i_items = P1.add(NARROW_COLS * sizeof(FinItem)), i_maps = P1.add(sizeof(BinMap)),
+                 i_slot = P1.add(NARROW_COLS * 4), i_mark = P1.add(NARROW_COLS * 4),
+                 i_small = P1.add(256 + final_big_ctl_bytes());
+    HG_TRY(arena_ensure(c, 0, P0.total()));
+    HG_TRY(arena_ensure(c, 1, P1.total()));
+    Carve c0, c1;
+    c0.init(c, 0, P0);
+    c1.init(c, 1, P1);
+    // the cursor and the gates end where the list of oversized buckets begins
+    pr.big_ctl = c1.get<char>(i_small) + 256;
+    pr.cursor = (unsigned long long *)pr.big_ctl - 2;
+    pr.gate = (unsigned int *)(pr.cursor + 1);
+    pr.hmark = c1.get<unsigned int>(i_mark);
+    pr.big_slot = c1.get<uint32_t>(i_slot);
+    p.keys = d_probe;
+    p.out = c0.get<void>(i_part);
+    p.cmat = c1.get<uint32_t>(i_cmat);
+    p.tot = c1.get<uint32_t>(i_tot);
+    p.items = c1.get<FinItem>(i_items);
+    p.maps = c1.get<BinMap>(i_maps);
+    p.zero = pr.cursor;
+    p.nzero = 2 + BIG_CTL_ZERO;
+    p.zero_col = pr.hmark;
+    {
+      Prof pf(c, "part_scatter");
+      HG_HIP(launch_narrow(p, c->stream));
+    }
+    if (done) HG_HIP(launch_fill_u64(pr.cursor, done, 1, c->stream));
+    pr.hk = (int)map.kind;
+    pr.nitems = p.geom.ncols;
+    pr.bpart = p.out;
+    pr.items = p.items;
+    pr.maps = p.maps;
+    pr.one_keys = one;
+    pr.one_lds = lds;
+  } else {
+    HG_TRY(probe_wide(c, map, kb, descA->n_keys, M, d_probe, n_probe, done, pr));
+  }
   pr.key_bytes = kb;
   pr.off_bytes = ob;
-  pr.hk = L.hash_kind();
-  pr.nitems = L.ncols_total;
   pr.akey_cap = probe_akey_cap(kb, ob);
-  pr.bpart = part;
-  pr.items = d.fin;
-  pr.maps = d.maps;
   pr.offA = d_offA;
   pr.keysA = d_keysA;
   pr.out = d_out;
   pr.capacity = d_out ? capacity : 0;
-  pr.cursor = small;
-  pr.gate = z.gate;
-  pr.hmark = hmark;
-  pr.big_slot = d.big_slot;
-  pr.big_ctl = d.big_ctl;
   // long bins are known of (listed keys) or likely (long on average): the
   // kernels that answer them follow at once, else only if a gate asks for them
   const bool rest = done_direct || descA->n_keys > 8 * M;
@@ -1584,13 +1679,13 @@ hg_status hg_probe(hg_ctx c, const hg_table_desc *descA, const void *d_offA, con
     if (rest) HG_HIP(launch_probe_rest(pr, c->stream));
   }
   unsigned long long res[2] = {0, 0};  // matches, both gates
-  HG_TRY(sync_read(c, res, small, 16));
+  HG_TRY(sync_read(c, res, pr.cursor, 16));
   if (res[1] && !rest) {  // items or bins left (skewed keys)
     {
       Prof pf(c, "probe");
       HG_HIP(launch_probe_rest(pr, c->stream));
     }
-    HG_TRY(sync_read(c, res, small, 8));
+    HG_TRY(sync_read(c, res, pr.cursor, 8));
   }
   const unsigned long long cnt = res[0];
   *h_count = cnt;
@@ -2842,6 +2937,8 @@ hg_status batch_launch_probe(hg_ctx c, const hg_batch_desc *bd, BatchSide &S, co
   pr.hk = S.L.hash_kind();
   pr.nitems = S.L.ncols_total;
   pr.akey_cap = probe_akey_cap(pr.key_bytes, 4);
+  pr.one_keys = probe_one_keys(pr.key_bytes);
+  pr.one_lds = PROBE1_LDS;
   pr.bpart = S.part;
   pr.items = S.d.fin;
   pr.maps = S.d.maps;

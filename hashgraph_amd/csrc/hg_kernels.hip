@@ -2801,17 +2801,32 @@ size_t final_big_ctl_bytes() { return sizeof(BigCtl); }
 
 // One-pass probe's bucket limits: keys of B per workgroup, keys of A in LDS.
 template <typename K> constexpr int probe1_kpt() { return sizeof(K) == 4 ? 32 : 16; }
-constexpr uint32_t PROBE1_LDS = 156 * 1024;  // keys of A + 16-bit offsets
+uint32_t probe_one_keys(int key_bytes) {
+  return 1024u * (uint32_t)(key_bytes == 4 ? probe1_kpt<uint32_t>() : probe1_kpt<uint64_t>());
+}
+uint32_t probe_one_lds(uint32_t W, uint64_t keys_a, int key_bytes) {
+  return (uint32_t)std::min<uint64_t>(probe1_off_bytes(W) + keys_a * (uint64_t)key_bytes + 16 + PROBE1_LEAF_BYTES,
+                                      1u << 30);
+}
 
 template <typename K, typename OFF>
 static hipError_t launch_probe_one_t(const LaunchProbe &p, hipStream_t st) {
   constexpr int KPT = sizeof(K) == 4 ? KPT_U32 : 32;
   return dispatch_hk(p.hk, [&](auto h) {
-    hipLaunchKernelGGL((k_probe1<K, OFF, 1024, probe1_kpt<K>(), decltype(h)::value>), dim3(p.nitems), dim3(1024),
-                       (size_t)PROBE1_LDS, st, (const K *)p.bpart, p.items, p.maps, (const OFF *)p.offA,
-                       (const K *)p.keysA, (K *)p.out, p.capacity, p.cursor, PROBE1_LDS, p.hmark, p.gate, p.out_off,
-                       std::min(1024u * KPT, 65535u), (BigCtl *)p.big_ctl, p.big_slot);
-    return hipGetLastError();
+    constexpr int H = decltype(h)::value;
+    auto go = [&](auto kern, uint32_t block) {
+      hipLaunchKernelGGL(kern, dim3(p.nitems), dim3(block), (size_t)p.one_lds, st, (const K *)p.bpart, p.items, p.maps,
+                         (const OFF *)p.offA, (const K *)p.keysA, (K *)p.out, p.capacity, p.cursor, p.one_lds, p.hmark,
+                         p.gate, p.out_off, std::min(1024u * KPT, 65535u), (BigCtl *)p.big_ctl, p.big_slot);
+      return hipGetLastError();
+    };
+    if constexpr (H != HK_ANY) {  // the small classes serve one table, murmur3 or learned
+      if (p.one_keys == 4096) return go(&k_probe1<K, OFF, 256, 16, H>, 256);
+      if (p.one_keys == 8192) return go(&k_probe1<K, OFF, 512, 16, H>, 512);
+      if (p.one_keys == 16384) return go(&k_probe1<K, OFF, 1024, 16, H>, 1024);
+    }
+    if (p.one_keys != probe_one_keys((int)sizeof(K))) return hipErrorInvalidValue;
+    return go(&k_probe1<K, OFF, 1024, probe1_kpt<K>(), H>, 1024);
   });
 }
 
@@ -2824,8 +2839,7 @@ static hipError_t launch_probe_rest_t(const LaunchProbe &p, hipStream_t st) {
   const hipError_t e = dispatch_hk(p.hk, [&](auto h) {
     hipLaunchKernelGGL((k_probe<K, OFF, 1024, KPT, SUB, decltype(h)::value>), dim3(p.nitems), dim3(1024), lds, st,
                        (const K *)p.bpart, p.items, p.maps, (const OFF *)p.offA, (const K *)p.keysA, (K *)p.out,
-                       p.capacity, p.cursor, p.akey_cap, p.hmark, (uint32_t)(1024 * probe1_kpt<K>()), PROBE1_LDS,
-                       p.gate, p.out_off);
+                       p.capacity, p.cursor, p.akey_cap, p.hmark, p.one_keys, p.one_lds, p.gate, p.out_off);
     return hipGetLastError();
   });
   if (e != hipSuccess) return e;
@@ -3253,6 +3267,14 @@ static hipError_t set_final_classes() {
   return r;
 }
 
+template <typename K, typename OFF, int H>
+static hipError_t set_probe_classes() {
+  hipError_t r = set_lds(&k_probe1<K, OFF, 256, 16, H>);
+  if (r == hipSuccess) r = set_lds(&k_probe1<K, OFF, 512, 16, H>);
+  if (r == hipSuccess) r = set_lds(&k_probe1<K, OFF, 1024, 16, H>);
+  return r;
+}
+
 hipError_t set_kernel_attributes() {
   hipError_t e = hipSuccess;
 #define HG_SET(...) do { hipError_t e_ = set_lds(__VA_ARGS__); if (e_ != hipSuccess) e = e_; } while (0)
@@ -3294,6 +3316,12 @@ hipError_t set_kernel_attributes() {
       if (r == hipSuccess) r = set_lds(&k_probe1<uint32_t, uint64_t, 1024, probe1_kpt<uint32_t>(), H>);
       if (r == hipSuccess) r = set_lds(&k_probe1<uint64_t, uint32_t, 1024, probe1_kpt<uint64_t>(), H>);
       if (r == hipSuccess) r = set_lds(&k_probe1<uint64_t, uint64_t, 1024, probe1_kpt<uint64_t>(), H>);
+      if constexpr (H != HK_ANY) {
+        if (r == hipSuccess) r = set_probe_classes<uint32_t, uint32_t, H>();
+        if (r == hipSuccess) r = set_probe_classes<uint32_t, uint64_t, H>();
+        if (r == hipSuccess) r = set_probe_classes<uint64_t, uint32_t, H>();
+        if (r == hipSuccess) r = set_probe_classes<uint64_t, uint64_t, H>();
+      }
       if (r == hipSuccess) r = set_lds(&k_probe<uint32_t, uint32_t, 1024, KPT_U32, probe_sub<uint32_t>(), H>);
       if (r == hipSuccess) r = set_lds(&k_probe<uint32_t, uint64_t, 1024, KPT_U32, probe_sub<uint64_t>(), H>);
       if (r == hipSuccess) r = set_lds(&k_probe<uint64_t, uint32_t, 1024, 32, probe_sub<uint32_t>(), H>);

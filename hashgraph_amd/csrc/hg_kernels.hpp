@@ -74,6 +74,8 @@ struct LaunchProbe {
   int hk;
   uint32_t nitems;
   uint32_t akey_cap;
+  uint32_t one_keys, one_lds;  // one-pass kernel: keys of B a workgroup holds (4096, 8192, 16384 or
+                               // probe_one_keys) and its LDS (probe_one_lds of what it should take)
   const void *bpart;
   const FinItem *items;
   const BinMap *maps;
@@ -138,8 +140,9 @@ struct LaunchNarrow {
   uint32_t *cmat, *tot;        // rows * ncols, ncols
   FinItem *items;              // ncols, for the final stage
   BinMap *maps;                // one
-  unsigned long long *zero;    // nzero words cleared for the final stage
+  unsigned long long *zero;    // nzero words cleared for the final stage or the probe
   uint32_t nzero;
+  unsigned int *zero_col;      // ncols more (or null)
 };
 
 // Bins longer than this are not walked by the probe kernels but answered from
@@ -336,6 +339,10 @@ hipError_t launch_colscan(const LaunchCol &lc, hipStream_t st);
 hipError_t launch_final(const LaunchFinal &lf, hipStream_t st);
 // The one-pass kernel, then the kernels of the items and bins it left: they
 // need not run when both gates are still 0 (and return at once if they do).
+constexpr uint32_t PROBE1_LDS = 156 * 1024;  // most LDS of a one-pass workgroup
+uint32_t probe_one_keys(int key_bytes);
+// LDS the one-pass probe needs for a bucket of W bins and keys_a keys of A
+uint32_t probe_one_lds(uint32_t W, uint64_t keys_a, int key_bytes);
 hipError_t launch_probe_one(const LaunchProbe &p, hipStream_t st);
 hipError_t launch_probe_rest(const LaunchProbe &p, hipStream_t st);
 hipError_t launch_join(const LaunchJoin &j, hipStream_t st);

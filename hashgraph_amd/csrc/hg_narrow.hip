@@ -86,7 +86,8 @@ __global__ __launch_bounds__(NB) void k_narrow_scatter(const void *__restrict__ 
                                                        const uint32_t *__restrict__ cmat,
                                                        const uint32_t *__restrict__ tot, K *__restrict__ out,
                                                        FinItem *__restrict__ items, BinMap *__restrict__ maps,
-                                                       unsigned long long *__restrict__ zero, uint32_t nzero) {
+                                                       unsigned long long *__restrict__ zero, uint32_t nzero,
+                                                       unsigned int *__restrict__ zero_col) {
   constexpr int KPT = sizeof(K) == 4 ? 16 : 8;
   constexpr uint32_t T = NB * KPT;
   using IN = typename std::conditional<PACK, uint32_t, K>::type;
@@ -112,6 +113,7 @@ __global__ __launch_bounds__(NB) void k_narrow_scatter(const void *__restrict__ 
       it.bin_lo = (uint32_t)(g.bin_lo + lo);
       it.table = 0;
       items[b] = it;
+      if (zero_col) zero_col[b] = 0;
     }
     if (b == 0) maps[0] = g.map;
     if (b < nzero) zero[b] = 0;
@@ -180,7 +182,8 @@ hipError_t launch_narrow_t(const LaunchNarrow &p, hipStream_t st) {
   if constexpr (sizeof(K) == 8 && HK == HK_MURMUR)
     if (p.pack) kern = &k_narrow_scatter<K, HK, true>;
   hipLaunchKernelGGL(kern, dim3(p.rows), dim3(NB), 0, st, p.keys, g, (const uint32_t *)p.cmat,
-                     (const uint32_t *)p.tot, (K *)p.out, p.items, p.maps, p.zero, p.nzero);
+                     (const uint32_t *)p.tot, (K *)p.out, p.items, p.maps, p.zero, p.nzero,
+                     p.zero_col);
   return hipGetLastError();
 }
 

@@ -192,3 +192,43 @@ def test_narrow_learned_build(dev):
     assert torch.equal(hg.table_bins(csr, M, **kw).to(torch.int64),
                        torch.repeat_interleave(torch.arange(M, device=dev), deg))
     assert torch.equal(torch.sort(csr).values, torch.sort(dk).values)
+
+
+@pytest.mark.parametrize("kb,ob", [(4, 4), (8, 8)])
+@pytest.mark.parametrize("nA,nB,M", [(1310723, 1310721, 1310719), (100003, 3000017, 65537), (3000017, 1400003, 1000003),
+                                     (200003, 1500007, 5000011), (6000011, 6000007, 6000013)])
+def test_narrow_probe(nA, nB, M, kb, ob, dev):
+    """Every bucket class of the narrow probe: balanced, many more probe keys
+    than table keys, long and sparse bins."""
+    import hashgraph_amd as hg
+    print(f"narrow probe nA={nA} nB={nB} M={M} kb={kb} ob={ob}", flush=True)
+    A = wl.uniform_keys(41, nA, kb)
+    off, csr = hg.build(_to_dev(A, dev), M, offset_bytes=ob)
+    _probe_equal(hg, off, csr, M, A, wl.probe_keys(A, 42, nB, 0.4, kb), dev, ob)
+
+
+@pytest.mark.parametrize("kb", [4, 8])
+def test_narrow_probe_skewed(kb, dev):
+    """Buckets of B beyond every class, of A beyond the LDS, and long bins."""
+    import hashgraph_amd as hg
+    n = 1400003
+    A = wl.uniform_keys(43, n, kb)
+    A[10:40000] = A[10]
+    B = wl.probe_keys(A, 44, n, 0.4, kb)
+    B[1000:200000] = A[50000]   # a hot key with a short bin
+    B[300000:300040] = A[10]    # a few of the long bin
+    off, csr = hg.build(_to_dev(A, dev), n)
+    _probe_equal(hg, off, csr, n, A, B, dev)
+
+
+def test_narrow_probe_learned(dev):
+    import torch
+    import hashgraph_amd as hg
+    n, M = 1500007, 1400003
+    A = wl.lognormal_keys(51, n, device=dev)
+    B = wl.mixed_probe(A, wl.lognormal_keys(52, n, device=dev), 53, 0.5)
+    model, _ = hg.rmi_train(A, M, seed=2)
+    kw = {"hash_kind": hg.HG_HASH_RMI, "rmi_model": model}
+    cnt, out = hg.probe(*hg.build(A, M, **kw), M, B, **kw)
+    ecnt, eout = hg.probe(*hg.build(A, M), M, B)
+    assert cnt == ecnt and torch.equal(torch.sort(out).values, torch.sort(eout).values)
