@@ -998,103 +998,30 @@ __global__ __launch_bounds__(1024) void k_range_hist(const K *__restrict__ keys,
 
 // ---------------------------------------------------------------------------
 // Run-length join of two built tables: one record (key, cA, cB) per value
-// present in both tables.  Small bins (|A_b|, |B_b| <= RLE_SMALL) are done by
-// one thread each (quadratic in the bin, in bin order); a bin above that is
-// appended to a heavy list and handled by k_rle_heavy.
-// A workgroup takes a chunk of RLE_CHUNK bins: both sides' offsets, and their
-// keys when the chunk holds at most RLE_KCAP keys per side (no heavy bin),
-// are read coalesced into LDS first; thread t then walks bins t*PER.. there.
-// Pass 0 counts records per chunk, pass 1 writes them at the chunk's
-// exclusive prefix.
+// present in both tables.  Bins with at most RLE_SMALL keys a side are done
+// here; a bin above that is appended to a heavy list and handled by
+// k_rle_heavy.
+// A workgroup takes a chunk of RLE_CHUNK bins.  The keys of its light bins
+// (both sides present, neither above RLE_SMALL) are packed into LDS, in rounds
+// of whole bins when they exceed RLE_KCAP a side: a heavy bin among them costs
+// nothing.  Then every key of A is one thread's: it looks for an earlier copy
+// in its bin, counts the later ones and B's, and holds a record if it is the
+// first and B has it.  Records leave in bin order through one block scan.
+// The kernel is bound by the latency of these LDS walks: at most 128 reads a
+// key, spread over all threads (one thread a bin took up to |A_b| (|A_b| +
+// |B_b|) of them, and a chunk with a heavy bin walked global memory: 97 us for
+// 2 M Zipf(1.1) uint64 keys against 1 M, 37 us now).
+// Pass 0 counts the chunk's records, heavy bins and pairs (plain stores: one
+// atomic per chunk on a shared counter would serialise the grid); pass 1, after
+// the first two were scanned, lists the heavy bins and, when emit, writes the
+// records at the chunk's prefixes; pass 3 does both at padded bases.
 // ---------------------------------------------------------------------------
 constexpr uint32_t RLE_SMALL = 64;
-constexpr uint32_t RLE_CHUNK = 1024;
-constexpr uint32_t RLE_KCAP = 768;
-constexpr uint32_t RLE_TINY = 8;  // bins above this on a side (up to RLE_SMALL) are walked by a wave
+constexpr uint32_t RLE_CHUNK = 512;
+constexpr uint32_t RLE_KCAP = 1024;
 
-// A medium bin (A's keys a0.., a of them; B's x0.., b of them; a, b <= 64)
-// walked by one wave: lane i takes A's i-th key and counts its copies on both
-// sides by broadcast reads; it holds a record if the key occurs first at i
-// and B has it.
-template <typename K, typename GA, typename GB>
-__device__ __forceinline__ bool rle_medium(uint64_t a0, uint32_t a, uint64_t x0, uint32_t b, GA getA, GB getB,
-                                           uint32_t lane, K &v, uint32_t &ca, uint32_t &cb) {
-  const bool mine = lane < a;
-  v = getA(a0 + (mine ? lane : 0u));
-  ca = 0;
-  cb = 0;
-  bool first = true;
-  for (uint32_t j = 0; j < a; j++) {
-    const bool eq = getA(a0 + j) == v;
-    ca += eq ? 1u : 0u;
-    first &= !(eq && j < lane);
-  }
-  for (uint32_t j = 0; j < b; j++) cb += getB(x0 + j) == v ? 1u : 0u;
-  return mine && first && cb > 0;
-}
-
-// A thread's walk over its PER bins of the chunk.  WRITE == false counts the
-// tiny bins' records and pairs, the heavy bins, and marks the medium bins in
-// medmask; WRITE == true lists the heavy bins from hw on and writes the tiny
-// bins' records from w on.  Without emit only the heavy bins are looked at.
-template <typename K, int PER, bool WRITE, typename OFF, typename GA, typename GB>
-__device__ __forceinline__ void rle_walk(const OFF *s_oa, const OFF *s_ob, uint32_t lo, uint32_t hi, bool emit,
-                                         GA getA, GB getB,
-                                         uint64_t b0, uint32_t &nrec, unsigned long long &npair, uint32_t &nheavy,
-                                         uint32_t &medmask, unsigned long long w, uint64_t hw, uint32_t *heavy,
-                                         uint64_t heavy_cap, K *rk, unsigned long long *rca, unsigned long long *rcb,
-                                         uint64_t capacity) {
-  for (int q = 0; q < PER; q++) {
-    const uint32_t l = threadIdx.x * PER + q;
-    if (l >= hi) break;
-    if (l < lo) continue;
-    const uint64_t a0 = s_oa[l], a1 = s_oa[l + 1], x0 = s_ob[l], x1 = s_ob[l + 1];
-    if (a1 == a0 || x1 == x0) continue;
-    if (a1 - a0 > RLE_SMALL || x1 - x0 > RLE_SMALL) {
-      if (WRITE) {
-        if (hw < heavy_cap) heavy[hw] = (uint32_t)(b0 + l);
-        hw++;
-      } else {
-        nheavy++;
-      }
-      continue;
-    }
-    if (!emit) continue;
-    if (a1 - a0 > RLE_TINY || x1 - x0 > RLE_TINY) {  // a wave takes it (rle_medium)
-      if (!WRITE) medmask |= 1u << q;
-      continue;
-    }
-    for (uint64_t i = a0; i < a1; i++) {
-      const K v = getA(i);
-      bool first = true;
-      for (uint64_t j = a0; j < i; j++) first &= getA(j) != v;
-      if (!first) continue;
-      unsigned long long ca = 0, cb = 0;
-      for (uint64_t j = i; j < a1; j++) ca += getA(j) == v;
-      for (uint64_t j = x0; j < x1; j++) cb += getB(j) == v;
-      if (!cb) continue;
-      if (!WRITE) {
-        nrec++;
-        npair += ca * cb;
-      } else {
-        if (w < capacity) {
-          rk[w] = v;
-          rca[w] = ca;
-          rcb[w] = cb;
-        }
-        w++;
-      }
-    }
-  }
-}
-
-// Pass 0 stores per chunk its record count, heavy-bin count and pair count
-// (plain stores: one atomic per chunk on a shared counter would serialise the
-// whole grid); pass 1, after the host scanned the first two, lists the heavy
-// bins at the chunk's heavy prefix and, when emit, writes the records at the
-// chunk's record prefix.  Pass 1 without emit only lists the heavy bins.
 template <typename K, typename OFF, int BLOCK>
-__global__ __launch_bounds__(BLOCK, 6) void k_rle_small(const OFF *__restrict__ offA, const K *__restrict__ keysA,
+__global__ __launch_bounds__(BLOCK, 5) void k_rle_small(const OFF *__restrict__ offA, const K *__restrict__ keysA,
                                                      const OFF *__restrict__ offB, const K *__restrict__ keysB, uint64_t M,
                                                      int pass, unsigned long long *__restrict__ chunk_cnt,
                                                      const unsigned long long *__restrict__ chunk_base,
@@ -1104,11 +1031,14 @@ __global__ __launch_bounds__(BLOCK, 6) void k_rle_small(const OFF *__restrict__ 
                                                      unsigned long long *__restrict__ rca,
                                                      unsigned long long *__restrict__ rcb, uint64_t capacity,
                                                      uint32_t *__restrict__ heavy, uint64_t heavy_cap) {
-  constexpr int PER = RLE_CHUNK / BLOCK;
-  constexpr int KPT = RLE_KCAP / BLOCK;
+  constexpr uint32_t PER = RLE_CHUNK / BLOCK;
+  constexpr uint32_t KPT = RLE_KCAP / BLOCK;
   __shared__ unsigned long long s_t64[BLOCK / 64 + 1];
   __shared__ OFF s_oa[RLE_CHUNK + 1], s_ob[RLE_CHUNK + 1];
+  __shared__ uint16_t s_pa[RLE_CHUNK + 1], s_pb[RLE_CHUNK + 1];  // light keys before the bin (<= 64 * 512)
   __shared__ K s_ka[RLE_KCAP], s_kb[RLE_KCAP];
+  __shared__ uint16_t s_ba[RLE_KCAP], s_bb[RLE_KCAP];  // bin of each packed key
+  __shared__ uint32_t s_hi;
   const uint64_t b0 = (uint64_t)blockIdx.x * RLE_CHUNK;
   const uint32_t nb = (uint32_t)min((uint64_t)RLE_CHUNK, M - b0);
   const bool emit = pass != 1 || capacity != 0;
@@ -1116,7 +1046,7 @@ __global__ __launch_bounds__(BLOCK, 6) void k_rle_small(const OFF *__restrict__ 
     // all offset loads of the thread in flight together (one round trip)
     OFF va[PER + 1], vb[PER + 1];
 #pragma unroll
-    for (int j = 0; j <= PER; j++) {
+    for (uint32_t j = 0; j <= PER; j++) {
       const uint32_t i = threadIdx.x + j * BLOCK;
       if (i <= nb) {
         va[j] = offA[b0 + i];
@@ -1124,7 +1054,7 @@ __global__ __launch_bounds__(BLOCK, 6) void k_rle_small(const OFF *__restrict__ 
       }
     }
 #pragma unroll
-    for (int j = 0; j <= PER; j++) {
+    for (uint32_t j = 0; j <= PER; j++) {
       const uint32_t i = threadIdx.x + j * BLOCK;
       if (i <= nb) {
         s_oa[i] = va[j];
@@ -1133,173 +1063,154 @@ __global__ __launch_bounds__(BLOCK, 6) void k_rle_small(const OFF *__restrict__ 
     }
   }
   __syncthreads();
-  // Sub-ranges: a chunk whose keys exceed RLE_KCAP on a side is walked in
-  // 2 or 4 sub-ranges of bins, each staged on its own (dense tables); when
-  // none fits, in one range reading the keys from global memory.
-  uint32_t nsub = 1;
-  bool staged = false;
-  if (emit) {
-    for (uint32_t ns = 1; ns <= 4 && !staged; ns <<= 1) {
-      const uint32_t span = RLE_CHUNK / ns;
-      bool fits = true;
-      for (uint32_t r = 0; r < ns && r * span < nb; r++) {
-        const uint32_t lo = r * span, hi = min(lo + span, nb);
-        fits &= (uint64_t)s_oa[hi] - (uint64_t)s_oa[lo] <= RLE_KCAP && (uint64_t)s_ob[hi] - (uint64_t)s_ob[lo] <= RLE_KCAP;
-      }
-      if (fits) {
-        nsub = ns;
-        staged = true;
-      }
-    }
-  }
-  // list of the medium bins (thread order: deterministic)
-  __shared__ uint16_t s_med[RLE_CHUNK];
-  __shared__ uint16_t s_mcnt[RLE_CHUNK];  // records of a medium bin, then its base in the sub-range (< 2^16)
-  __shared__ unsigned long long s_mbase;
-  __shared__ uint32_t s_mtot;
-  const uint32_t lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  constexpr uint32_t NW = BLOCK / 64;
-  // pass 0: the chunk's totals (records | heavy << 32, pairs); passes 1
-  // and 3: the records and heavy bins written so far (pass 3 also sums the
-  // pairs)
-  unsigned long long acc = 0, accp = 0;
-  const unsigned long long cbase = pass == 0 ? 0ull : chunk_base[blockIdx.x];
-  const uint64_t hbase = pass == 0 ? 0ull : (uint64_t)heavy_base[blockIdx.x];
-  const uint32_t span = RLE_CHUNK / nsub;
-  for (uint32_t r = 0; r < nsub; r++) {
-    const uint32_t lo = r * span, hi = min(lo + span, nb);
-    if (lo >= nb) break;  // uniform
-    const uint64_t ka0 = uni64(s_oa[lo]), kb0 = uni64(s_ob[lo]);
-    const uint64_t na = uni64((uint64_t)s_oa[hi] - ka0), nx = uni64((uint64_t)s_ob[hi] - kb0);
-    if (staged) {
-      if (r) __syncthreads();  // the previous sub-range is done with s_ka / s_kb
-      K ta[KPT], tb[KPT];
+  // this thread's bins l0 .. l0 + PER - 1: keys of the light ones, heavy ones
+  const uint32_t l0 = threadIdx.x * PER;
+  uint32_t la[PER], lb[PER], hm = 0;
+  unsigned long long sum = 0;  // light keys of A | of B << 20 | heavy bins << 40
 #pragma unroll
-      for (int j = 0; j < KPT; j++) {
-        const uint32_t i = threadIdx.x + j * BLOCK;
-        if (i < na) ta[j] = keysA[ka0 + i];
-        if (i < nx) tb[j] = keysB[kb0 + i];
-      }
-#pragma unroll
-      for (int j = 0; j < KPT; j++) {
-        const uint32_t i = threadIdx.x + j * BLOCK;
-        if (i < na) s_ka[i] = ta[j];
-        if (i < nx) s_kb[i] = tb[j];
-      }
-      __syncthreads();
-    }
-    auto lA = [&](uint64_t i) { return s_ka[i - ka0]; };
-    auto lB = [&](uint64_t i) { return s_kb[i - kb0]; };
-    auto gA = [&](uint64_t i) { return keysA[i]; };
-    auto gB = [&](uint64_t i) { return keysB[i]; };
-    uint32_t nrec = 0, nheavy = 0, medmask = 0;
-    unsigned long long npair = 0;
-    if (staged)
-      rle_walk<K, PER, false>(s_oa, s_ob, lo, hi, emit, lA, lB, b0, nrec, npair, nheavy, medmask, 0ull, 0ull, heavy, 0,
-                              rk, rca, rcb, 0);
-    else
-      rle_walk<K, PER, false>(s_oa, s_ob, lo, hi, emit, gA, gB, b0, nrec, npair, nheavy, medmask, 0ull, 0ull, heavy, 0,
-                              rk, rca, rcb, 0);
-    unsigned long long nmed_tot;
-    const unsigned long long mex = block_exclusive_sum<BLOCK, unsigned long long>(
-        (unsigned long long)__popc(medmask), s_t64, nmed_tot);
-    {
-      uint32_t k = (uint32_t)mex;
-      for (int q = 0; q < PER; q++)
-        if (medmask & (1u << q)) s_med[k++] = (uint16_t)(threadIdx.x * PER + q);
-    }
-    __syncthreads();
-    const uint32_t nmed = uni32((uint32_t)nmed_tot);
-    // medium bins: one wave each
-    uint32_t mrec = 0;
-    unsigned long long mpair = 0;
-    if (pass == 0)
-      for (uint32_t k = wv; k < nmed; k += NW) {
-        const uint32_t l = s_med[k];
-        const uint64_t a0 = s_oa[l], x0 = s_ob[l];
-        const uint32_t a = (uint32_t)((uint64_t)s_oa[l + 1] - a0), b = (uint32_t)((uint64_t)s_ob[l + 1] - x0);
-        K v;
-        uint32_t ca, cb;
-        const bool rec = staged ? rle_medium<K>(a0, a, x0, b, lA, lB, lane, v, ca, cb)
-                                : rle_medium<K>(a0, a, x0, b, gA, gB, lane, v, ca, cb);
-        mrec += rec ? 1u : 0u;
-        mpair += rec ? (unsigned long long)ca * cb : 0ull;
-      }
-    // records in the low word, heavy bins in the high word (a chunk holds at
-    // most 64 K records and 1024 heavy bins)
-    unsigned long long tot;
-    const unsigned long long ex = block_exclusive_sum<BLOCK, unsigned long long>(
-        (unsigned long long)(nrec + mrec) | ((unsigned long long)nheavy << 32), s_t64, tot);
-    if (pass == 0) {
-      acc += uni64(tot);
-      accp += uni64(block_sum<BLOCK, unsigned long long>(npair + mpair, s_t64));
+  for (uint32_t q = 0; q < PER; q++) {
+    la[q] = lb[q] = 0;
+    const uint32_t l = l0 + q;
+    if (l >= nb) continue;
+    const uint64_t a = (uint64_t)(s_oa[l + 1] - s_oa[l]), b = (uint64_t)(s_ob[l + 1] - s_ob[l]);
+    if (a == 0 || b == 0) continue;
+    if (a > RLE_SMALL || b > RLE_SMALL) {
+      hm |= 1u << q;
       continue;
     }
-    if (pass == 3) accp += uni64(block_sum<BLOCK, unsigned long long>(npair, s_t64));  // the tiny bins' pairs
-    // pass 1: the tiny bins' records at the sub-range's base plus the threads
-    // before, then the medium bins' records after all of them
-    const unsigned long long rbase = cbase + (acc & 0xFFFFFFFFull);
-    const uint64_t hw = hbase + (acc >> 32) + (ex >> 32);
-    if (staged)
-      rle_walk<K, PER, true>(s_oa, s_ob, lo, hi, emit, lA, lB, b0, nrec, npair, nheavy, medmask,
-                             rbase + (ex & 0xFFFFFFFFull), hw, heavy, heavy_cap, rk, rca, rcb, capacity);
-    else
-      rle_walk<K, PER, true>(s_oa, s_ob, lo, hi, emit, gA, gB, b0, nrec, npair, nheavy, medmask,
-                             rbase + (ex & 0xFFFFFFFFull), hw, heavy, heavy_cap, rk, rca, rcb, capacity);
-    acc += uni64(tot);  // tiny records and heavy bins of the sub-range
-    if (nmed == 0) continue;  // uniform
-    // medium bins: count each bin's records, then the bins' bases in bin order
-    for (uint32_t k = wv; k < nmed; k += NW) {
-      const uint32_t l = s_med[k];
-      const uint64_t a0 = s_oa[l], x0 = s_ob[l];
-      const uint32_t a = (uint32_t)((uint64_t)s_oa[l + 1] - a0), b = (uint32_t)((uint64_t)s_ob[l + 1] - x0);
-      K v;
-      uint32_t ca, cb;
-      const bool rec = staged ? rle_medium<K>(a0, a, x0, b, lA, lB, lane, v, ca, cb)
-                              : rle_medium<K>(a0, a, x0, b, gA, gB, lane, v, ca, cb);
-      const uint64_t bal = __ballot(rec);
-      if (lane == 0) s_mcnt[k] = (uint16_t)__popcll(bal);
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      uint32_t m = 0;
-      for (uint32_t k = 0; k < nmed; k++) {  // record base of each medium bin past the tiny bins' records
-        const uint32_t c = s_mcnt[k];
-        s_mcnt[k] = (uint16_t)m;
-        m += c;
-      }
-      s_mbase = cbase + (acc & 0xFFFFFFFFull);
-      s_mtot = m;
-    }
-    __syncthreads();
-    const unsigned long long mb = uni64(s_mbase);
-    acc += uni32(s_mtot);  // the medium bins' records
-    unsigned long long mp = 0;  // pass 3: the medium bins' pairs
-    for (uint32_t k = wv; k < nmed; k += NW) {
-      const uint32_t l = s_med[k];
-      const uint64_t a0 = s_oa[l], x0 = s_ob[l];
-      const uint32_t a = (uint32_t)((uint64_t)s_oa[l + 1] - a0), b = (uint32_t)((uint64_t)s_ob[l + 1] - x0);
-      K v;
-      uint32_t ca, cb;
-      const bool rec = staged ? rle_medium<K>(a0, a, x0, b, lA, lB, lane, v, ca, cb)
-                              : rle_medium<K>(a0, a, x0, b, gA, gB, lane, v, ca, cb);
-      const uint64_t bal = __ballot(rec);
-      if (rec) {
-        const unsigned long long p = mb + s_mcnt[k] + (unsigned long long)__popcll(bal & ((1ull << lane) - 1ull));
-        if (p < capacity) {
-          rk[p] = v;
-          rca[p] = ca;
-          rcb[p] = cb;
-        }
-        mp += (unsigned long long)ca * cb;
-      }
-    }
-    if (pass == 3) accp += uni64(block_sum<BLOCK, unsigned long long>(mp, s_t64));
+    la[q] = (uint32_t)a;
+    lb[q] = (uint32_t)b;
+    sum += a | (b << 20);
   }
-  if ((pass == 0 || pass == 3) && threadIdx.x == 0) {
-    chunk_cnt[blockIdx.x] = acc & 0xFFFFFFFFull;
-    chunk_heavy[blockIdx.x] = (uint32_t)(acc >> 32);
-    chunk_pairs[blockIdx.x] = accp;
+  sum += (unsigned long long)__popc(hm) << 40;
+  unsigned long long tot;
+  const unsigned long long ex = block_exclusive_sum<BLOCK, unsigned long long>(sum, s_t64, tot);
+  {
+    uint32_t pa = (uint32_t)ex & 0xFFFFFu, pb = (uint32_t)(ex >> 20) & 0xFFFFFu;
+#pragma unroll
+    for (uint32_t q = 0; q < PER; q++) {
+      if (l0 + q <= nb) {
+        s_pa[l0 + q] = (uint16_t)pa;
+        s_pb[l0 + q] = (uint16_t)pb;
+      }
+      pa += la[q];
+      pb += lb[q];
+    }
+    if (threadIdx.x == BLOCK - 1 && nb == RLE_CHUNK) {
+      s_pa[RLE_CHUNK] = (uint16_t)pa;
+      s_pb[RLE_CHUNK] = (uint16_t)pb;
+    }
+  }
+  if (pass != 0 && hm) {
+    uint64_t hw = (uint64_t)heavy_base[blockIdx.x] + (ex >> 40);
+#pragma unroll
+    for (uint32_t q = 0; q < PER; q++)
+      if ((hm >> q) & 1u) {
+        if (hw < heavy_cap) heavy[hw] = (uint32_t)(b0 + l0 + q);
+        hw++;
+      }
+  }
+  const uint32_t ta = uni32((uint32_t)tot & 0xFFFFFu), tb = uni32((uint32_t)(tot >> 20) & 0xFFFFFu);
+  const unsigned long long cbase = pass == 0 ? 0ull : chunk_base[blockIdx.x];
+  uint32_t nrec = 0;             // records of the rounds so far
+  unsigned long long pairs = 0;  // this thread's pairs
+  __syncthreads();
+  for (uint32_t lo = 0, ka0 = 0, kb0 = 0; emit && ka0 < ta;) {
+    // bins [lo, hi): as many whole bins as fit
+    uint32_t hi = nb;
+    if (ta - ka0 > RLE_KCAP || tb - kb0 > RLE_KCAP) {
+      if (threadIdx.x == 0) s_hi = lo + 1;
+      __syncthreads();
+      uint32_t h = lo + 1;
+#pragma unroll
+      for (uint32_t q = 0; q < PER; q++) {
+        const uint32_t l = l0 + q + 1;
+        if (l > lo && l <= nb && s_pa[l] - ka0 <= RLE_KCAP && s_pb[l] - kb0 <= RLE_KCAP) h = max(h, l);
+      }
+      if (h > lo + 1) atomicMax(&s_hi, h);
+      __syncthreads();
+      hi = uni32(s_hi);
+    }
+    const uint32_t na = uni32(s_pa[hi] - ka0), nx = uni32(s_pb[hi] - kb0);
+#pragma unroll
+    for (uint32_t q = 0; q < PER; q++) {
+      const uint32_t l = l0 + q;
+      if (l < lo || l >= hi) continue;
+      for (uint32_t i = 0; i < la[q]; i++) s_ba[s_pa[l] - ka0 + i] = (uint16_t)l;
+      for (uint32_t i = 0; i < lb[q]; i++) s_bb[s_pb[l] - kb0 + i] = (uint16_t)l;
+    }
+    __syncthreads();
+    {
+      K va[KPT], vb[KPT];
+#pragma unroll
+      for (uint32_t j = 0; j < KPT; j++) {
+        const uint32_t i = threadIdx.x + j * BLOCK;
+        if (i < na) {
+          const uint32_t l = s_ba[i];
+          va[j] = keysA[s_oa[l] + (i + ka0 - s_pa[l])];
+        }
+        if (i < nx) {
+          const uint32_t l = s_bb[i];
+          vb[j] = keysB[s_ob[l] + (i + kb0 - s_pb[l])];
+        }
+      }
+#pragma unroll
+      for (uint32_t j = 0; j < KPT; j++) {
+        const uint32_t i = threadIdx.x + j * BLOCK;
+        if (i < na) s_ka[i] = va[j];
+        if (i < nx) s_kb[i] = vb[j];
+      }
+    }
+    __syncthreads();
+    // this thread's keys of A (neighbours, so that records keep bin order)
+    const uint32_t per = (na + BLOCK - 1) / BLOCK;
+    uint32_t rec[KPT], mine = 0;  // cA | cB << 16 of a record, 0 otherwise
+#pragma unroll
+    for (uint32_t u = 0; u < KPT; u++) {
+      rec[u] = 0;
+      const uint32_t i = threadIdx.x * per + u;
+      if (u >= per || i >= na) continue;
+      const K v = s_ka[i];
+      const uint32_t l = s_ba[i];
+      uint32_t j = s_pa[l] - ka0;
+      while (j < i && s_ka[j] != v) j++;
+      if (j < i) continue;  // not the value's first key
+      uint32_t cb = 0;
+      for (uint32_t x = s_pb[l] - kb0, e = s_pb[l + 1] - kb0; x < e; x++) cb += s_kb[x] == v ? 1u : 0u;
+      if (!cb) continue;
+      uint32_t ca = 1;
+      for (uint32_t x = i + 1, e = s_pa[l + 1] - ka0; x < e; x++) ca += s_ka[x] == v ? 1u : 0u;
+      rec[u] = ca | (cb << 16);
+      pairs += ca * cb;
+      mine++;
+    }
+    unsigned long long rt;
+    unsigned long long w = block_exclusive_sum<BLOCK, unsigned long long>(mine, s_t64, rt) + cbase + nrec;
+    nrec += uni32((uint32_t)rt);
+    if (pass != 0) {
+#pragma unroll
+      for (uint32_t u = 0; u < KPT; u++) {
+        if (!rec[u]) continue;
+        if (w < capacity) {
+          rk[w] = s_ka[threadIdx.x * per + u];
+          rca[w] = rec[u] & 0xFFFFu;
+          rcb[w] = rec[u] >> 16;
+        }
+        w++;
+      }
+    }
+    ka0 += na;
+    kb0 += nx;
+    lo = hi;
+    __syncthreads();  // the next round overwrites the packed keys
+  }
+  if (pass == 0 || pass == 3) {
+    pairs = block_sum<BLOCK, unsigned long long>(pairs, s_t64);
+    if (threadIdx.x == 0) {
+      chunk_cnt[blockIdx.x] = nrec;
+      chunk_heavy[blockIdx.x] = (uint32_t)(tot >> 40);
+      chunk_pairs[blockIdx.x] = pairs;
+    }
   }
 }
 
