@@ -1932,81 +1932,104 @@ hg_status hg_intersect_rle(hg_ctx c, const hg_table_desc *descA, const void *d_o
     r.gcb = r.gca + rle_giant_slots();
   }
   void *status = cv.get<void>(i_status);
-  unsigned long long nsmall = 0;
-  uint32_t nheavy = 0;
   // With an output, one pass of the small-bin kernel counts and writes the
   // records and heavy bins at padded places bounded from the offsets alone,
   // and a gather packs them; without one (or when the padded records would
   // take more than kRleOnePassBytes) a count pass sizes the output first.
+  // What the host needs to know of the chunks stays on the device: their
+  // totals size the heavy bins' kernels there, and the call reads back once.
   bool one_pass = false;
   unsigned long long *pbase = cv.get<unsigned long long>(i_pbase);
   uint32_t *phbase = cv.get<uint32_t>(i_phbase);
-  unsigned long long s_rec = 0;
-  uint32_t s_heavy = 0;
+  uint64_t s_rec = 0, s_heavy = 0;
+  LaunchRleScan sc{};
+  sc.n = nch;
   if (capacity) {
     HG_HIP(launch_rle_caps(d_offA, d_offB, r.off_bytes, M, cv.get<unsigned long long>(i_caprec),
                            cv.get<uint32_t>(i_caph), c->stream));
-    HG_HIP(launch_scan(cv.get<unsigned long long>(i_caprec), (void *)pbase, nch, 8, status, c->stream));
-    HG_HIP(launch_scan(cv.get<uint32_t>(i_caph), (void *)phbase, nch, 4, status, c->stream));
-    HG_TRY(sync_read(c, &s_rec, pbase + nch, 8));
-    HG_TRY(sync_read(c, &s_heavy, phbase + nch, 4));
-    one_pass = (double)s_rec * (descA->key_bytes + 16) + (double)s_heavy * 4 <= (double)kRleOnePassBytes;
-  }
-  if (one_pass) {
+    sc.in64 = cv.get<unsigned long long>(i_caprec);
+    sc.out64 = pbase;
+    sc.in32 = cv.get<uint32_t>(i_caph);
+    sc.out32 = phbase;
+    HG_HIP(launch_rle_scan(sc, status, c->stream));
+    // the chunks' bounds add up to at most one record per key of the smaller
+    // side; only when that is too much are the sums themselves read back
+    const auto fits = [&] {
+      return (double)s_rec * (descA->key_bytes + 16) + (double)s_heavy * 4 <= (double)kRleOnePassBytes;
+    };
     Plan P0;
-    const size_t j_rk = P0.add(std::max<uint64_t>(s_rec, 1) * descA->key_bytes),
-                 j_ca = P0.add(std::max<uint64_t>(s_rec, 1) * 8), j_cb = P0.add(std::max<uint64_t>(s_rec, 1) * 8),
-                 j_h = P0.add(((uint64_t)s_heavy + 1) * 4);
-    HG_TRY(arena_ensure(c, 0, P0.total()));
-    Carve cv0;
-    cv0.init(c, 0, P0);
-    LaunchRle r3 = r;
-    r3.pass = 3;
-    r3.chunk_base = pbase;
-    r3.heavy_base = phbase;
-    r3.rk = cv0.get<void>(j_rk);
-    r3.rca = cv0.get<unsigned long long>(j_ca);
-    r3.rcb = cv0.get<unsigned long long>(j_cb);
-    r3.capacity = s_rec;
-    r3.heavy = cv0.get<uint32_t>(j_h);
-    r3.heavy_cap = s_heavy;
-    {
-      Prof pf(c, "rle_small");
-      HG_HIP(launch_rle(r3, c->stream));
+    const auto layout = [&] {
+      P0.sizes.clear();
+      P0.add(std::max<uint64_t>(s_rec, 1) * descA->key_bytes);
+      P0.add(std::max<uint64_t>(s_rec, 1) * 8);
+      P0.add(std::max<uint64_t>(s_rec, 1) * 8);
+      P0.add((s_heavy + 1) * 4);
+      return P0.total();
+    };
+    s_rec = std::min(descA->n_keys, descB->n_keys);
+    s_heavy = heavy_cap;
+    one_pass = fits() && arena_ensure(c, 0, layout()) == HG_OK;
+    if (!one_pass) {
+      unsigned long long sr = 0;
+      uint32_t sh = 0;
+      HG_TRY(sync_read(c, &sr, pbase + nch, 8));
+      HG_TRY(sync_read(c, &sh, phbase + nch, 4));
+      s_rec = sr;
+      s_heavy = sh;
+      one_pass = fits();
+      if (one_pass) HG_TRY(arena_ensure(c, 0, layout()));
     }
-    HG_HIP(launch_scan(r.chunk_cnt, (void *)r.chunk_base, nch, 8, status, c->stream));
-    HG_HIP(launch_scan(r.chunk_heavy, (void *)r.heavy_base, nch, 4, status, c->stream));
-    LaunchRleGather gt{};
-    gt.key_bytes = r.key_bytes;
-    gt.nch = (uint32_t)nch;
-    gt.pbase = pbase;
-    gt.cbase = r.chunk_base;
-    gt.cnt = r.chunk_cnt;
-    gt.srk = r3.rk;
-    gt.srca = r3.rca;
-    gt.srcb = r3.rcb;
-    gt.rk = r.rk;
-    gt.rca = r.rca;
-    gt.rcb = r.rcb;
-    gt.capacity = capacity;
-    gt.phbase = phbase;
-    gt.hbase = r.heavy_base;
-    gt.hcnt = r.chunk_heavy;
-    gt.sheavy = r3.heavy;
-    gt.heavy = r.heavy;
-    gt.heavy_cap = heavy_cap;
-    gt.bad = (unsigned int *)(small + 5);
-    {
+    if (one_pass) {
+      Carve cv0;
+      cv0.init(c, 0, P0);
+      LaunchRle r3 = r;
+      r3.pass = 3;
+      r3.chunk_base = pbase;
+      r3.heavy_base = phbase;
+      r3.rk = cv0.get<void>(0);
+      r3.rca = cv0.get<unsigned long long>(1);
+      r3.rcb = cv0.get<unsigned long long>(2);
+      r3.capacity = s_rec;
+      r3.heavy = cv0.get<uint32_t>(3);
+      r3.heavy_cap = s_heavy;
+      {
+        Prof pf(c, "rle_small");
+        HG_HIP(launch_rle(r3, c->stream));
+      }
+      LaunchRleGather gt{};
+      gt.key_bytes = r.key_bytes;
+      gt.nch = (uint32_t)nch;
+      gt.pbase = pbase;
+      gt.cbase = r.chunk_base;
+      gt.cnt = r.chunk_cnt;
+      gt.srk = r3.rk;
+      gt.srca = r3.rca;
+      gt.srcb = r3.rcb;
+      gt.rk = r.rk;
+      gt.rca = r.rca;
+      gt.rcb = r.rcb;
+      gt.capacity = capacity;
+      gt.phbase = phbase;
+      gt.hbase = r.heavy_base;
+      gt.hcnt = r.chunk_heavy;
+      gt.sheavy = r3.heavy;
+      gt.heavy = r.heavy;
+      gt.heavy_cap = heavy_cap;
+      gt.bad = (unsigned int *)(small + 5);
+      sc.in64 = r.chunk_cnt;
+      sc.out64 = (unsigned long long *)r.chunk_base;
+      sc.in32 = r.chunk_heavy;
+      sc.out32 = (uint32_t *)r.heavy_base;
+      sc.add = r.chunk_pairs;
+      sc.acc = r.pairs;
+      sc.zero = (uint32_t *)r.gctl;
+      sc.nzero = RLE_GIANT_ZERO;
+      HG_HIP(launch_rle_scan(sc, status, c->stream));
       Prof pf(c, "rle_gather");
       HG_HIP(launch_rle_gather(gt, c->stream));
     }
-    HG_TRY(sync_read(c, &nsmall, r.chunk_base + nch, 8));
-    HG_TRY(sync_read(c, &nheavy, r.heavy_base + nch, 4));
-    unsigned int bad = 0;
-    HG_TRY(sync_read(c, &bad, small + 5, 4));
-    if (bad) return fail(HG_ERR_DEVICE, "a chunk of the run-length join exceeded its bound");
-    if (nheavy > heavy_cap) return fail(HG_ERR_DEVICE, "heavy bins exceed their bound");
-  } else {
+  }
+  if (!one_pass) {
     r.pass = 0;
     {
       Prof pf(c, "rle_small");
@@ -2014,11 +2037,15 @@ hg_status hg_intersect_rle(hg_ctx c, const hg_table_desc *descA, const void *d_o
     }
     // record positions of the small bins and heavy-list positions: exclusive
     // scans of the chunk counts
-    HG_HIP(launch_scan(r.chunk_cnt, (void *)r.chunk_base, nch, 8, status, c->stream));
-    HG_HIP(launch_scan(r.chunk_heavy, (void *)r.heavy_base, nch, 4, status, c->stream));
-    HG_TRY(sync_read(c, &nsmall, r.chunk_base + nch, 8));
-    HG_TRY(sync_read(c, &nheavy, r.heavy_base + nch, 4));
-    if (nheavy > heavy_cap) return fail(HG_ERR_DEVICE, "heavy bins exceed their bound");
+    sc.in64 = r.chunk_cnt;
+    sc.out64 = (unsigned long long *)r.chunk_base;
+    sc.in32 = r.chunk_heavy;
+    sc.out32 = (uint32_t *)r.heavy_base;
+    sc.add = r.chunk_pairs;
+    sc.acc = r.pairs;
+    sc.zero = (uint32_t *)r.gctl;
+    sc.nzero = RLE_GIANT_ZERO;
+    HG_HIP(launch_rle_scan(sc, status, c->stream));
     // pass 1 lists the heavy bins and, with a capacity, writes the records
     r.pass = 1;
     {
@@ -2027,15 +2054,18 @@ hg_status hg_intersect_rle(hg_ctx c, const hg_table_desc *descA, const void *d_o
     }
   }
   // heavy bins append after the small bins' records
-  HG_HIP(launch_fill_u64(small + 2, nsmall, 1, c->stream));
   r.pass = 2;
-  r.nheavy = nheavy;
+  r.nheavy = r.heavy_base + nch;
+  r.nsmall = r.chunk_base + nch;
+  r.heavy_seen = small + 6;
   {
     Prof pf(c, "rle_heavy");
     HG_HIP(launch_rle(r, c->stream));
   }
-  unsigned long long res[5];
-  HG_TRY(sync_read(c, res, small, 40));
+  unsigned long long res[7];
+  HG_TRY(sync_read(c, res, small, sizeof(res)));
+  if (res[5] & 0xFFFFFFFFull) return fail(HG_ERR_DEVICE, "a chunk of the run-length join exceeded its bound");
+  if (res[6] > heavy_cap) return fail(HG_ERR_DEVICE, "heavy bins exceed their bound");
   if (res[3] & 0xFFFFFFFFull) return fail(HG_ERR_UNSUPPORTED, "a heavy bin holds 2^32 or more keys on a side");
   const uint64_t novf = res[4] & 0xFFFFFFFFull;
   if (novf > heavy_cap) return fail(HG_ERR_DEVICE, "value-rich bins exceed their bound");

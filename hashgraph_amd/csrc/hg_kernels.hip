@@ -1458,9 +1458,10 @@ __device__ __forceinline__ void wave_append(bool p, uint32_t *ctr, uint32_t *lis
 // to the lists of k_rle_heavy's two forms (lists[0..), lists[heavy_cap..)).
 template <typename OFF>
 __global__ __launch_bounds__(256) void k_giant_mark(const OFF *__restrict__ offA, const OFF *__restrict__ offB,
-                                                    const uint32_t *__restrict__ heavy, uint64_t nheavy,
-                                                    uint32_t *__restrict__ lists, uint64_t heavy_cap,
+                                                    const uint32_t *__restrict__ heavy,
+                                                    const uint32_t *__restrict__ heavy_n, uint32_t *__restrict__ lists, uint64_t heavy_cap,
                                                     GiantCtl *__restrict__ ctl) {
+  const uint64_t nheavy = min((uint64_t)*heavy_n, heavy_cap);
   for (uint64_t h = (uint64_t)blockIdx.x * 256 + threadIdx.x; h < nheavy; h += (uint64_t)gridDim.x * 256) {
     const uint32_t b = heavy[h];
     const uint64_t na = (uint64_t)(offA[b + 1] - offA[b]);
@@ -1480,8 +1481,14 @@ __global__ __launch_bounds__(256) void k_giant_mark(const OFF *__restrict__ offA
 
 template <typename OFF>
 __global__ __launch_bounds__(64) void k_giant_prefix(const OFF *__restrict__ offA, const OFF *__restrict__ offB,
-                                                     const uint32_t *__restrict__ heavy, GiantCtl *__restrict__ ctl) {
+                                                     const uint32_t *__restrict__ heavy, GiantCtl *__restrict__ ctl,
+                                                    const uint32_t *__restrict__ heavy_n,
+                                                    const unsigned long long *__restrict__ nsmall,
+                                                    unsigned long long *__restrict__ cursor,
+                                                    unsigned long long *__restrict__ heavy_seen) {
   if (threadIdx.x != 0) return;
+  *cursor = *nsmall;  // the heavy bins' records follow the small bins'
+  *heavy_seen = *heavy_n;
   const uint32_t n = min(ctl->n, GIANT_CAP);
   uint32_t a = 0, b = 0;
   for (uint32_t s = 0; s < n; s++) {
@@ -1983,6 +1990,55 @@ __global__ __launch_bounds__(1024) void k_sum_add(const unsigned long long *__re
   for (uint64_t i = threadIdx.x; i < n; i += 1024) s += in[i];
   s = block_sum<1024, unsigned long long>(s, s_t64);
   if (threadIdx.x == 0 && s) atomicAdd(acc, s);
+}
+
+// Exclusive scans of the run-length join's chunk arrays by one workgroup each
+// (block 0: in64 -> out64, block 1: in32 -> out32; totals at [n]), and in the
+// same launch the pair sum (block 2: *acc += sum of add) and nzero cleared
+// words.  For up to SCAN_ONE chunks one workgroup's pass is shorter than the
+// look-back scan's two clearing launches and its own.
+constexpr uint64_t SCAN_ONE = 1u << 16;
+template <typename T>
+__device__ void scan_one(const T *__restrict__ in, T *__restrict__ out, uint64_t n) {
+  constexpr int U = 4;
+  __shared__ T s_tmp[1024 / 64 + 1];
+  T run = 0;
+  for (uint64_t i0 = 0; i0 < n; i0 += 1024 * U) {
+    const uint64_t i = i0 + (uint64_t)threadIdx.x * U;
+    T v[U], s = 0;
+#pragma unroll
+    for (int u = 0; u < U; u++) v[u] = i + u < n ? in[i + u] : (T)0;
+#pragma unroll
+    for (int u = 0; u < U; u++) s += v[u];
+    T tot;
+    T ex = run + block_exclusive_sum<1024, T>(s, s_tmp, tot);
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      if (i + u < n) out[i + u] = ex;
+      ex += v[u];
+    }
+    run += tot;
+  }
+  if (threadIdx.x == 0) out[n] = run;
+}
+__global__ __launch_bounds__(1024) void k_rle_scan(const unsigned long long *__restrict__ in64,
+                                                   unsigned long long *__restrict__ out64,
+                                                   const uint32_t *__restrict__ in32, uint32_t *__restrict__ out32,
+                                                   uint64_t n, const unsigned long long *__restrict__ add,
+                                                   unsigned long long *__restrict__ acc, uint32_t *__restrict__ zero,
+                                                   uint32_t nzero) {
+  if (blockIdx.x == 0) {
+    scan_one<unsigned long long>(in64, out64, n);
+  } else if (blockIdx.x == 1) {
+    if (threadIdx.x < nzero) zero[threadIdx.x] = 0;
+    scan_one<uint32_t>(in32, out32, n);
+  } else {
+    __shared__ unsigned long long s_t64[1024 / 64 + 1];
+    unsigned long long s = 0;
+    for (uint64_t i = threadIdx.x; i < n; i += 1024) s += add[i];
+    s = block_sum<1024, unsigned long long>(s, s_t64);
+    if (threadIdx.x == 0 && s) atomicAdd(acc, s);
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -3020,6 +3076,23 @@ __global__ __launch_bounds__(256) void k_rle_gather(LaunchRleGather g) {
   }
 }
 
+hipError_t launch_rle_scan(const LaunchRleScan &p, void *status, hipStream_t st) {
+  const uint32_t blocks = p.add ? 3 : 2;
+  if (p.n <= SCAN_ONE) {
+    hipLaunchKernelGGL(k_rle_scan, dim3(blocks), dim3(1024), 0, st, p.in64, p.out64, p.in32, p.out32, p.n, p.add, p.acc,
+                       p.zero, p.nzero);
+    return hipGetLastError();
+  }
+  hipError_t e = launch_scan(p.in64, p.out64, p.n, 8, status, st);
+  if (e == hipSuccess) e = launch_scan(p.in32, p.out32, p.n, 4, status, st);
+  if (e == hipSuccess && p.nzero) e = launch_fill_u32(p.zero, 0u, p.nzero, st);
+  if (e == hipSuccess && p.add) {
+    hipLaunchKernelGGL(k_sum_add, dim3(1), dim3(1024), 0, st, p.add, p.n, p.acc);
+    e = hipGetLastError();
+  }
+  return e;
+}
+
 hipError_t launch_rle_caps(const void *offA, const void *offB, int off_bytes, uint64_t M,
                            unsigned long long *cap_rec, uint32_t *cap_h, hipStream_t st) {
   const uint32_t nch = (uint32_t)((M + RLE_CHUNK - 1) / RLE_CHUNK);
@@ -3052,19 +3125,17 @@ static hipError_t launch_rle_t(const LaunchRle &r, hipStream_t st) {
                        (const K *)r.keysA, (const OFF *)r.offB, (const K *)r.keysB, r.M, r.pass, r.chunk_cnt,
                        r.chunk_base, r.chunk_heavy, r.heavy_base, r.chunk_pairs, (K *)r.rk, r.rca, r.rcb, r.capacity,
                        r.heavy, r.heavy_cap);
-    if (r.pass == 0 || r.pass == 3)
-      hipLaunchKernelGGL(k_sum_add, dim3(1), dim3(1024), 0, st, (const unsigned long long *)r.chunk_pairs,
-                         (uint64_t)nchunks, r.pairs);
   }
-  if (r.pass == 2 && r.nheavy) {
+  if (r.pass == 2) {
+    // how many heavy bins there are is known on the device only (*nheavy, at
+    // most heavy_cap): grids are sized for heavy_cap and return when it is 0
     GiantCtl *ctl = (GiantCtl *)r.gctl;
-    hipLaunchKernelGGL(k_fill<uint32_t>, dim3(1), dim3(64), 0, st, (uint32_t *)&ctl->n, 0u, (uint64_t)8);
-    hipLaunchKernelGGL((k_giant_mark<OFF>), dim3((uint32_t)std::min<uint64_t>((r.nheavy + 255) / 256, 4096)), dim3(256), 0,
-                       st, (const OFF *)r.offA, (const OFF *)r.offB, (const uint32_t *)r.heavy, r.nheavy, r.gmark,
+    hipLaunchKernelGGL((k_giant_mark<OFF>), dim3((uint32_t)std::min<uint64_t>((r.heavy_cap + 255) / 256, 512)), dim3(256),
+                       0, st, (const OFF *)r.offA, (const OFF *)r.offB, (const uint32_t *)r.heavy, r.nheavy, r.gmark,
                        r.heavy_cap, ctl);
     hipLaunchKernelGGL((k_giant_prefix<OFF>), dim3(1), dim3(64), 0, st, (const OFF *)r.offA, (const OFF *)r.offB,
-                       (const uint32_t *)r.heavy, ctl);
-    hipLaunchKernelGGL((k_giant_clear<K>), dim3(1024), dim3(256), 0, st, (const GiantCtl *)ctl, (K *)r.gkey, r.gca, r.gcb);
+                       (const uint32_t *)r.heavy, ctl, r.nheavy, r.nsmall, r.cursor, r.heavy_seen);
+    hipLaunchKernelGGL((k_giant_clear<K>), dim3(512), dim3(256), 0, st, (const GiantCtl *)ctl, (K *)r.gkey, r.gca, r.gcb);
     hipLaunchKernelGGL((k_giant_fold<K, OFF, 0>), dim3(1024), dim3(1024), 0, st, (const OFF *)r.offA, (const K *)r.keysA,
                        (const uint32_t *)r.heavy, ctl, (K *)r.gkey, r.gca);
     hipLaunchKernelGGL((k_giant_fold<K, OFF, 1>), dim3(1024), dim3(1024), 0, st, (const OFF *)r.offB, (const K *)r.keysB,
@@ -3072,8 +3143,8 @@ static hipError_t launch_rle_t(const LaunchRle &r, hipStream_t st) {
     hipLaunchKernelGGL((k_giant_emit<K>), dim3(GIANT_CAP), dim3(1024), 0, st, (const GiantCtl *)ctl, (const K *)r.gkey,
                        (const unsigned long long *)r.gca, (const unsigned long long *)r.gcb, (K *)r.rk, r.rca, r.rcb,
                        r.capacity, r.cursor, r.pairs, (const uint32_t *)r.heavy, r.ovf_list, r.ovf_n, r.heavy_cap);
-    const uint32_t gs = (uint32_t)std::min<uint64_t>(r.nheavy, RLE_HEAVY_GRID_S);
-    const uint32_t gb = (uint32_t)std::min<uint64_t>(r.nheavy, RLE_HEAVY_GRID);
+    const uint32_t gs = (uint32_t)std::min<uint64_t>(r.heavy_cap, RLE_HEAVY_GRID_S);
+    const uint32_t gb = (uint32_t)std::min<uint64_t>(r.heavy_cap, RLE_HEAVY_GRID);
     hipLaunchKernelGGL((k_rle_heavy<K, OFF, 256, RLE_HEAVY_SMALL_TS>), dim3(gs), dim3(256), 0, st, (const OFF *)r.offA,
                        (const K *)r.keysA, (const OFF *)r.offB, (const K *)r.keysB, (K *)r.rk, r.rca,
                        r.rcb, r.capacity, r.cursor, r.pairs, r.overflow, (const uint32_t *)r.gmark,

@@ -212,7 +212,12 @@ struct LaunchRle {
   unsigned long long *rca, *rcb;
   uint64_t capacity;
   uint32_t *heavy;
-  uint64_t heavy_cap, nheavy;
+  uint64_t heavy_cap;
+  // pass 2: number of heavy bins and of the small bins' records (device), and
+  // where the former goes for the host to check
+  const uint32_t *nheavy;
+  const unsigned long long *nsmall;
+  unsigned long long *heavy_seen;
   unsigned long long *cursor, *pairs;
   unsigned int *overflow;
   // giant heavy bins: per-heavy-bin slot (heavy_cap), control block, tables
@@ -228,6 +233,20 @@ struct LaunchRle {
   // list (heavy_cap entries) and its zeroed counter
   uint32_t *ovf_list;
   unsigned int *ovf_n;
+};
+
+// Exclusive scans of two chunk arrays (n elements, totals at [n]); add (or
+// null): an array whose sum is added to *acc; nzero words cleared.
+struct LaunchRleScan {
+  const unsigned long long *in64;
+  unsigned long long *out64;
+  const uint32_t *in32;
+  uint32_t *out32;
+  uint64_t n;
+  const unsigned long long *add;
+  unsigned long long *acc;
+  uint32_t *zero;
+  uint32_t nzero;
 };
 
 // One batch of the run-length join's global-table path (value-rich bins).
@@ -320,6 +339,7 @@ hipError_t launch_rle(const LaunchRle &r, hipStream_t st);
 // heavy bins <= keys of A / 65 + keys of B / 65 (from the offsets alone)
 hipError_t launch_rle_caps(const void *offA, const void *offB, int off_bytes, uint64_t M,
                            unsigned long long *cap_rec, uint32_t *cap_h, hipStream_t st);
+hipError_t launch_rle_scan(const LaunchRleScan &p, void *status, hipStream_t st);
 hipError_t launch_rle_gather(const LaunchRleGather &g, hipStream_t st);
 hipError_t launch_rle_ovf(const LaunchRleOvf &o, hipStream_t st);
 // (a0, a1, x0, x1) of each listed bin -> out (4 entries per bin)
@@ -332,6 +352,7 @@ size_t rle_giant_slots();
 size_t rle_priv_records();
 uint32_t rle_heavy_grid();
 size_t rle_giant_ctl_bytes();
+constexpr uint32_t RLE_GIANT_ZERO = 8;  // leading words of the control block cleared before pass 2
 hipError_t launch_part_hist(const LaunchPart &lp, hipStream_t st);
 hipError_t launch_part_scatter(const LaunchPart &lp, hipStream_t st);
 hipError_t launch_narrow(const LaunchNarrow &p, hipStream_t st);
