@@ -123,6 +123,15 @@ uint32_t choose_width(uint64_t n, uint64_t M, int kb, double fill = 0.875) {
   return (uint32_t)w;
 }
 
+// The same for a smaller bucket class.  Sparse tables get more buckets of
+// fewer bins, up to `cols` of them, since a bucket's time then goes to its bins.
+uint32_t class_width(uint64_t n, uint64_t M, int cls, double fill, uint64_t cols) {
+  const double keys = final_class_keys(cls);
+  double w = n ? std::floor(fill * keys * (double)M / (double)n) : 65535.0;
+  w = std::min(w, std::max(2 * keys, std::ceil((double)M / (double)cols)));
+  return (uint32_t)std::min(std::max(w, 1.0), 65535.0);
+}
+
 }  // namespace
 
 struct hg_ctx_s {
@@ -322,6 +331,7 @@ struct Level {
   uint64_t cmat_elems = 0, psum_elems = 0;
   uint32_t tile_keys = kTile;   // keys per partition tile
   uint32_t big_cap = 1;         // per-bin counters of the final stage's oversized buckets
+  int cls = FINAL_CLASSES - 1;  // bucket class of the final stage / the probe
 
   bool any_kind = false;        // kinds change on the device (trained in a plan): general kernels
   // One kind shared by all segments selects a specialised kernel.
@@ -546,7 +556,15 @@ hg_status run_final(hg_ctx c, const Level &L, const LevelDev &d, int kb, int ob,
   f.off_bytes = ob;
   f.hk = L.hash_kind();
   f.nitems = L.ncols_total;
-  f.lds_bytes = 128 * 1024;
+  f.cls = L.cls;
+  f.many = L.segs.size() >= MANY_TABLES && L.maps.size() >= MANY_TABLES;
+  if (L.cls == FINAL_CLASSES - 1) {
+    f.lds_bytes = 128 * 1024;
+  } else {  // the widest bucket's counters, then the staged keys (64 KB of them at a time)
+    uint32_t W = 1;
+    for (const SegDesc &sd : L.segs) W = std::max(W, (uint32_t)std::min<uint64_t>(sd.div.d, sd.seg_nbins));
+    f.lds_bytes = std::max<uint32_t>((W + 1) / 2 * 4, std::min<uint32_t>(final_class_keys(L.cls) * (uint32_t)kb, 64 * 1024));
+  }
   f.part = part;
   f.csr = csr;
   f.off = off;
@@ -2888,9 +2906,16 @@ BinMap batch_map(const hg_batch_desc *bd, uint32_t t) {
   return make_map(bd->h_n_bins[t], k, m);
 }
 
+// Buckets of one table beyond which a batch keeps to the largest bucket class.
+constexpr uint64_t kBatchCols = 1024;
+constexpr int kBatchCls = 1;  // the smaller class a plan tries: 8192 keys
 struct BatchCfg {
   uint32_t tile_keys = kTile;
   double fill = 0.875;
+  // bucket class (the largest when a table needs too many smaller buckets).
+  // 1024 tables of 2^8..2^20 keys, half of them Zipf(1.2), build and counts:
+  // 3.8 ms with 8 K-key buckets, 4.2 with 32 K
+  int cls = kBatchCls;
   bool train = false;  // models trained inside the plan: kinds set on the device
 };
 
@@ -2913,11 +2938,19 @@ hg_status batch_prepare(hg_ctx c, const hg_batch_desc *bd, const uint64_t *probe
   S.L = Level();
   const uint64_t *ko = bd->h_key_off;
   const uint64_t *src = probe_off ? probe_off : ko;
-  for (uint32_t t = 0; t < bd->n_tables; t++) {
+  const auto width = [&](uint32_t t, int cls) {
     const uint64_t n = ko[t + 1] - ko[t], np = src[t + 1] - src[t], M = bd->h_n_bins[t];
+    const uint64_t k = probe_off ? std::max(n, np) : n;
+    if (cls == FINAL_CLASSES - 1) return choose_width(k, M, kb, probe_off ? std::min(cfg.fill, probe_fill(kb)) : cfg.fill);
+    return class_width(k, M, cls, probe_off ? 0.72 : cfg.fill, kBatchCols);
+  };
+  S.L.cls = cfg.cls;
+  for (uint32_t t = 0; t < bd->n_tables && S.L.cls != FINAL_CLASSES - 1; t++)
+    if ((bd->h_n_bins[t] - 1) / width(t, S.L.cls) >= kBatchCols) S.L.cls = FINAL_CLASSES - 1;
+  for (uint32_t t = 0; t < bd->n_tables; t++) {
+    const uint64_t M = bd->h_n_bins[t];
     const BinMap map = batch_map(bd, t);
-    const uint32_t W = choose_width(probe_off ? std::max(n, np) : n, M, kb,
-                                    probe_off ? std::min(cfg.fill, probe_fill(kb)) : cfg.fill);
+    const uint32_t W = width(t, S.L.cls);
     SegDesc s = range_seg(src[t], src[t + 1], 0, M, W, map);
     if (s.nbuckets > kFMax) return fail(HG_ERR_UNSUPPORTED, "a batched table is too large for one partition level");
     s.fin_off_base = bd->h_off_off[t];
@@ -2967,8 +3000,14 @@ hg_status batch_launch_probe(hg_ctx c, const hg_batch_desc *bd, BatchSide &S, co
   pr.hk = S.L.hash_kind();
   pr.nitems = S.L.ncols_total;
   pr.akey_cap = probe_akey_cap(pr.key_bytes, 4);
-  pr.one_keys = probe_one_keys(pr.key_bytes);
-  pr.one_lds = PROBE1_LDS;
+  pr.many = bd->n_tables >= MANY_TABLES;
+  if (S.L.cls == FINAL_CLASSES - 1) {
+    pr.one_keys = probe_one_keys(pr.key_bytes);
+    pr.one_lds = PROBE1_LDS;
+  } else {  // 0.72 of a class's keys with their offsets fit with 10% to spare; 3 (uint64: 2) workgroups a CU
+    pr.one_keys = final_class_keys(S.L.cls);
+    pr.one_lds = pr.key_bytes == 4 ? 52 * 1024 : 78 * 1024;
+  }
   pr.bpart = S.part;
   pr.items = S.d.fin;
   pr.maps = S.d.maps;
@@ -3259,10 +3298,10 @@ hg_status hg_batch_plan_create(hg_ctx c, const hg_batch_desc *bd, const void *d_
   }
   std::vector<BatchCfg> cands;
   if (autotune & HG_PLAN_AUTOTUNE) {
-    for (double f : {0.875, 0.5})
+    for (int cls : {FINAL_CLASSES - 1, kBatchCls})
       for (uint32_t tk : {kTile / 4, kTile, kTile * 4}) {
         BatchCfg x;
-        x.fill = f;
+        x.cls = cls;
         x.tile_keys = tk;
         x.train = p->train;
         cands.push_back(x);
@@ -3295,7 +3334,7 @@ hg_status hg_batch_plan_create(hg_ctx c, const hg_batch_desc *bd, const void *d_
   st = plan_capture(p, best);
   if (st != HG_OK) return bail(st);
   p->info.tile_keys = best.tile_keys;
-  p->info.fill = (float)best.fill;
+  p->info.fill = (float)(best.fill * final_class_keys(best.cls) / final_class_keys(FINAL_CLASSES - 1));
   p->info.candidates = (uint32_t)cands.size();
   p->info.tuned_ms = best_ms;
   *out = p;

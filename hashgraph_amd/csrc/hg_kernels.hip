@@ -368,15 +368,18 @@ struct BigCtl {
   unsigned long long packed;    // listed slots << 40 | chunks
   unsigned long long bins;      // per-bin counters asked for
   unsigned long long unlisted;  // some item did not fit
+  unsigned long long nmid;      // items between a small bucket class and the largest (up to BIG_CAP listed)
   uint32_t item[BIG_CAP];
   uint32_t chunk_start[BIG_CAP];
   uint32_t bin_base[BIG_CAP];
+  uint32_t mid[BIG_CAP];
 };
 
 __device__ void big_clear(BigCtl *ctl) {
   ctl->packed = 0;
   ctl->bins = 0;
   ctl->unlisted = 0;
+  ctl->nmid = 0;
 }
 
 // One thread: lists item i (count keys, nbins per-bin counters from *bin0 on)
@@ -416,15 +419,51 @@ __device__ __forceinline__ uint32_t big_chunks(const BigCtl *ctl, const FinItem 
 // ---------------------------------------------------------------------------
 // Final stage: one workgroup per bucket (final_bucket).
 // ---------------------------------------------------------------------------
+constexpr uint32_t FINAL_MAX = final_class_keys(FINAL_CLASSES - 1);
+
+// The items a small class left to the largest one (skewed keys: a few
+// thousand keys too many for their bucket), shared by a fixed grid: for
+// batches of many tables, where the three passes of the oversized-bucket
+// kernels cost more (1024 tables, half of them Zipf(1.2): 810 us without this
+// kernel, 600 us with it).  The few such items of one table are done sooner by
+// those kernels, which cut them into chunks (10^6 Zipf keys: 177 against 229 us).
+template <typename K, typename OFF, int BLOCK, int KPT, int HK, bool SPLIT = false>
+__global__ __launch_bounds__(BLOCK) void k_final_mid(const K *__restrict__ part, K *__restrict__ csr, OFF *__restrict__ off,
+                                                     const FinItem *__restrict__ items, const BinMap *__restrict__ maps,
+                                                     uint32_t lds_bytes, const BigCtl *__restrict__ ctl,
+                                                     uint64_t *__restrict__ csr_index) {
+  extern __shared__ __align__(16) uint32_t smem32[];
+  const uint32_t n = (uint32_t)min(ctl->nmid, (unsigned long long)BIG_CAP);
+  for (uint32_t i = blockIdx.x; i < n; i += gridDim.x) {
+    const FinItem it = items[ctl->mid[i]];
+    const BinMap mp = maps[it.table];
+    final_bucket<K, OFF, BLOCK, KPT, HK, SPLIT>(part, csr, off, it, mp, smem32, lds_bytes, csr_index);
+    __syncthreads();
+  }
+}
+
 template <typename K, typename OFF, int BLOCK, int KPT, int HK, bool SPLIT = false>
 __global__ __launch_bounds__(BLOCK) void k_final(const K *__restrict__ part, K *__restrict__ csr, OFF *__restrict__ off,
                                                  const FinItem *__restrict__ items, const BinMap *__restrict__ maps,
                                                  uint32_t lds_bytes, BigCtl *__restrict__ ctl,
                                                  uint32_t *__restrict__ big_slot, uint32_t *__restrict__ big_cnt,
-                                                 uint32_t big_cap, uint64_t *__restrict__ csr_index) {
+                                                 uint32_t big_cap, uint64_t *__restrict__ csr_index, bool use_mid) {
   extern __shared__ __align__(16) uint32_t smem32[];
   const FinItem it = items[blockIdx.x];
   if (it.count > BLOCK * KPT || it.count > 65535u) {  // the oversized-bucket kernels' item: listed, its counters cleared
+    if (BLOCK * KPT < FINAL_MAX && use_mid && it.count <= FINAL_MAX) {  // one workgroup of the largest class still holds it
+      if (threadIdx.x == 0) smem32[0] = (uint32_t)min(atomicAdd(&ctl->nmid, 1ull), (unsigned long long)BIG_CAP);
+      __syncthreads();
+      const uint32_t slot = smem32[0];
+      if (slot < BIG_CAP) {
+        if (threadIdx.x == 0) {
+          ctl->mid[slot] = blockIdx.x;
+          big_slot[blockIdx.x] = 0;  // not an unlisted item
+        }
+        return;
+      }
+      __syncthreads();
+    }
     if (threadIdx.x == 0)
       smem32[0] = big_register(ctl, big_slot, blockIdx.x, it.count, it.nbins, big_cap, BIG_CHUNK, &smem32[1]);
     __syncthreads();
@@ -1388,6 +1427,27 @@ __device__ __forceinline__ void vt_fold_seq(uint64_t n, AT &&key_at, K *s_key, u
     for (int u = 0; u < FOLD_U; u++) {
       const uint64_t i = c0 + (uint64_t)u * BLOCK + threadIdx.x;
       v[u] = i < n ? key_at(i) : EMPTY;
+    }
+    if constexpr ((uint32_t)(BLOCK * FOLD_U) <= HT_SLOTS / 2) {
+      // the group's inserts always fit behind one check
+      const bool full = *s_fill > HT_SLOTS / 2;  // uniform: read after a barrier
+      __syncthreads();                           // every thread has read it before it changes
+      if (full) {
+        answer();
+        vt_clear<K, BLOCK>(s_key, s_cnt, s_fill, s_ecnt);
+      }
+#pragma unroll
+      for (int u = 0; u < FOLD_U; u++) {
+        if (c0 + (uint64_t)u * BLOCK + threadIdx.x >= n) continue;
+        const uint32_t c = wave_same_value(v[u]);
+        if (c) {
+          if (v[u] == EMPTY) atomicAdd(s_ecnt, c);
+          else vt_insert(s_key, s_cnt, s_fill, v[u], c);
+        }
+      }
+      __syncthreads();
+      pending = true;
+      continue;
     }
 #pragma unroll
     for (int u = 0; u < FOLD_U; u++) {
@@ -2506,7 +2566,11 @@ __global__ __launch_bounds__(BLOCK) void k_probe_big(const K *__restrict__ bpart
 // Bins longer than PROBE_BIN_LIMIT (duplicates) of the items k_probe1, k_probe
 // and k_probe_big marked: one workgroup per marked item folds the bucket's
 // long bins of A into one LDS value table (a value lives in one bin, so the
-// bins share the table).  The bucket's offsets are read HEAVY_UB bins per
+// bins share the table).  Many marked items (a batch of tables) are bound by
+// the latency of each one's phases and take small workgroups (512 threads:
+// 661 us on 1024 tables, half of them Zipf(1.2), where 1024 threads took 1048);
+// a table or few are bound by the workgroup with the hottest value and take
+// 1024 (4 M Zipf keys: 1.10 ms, with 512 threads 1.44).  The bucket's offsets are read HEAVY_UB bins per
 // thread at a time; the long bins found are listed in LDS (HEAVY_LIST at a
 // time, with the exclusive prefix of their lengths) and their keys are
 // folded as one concatenated sequence (vt_fold_seq: a key's bin is found by
@@ -2514,29 +2578,30 @@ __global__ __launch_bounds__(BLOCK) void k_probe_big(const K *__restrict__ bpart
 // answer of the table looks every probe key of the bucket up (a value found
 // is in a long bin; the walking kernels skipped those).  Bins with more
 // distinct values than the table holds are folded over several rounds.
-constexpr int HEAVY_UB = 8;
-constexpr uint32_t HEAVY_LIST = 1024;
 template <typename K, typename OFF, int BLOCK>
-__global__ __launch_bounds__(BLOCK) void k_probe_heavy(const K *__restrict__ bpart, const FinItem *__restrict__ items,
+__global__ __launch_bounds__(BLOCK, BLOCK == 512 && sizeof(K) == 4 ? 6 : 4) void k_probe_heavy(const K *__restrict__ bpart, const FinItem *__restrict__ items,
                                                        const OFF *__restrict__ offA, const K *__restrict__ keysA,
                                                        K *__restrict__ out, uint64_t capacity,
                                                        unsigned long long *__restrict__ cursor,
                                                        const unsigned int *__restrict__ hmark,
                                                        const unsigned int *__restrict__ gate,
                                                        const uint64_t *__restrict__ out_off) {
-  static_assert(HEAVY_LIST == BLOCK, "one listed bin per thread in the prefix step");
+  constexpr int HEAVY_UB = BLOCK == 512 ? 12 : 8;
+  constexpr uint32_t HEAVY_LIST = BLOCK;  // one listed bin per thread in the prefix step
   __shared__ K s_key[HT_SLOTS];
   __shared__ uint32_t s_cnt[HT_SLOTS];
-  __shared__ uint64_t s_hs[HEAVY_LIST];      // first key (index into A's bucket) of each listed bin
-  __shared__ uint64_t s_hx[HEAVY_LIST + 1];  // exclusive prefix of the listed bins' lengths
+  // first key of each listed bin (relative to the bucket's first: a table has
+  // fewer than 2^32 keys) and the exclusive prefix of the bins' lengths
+  __shared__ uint32_t s_hs[HEAVY_LIST], s_hx[HEAVY_LIST + 1];
   __shared__ uint32_t s_fill, s_ecnt;
   __shared__ uint32_t s_t32[BLOCK / 64 + 1];
   __shared__ unsigned long long s_t64[BLOCK / 64 + 1], s_base;
   if (gate[1] == 0 || !hmark[blockIdx.x]) return;
   const FinItem it = items[blockIdx.x];
   const K *kp = bpart + it.key_start;
-  const K *ka = keysA + it.key_rel;
   const OFF *of = offA + it.off_pos;  // of[0..nbins] are the bucket's offsets
+  const OFF of0 = of[0];
+  const K *ka = keysA + it.key_rel + of0;
   uint64_t cap;
   K *o = out_region(out, capacity, out_off, it.table, cap);
   auto answer = [&]() {
@@ -2547,9 +2612,9 @@ __global__ __launch_bounds__(BLOCK) void k_probe_heavy(const K *__restrict__ bpa
   for (uint64_t w0 = 0; w0 < it.nbins; w0 += (uint64_t)BLOCK * HEAVY_UB) {
     // this thread's bins: l0 .. l0 + HEAVY_UB - 1
     const uint64_t l0 = w0 + (uint64_t)threadIdx.x * HEAVY_UB;
-    uint64_t o[HEAVY_UB + 1];
+    uint32_t o[HEAVY_UB + 1];
 #pragma unroll
-    for (int i = 0; i <= HEAVY_UB; i++) o[i] = l0 + i <= it.nbins ? (uint64_t)of[l0 + i] : 0ull;
+    for (int i = 0; i <= HEAVY_UB; i++) o[i] = l0 + i <= it.nbins ? (uint32_t)(of[l0 + i] - of0) : 0u;
     uint32_t hm = 0;
 #pragma unroll
     for (int i = 0; i < HEAVY_UB; i++)
@@ -2570,9 +2635,9 @@ __global__ __launch_bounds__(BLOCK) void k_probe_heavy(const K *__restrict__ bpa
         }
       }
       __syncthreads();
-      const uint64_t len = threadIdx.x < nh ? s_hx[threadIdx.x] : 0ull;
-      unsigned long long tot;
-      const unsigned long long lx = block_exclusive_sum<BLOCK, unsigned long long>(len, s_t64, tot);
+      const uint32_t len = threadIdx.x < nh ? s_hx[threadIdx.x] : 0u;
+      uint32_t tot;
+      const uint32_t lx = block_exclusive_sum<BLOCK, uint32_t>(len, s_t32, tot);
       if (threadIdx.x < nh) s_hx[threadIdx.x] = lx;
       if (threadIdx.x == 0) s_hx[nh] = tot;
       __syncthreads();
@@ -2729,22 +2794,24 @@ static hipError_t launch_final_t(const LaunchFinal &lf, hipStream_t st) {
     auto go = [&](auto kern, uint32_t block) {
       hipLaunchKernelGGL(kern, dim3(lf.nitems), dim3(block), lf.lds_bytes, st, (const K *)lf.part, (K *)lf.csr,
                          (OFF *)lf.off, lf.items, lf.maps, lf.lds_bytes, ctl, lf.big_slot, lf.big_cnt, lf.big_cap,
-                         lf.csr_index);
+                         lf.csr_index, lf.many);
       return hipGetLastError();
     };
-    // the small classes serve one table, murmur3 or learned
-    if constexpr (H != HK_ANY) {
-      if (lf.cls == 0) return go(&k_final<K, OFF, 256, 16, H, S>, 256);
-      if (lf.cls == 1) return go(&k_final<K, OFF, 512, 16, H, S>, 512);
-      if (lf.cls == 2) return go(&k_final<K, OFF, 1024, 16, H, S>, 1024);
-    }
-    return go(&k_final<K, OFF, 1024, KPT, H, S>, 1024);
+    if (lf.cls == FINAL_CLASSES - 1) return go(&k_final<K, OFF, 1024, KPT, H, S>, 1024);
+    hipError_t r = lf.cls == 0   ? go(&k_final<K, OFF, 256, 16, H, S>, 256)
+                   : lf.cls == 1 ? go(&k_final<K, OFF, 512, 16, H, S>, 512)
+                                 : go(&k_final<K, OFF, 1024, 16, H, S>, 1024);
+    if (r != hipSuccess || !lf.many) return r;
+    const uint32_t lds = std::max(lf.lds_bytes, 128u * 1024);
+    hipLaunchKernelGGL((k_final_mid<K, OFF, 1024, KPT, H, S>), dim3(256), dim3(1024), lds, st, (const K *)lf.part,
+                       (K *)lf.csr, (OFF *)lf.off, lf.items, lf.maps, lds, (const BigCtl *)ctl, lf.csr_index);
+    return hipGetLastError();
   });
   if (e != hipSuccess) return e;
   // three kernels that return at once when no item was oversized: two
   // workgroups per CU (their 128 KB of LDS admit one at a time) dispatch in
   // under 2 us, the 2048 they had took 4.5 us
-  const uint32_t small_cap = std::min(final_class_keys(lf.cls), 65535u);
+  const uint32_t small_cap = final_class_keys(lf.cls);
   hipLaunchKernelGGL((k_big_count<K, 1024>), dim3(BIG_GRID), dim3(1024), 0, st, (const K *)lf.part, lf.items, lf.maps,
                      (const BigCtl *)ctl, lf.big_cnt);
   hipLaunchKernelGGL((k_big_scan<OFF>), dim3(256), dim3(1024), 0, st, lf.items, (const BigCtl *)ctl, lf.big_cnt,
@@ -2757,7 +2824,7 @@ static hipError_t launch_final_t(const LaunchFinal &lf, hipStream_t st) {
 
 static_assert(final_class_keys(FINAL_CLASSES - 1) == 1024u * KPT_U32, "largest final-stage class");
 hipError_t launch_final(const LaunchFinal &lf, hipStream_t st) {
-  if (lf.cls < 0 || lf.cls >= FINAL_CLASSES || (lf.cls != FINAL_CLASSES - 1 && lf.hk == HK_ANY)) return hipErrorInvalidValue;
+  if (lf.cls < 0 || lf.cls >= FINAL_CLASSES) return hipErrorInvalidValue;
   if (lf.csr_index) {  // index-carrying build of 32-bit keys: 8-byte murmur3 records split on store
     if (lf.key_bytes != 8 || lf.hk != HK_MURMUR) return hipErrorInvalidValue;
     return lf.off_bytes == 4 ? launch_final_t<uint64_t, uint32_t, true>(lf, st)
@@ -2794,11 +2861,9 @@ static hipError_t launch_probe_one_t(const LaunchProbe &p, hipStream_t st) {
                          p.gate, p.out_off, std::min(1024u * KPT, 65535u), (BigCtl *)p.big_ctl, p.big_slot);
       return hipGetLastError();
     };
-    if constexpr (H != HK_ANY) {  // the small classes serve one table, murmur3 or learned
-      if (p.one_keys == 4096) return go(&k_probe1<K, OFF, 256, 16, H>, 256);
-      if (p.one_keys == 8192) return go(&k_probe1<K, OFF, 512, 16, H>, 512);
-      if (p.one_keys == 16384) return go(&k_probe1<K, OFF, 1024, 16, H>, 1024);
-    }
+    if (p.one_keys == 4096) return go(&k_probe1<K, OFF, 256, 16, H>, 256);
+    if (p.one_keys == 8192) return go(&k_probe1<K, OFF, 512, 16, H>, 512);
+    if (p.one_keys == 16384) return go(&k_probe1<K, OFF, 1024, 16, H>, 1024);
     if (p.one_keys != probe_one_keys((int)sizeof(K))) return hipErrorInvalidValue;
     return go(&k_probe1<K, OFF, 1024, probe1_kpt<K>(), H>, 1024);
   });
@@ -2821,9 +2886,13 @@ static hipError_t launch_probe_rest_t(const LaunchProbe &p, hipStream_t st) {
                      p.items, p.maps, (const OFF *)p.offA, (const K *)p.keysA, (K *)p.out, p.capacity, p.cursor,
                      (const BigCtl *)p.big_ctl, (const uint32_t *)p.big_slot, p.nitems, std::min(1024u * KPT, 65535u),
                      p.hmark, p.gate, p.out_off);
-  hipLaunchKernelGGL((k_probe_heavy<K, OFF, 1024>), dim3(p.nitems), dim3(1024), 0, st, (const K *)p.bpart, p.items,
-                     (const OFF *)p.offA, (const K *)p.keysA, (K *)p.out, p.capacity, p.cursor,
-                     (const unsigned int *)p.hmark, (const unsigned int *)p.gate, p.out_off);
+  const auto heavy = [&](auto kern, uint32_t block) {
+    hipLaunchKernelGGL(kern, dim3(p.nitems), dim3(block), 0, st, (const K *)p.bpart, p.items, (const OFF *)p.offA,
+                       (const K *)p.keysA, (K *)p.out, p.capacity, p.cursor, (const unsigned int *)p.hmark,
+                       (const unsigned int *)p.gate, p.out_off);
+  };
+  if (p.many) heavy(&k_probe_heavy<K, OFF, 512>, 512);
+  else heavy(&k_probe_heavy<K, OFF, 1024>, 1024);
   return hipGetLastError();
 }
 
@@ -3253,6 +3322,7 @@ static hipError_t set_final_classes() {
   hipError_t r = set_lds(&k_final<K, OFF, 256, 16, H, S>);
   if (r == hipSuccess) r = set_lds(&k_final<K, OFF, 512, 16, H, S>);
   if (r == hipSuccess) r = set_lds(&k_final<K, OFF, 1024, 16, H, S>);
+  if (r == hipSuccess) r = set_lds(&k_final_mid<K, OFF, 1024, 32, H, S>);
   return r;
 }
 
@@ -3295,22 +3365,18 @@ hipError_t set_kernel_attributes() {
         if (r == hipSuccess) r = set_final_classes<uint64_t, uint32_t, H, true>();
         if (r == hipSuccess) r = set_final_classes<uint64_t, uint64_t, H, true>();
       }
-      if constexpr (H != HK_ANY) {
-        if (r == hipSuccess) r = set_final_classes<uint32_t, uint32_t, H, false>();
-        if (r == hipSuccess) r = set_final_classes<uint32_t, uint64_t, H, false>();
-        if (r == hipSuccess) r = set_final_classes<uint64_t, uint32_t, H, false>();
-        if (r == hipSuccess) r = set_final_classes<uint64_t, uint64_t, H, false>();
-      }
+      if (r == hipSuccess) r = set_final_classes<uint32_t, uint32_t, H, false>();
+      if (r == hipSuccess) r = set_final_classes<uint32_t, uint64_t, H, false>();
+      if (r == hipSuccess) r = set_final_classes<uint64_t, uint32_t, H, false>();
+      if (r == hipSuccess) r = set_final_classes<uint64_t, uint64_t, H, false>();
       if (r == hipSuccess) r = set_lds(&k_probe1<uint32_t, uint32_t, 1024, probe1_kpt<uint32_t>(), H>);
       if (r == hipSuccess) r = set_lds(&k_probe1<uint32_t, uint64_t, 1024, probe1_kpt<uint32_t>(), H>);
       if (r == hipSuccess) r = set_lds(&k_probe1<uint64_t, uint32_t, 1024, probe1_kpt<uint64_t>(), H>);
       if (r == hipSuccess) r = set_lds(&k_probe1<uint64_t, uint64_t, 1024, probe1_kpt<uint64_t>(), H>);
-      if constexpr (H != HK_ANY) {
-        if (r == hipSuccess) r = set_probe_classes<uint32_t, uint32_t, H>();
-        if (r == hipSuccess) r = set_probe_classes<uint32_t, uint64_t, H>();
-        if (r == hipSuccess) r = set_probe_classes<uint64_t, uint32_t, H>();
-        if (r == hipSuccess) r = set_probe_classes<uint64_t, uint64_t, H>();
-      }
+      if (r == hipSuccess) r = set_probe_classes<uint32_t, uint32_t, H>();
+      if (r == hipSuccess) r = set_probe_classes<uint32_t, uint64_t, H>();
+      if (r == hipSuccess) r = set_probe_classes<uint64_t, uint32_t, H>();
+      if (r == hipSuccess) r = set_probe_classes<uint64_t, uint64_t, H>();
       if (r == hipSuccess) r = set_lds(&k_probe<uint32_t, uint32_t, 1024, KPT_U32, probe_sub<uint32_t>(), H>);
       if (r == hipSuccess) r = set_lds(&k_probe<uint32_t, uint64_t, 1024, KPT_U32, probe_sub<uint64_t>(), H>);
       if (r == hipSuccess) r = set_lds(&k_probe<uint64_t, uint32_t, 1024, 32, probe_sub<uint32_t>(), H>);

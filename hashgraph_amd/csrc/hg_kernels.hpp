@@ -46,12 +46,16 @@ struct LaunchCol {
 // tables take small buckets, so that there are workgroups for every CU.
 constexpr int FINAL_CLASSES = 4;
 constexpr uint32_t final_class_keys(int cls) { return 4096u << cls; }
+// Tables from which a batch's skewed items are bound by throughput, not by the
+// hottest one (a table per CU).
+constexpr uint32_t MANY_TABLES = 256;
 struct LaunchFinal {
   int key_bytes, off_bytes;
   int hk;
   uint32_t nitems;
   uint32_t lds_bytes;
   int cls = FINAL_CLASSES - 1;  // bucket size class (final_class_keys)
+  bool many = false;            // items of MANY_TABLES tables or more
   const void *part;
   void *csr;
   void *off;
@@ -74,6 +78,7 @@ struct LaunchProbe {
   int hk;
   uint32_t nitems;
   uint32_t akey_cap;
+  bool many = false;           // items of MANY_TABLES tables or more
   uint32_t one_keys, one_lds;  // one-pass kernel: keys of B a workgroup holds (4096, 8192, 16384 or
                                // probe_one_keys) and its LDS (probe_one_lds of what it should take)
   const void *bpart;
@@ -406,7 +411,7 @@ hipError_t launch_make_items(const SegDesc *segs, uint32_t nsegs, const uint32_t
 
 int final_kpt(int key_bytes);
 // words of a final_big_ctl_bytes() area that are zero when no item is listed
-constexpr uint32_t BIG_CTL_ZERO = 3;
+constexpr uint32_t BIG_CTL_ZERO = 4;
 size_t final_big_ctl_bytes();
 // keys staged per LDS round of the scatter for a level whose widest segment
 // has max_cols columns (0: the columns do not leave room for staging)

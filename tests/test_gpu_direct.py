@@ -232,3 +232,42 @@ def test_narrow_probe_learned(dev):
     cnt, out = hg.probe(*hg.build(A, M, **kw), M, B, **kw)
     ecnt, eout = hg.probe(*hg.build(A, M), M, B)
     assert cnt == ecnt and torch.equal(torch.sort(out).values, torch.sort(eout).values)
+
+
+@pytest.mark.parametrize("kb", [4, 8])
+def test_batch_of_many_tables_skewed(kb, dev):
+    """A batch of more than 256 tables whose buckets fall into every size tier:
+    ordinary, between the small and the largest class, beyond both; long bins."""
+    import hashgraph_amd as hg
+    T = 260
+    sizes = [100 + 37 * t for t in range(T)]
+    sizes[7], sizes[100], sizes[200] = 60000, 90000, 45000
+    tabs, probes = [], []
+    for t, n in enumerate(sizes):
+        a = wl.uniform_keys(900 + t, n, kb)
+        if t == 7:
+            a[:12000] = a[0]          # one bucket between the classes
+        elif t == 100:
+            a[:50000] = a[0]          # one bucket beyond both
+        elif t == 200:
+            a[:300], a[300:700] = a[0], a[300]
+        tabs.append(a)
+        probes.append(wl.probe_keys(a, 5000 + 2 * t, n // 2 + 1, 0.4, kb))
+        if t in (7, 100):
+            probes[-1][:40] = a[0]
+    ko = np.concatenate([[0], np.cumsum(sizes)])
+    po = np.concatenate([[0], np.cumsum([len(b) for b in probes])])
+    off, csr, oo = hg.batch_build(_to_dev(np.concatenate(tabs), dev), ko, sizes)
+    total, counts = hg.batch_probe(off, csr, ko, sizes, oo, _to_dev(np.concatenate(probes), dev), po)
+    goff, gcsr = off.cpu().numpy().view(np.uint32), csr.cpu().numpy().view(tabs[0].dtype)
+    exp = []
+    for t, n in enumerate(sizes):
+        eo, ek = o.build_csr(tabs[t], n)
+        assert np.array_equal(goff[oo[t]:oo[t] + n + 1].astype(np.uint64), eo), f"table {t}: offsets differ"
+        g = gcsr[ko[t]:ko[t + 1]].copy()
+        o.canon(eo, g)
+        o.canon(eo, ek)
+        assert np.array_equal(g, ek), f"table {t}: bins differ"
+        bo, bk = o.build_csr(probes[t], n)
+        exp.append(o.intersect(eo, ek, bo, bk)[0])
+    assert counts.cpu().numpy().tolist() == exp and total == sum(exp)
