@@ -1,0 +1,272 @@
+// hg_deep.hip -- gfx950 kernels of the two-step partition of a large table:
+// up to DEEP_FINE buckets reached through about their square root of groups.
+//
+// One pass over thousands of buckets writes runs of a few keys (2^28 uint32
+// keys over 9363 buckets: 3.5 keys a run, 2.6 times the bytes) from one
+// workgroup a CU, whose counters alone fill half of its LDS.  Here every pass
+// has at most about 200 columns: runs of 40 keys and more, three workgroups a
+// CU.  The first step's histogram counts the buckets themselves and sums their
+// counts to the groups', so the second step needs no histogram: a tile of it
+// reserves its places in the buckets.  The buckets can then be small ones
+// (8 K keys), which the final stage and the probe take several of to a CU.
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+#include <algorithm>
+#include "hg_common.hpp"
+#include "hg_device.hpp"
+#include "hg_kernels.hpp"
+#include "hg_scatter.hpp"
+
+namespace hg {
+
+constexpr int HB = 1024;        // threads of the histogram
+constexpr int SB = 512;         // threads of the scatter steps
+constexpr int SUM_COLS = 32;    // columns of a column-sum workgroup
+constexpr uint32_t XCDS = 8;
+constexpr uint32_t XROWS = DEEP_ROWS / XCDS;  // key ranges of an XCD
+static_assert(DEEP_ROWS % XCDS == 0 && DEEP_ROWS % (1024 / SUM_COLS) == 0 && DEEP_GROUPS <= SB, "two-step geometry");
+
+// Counts of the buckets over key range blockIdx.x (a row of fmat) and of the
+// groups (a row of cmat).  One workgroup a CU: its LDS holds a counter for
+// every bucket.
+template <typename K>
+__global__ __launch_bounds__(HB) void k_deep_hist(const K *__restrict__ keys, DeepGeom g, uint32_t *__restrict__ cmat,
+                                                  uint32_t *__restrict__ fmat) {
+  constexpr int U = sizeof(K) == 4 ? 16 : 8;
+  extern __shared__ __align__(16) uint32_t s_cnt[];
+  for (uint32_t i = threadIdx.x; i < g.nfine; i += HB) s_cnt[i] = 0;
+  __syncthreads();
+  const uint64_t k0 = (uint64_t)blockIdx.x * g.per;
+  const uint32_t n = (uint32_t)min((uint64_t)g.per, g.n - k0);
+  for (uint32_t base = 0; base < n; base += HB * U) {
+    const uint32_t cnt = min((uint32_t)(HB * U), n - base);
+    const __amdgpu_buffer_rsrc_t rs = make_rsrc(keys + k0 + base, cnt * (uint32_t)sizeof(K));
+    K kr[U];
+#pragma unroll
+    for (int j = 0; j < U; j++) kr[j] = buf_load<K>(rs, threadIdx.x * (uint32_t)sizeof(K), j * HB * (uint32_t)sizeof(K));
+#pragma unroll
+    for (int j = 0; j < U; j++)
+      if (j * HB + threadIdx.x < cnt) atomicAdd(&s_cnt[divq(bin_of<K, HK_MURMUR>(kr[j], g.map) - g.bin_lo, g.fine)], 1u);
+  }
+  __syncthreads();
+  for (uint32_t s = threadIdx.x >> 6; s < g.ngroups; s += HB / 64) {  // a wave a group
+    uint32_t v = 0;
+    const uint32_t f1 = min(g.nfine, (s + 1) * g.group);
+    for (uint32_t f = s * g.group + (threadIdx.x & 63); f < f1; f += 64) v += s_cnt[f];
+    v = wave_inclusive_sum<uint32_t>(v);
+    if ((threadIdx.x & 63) == 63) cmat[(uint64_t)blockIdx.x * g.ngroups + s] = v;
+  }
+  for (uint32_t i = threadIdx.x; i < g.nfine; i += HB) fmat[(uint64_t)blockIdx.x * g.nfine + i] = s_cnt[i];
+}
+
+// 32 columns of a count matrix, PER rows a thread in registers.  SCAN: the
+// counts become exclusive sums down the column; else only its total is kept.
+template <int PER, bool SCAN>
+__device__ __forceinline__ void sum_columns(uint32_t *mat, uint32_t rows, uint32_t ncols, uint32_t block,
+                                            uint32_t (*s_sum)[SUM_COLS], uint32_t *tot) {
+  constexpr int CH = 1024 / SUM_COLS;
+  const uint32_t c = threadIdx.x % SUM_COLS, ch = threadIdx.x / SUM_COLS;
+  const uint32_t col = block * SUM_COLS + c, r0 = ch * PER;
+  uint32_t v[PER], s = 0;
+#pragma unroll
+  for (int i = 0; i < PER; i++) v[i] = col < ncols && r0 + i < rows ? mat[(uint64_t)(r0 + i) * ncols + col] : 0u;
+#pragma unroll
+  for (int i = 0; i < PER; i++) s += v[i];
+  s_sum[ch][c] = s;
+  __syncthreads();
+  if (col >= ncols || (!SCAN && ch != CH - 1)) return;
+  uint32_t run = 0;
+  for (uint32_t q = 0; q < ch; q++) run += s_sum[q][c];
+  if (ch == CH - 1 && tot) tot[col] = run + s;
+  if constexpr (SCAN) {
+#pragma unroll
+    for (int i = 0; i < PER; i++) {
+      if (r0 + i < rows) mat[(uint64_t)(r0 + i) * ncols + col] = run;
+      run += v[i];
+    }
+  }
+}
+
+// The first blocks: totals of the buckets' columns; the others: exclusive sums
+// of the groups' columns.
+__global__ __launch_bounds__(1024) void k_deep_sum(uint32_t *__restrict__ cmat, uint32_t rows, uint32_t ngroups,
+                                                   uint32_t *__restrict__ fmat, uint32_t nfine,
+                                                   uint32_t *__restrict__ ftot) {
+  constexpr int PER = DEEP_ROWS * SUM_COLS / 1024;
+  __shared__ uint32_t s_sum[1024 / SUM_COLS][SUM_COLS];
+  const uint32_t nb = (nfine + SUM_COLS - 1) / SUM_COLS;
+  if (blockIdx.x < nb)
+    sum_columns<PER, false>(fmat, rows, nfine, blockIdx.x, s_sum, ftot);
+  else
+    sum_columns<PER, true>(cmat, rows, ngroups, blockIdx.x - nb, s_sum, nullptr);
+}
+
+// Starts of the buckets (fstart, nfine + 1), each XCD's first places in the
+// groups (gstart) and the second step's chunks, group by group.  One workgroup.
+__global__ __launch_bounds__(1024) void k_deep_starts(const uint32_t *__restrict__ ftot, DeepGeom g, uint32_t rows,
+                                                      const uint32_t *__restrict__ cmat, uint32_t chunk_keys,
+                                                      uint32_t *__restrict__ fstart, uint32_t *__restrict__ gstart,
+                                                      DeepChunk *__restrict__ chunks, uint32_t *__restrict__ nchunks) {
+  extern __shared__ __align__(16) uint32_t s_a[];  // nfine + 1
+  __shared__ uint32_t s_tmp[1024 / 64 + 1];
+  lds_fill<uint32_t, 1024, 8>(s_a, ftot, g.nfine);
+  __syncthreads();
+  const uint32_t tot = lds_exclusive_scan<1024>(s_a, g.nfine, s_tmp);
+  if (threadIdx.x == 0) s_a[g.nfine] = tot;
+  __syncthreads();
+  for (uint32_t f = threadIdx.x; f <= g.nfine; f += 1024) fstart[f] = s_a[f];
+  const uint32_t s = threadIdx.x;
+  uint32_t a = 0, e = 0;
+  if (s < g.ngroups) {
+    a = s_a[s * g.group];
+    e = s_a[min(g.nfine, (s + 1) * g.group)];
+  }
+  if (s < g.ngroups)
+    for (uint32_t x = 0; x < XCDS; x++)
+      if (x * XROWS < rows) gstart[x * g.ngroups + s] = a + cmat[(uint64_t)x * XROWS * g.ngroups + s];
+  const uint32_t nc = (uint32_t)(((uint64_t)(e - a) + chunk_keys - 1) / chunk_keys);
+  uint32_t all;
+  const uint32_t c0 = block_exclusive_sum<1024, uint32_t>(nc, s_tmp, all);
+  if (threadIdx.x == 0) *nchunks = all;
+  for (uint32_t i = 0; i < nc; i++) {
+    DeepChunk d;
+    d.start = a + i * chunk_keys;
+    d.count = min(chunk_keys, e - d.start);
+    d.group = s;
+    d.pad = 0;
+    chunks[c0 + i] = d;
+  }
+}
+
+// First step: chunks of the keys into the groups; a tile reserves its places.
+// XCD x takes the x-th eighth of the keys in order and writes one part of each
+// group, so the tiles in flight on an XCD write next to each other (with a
+// contiguous key range for each workgroup instead: 747 against 519 us for the
+// second step, which writes 5 MB at a time; 2^28 uint32 keys).
+// The first workgroups also write the buckets' items and clear what the items'
+// kernels need.
+template <typename K, bool PACK>
+__global__ __launch_bounds__(SB) void k_deep_first(const void *__restrict__ keys, DeepGeom g, uint32_t chunk_keys,
+                                                   uint32_t *__restrict__ gstart,
+                                                   const uint32_t *__restrict__ fstart, K *__restrict__ out,
+                                                   FinItem *__restrict__ items, BinMap *__restrict__ maps,
+                                                   unsigned long long *__restrict__ zero, uint32_t nzero,
+                                                   unsigned int *__restrict__ zero_col) {
+  constexpr uint32_t T = scatter_tile_keys<K>(SB);
+  using IN = typename std::conditional<PACK, uint32_t, K>::type;
+  __shared__ ScatterLds<K, SB> s;
+  const uint32_t b = threadIdx.x;
+  for (uint32_t f = blockIdx.x * SB + b; f < g.nfine; f += gridDim.x * SB) {
+    FinItem it;
+    const uint64_t lo = (uint64_t)f * g.fine.d;
+    it.key_start = fstart[f];
+    it.key_rel = 0;
+    it.off_pos = lo;
+    it.end_pos = f + 1 == g.nfine ? g.nbins : ~0ull;
+    it.count = fstart[f + 1] - fstart[f];
+    it.nbins = (uint32_t)min((uint64_t)g.fine.d, g.nbins - lo);
+    it.bin_lo = (uint32_t)(g.bin_lo + lo);
+    it.table = 0;
+    items[f] = it;
+    if (zero_col) zero_col[f] = 0;
+  }
+  if (blockIdx.x == 0) {
+    if (b == 0) maps[0] = g.map;
+    if (b < nzero) zero[b] = 0;
+  }
+  const uint32_t x = blockIdx.x % XCDS;
+  const uint64_t share = (uint64_t)XROWS * g.per, end = min(g.n, (x + 1) * share);
+  const uint64_t k0 = x * share + (uint64_t)(blockIdx.x / XCDS) * chunk_keys;
+  if (k0 >= end) return;
+  const uint32_t n = (uint32_t)min((uint64_t)chunk_keys, end - k0);
+  for (uint32_t base = 0; base < n; base += T)
+    scatter_tile<K, SB, PACK>(keys, k0 + base, min(T, n - base), g.ngroups, s, out,
+                              [&](IN key) { return divq(bin_of<IN, HK_MURMUR>(key, g.map) - g.bin_lo, g.coarse); },
+                              [&](uint32_t c) { return c ? atomicAdd(&gstart[x * g.ngroups + b], c) : 0u; });
+}
+
+// Second step: a chunk of one group into the group's buckets; every tile
+// reserves its places (fstart ends as the buckets' ends).  Consecutive chunks
+// run on one XCD, so the runs of a bucket meet in its L2.
+template <typename K>
+__global__ __launch_bounds__(SB) void k_deep_second(const K *__restrict__ keys, DeepGeom g,
+                                                    const DeepChunk *__restrict__ chunks,
+                                                    const uint32_t *__restrict__ nchunks, uint32_t *__restrict__ fstart,
+                                                    K *__restrict__ out) {
+  constexpr uint32_t T = scatter_tile_keys<K>(SB);
+  __shared__ ScatterLds<K, SB> s;
+  const uint32_t nc = *nchunks;
+  if (blockIdx.x >= nc) return;
+  const uint32_t q = nc >> 3, r = nc & 7, x = blockIdx.x & 7;
+  const DeepChunk d = chunks[x * q + min(x, r) + (blockIdx.x >> 3)];
+  const uint32_t f0 = d.group * g.group, ncols = min(g.group, g.nfine - f0);
+  const uint32_t lo = g.bin_lo + f0 * g.fine.d;  // first bin of the group
+  for (uint32_t base = 0; base < d.count; base += T)
+    scatter_tile<K, SB, false>(keys, (uint64_t)d.start + base, min(T, d.count - base), ncols, s, out,
+                               [&](K key) { return divq(bin_of<K, HK_MURMUR>(key, g.map) - lo, g.fine); },
+                               [&](uint32_t c) { return c ? atomicAdd(&fstart[f0 + threadIdx.x], c) : 0u; });
+}
+
+namespace {
+
+// Keys of a scatter workgroup: four tiles, fewer where that would leave less
+// than a few workgroups for each of the chip's 768 places.
+uint32_t chunk_keys(uint64_t n, int key_bytes) {
+  const uint64_t t = key_bytes == 4 ? scatter_tile_keys<uint32_t>(SB) : scatter_tile_keys<uint64_t>(SB);
+  return (uint32_t)(t * std::min<uint64_t>(4, std::max<uint64_t>(1, n / (t * 3072))));
+}
+
+template <typename K>
+hipError_t launch_deep_t(const LaunchDeep &p, hipStream_t st) {
+  const DeepGeom &g = p.geom;
+  const uint32_t chunk = chunk_keys(g.n, p.key_bytes);
+  const size_t hlds = (size_t)g.nfine * 4;
+  if (p.pack)
+    hipLaunchKernelGGL(k_deep_hist<uint32_t>, dim3(p.rows), dim3(HB), hlds, st, (const uint32_t *)p.keys, g, p.cmat,
+                       p.fmat);
+  else
+    hipLaunchKernelGGL(k_deep_hist<K>, dim3(p.rows), dim3(HB), hlds, st, (const K *)p.keys, g, p.cmat, p.fmat);
+  hipLaunchKernelGGL(k_deep_sum, dim3((g.nfine + SUM_COLS - 1) / SUM_COLS + (g.ngroups + SUM_COLS - 1) / SUM_COLS),
+                     dim3(1024), 0, st, p.cmat, p.rows, g.ngroups, p.fmat, g.nfine, p.ftot);
+  hipLaunchKernelGGL(k_deep_starts, dim3(1), dim3(1024), ((size_t)g.nfine + 1) * 4, st, (const uint32_t *)p.ftot, g,
+                     p.rows, (const uint32_t *)p.cmat, chunk, p.fstart, p.gstart, p.chunks, p.nchunks);
+  auto first = &k_deep_first<K, false>;
+  if constexpr (sizeof(K) == 8)
+    if (p.pack) first = &k_deep_first<K, true>;
+  const uint64_t share = std::min<uint64_t>((uint64_t)XROWS * g.per, g.n);
+  hipLaunchKernelGGL(first, dim3((uint32_t)((share + chunk - 1) / chunk) * XCDS), dim3(SB), 0, st, p.keys, g, chunk,
+                     p.gstart, (const uint32_t *)p.fstart, (K *)p.mid, p.items, p.maps, p.zero, p.nzero, p.zero_col);
+  hipLaunchKernelGGL(k_deep_second<K>, dim3(deep_max_chunks(g, p.key_bytes)), dim3(SB), 0, st, (const K *)p.mid, g,
+                     (const DeepChunk *)p.chunks, (const uint32_t *)p.nchunks, p.fstart, (K *)p.out);
+  return hipGetLastError();
+}
+
+}  // namespace
+
+uint32_t deep_max_chunks(const DeepGeom &g, int key_bytes) {
+  return (uint32_t)(g.n / chunk_keys(g.n, key_bytes) + g.ngroups);
+}
+
+hipError_t launch_deep(const LaunchDeep &p, hipStream_t st) {
+  const DeepGeom &g = p.geom;
+  if (!g.n || g.n >= (1ull << 32) || !g.nfine || g.nfine > DEEP_FINE || !g.group || g.group > (uint32_t)SB ||
+      !g.ngroups || g.ngroups > DEEP_GROUPS || (uint64_t)g.ngroups * g.group < g.nfine ||
+      (uint64_t)(g.ngroups - 1) * g.group >= g.nfine || !p.rows || p.rows > DEEP_ROWS ||
+      (uint64_t)p.rows * g.per < g.n || (uint64_t)(p.rows - 1) * g.per >= g.n || p.nzero > (uint32_t)SB ||
+      g.map.kind != 0 || (uint64_t)g.nfine * g.fine.d < g.nbins || (p.pack && p.key_bytes != 8))
+    return hipErrorInvalidValue;
+  return p.key_bytes == 4 ? launch_deep_t<uint32_t>(p, st) : launch_deep_t<uint64_t>(p, st);
+}
+
+hipError_t set_deep_kernel_attributes() {
+  const auto lds = [](const void *f) {
+    return hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (DEEP_FINE + 1) * 4);
+  };
+  hipError_t e = hipSuccess;
+  for (hipError_t x : {lds((const void *)&k_deep_hist<uint32_t>), lds((const void *)&k_deep_hist<uint64_t>),
+                       lds((const void *)&k_deep_starts)})
+    if (x != hipSuccess) e = x;
+  return e;
+}
+
+}  // namespace hg

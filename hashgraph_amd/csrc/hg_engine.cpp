@@ -723,14 +723,15 @@ hg_status build_narrow(hg_ctx c, const BinMap &map, int kb, int ob, uint64_t n, 
 // exceeds it takes k_probe).  Returns 0 when no class does: the wide pass.
 // Narrow against wide, as many uint32 probe keys as table keys: 60 against
 // 113 us at 2^21, 80 against 121 us at 2^22, 153 against 200 us at 12 M.
-uint32_t narrow_probe(uint64_t nb, uint64_t na, uint64_t M, int kb, uint32_t &W, uint32_t &lds) {
+uint32_t probe_geometry(uint64_t nb, uint64_t na, uint64_t M, int kb, int first, double fill, uint32_t cols, uint32_t &W,
+                        uint32_t &lds) {
   const double r = (double)na / (double)M;
-  for (int cls = 0; cls < 4; cls++) {
+  for (int cls = first; cls < 4; cls++) {
     // the last two classes: 16 K keys with the whole LDS, then what the wide probe holds
     const uint32_t keys = cls < 3 ? 4096u << cls : probe_one_keys(kb);
     const uint32_t room = cls == 0 ? 52 * 1024 : cls < 3 ? 78 * 1024 : PROBE1_LDS;
-    double w = std::min(0.8 * keys * (double)M / (double)nb, 65535.0);
-    w = std::min(w, std::max(2.0 * keys, std::ceil((double)M / NARROW_COLS)));
+    double w = std::min(fill * keys * (double)M / (double)nb, 65535.0);
+    w = std::min(w, std::max(2.0 * keys, std::ceil((double)M / cols)));
     for (; w >= 1; w *= 0.97) {
       const double mean = w * r;
       lds = probe_one_lds((uint32_t)w, (uint64_t)(mean + 8 * std::sqrt(mean) + 64), kb);
@@ -738,9 +739,126 @@ uint32_t narrow_probe(uint64_t nb, uint64_t na, uint64_t M, int kb, uint32_t &W,
     }
     if (w < 1) continue;
     W = (uint32_t)w;
-    if ((M + W - 1) / W <= NARROW_COLS) return keys;
+    if ((M + W - 1) / W <= cols) return keys;
   }
   return 0;
+}
+uint32_t narrow_probe(uint64_t nb, uint64_t na, uint64_t M, int kb, uint32_t &W, uint32_t &lds) {
+  return probe_geometry(nb, na, M, kb, 0, 0.8, NARROW_COLS, W, lds);
+}
+// The same for a probe's two-step partition (8 K-key buckets first).
+uint32_t deep_probe(uint64_t nb, uint64_t na, uint64_t M, int kb, uint32_t &W, uint32_t &lds) {
+  return probe_geometry(nb, na, M, kb, 1, 0.875, DEEP_FINE, W, lds);
+}
+
+// Bucket class and width of a build's two-step partition; -1: none (the wide
+// pass).  Buckets of 8 K keys first: the final stage takes three of them to a
+// CU (2^28 uint32 keys: 0.57 ms against 0.90 with 32 K).
+int deep_class(uint64_t n, uint64_t R, uint32_t &W) {
+  for (int cls = 1; cls < FINAL_CLASSES; cls++) {
+    if (0.875 * final_class_keys(cls) * (double)R < (double)n) continue;  // less than a bin a bucket
+    W = class_width(n, R, cls, 0.875, DEEP_FINE);
+    if ((R + W - 1) / W <= DEEP_FINE) return cls;
+  }
+  return -1;
+}
+
+// Geometry of a two-step partition, its scratch in arena 1 (extra bytes of the
+// caller's behind it, at *rest) and its pointers, but for the keys' own.
+hg_status deep_launch(hg_ctx c, const BinMap &map, int kb, uint64_t n, uint64_t lo, uint64_t R, uint32_t W,
+                      size_t extra, LaunchDeep &p, char *&rest) {
+  p = LaunchDeep{};
+  DeepGeom &g = p.geom;
+  g.n = n;
+  g.nbins = R;
+  g.per = (uint32_t)(((n + DEEP_ROWS - 1) / DEEP_ROWS + 1023) & ~1023ull);
+  g.nfine = (uint32_t)((R + W - 1) / W);
+  g.group = (uint32_t)std::ceil(std::sqrt((double)g.nfine));
+  g.ngroups = (g.nfine + g.group - 1) / g.group;
+  g.bin_lo = (uint32_t)lo;
+  g.fine = make_div(W);
+  g.coarse = make_div(W * g.group);
+  g.map = map;
+  p.key_bytes = kb;
+  p.rows = (uint32_t)((n + g.per - 1) / g.per);
+  Plan P;
+  const size_t i_cmat = P.add((size_t)DEEP_ROWS * g.ngroups * 4), i_fmat = P.add((size_t)DEEP_ROWS * g.nfine * 4),
+               i_ftot = P.add(g.nfine * 4), i_fstart = P.add(((size_t)g.nfine + 1) * 4),
+               i_gstart = P.add((size_t)8 * g.ngroups * 4),
+               i_chunks = P.add((size_t)deep_max_chunks(g, kb) * sizeof(DeepChunk)), i_nch = P.add(4),
+               i_items = P.add((size_t)g.nfine * sizeof(FinItem)), i_maps = P.add(sizeof(BinMap)), i_rest = P.add(extra);
+  HG_TRY(arena_ensure(c, 1, P.total()));
+  Carve cv;
+  cv.init(c, 1, P);
+  p.cmat = cv.get<uint32_t>(i_cmat);
+  p.fmat = cv.get<uint32_t>(i_fmat);
+  p.ftot = cv.get<uint32_t>(i_ftot);
+  p.fstart = cv.get<uint32_t>(i_fstart);
+  p.gstart = cv.get<uint32_t>(i_gstart);
+  p.chunks = cv.get<DeepChunk>(i_chunks);
+  p.nchunks = cv.get<uint32_t>(i_nch);
+  p.items = cv.get<FinItem>(i_items);
+  p.maps = cv.get<BinMap>(i_maps);
+  rest = cv.get<char>(i_rest);
+  return HG_OK;
+}
+
+bool overlap(const void *a, uint64_t na, const void *b, uint64_t nb) {
+  const uintptr_t x = (uintptr_t)a, y = (uintptr_t)b;
+  return x < y + nb && y < x + na;
+}
+
+hg_status build_deep(hg_ctx c, const BinMap &map, int kb, int ob, uint64_t n, uint64_t lo, uint64_t R, int cls,
+                     uint32_t W, const void *d_keys, void *d_off, void *d_csr, uint64_t *d_csr_index, bool pack_in) {
+  const uint64_t F = (R + W - 1) / W, big_cap = std::max<uint64_t>(1, std::min<uint64_t>(R, 1ull << 28));
+  Plan Px;
+  const size_t i_ctl = Px.add(final_big_ctl_bytes()), i_slot = Px.add(F * 4), i_cnt = Px.add(big_cap * 4);
+  LaunchDeep p;
+  char *rest;
+  HG_TRY(deep_launch(c, map, kb, n, lo, R, W, Px.total(), p, rest));
+  // the grouped keys pass through the CSR, which only the final stage writes
+  // otherwise, unless the caller builds over the keys themselves
+  void *mid = d_csr_index ? (void *)d_csr_index : d_csr;
+  const bool own = overlap(mid, n * kb, d_keys, n * (pack_in ? 4 : kb));
+  Plan P0;
+  const size_t i_part = P0.add(n * kb), i_mid = P0.add(own ? n * kb : 1);
+  HG_TRY(arena_ensure(c, 0, P0.total()));
+  Carve c0;
+  c0.init(c, 0, P0);
+  p.pack = pack_in;
+  p.keys = d_keys;
+  p.mid = own ? c0.get<void>(i_mid) : mid;
+  p.out = c0.get<void>(i_part);
+  const size_t o_slot = Px.sizes[i_ctl], o_cnt = o_slot + Px.sizes[i_slot];
+  p.zero = (unsigned long long *)rest;
+  p.nzero = BIG_CTL_ZERO;
+  {
+    Prof pf(c, "part_scatter");
+    HG_HIP(launch_deep(p, c->stream));
+  }
+  (void)i_cnt;
+  LaunchFinal f{};
+  f.key_bytes = kb;
+  f.off_bytes = ob;
+  f.hk = (int)map.kind;
+  f.nitems = p.geom.nfine;
+  f.cls = cls;
+  f.many = true;  // so many buckets that a few thousand keys too many are a throughput matter
+  f.lds_bytes = std::max<uint32_t>((W + 1) / 2 * 4, std::min<uint32_t>(final_class_keys(cls) * (uint32_t)kb, 64 * 1024));
+  if (cls == FINAL_CLASSES - 1) f.lds_bytes = 128 * 1024;
+  f.part = p.out;
+  f.csr = d_csr;
+  f.off = d_off;
+  f.items = p.items;
+  f.maps = p.maps;
+  f.big_ctl = rest;
+  f.big_slot = (uint32_t *)(rest + o_slot);
+  f.big_cnt = (uint32_t *)(rest + o_cnt);
+  f.big_cap = (uint32_t)big_cap;
+  f.csr_index = d_csr_index;
+  Prof pf(c, "final");
+  HG_HIP(launch_final(f, c->stream));
+  return HG_OK;
 }
 
 // CSR of n keys whose bins all lie in [lo, lo + R): d_off[0..R] with values
@@ -768,6 +886,8 @@ hg_status build_range(hg_ctx c, const BinMap &map, int kb, int ob, uint64_t n, u
   uint32_t Wn;
   if (const int cls = narrow_class(n, R, Wn); cls >= 0)
     return build_narrow(c, map, kb, ob, n, lo, R, cls, Wn, d_keys, d_off, d_csr, d_csr_index, pack_in);
+  if (const int cls = map.kind == 0 && n < (1ull << 32) ? deep_class(n, R, Wn) : -1; cls >= 0)
+    return build_deep(c, map, kb, ob, n, lo, R, cls, Wn, d_keys, d_off, d_csr, d_csr_index, pack_in);
   const uint32_t W = choose_width(n, R, kb, build_fill());
   const uint64_t F = (R + W - 1) / W;
   const uint64_t k = level1_group(F);
@@ -1109,6 +1229,53 @@ static hg_status probe_wide(hg_ctx c, const BinMap &map, int kb, uint64_t n_keys
   pr.big_ctl = d.big_ctl;
   pr.one_keys = probe_one_keys(kb);
   pr.one_lds = PROBE1_LDS;
+  return HG_OK;
+}
+
+// Two-step partition of hg_probe's keys and pr's items and state; taken stays
+// false when its geometry or the memory for its second copy of the keys does
+// not allow it.
+static hg_status probe_deep(hg_ctx c, const BinMap &map, int kb, uint64_t n_keys, uint64_t M, const void *d_probe,
+                            uint64_t n_probe, uint64_t done, LaunchProbe &pr, bool &taken) {
+  uint32_t W, lds = 0;
+  const uint32_t one = map.kind == 0 ? deep_probe(n_probe, n_keys, M, kb, W, lds) : 0;
+  if (!one) return HG_OK;
+  const uint64_t F = (M + W - 1) / W;
+  Plan P0, Px;
+  const size_t i_part = P0.add(n_probe * kb), i_mid = P0.add(n_probe * kb);
+  if (arena_ensure(c, 0, P0.total()) != HG_OK) return HG_OK;
+  const size_t i_slot = Px.add(F * 4), i_mark = Px.add(F * 4), i_ctl = Px.add(256 + final_big_ctl_bytes());
+  LaunchDeep p;
+  char *rest;
+  HG_TRY(deep_launch(c, map, kb, n_probe, 0, M, W, Px.total(), p, rest));
+  Carve c0;
+  c0.init(c, 0, P0);
+  // the cursor and the gates end where the list of oversized buckets begins
+  pr.big_slot = (uint32_t *)rest;
+  pr.hmark = (unsigned int *)(rest + Px.sizes[i_slot]);
+  pr.big_ctl = rest + Px.sizes[i_slot] + Px.sizes[i_mark] + 256;
+  pr.cursor = (unsigned long long *)pr.big_ctl - 2;
+  pr.gate = (unsigned int *)(pr.cursor + 1);
+  (void)i_ctl;
+  p.keys = d_probe;
+  p.mid = c0.get<void>(i_mid);
+  p.out = c0.get<void>(i_part);
+  p.zero = pr.cursor;
+  p.nzero = 2 + BIG_CTL_ZERO;
+  p.zero_col = pr.hmark;
+  {
+    Prof pf(c, "part_scatter");
+    HG_HIP(launch_deep(p, c->stream));
+  }
+  if (done) HG_HIP(launch_fill_u64(pr.cursor, done, 1, c->stream));
+  pr.hk = (int)map.kind;
+  pr.nitems = p.geom.nfine;
+  pr.bpart = p.out;
+  pr.items = p.items;
+  pr.maps = p.maps;
+  pr.one_keys = one;
+  pr.one_lds = lds;
+  taken = true;
   return HG_OK;
 }
 
@@ -1679,7 +1846,9 @@ hg_status hg_probe(hg_ctx c, const hg_table_desc *descA, const void *d_offA, con
     pr.one_keys = one;
     pr.one_lds = lds;
   } else {
-    HG_TRY(probe_wide(c, map, kb, descA->n_keys, M, d_probe, n_probe, done, pr));
+    bool two = false;
+    HG_TRY(probe_deep(c, map, kb, descA->n_keys, M, d_probe, n_probe, done, pr, two));
+    if (!two) HG_TRY(probe_wide(c, map, kb, descA->n_keys, M, d_probe, n_probe, done, pr));
   }
   pr.key_bytes = kb;
   pr.off_bytes = ob;

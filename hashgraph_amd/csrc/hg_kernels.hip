@@ -3390,6 +3390,7 @@ hipError_t set_kernel_attributes() {
   HG_SET(&k_range_hist<uint64_t>);
   HG_SET_D(set_rmi_kernel_attributes());
   HG_SET_D(set_direct_kernel_attributes());
+  HG_SET_D(set_deep_kernel_attributes());
 #undef HG_SET
 #undef HG_SET_D
   return e;

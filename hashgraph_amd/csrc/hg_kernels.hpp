@@ -150,6 +150,43 @@ struct LaunchNarrow {
   unsigned int *zero_col;      // ncols more (or null)
 };
 
+// Two-step partition: keys whose bins lie in [bin_lo, bin_lo + nbins) into
+// nfine buckets of fine.d bins, by way of ngroups groups of `group` buckets;
+// key range r of per keys is counted in row r.
+constexpr uint32_t DEEP_ROWS = 256;     // a histogram workgroup on every CU
+constexpr uint32_t DEEP_GROUPS = 256;
+constexpr uint32_t DEEP_FINE = 39424;   // a counter each in the histogram's LDS
+struct DeepGeom {
+  uint64_t n, nbins;
+  uint32_t per, nfine, group, ngroups, bin_lo;
+  Div32 fine, coarse;
+  BinMap map;  // murmur3
+};
+struct DeepChunk {
+  uint32_t start, count, group, pad;
+};
+struct LaunchDeep {
+  int key_bytes;
+  bool pack;                   // 32-bit keys made into 8-byte records (key_bytes 8)
+  uint32_t rows;
+  DeepGeom geom;
+  const void *keys;
+  void *mid, *out;             // n keys each: grouped, then in buckets
+  uint32_t *cmat, *fmat;       // DEEP_ROWS * ngroups, DEEP_ROWS * nfine
+  uint32_t *ftot, *fstart;     // nfine, nfine + 1
+  uint32_t *gstart;            // 8 * ngroups
+  DeepChunk *chunks;           // deep_max_chunks
+  uint32_t *nchunks;
+  FinItem *items;              // nfine
+  BinMap *maps;                // one
+  unsigned long long *zero;    // as in LaunchNarrow
+  uint32_t nzero;
+  unsigned int *zero_col;      // nfine more (or null)
+};
+uint32_t deep_max_chunks(const DeepGeom &g, int key_bytes);
+hipError_t launch_deep(const LaunchDeep &p, hipStream_t st);
+hipError_t set_deep_kernel_attributes();
+
 // Bins longer than this are not walked by the probe kernels but answered from
 // a value table by k_probe_heavy (duplicates: a walk would cost
 // |A_bin| x |B_bin| comparisons).

@@ -17,6 +17,7 @@
 #include "hg_common.hpp"
 #include "hg_device.hpp"
 #include "hg_kernels.hpp"
+#include "hg_scatter.hpp"
 
 namespace hg {
 
@@ -75,11 +76,8 @@ __global__ __launch_bounds__(1024) void k_narrow_scan(uint32_t *__restrict__ cma
   }
 }
 
-// Scatter of key range g.  A tile of NB*KPT keys is ranked with LDS atomics,
-// staged bucket by bucket in LDS and written run by run; thread b carries
-// bucket b's next place in a register from tile to tile.  44-53 KB of LDS, so
-// three workgroups share a CU and one's loads and stores run under another's
-// LDS phases.  Workgroup 0 also writes the final stage's items.
+// Scatter of key range g, tile by tile (scatter_tile); thread b carries bucket
+// b's next place in a register.  Workgroup 0 also writes the final stage's items.
 // PACK: the keys are 32-bit and the output 8-byte records (position << 32 | key).
 template <typename K, int HK, bool PACK>
 __global__ __launch_bounds__(NB) void k_narrow_scatter(const void *__restrict__ keys, NarrowGeom g,
@@ -88,18 +86,14 @@ __global__ __launch_bounds__(NB) void k_narrow_scatter(const void *__restrict__ 
                                                        FinItem *__restrict__ items, BinMap *__restrict__ maps,
                                                        unsigned long long *__restrict__ zero, uint32_t nzero,
                                                        unsigned int *__restrict__ zero_col) {
-  constexpr int KPT = sizeof(K) == 4 ? 16 : 8;
-  constexpr uint32_t T = NB * KPT;
+  constexpr uint32_t T = scatter_tile_keys<K>(NB);
   using IN = typename std::conditional<PACK, uint32_t, K>::type;
-  __shared__ K s_key[T];
-  __shared__ uint16_t s_bkt[T];
-  __shared__ uint32_t s_cnt[NARROW_COLS], s_adj[NARROW_COLS];
-  __shared__ uint32_t s_tmp[NB / 64 + 1];
+  __shared__ ScatterLds<K, NB> s;
   const uint32_t b = threadIdx.x;
   const bool col = b < g.ncols;
   const uint32_t mine = col ? tot[b] : 0u;
   uint32_t all;
-  const uint32_t start = block_exclusive_sum<NB, uint32_t>(mine, s_tmp, all);
+  const uint32_t start = block_exclusive_sum<NB, uint32_t>(mine, s.tmp, all);
   if (blockIdx.x == 0) {
     if (col) {
       FinItem it;
@@ -121,50 +115,14 @@ __global__ __launch_bounds__(NB) void k_narrow_scatter(const void *__restrict__ 
   uint32_t next = col ? start + cmat[(uint64_t)blockIdx.x * g.ncols + b] : 0u;
   const uint64_t k0 = (uint64_t)blockIdx.x * g.per;
   const uint32_t n = (uint32_t)min((uint64_t)g.per, g.n - k0);
-  const IN *kp = (const IN *)keys + k0;
-  for (uint32_t base = 0; base < n; base += T) {
-    const uint32_t cnt = min(T, n - base);
-    const __amdgpu_buffer_rsrc_t rs = make_rsrc(kp + base, cnt * (uint32_t)sizeof(IN));
-    IN kr[KPT];
-#pragma unroll
-    for (int j = 0; j < KPT; j++)
-      kr[j] = buf_load<IN>(rs, threadIdx.x * (uint32_t)sizeof(IN), j * NB * (uint32_t)sizeof(IN));
-    if (col) s_cnt[b] = 0;
-    __syncthreads();
-    uint32_t pk[KPT];
-#pragma unroll
-    for (int j = 0; j < KPT; j++) pk[j] = divq(bin_of<IN, HK>(kr[j], g.map) - g.bin_lo, g.div);
-#pragma unroll
-    for (int j = 0; j < KPT; j++)
-      if (j * NB + threadIdx.x < cnt) pk[j] = (pk[j] << 16) | atomicAdd(&s_cnt[pk[j]], 1u);
-    __syncthreads();
-    const uint32_t c = col ? s_cnt[b] : 0u;
-    uint32_t tt;
-    const uint32_t ex = block_exclusive_sum<NB, uint32_t>(c, s_tmp, tt);
-    if (col) {
-      s_cnt[b] = ex;
-      s_adj[b] = next - ex;
-      next += c;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int j = 0; j < KPT; j++)
-      if (j * NB + threadIdx.x < cnt) {
-        const uint32_t q = s_cnt[pk[j] >> 16] + (pk[j] & 0xFFFFu);
-        if constexpr (PACK)
-          s_key[q] = ((k0 + base + j * NB + threadIdx.x) << 32) | kr[j];
-        else
-          s_key[q] = kr[j];
-        s_bkt[q] = (uint16_t)(pk[j] >> 16);
-      }
-    __syncthreads();
-#pragma unroll
-    for (int j = 0; j < KPT; j++) {
-      const uint32_t q = j * NB + threadIdx.x;
-      if (q < cnt) out[s_adj[s_bkt[q]] + q] = s_key[q];
-    }
-    __syncthreads();
-  }
+  for (uint32_t base = 0; base < n; base += T)
+    scatter_tile<K, NB, PACK>(keys, k0 + base, min(T, n - base), g.ncols, s, out,
+                              [&](IN key) { return divq(bin_of<IN, HK>(key, g.map) - g.bin_lo, g.div); },
+                              [&](uint32_t c) {
+                                const uint32_t at = next;
+                                next += c;
+                                return at;
+                              });
 }
 
 namespace {

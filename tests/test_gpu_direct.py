@@ -271,3 +271,54 @@ def test_batch_of_many_tables_skewed(kb, dev):
         bo, bk = o.build_csr(probes[t], n)
         exp.append(o.intersect(eo, ek, bo, bk)[0])
     assert counts.cpu().numpy().tolist() == exp and total == sum(exp)
+
+
+def _csr_matches(hg, dk, off, csr, M):
+    """Table of dk on the device: degrees, bins in order, the same keys."""
+    import torch
+    deg = torch.bincount(hg.table_bins(dk, M).to(torch.int64) & 0xFFFFFFFF, minlength=M)
+    assert int(off[0]) == 0 and torch.equal(off[1:].to(torch.int64) & 0xFFFFFFFF, torch.cumsum(deg, 0))
+    assert torch.equal(hg.table_bins(csr, M).to(torch.int64) & 0xFFFFFFFF,
+                       torch.repeat_interleave(torch.arange(M, device=dk.device), deg))
+    assert torch.equal(torch.sort(csr).values, torch.sort(dk).values)
+
+
+# two-step partitions: as many keys as bins, long bins, a table of few keys a
+# bin (every bucket at its widest), sizes that leave short rows and tiles
+@pytest.mark.parametrize("kb,ob", [(4, 4), (8, 8)])
+@pytest.mark.parametrize("n,M", [(15000011, 15000017), (20000003, 1000003), (16777217, 900000011), (40000003, 39999983)])
+def test_two_step_build_and_probe(n, M, kb, ob, dev):
+    import torch
+    import hashgraph_amd as hg
+    print(f"two-step n={n} M={M} kb={kb} ob={ob}", flush=True)
+    dk = wl.uniform_keys(n, n, kb, device=dev)
+    dk[5:3000] = dk[5]                 # a long bin
+    dk[1000000:1009000] = dk[1000000]  # a bucket beyond the small class
+    off, csr = hg.build(dk, M, offset_bytes=ob)
+    _csr_matches(hg, dk, off, csr, M)
+    q = wl.probe_keys(dk, n + 1, n // 2 + 1, 0.3, kb, device=dev)
+    q[100:50000] = dk[77]              # a bucket of B beyond every class
+    cnt, out = hg.probe(off, csr, M, q)
+    vals, num = torch.unique(csr, return_counts=True)
+    at = torch.searchsorted(vals, q).clamp_(max=vals.numel() - 1)
+    m = torch.where(vals[at] == q, num[at], 0)
+    assert cnt == int(m.sum())
+    assert torch.equal(torch.sort(out).values, torch.sort(torch.repeat_interleave(q, m)).values)
+
+
+@pytest.mark.parametrize("kb", [4, 8])
+def test_two_step_build_in_place_and_indexed(kb, dev):
+    """The CSR written over the input keys; the index-carrying form; one value
+    in more copies than a bucket, a group's share of them, half the table."""
+    import torch
+    import hashgraph_amd as hg
+    n, M = 16000001, 15000013
+    dk = wl.uniform_keys(3, n, kb, device=dev)
+    off, csr, ind = hg.build_indexed(dk, M)
+    _csr_matches(hg, dk, off, csr, M)
+    assert torch.equal(dk[ind], csr) and torch.equal(torch.sort(ind).values, torch.arange(n, device=dev))
+    dk[::2] = dk[1]
+    keep = dk.clone()
+    off = torch.empty(M + 1, dtype=torch.int32, device=dev)
+    hg.build(dk, M, out=(off, dk))
+    _csr_matches(hg, keep, off, dk, M)
