@@ -29,7 +29,7 @@ DEVFLAGS = ["-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", "-ffp-c
 CFLAGS = ["-O3", "-std=c++17", "-fPIC", "-Wall", "-Wno-unused-function", f"--offload-arch={ARCH}",
           "-I", os.path.join(ROOT, "include"), "-I", CSRC]
 
-SOURCES = ["hg_kernels.hip", "hg_direct.hip", "hg_narrow.hip", "hg_deep.hip", "hg_rmi.hip", "hg_engine.cpp",
+SOURCES = ["hg_kernels.hip", "hg_direct.hip", "hg_narrow.hip", "hg_deep.hip", "hg_stage.hip", "hg_rmi.hip", "hg_engine.cpp",
            "SingleHashGraph.cpp", "MultiHashGraph.cpp"]
 # driver programs: name -> (source, extra flags).  multi-hash-32,
 # multi-hash-idx and the -managed ones are the reference's B32, INDEX_TRACK

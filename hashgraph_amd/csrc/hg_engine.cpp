@@ -2602,6 +2602,23 @@ bool device_only(const void *p) {
   return a.type == hipMemoryTypeDevice;
 }
 
+// Device address of a range of pinned host memory that kernels can write, else
+// null (pageable, managed or device memory, a range beyond its allocation,
+// elements of kb bytes off their alignment).
+void *mapped_host(const void *p, size_t bytes, int kb) {
+  hipPointerAttribute_t a{}, e{};
+  if ((uintptr_t)p % (size_t)kb) return nullptr;
+  if (hipPointerGetAttributes(&a, p) != hipSuccess ||
+      hipPointerGetAttributes(&e, (const char *)p + bytes - 1) != hipSuccess) {
+    (void)hipGetLastError();
+    return nullptr;
+  }
+  if (a.type != hipMemoryTypeHost || e.type != hipMemoryTypeHost || !a.devicePointer ||
+      (char *)a.devicePointer + bytes - 1 != (char *)e.devicePointer)
+    return nullptr;
+  return a.devicePointer;
+}
+
 hg_status stage_streams(hg_ctx c, StageStreams &s) {
   if (!c->st_in) HG_HIP(hipStreamCreateWithFlags(&c->st_in, hipStreamNonBlocking));
   if (!c->st_out) HG_HIP(hipStreamCreateWithFlags(&c->st_out, hipStreamNonBlocking));
@@ -2637,37 +2654,50 @@ hg_status staged_partitioned(hg_ctx c, const hg_table_desc *desc, const void *h_
   const uint64_t nch = (n + C - 1) / C;
   // passes 1 and 2: arena 3 = two upload buffers and two partition buffers
   Plan P3;
-  const size_t i_in0 = P3.add(C * kb), i_in1 = P3.add(C * kb), i_pt0 = P3.add(C * kb), i_pt1 = P3.add(C * kb);
+  const size_t i_in0 = P3.add(C * kb), i_in1 = P3.add(C * kb), i_pt0 = P3.add(C * kb), i_pt1 = P3.add(C * kb),
+               i_acc = P3.add((size_t)np * 8), i_slab = P3.add((size_t)np * sizeof(StageSlab)),
+               i_cur = P3.add(((size_t)np + 1) * 8), i_mv0 = P3.add((size_t)np * sizeof(StageMove)),
+               i_mv1 = P3.add((size_t)np * sizeof(StageMove));
   HG_TRY(arena_ensure(c, 3, P3.total()));
   Carve cv3;
   cv3.init(c, 3, P3);
   char *d_in[2] = {cv3.get<char>(i_in0), cv3.get<char>(i_in1)};
   char *d_pt[2] = {cv3.get<char>(i_pt0), cv3.get<char>(i_pt1)};
   // chunk j goes to buffer j & 1 once chunk j - 2's kernels are done with it
-  auto upload = [&](uint64_t j) -> hg_status {
+  auto upload_chunk = [&](uint64_t j) -> hg_status {
     const int b = (int)(j & 1);
     if (j >= 2) HG_HIP(hipStreamWaitEvent(ss->in, ss->ev_done[b], 0));
     HG_TRY(stage_copy(ss->in, d_in[b], (const char *)h_keys + j * C * kb, std::min(C, n - j * C) * kb));
     HG_HIP(hipEventRecord(ss->ev_in[b], ss->in));
     return HG_OK;
   };
-  std::vector<uint32_t> cnt(np + 1), st(np + 1);
-  // pass 1: keys per piece
-  std::vector<uint64_t> T(np, 0);
-  if (nch) HG_TRY(upload(0));
+  // the piece level of a chunk of m keys, laid out and uploaded when m changes
+  // (an upload waits behind the next chunk's in the copy engine)
+  Level L;
+  LevelDev d;
+  uint64_t laid = 0;
+  auto level = [&](uint64_t m) -> hg_status {
+    if (m == laid) return HG_OK;
+    laid = m;
+    L = Level();
+    piece_level(L, map, pc, m);
+    return setup_level(c, L, d);
+  };
+  // pass 1: keys per piece, summed on the device
+  unsigned long long *acc = cv3.get<unsigned long long>(i_acc);
+  HG_HIP(launch_fill_u64(acc, 0ull, np, c->stream));
+  if (nch) HG_TRY(upload_chunk(0));
   for (uint64_t j = 0; j < nch; j++) {
     const int b = (int)(j & 1);
-    if (j + 1 < nch) HG_TRY(upload(j + 1));
+    if (j + 1 < nch) HG_TRY(upload_chunk(j + 1));
     HG_HIP(hipStreamWaitEvent(c->stream, ss->ev_in[b], 0));
-    Level L;
-    piece_level(L, map, pc, std::min(C, n - j * C));
-    LevelDev d;
-    HG_TRY(setup_level(c, L, d));
+    HG_TRY(level(std::min(C, n - j * C)));
     HG_TRY(run_level(c, L, d, kb, d_in[b], nullptr, false));
+    HG_HIP(launch_stage_count(d.coltot, np, acc, c->stream));
     HG_HIP(hipEventRecord(ss->ev_done[b], c->stream));
-    HG_TRY(sync_read(c, cnt.data(), d.coltot, (np + 1) * 4));
-    for (uint32_t p = 0; p < np; p++) T[p] += cnt[p];
   }
+  std::vector<uint64_t> T(np, 0);
+  HG_TRY(sync_read(c, T.data(), acc, (size_t)np * 8));
   // slabs: consecutive pieces of one partition within the budget
   std::vector<Slab> slabs;
   std::vector<uint64_t> po(n_parts + 1, 0);
@@ -2696,24 +2726,44 @@ hg_status staged_partitioned(hg_ctx c, const hg_table_desc *desc, const void *h_
   }
   for (const Slab &sl : slabs) po[sl.part + 1] += sl.count;
   for (uint32_t p = 0; p < n_parts; p++) po[p + 1] += po[p];
-  // pass 2: every chunk's share of a slab goes to the slab's final region
-  std::vector<uint64_t> cur(slabs.size(), 0);
-  if (nch) HG_TRY(upload(0));
+  // pass 2: every chunk's share of a slab goes to the slab's final region.
+  // Pinned memory is written by one kernel a chunk, which takes the shares from
+  // the device's own counts; a copy a slab (28 slabs: 0.67 ms a chunk of 5.5 MB,
+  // nearly all of it the host's calls) and a read-back a chunk serve the rest.
+  StageMove *mv[2] = {cv3.get<StageMove>(i_mv0), cv3.get<StageMove>(i_mv1)};
+  unsigned long long *d_cur = cv3.get<unsigned long long>(i_cur);  // keys placed per slab; then: a share did not fit
+  const uint32_t ns = (uint32_t)slabs.size();
+  void *const map_csr = n ? mapped_host(h_csr, n * kb, kb) : nullptr;
+  void *const map_off = mapped_host(h_off, ((uint64_t)splits[n_parts] + n_parts) * ob, ob);
+  std::vector<uint64_t> cur(ns + 1, 0);
+  std::vector<uint32_t> cnt(np + 1), st(np + 1);
+  if (map_csr) {
+    std::vector<StageSlab> tab;
+    for (const Slab &sl : slabs) tab.push_back({sl.p0, sl.p1, sl.pos, sl.count});
+    HG_TRY(upload(c, cv3.get<void>(i_slab), tab.data(), tab.size() * sizeof(StageSlab)));
+    HG_HIP(launch_fill_u64(d_cur, 0ull, ns + 1, c->stream));
+  }
+  if (nch) HG_TRY(upload_chunk(0));
   for (uint64_t j = 0; j < nch; j++) {
     const int b = (int)(j & 1);
-    if (j + 1 < nch) HG_TRY(upload(j + 1));
+    if (j + 1 < nch) HG_TRY(upload_chunk(j + 1));
     HG_HIP(hipStreamWaitEvent(c->stream, ss->ev_in[b], 0));
     if (j >= 2) HG_HIP(hipStreamWaitEvent(c->stream, ss->ev_out[b], 0));  // chunk j - 2's copies are out
-    Level L;
-    piece_level(L, map, pc, std::min(C, n - j * C));
-    LevelDev d;
-    HG_TRY(setup_level(c, L, d));
+    HG_TRY(level(std::min(C, n - j * C)));
     HG_TRY(run_level(c, L, d, kb, d_in[b], d_pt[b]));
+    if (map_csr)
+      HG_HIP(launch_stage_shares(d.bstart, d.coltot, cv3.get<StageSlab>(i_slab), ns, d_cur, mv[b], c->stream));
     HG_HIP(hipEventRecord(ss->ev_done[b], c->stream));
+    if (map_csr) {
+      HG_HIP(hipStreamWaitEvent(ss->out, ss->ev_done[b], 0));
+      HG_HIP(launch_stage_out(d_pt[b], map_csr, kb, mv[b], ns, ss->out));
+      HG_HIP(hipEventRecord(ss->ev_out[b], ss->out));
+      continue;
+    }
     HG_TRY(sync_read(c, cnt.data(), d.coltot, (np + 1) * 4));
     HG_TRY(sync_read(c, st.data(), d.bstart, (np + 1) * 4));
     HG_HIP(hipStreamWaitEvent(ss->out, ss->ev_done[b], 0));
-    for (size_t s = 0; s < slabs.size(); s++) {
+    for (size_t s = 0; s < ns; s++) {
       const Slab &sl = slabs[s];
       const uint64_t a = st[sl.p0], e = (uint64_t)st[sl.p1 - 1] + cnt[sl.p1 - 1];
       if (cur[s] + (e - a) > sl.count) return fail(HG_ERR_DEVICE, "staged build: keys changed between passes");
@@ -2722,8 +2772,9 @@ hg_status staged_partitioned(hg_ctx c, const hg_table_desc *desc, const void *h_
     }
     HG_HIP(hipEventRecord(ss->ev_out[b], ss->out));
   }
-  for (size_t s = 0; s < slabs.size(); s++)
-    if (cur[s] != slabs[s].count) return fail(HG_ERR_DEVICE, "staged build: keys changed between passes");
+  if (map_csr) HG_TRY(sync_read(c, cur.data(), d_cur, ((size_t)ns + 1) * 8));
+  for (size_t s = 0; s < ns; s++)
+    if (cur[ns] || cur[s] != slabs[s].count) return fail(HG_ERR_DEVICE, "staged build: keys changed between passes");
   HG_HIP(hipStreamSynchronize(ss->out));
   HG_HIP(hipStreamSynchronize(ss->in));
   // pass 3: arena 3 = two upload, two CSR and two offsets buffers
@@ -2752,11 +2803,19 @@ hg_status staged_partitioned(hg_ctx c, const hg_table_desc *desc, const void *h_
     if (s >= 2) HG_HIP(hipStreamWaitEvent(c->stream, ss->ev_out[b], 0));  // slab s - 2's copies are out
     HG_TRY(build_range(c, map, kb, ob, sl.count, sl.lo, sl.R, s_in[b], s_off[b], s_out[b]));
     // offsets of a partitioned table count from the partition's first key
-    HG_HIP(launch_offsets_add(s_off[b], ob, sl.R + 1, sl.pos - po[sl.part], c->stream));
-    HG_HIP(hipEventRecord(ss->ev_done[b], c->stream));
-    HG_HIP(hipStreamWaitEvent(ss->out, ss->ev_done[b], 0));
-    HG_TRY(stage_copy(ss->out, (char *)h_csr + sl.pos * kb, s_out[b], sl.count * kb));
-    HG_TRY(stage_copy(ss->out, (char *)h_off + (sl.lo + sl.part) * ob, s_off[b], (sl.R + 1) * ob));
+    const uint64_t add = sl.pos - po[sl.part], at = sl.lo + sl.part;
+    if (map_csr && map_off) {
+      HG_HIP(hipEventRecord(ss->ev_done[b], c->stream));
+      HG_HIP(hipStreamWaitEvent(ss->out, ss->ev_done[b], 0));
+      HG_HIP(launch_stage_back(s_out[b], (char *)map_csr + sl.pos * kb, kb, sl.count, s_off[b],
+                               (char *)map_off + at * ob, ob, sl.R + 1, add, ss->out));
+    } else {
+      HG_HIP(launch_offsets_add(s_off[b], ob, sl.R + 1, add, c->stream));
+      HG_HIP(hipEventRecord(ss->ev_done[b], c->stream));
+      HG_HIP(hipStreamWaitEvent(ss->out, ss->ev_done[b], 0));
+      HG_TRY(stage_copy(ss->out, (char *)h_csr + sl.pos * kb, s_out[b], sl.count * kb));
+      HG_TRY(stage_copy(ss->out, (char *)h_off + at * ob, s_off[b], (sl.R + 1) * ob));
+    }
     HG_HIP(hipEventRecord(ss->ev_out[b], ss->out));
   }
   HG_HIP(hipStreamSynchronize(ss->out));
@@ -2811,9 +2870,9 @@ struct JoinStage {
   uint32_t used = 0;  // emissions so far (a buffer is waited for from its second use on)
 };
 
-// Matches of bins [x, y) of the slab: counted, then emitted into a stage
-// buffer and copied to the host list when they fit it (else the range is
-// halved).
+// Matches of bins [x, y) of the slab: emitted into a stage buffer and copied
+// to the host list when they fit it (else the range is halved); counted only
+// when the caller wants no list or it is full.
 hg_status join_range(hg_ctx c, const StageStreams &ss, const hg_table_desc *descA, const void *h_offA,
                      const void *h_offB, const JoinSlab &js, uint64_t x, uint64_t y, JoinStage &stg, void *h_out,
                      uint64_t capacity, uint64_t &written, uint64_t &total, bool &full) {
@@ -2824,7 +2883,14 @@ hg_status join_range(hg_ctx c, const StageStreams &ss, const hg_table_desc *desc
   dB.n_keys = off_at(h_offB, ob, y) - off_at(h_offB, ob, x);
   const void *oa = (const char *)js.offA + (x - js.lo) * ob, *obp = (const char *)js.offB + (x - js.lo) * ob;
   uint64_t cnt = 0;
-  HG_TRY(hg_intersect(c, &dA, oa, js.keysA, &dB, obp, js.keysB, nullptr, 0, &cnt));
+  const int e = stg.next;
+  if (h_out && !full) {
+    if (stg.used >= 2) HG_HIP(hipStreamWaitEvent(c->stream, ss.ev_out[e], 0));  // its last copy back is done
+    const hg_status st = hg_intersect(c, &dA, oa, js.keysA, &dB, obp, js.keysB, stg.buf[e], stg.cap, &cnt);
+    if (st != HG_OK && st != HG_ERR_CAPACITY) return st;
+  } else {
+    HG_TRY(hg_intersect(c, &dA, oa, js.keysA, &dB, obp, js.keysB, nullptr, 0, &cnt));
+  }
   total += cnt;
   if (!h_out || full || cnt == 0) return HG_OK;
   if (written + cnt > capacity) {
@@ -2841,11 +2907,6 @@ hg_status join_range(hg_ctx c, const StageStreams &ss, const hg_table_desc *desc
     HG_TRY(join_range(c, ss, descA, h_offA, h_offB, js, x, m, stg, h_out, capacity, written, total, full));
     return join_range(c, ss, descA, h_offA, h_offB, js, m, y, stg, h_out, capacity, written, total, full);
   }
-  const int e = stg.next;
-  if (stg.used >= 2) HG_HIP(hipStreamWaitEvent(c->stream, ss.ev_out[e], 0));  // its last copy back is done
-  uint64_t got = 0;
-  HG_TRY(hg_intersect(c, &dA, oa, js.keysA, &dB, obp, js.keysB, stg.buf[e], stg.cap, &got));
-  if (got != cnt) return fail(HG_ERR_DEVICE, "staged intersect: count changed between passes");
   // hg_intersect has synchronised the context's stream: the matches are in place
   HG_TRY(stage_copy(ss.out, (char *)h_out + written * kb, stg.buf[e], cnt * kb));
   HG_HIP(hipEventRecord(ss.ev_out[e], ss.out));
@@ -2956,18 +3017,16 @@ hg_status hg_intersect_staged(hg_ctx c, const hg_table_desc *descA, const void *
     device_budget = fr / 2;
   }
   if (device_budget < kStageMinBudget) return fail(HG_ERR_INVALID_ARG, "device_budget below 4 MiB");
-  // two slab buffers (each a quarter of the budget for keys of A and B and a
-  // twentieth for each table's offsets) and two stage buffers (an eighth each)
+  // two slab buffers (0.35 of the budget each, shared by both tables' keys and
+  // offsets as the slab has them) and two stage buffers (an eighth each)
   const uint64_t kmax = std::min<uint64_t>((uint64_t)(0.25 * (double)device_budget / kb), kStageMaxChunk);
-  const uint64_t rmax = std::min<uint64_t>((uint64_t)(0.05 * (double)device_budget / ob), (1ull << 32) - 2);
+  const size_t slab_bytes = (size_t)(0.35 * (double)device_budget);
   JoinStage stg;
   stg.cap = (uint64_t)(0.125 * (double)device_budget / kb);
   Plan P3;
-  size_t i_k[2], i_oa[2], i_ob[2], i_st[2];
+  size_t i_slab[2], i_st[2];
   for (int b = 0; b < 2; b++) {
-    i_k[b] = P3.add(kmax * kb);
-    i_oa[b] = P3.add((rmax + 1) * ob);
-    i_ob[b] = P3.add((rmax + 1) * ob);
+    i_slab[b] = P3.add(slab_bytes + 4 * 256);
     i_st[b] = P3.add(stg.cap * kb);
   }
   StageStreams ss;
@@ -2980,10 +3039,10 @@ hg_status hg_intersect_staged(hg_ctx c, const hg_table_desc *descA, const void *
   auto keys_in = [&](uint64_t lo, uint64_t hi) {
     return (off_at(h_offA, ob, hi) - off_at(h_offA, ob, lo)) + (off_at(h_offB, ob, hi) - off_at(h_offB, ob, lo));
   };
-  // slabs: the largest hi with the keys within kmax and the bins within rmax
+  // slabs: the largest hi whose keys and offsets fit a slab buffer
   std::vector<JoinSlab> slabs;
   for (uint64_t lo = 0; lo < M;) {
-    uint64_t top = std::min<uint64_t>(M, lo + rmax);
+    uint64_t top = std::min<uint64_t>(M, lo + slab_bytes / (2 * ob));
     if (keys_in(lo, lo + 1) > kmax)
       return fail(HG_ERR_UNSUPPORTED, "bin " + std::to_string(lo) + " holds " + std::to_string(keys_in(lo, lo + 1)) +
                                           " keys of A and B, more than this device_budget stages (" +
@@ -2991,7 +3050,8 @@ hg_status hg_intersect_staged(hg_ctx c, const hg_table_desc *descA, const void *
     uint64_t good = lo + 1;
     while (good < top) {
       const uint64_t mid = good + (top - good + 1) / 2;
-      if (keys_in(lo, mid) <= kmax) good = mid;
+      const uint64_t k = keys_in(lo, mid);
+      if (k <= kStageMaxChunk && k * kb + 2 * (mid - lo + 1) * ob <= slab_bytes) good = mid;
       else top = mid - 1;
     }
     JoinSlab js;
@@ -3002,23 +3062,24 @@ hg_status hg_intersect_staged(hg_ctx c, const hg_table_desc *descA, const void *
     slabs.push_back(js);
     lo = good;
   }
-  // slab s uploads into buffer s & 1 (its offsets rebased on the upload
-  // stream) once slab s - 2's joins are done with it
+  // slab s uploads into buffer s & 1 once slab s - 2's joins are done with it;
+  // its offsets are rebased before its join
   auto upload = [&](size_t s) -> hg_status {
     const int b = (int)(s & 1);
     JoinSlab &js = slabs[s];
     const uint64_t na = off_at(h_offA, ob, js.hi) - js.a0, nb = off_at(h_offB, ob, js.hi) - js.b0;
-    js.keysA = cv3.get<char>(i_k[b]);
-    js.keysB = js.keysA + na * kb;
-    js.offA = cv3.get<void>(i_oa[b]);
-    js.offB = cv3.get<void>(i_ob[b]);
+    const auto up = [](uint64_t x) { return (x + 255) & ~255ull; };
+    const uint64_t no = up((js.hi - js.lo + 1) * ob);
+    char *const buf = cv3.get<char>(i_slab[b]);
+    js.offA = buf;
+    js.offB = buf + no;
+    js.keysA = buf + 2 * no;
+    js.keysB = js.keysA + up(na * kb);
     if (s >= 2) HG_HIP(hipStreamWaitEvent(ss.in, ss.ev_done[b], 0));
     HG_TRY(stage_copy(ss.in, js.keysA, (const char *)h_keysA + js.a0 * kb, na * kb));
     HG_TRY(stage_copy(ss.in, js.keysB, (const char *)h_keysB + js.b0 * kb, nb * kb));
     HG_TRY(stage_copy(ss.in, js.offA, (const char *)h_offA + js.lo * ob, (js.hi - js.lo + 1) * ob));
     HG_TRY(stage_copy(ss.in, js.offB, (const char *)h_offB + js.lo * ob, (js.hi - js.lo + 1) * ob));
-    HG_HIP(launch_offsets_add(js.offA, ob, js.hi - js.lo + 1, (uint64_t)0 - js.a0, ss.in));
-    HG_HIP(launch_offsets_add(js.offB, ob, js.hi - js.lo + 1, (uint64_t)0 - js.b0, ss.in));
     HG_HIP(hipEventRecord(ss.ev_in[b], ss.in));
     return HG_OK;
   };
@@ -3029,6 +3090,11 @@ hg_status hg_intersect_staged(hg_ctx c, const hg_table_desc *descA, const void *
     const int b = (int)(s & 1);
     if (s + 1 < slabs.size()) HG_TRY(upload(s + 1));
     HG_HIP(hipStreamWaitEvent(c->stream, ss.ev_in[b], 0));
+    {
+      const JoinSlab &js = slabs[s];
+      HG_HIP(launch_offsets_add(js.offA, ob, js.hi - js.lo + 1, (uint64_t)0 - js.a0, c->stream));
+      HG_HIP(launch_offsets_add(js.offB, ob, js.hi - js.lo + 1, (uint64_t)0 - js.b0, c->stream));
+    }
     HG_TRY(join_range(c, ss, descA, h_offA, h_offB, slabs[s], slabs[s].lo, slabs[s].hi, stg, h_out, capacity,
                       written, total, full));
     HG_HIP(hipEventRecord(ss.ev_done[b], c->stream));

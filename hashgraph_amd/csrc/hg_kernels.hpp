@@ -187,6 +187,29 @@ uint32_t deep_max_chunks(const DeepGeom &g, int key_bytes);
 hipError_t launch_deep(const LaunchDeep &p, hipStream_t st);
 hipError_t set_deep_kernel_attributes();
 
+// Staged builds: a slab's pieces [p0, p1) and its place among the CSR keys; a
+// chunk's share of it (keys [src, src + count) of the chunk to dst).
+struct StageSlab {
+  uint32_t p0, p1;
+  uint64_t pos, count;
+};
+struct StageMove {
+  uint64_t src, dst, count;
+};
+// acc[p] += tot[p]
+hipError_t launch_stage_count(const uint32_t *tot, uint32_t np, unsigned long long *acc, hipStream_t st);
+// shares of a chunk whose piece p holds tot[p] keys from bstart[p] on; cur[s]:
+// keys of slab s placed so far, cur[ns] set when a share does not fit its slab
+hipError_t launch_stage_shares(const uint32_t *bstart, const uint32_t *tot, const StageSlab *slabs, uint32_t ns,
+                               unsigned long long *cur, StageMove *mv, hipStream_t st);
+// the shares written to pinned host memory (its device address)
+hipError_t launch_stage_out(const void *keys, void *host, int key_bytes, const StageMove *mv, uint32_t ns,
+                            hipStream_t st);
+
+// a built slab's CSR keys and its offsets (each plus add) to pinned host memory
+hipError_t launch_stage_back(const void *keys, void *host_keys, int key_bytes, uint64_t n, const void *off,
+                             void *host_off, int off_bytes, uint64_t noff, uint64_t add, hipStream_t st);
+
 // Bins longer than this are not walked by the probe kernels but answered from
 // a value table by k_probe_heavy (duplicates: a walk would cost
 // |A_bin| x |B_bin| comparisons).
