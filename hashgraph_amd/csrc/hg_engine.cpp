@@ -2656,7 +2656,7 @@ hg_status staged_partitioned(hg_ctx c, const hg_table_desc *desc, const void *h_
   Plan P3;
   const size_t i_in0 = P3.add(C * kb), i_in1 = P3.add(C * kb), i_pt0 = P3.add(C * kb), i_pt1 = P3.add(C * kb),
                i_acc = P3.add((size_t)np * 8), i_slab = P3.add((size_t)np * sizeof(StageSlab)),
-               i_cur = P3.add(((size_t)np + 1) * 8), i_mv0 = P3.add((size_t)np * sizeof(StageMove)),
+               i_bound = P3.add(((size_t)np + 1) * 4), i_cur = P3.add(((size_t)np + 1) * 8), i_mv0 = P3.add((size_t)np * sizeof(StageMove)),
                i_mv1 = P3.add((size_t)np * sizeof(StageMove));
   HG_TRY(arena_ensure(c, 3, P3.total()));
   Carve cv3;
@@ -2727,20 +2727,42 @@ hg_status staged_partitioned(hg_ctx c, const hg_table_desc *desc, const void *h_
   for (const Slab &sl : slabs) po[sl.part + 1] += sl.count;
   for (uint32_t p = 0; p < n_parts; p++) po[p + 1] += po[p];
   // pass 2: every chunk's share of a slab goes to the slab's final region.
-  // Pinned memory is written by one kernel a chunk, which takes the shares from
-  // the device's own counts; a copy a slab (28 slabs: 0.67 ms a chunk of 5.5 MB,
-  // nearly all of it the host's calls) and a read-back a chunk serve the rest.
+  // Up to 511 slabs in pinned memory: the chunk is partitioned by slab and one
+  // kernel writes the shares, which the device counts itself.  Else it is
+  // partitioned by piece, its counts are read back and every share is a copy
+  // (28 slabs: 0.67 ms a chunk of 5.5 MB, nearly all of it the host's calls).
   StageMove *mv[2] = {cv3.get<StageMove>(i_mv0), cv3.get<StageMove>(i_mv1)};
   unsigned long long *d_cur = cv3.get<unsigned long long>(i_cur);  // keys placed per slab; then: a share did not fit
   const uint32_t ns = (uint32_t)slabs.size();
   void *const map_csr = n ? mapped_host(h_csr, n * kb, kb) : nullptr;
   void *const map_off = mapped_host(h_off, ((uint64_t)splits[n_parts] + n_parts) * ob, ob);
+  const bool by_slab = map_csr && ns && ns < NARROW_COLS;
+  LaunchStagePart sp{};
   std::vector<uint64_t> cur(ns + 1, 0);
   std::vector<uint32_t> cnt(np + 1), st(np + 1);
-  if (map_csr) {
+  if (by_slab) {
     std::vector<StageSlab> tab;
-    for (const Slab &sl : slabs) tab.push_back({sl.p0, sl.p1, sl.pos, sl.count});
+    std::vector<uint32_t> bound;
+    for (const Slab &sl : slabs) {
+      tab.push_back({sl.pos, sl.count});
+      bound.push_back((uint32_t)sl.lo);
+    }
+    bound.push_back((uint32_t)pc.bounds[np]);
+    Plan P1;
+    const size_t i_cmat = P1.add((size_t)NARROW_ROWS * (ns + 1) * 4), i_tot = P1.add((ns + 1) * 4);
+    HG_TRY(arena_ensure(c, 1, P1.total()));
+    Carve cv1;
+    cv1.init(c, 1, P1);
+    sp.key_bytes = kb;
+    sp.map = map;
+    sp.ns = ns;
+    sp.bound = cv3.get<uint32_t>(i_bound);
+    sp.cmat = cv1.get<uint32_t>(i_cmat);
+    sp.tot = cv1.get<uint32_t>(i_tot);
+    sp.slabs = cv3.get<StageSlab>(i_slab);
+    sp.cur = d_cur;
     HG_TRY(upload(c, cv3.get<void>(i_slab), tab.data(), tab.size() * sizeof(StageSlab)));
+    HG_TRY(upload(c, cv3.get<void>(i_bound), bound.data(), bound.size() * 4));
     HG_HIP(launch_fill_u64(d_cur, 0ull, ns + 1, c->stream));
   }
   if (nch) HG_TRY(upload_chunk(0));
@@ -2749,17 +2771,24 @@ hg_status staged_partitioned(hg_ctx c, const hg_table_desc *desc, const void *h_
     if (j + 1 < nch) HG_TRY(upload_chunk(j + 1));
     HG_HIP(hipStreamWaitEvent(c->stream, ss->ev_in[b], 0));
     if (j >= 2) HG_HIP(hipStreamWaitEvent(c->stream, ss->ev_out[b], 0));  // chunk j - 2's copies are out
-    HG_TRY(level(std::min(C, n - j * C)));
-    HG_TRY(run_level(c, L, d, kb, d_in[b], d_pt[b]));
-    if (map_csr)
-      HG_HIP(launch_stage_shares(d.bstart, d.coltot, cv3.get<StageSlab>(i_slab), ns, d_cur, mv[b], c->stream));
-    HG_HIP(hipEventRecord(ss->ev_done[b], c->stream));
-    if (map_csr) {
+    if (by_slab) {
+      sp.keys = d_in[b];
+      sp.out = d_pt[b];
+      sp.n = (uint32_t)std::min(C, n - j * C);
+      sp.mv = mv[b];
+      {
+        Prof pf(c, "part_scatter");
+        HG_HIP(launch_stage_part(sp, c->stream));
+      }
+      HG_HIP(hipEventRecord(ss->ev_done[b], c->stream));
       HG_HIP(hipStreamWaitEvent(ss->out, ss->ev_done[b], 0));
       HG_HIP(launch_stage_out(d_pt[b], map_csr, kb, mv[b], ns, ss->out));
       HG_HIP(hipEventRecord(ss->ev_out[b], ss->out));
       continue;
     }
+    HG_TRY(level(std::min(C, n - j * C)));
+    HG_TRY(run_level(c, L, d, kb, d_in[b], d_pt[b]));
+    HG_HIP(hipEventRecord(ss->ev_done[b], c->stream));
     HG_TRY(sync_read(c, cnt.data(), d.coltot, (np + 1) * 4));
     HG_TRY(sync_read(c, st.data(), d.bstart, (np + 1) * 4));
     HG_HIP(hipStreamWaitEvent(ss->out, ss->ev_done[b], 0));
@@ -2772,7 +2801,7 @@ hg_status staged_partitioned(hg_ctx c, const hg_table_desc *desc, const void *h_
     }
     HG_HIP(hipEventRecord(ss->ev_out[b], ss->out));
   }
-  if (map_csr) HG_TRY(sync_read(c, cur.data(), d_cur, ((size_t)ns + 1) * 8));
+  if (by_slab) HG_TRY(sync_read(c, cur.data(), d_cur, ((size_t)ns + 1) * 8));
   for (size_t s = 0; s < ns; s++)
     if (cur[ns] || cur[s] != slabs[s].count) return fail(HG_ERR_DEVICE, "staged build: keys changed between passes");
   HG_HIP(hipStreamSynchronize(ss->out));

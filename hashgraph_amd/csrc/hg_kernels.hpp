@@ -187,21 +187,31 @@ uint32_t deep_max_chunks(const DeepGeom &g, int key_bytes);
 hipError_t launch_deep(const LaunchDeep &p, hipStream_t st);
 hipError_t set_deep_kernel_attributes();
 
-// Staged builds: a slab's pieces [p0, p1) and its place among the CSR keys; a
+// Staged builds: a slab's place among the CSR keys; a
 // chunk's share of it (keys [src, src + count) of the chunk to dst).
 struct StageSlab {
-  uint32_t p0, p1;
   uint64_t pos, count;
 };
 struct StageMove {
   uint64_t src, dst, count;
 };
+// Partition of a staged chunk into ns slabs (slab s: the bins [bound[s],
+// bound[s + 1])) and the keys of no slab, behind them.
+struct LaunchStagePart {
+  int key_bytes;
+  BinMap map;
+  const void *keys;
+  void *out;
+  uint32_t n, ns;           // ns < NARROW_COLS
+  const uint32_t *bound;    // ns + 1, ascending
+  uint32_t *cmat, *tot;     // NARROW_ROWS * (ns + 1), ns + 1
+  const StageSlab *slabs;
+  unsigned long long *cur;  // keys of each slab placed so far; [ns]: a share did not fit its slab
+  StageMove *mv;
+};
+hipError_t launch_stage_part(const LaunchStagePart &p, hipStream_t st);
 // acc[p] += tot[p]
 hipError_t launch_stage_count(const uint32_t *tot, uint32_t np, unsigned long long *acc, hipStream_t st);
-// shares of a chunk whose piece p holds tot[p] keys from bstart[p] on; cur[s]:
-// keys of slab s placed so far, cur[ns] set when a share does not fit its slab
-hipError_t launch_stage_shares(const uint32_t *bstart, const uint32_t *tot, const StageSlab *slabs, uint32_t ns,
-                               unsigned long long *cur, StageMove *mv, hipStream_t st);
 // the shares written to pinned host memory (its device address)
 hipError_t launch_stage_out(const void *keys, void *host, int key_bytes, const StageMove *mv, uint32_t ns,
                             hipStream_t st);
@@ -421,6 +431,8 @@ constexpr uint32_t RLE_GIANT_ZERO = 8;  // leading words of the control block cl
 hipError_t launch_part_hist(const LaunchPart &lp, hipStream_t st);
 hipError_t launch_part_scatter(const LaunchPart &lp, hipStream_t st);
 hipError_t launch_narrow(const LaunchNarrow &p, hipStream_t st);
+// columns of a count matrix to exclusive sums, their totals to tot
+hipError_t launch_narrow_scan(uint32_t *cmat, uint32_t rows, uint32_t ncols, uint32_t *tot, hipStream_t st);
 hipError_t launch_colscan(const LaunchCol &lc, hipStream_t st);
 hipError_t launch_final(const LaunchFinal &lf, hipStream_t st);
 // The one-pass kernel, then the kernels of the items and bins it left: they

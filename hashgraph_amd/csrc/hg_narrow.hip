@@ -125,6 +125,13 @@ __global__ __launch_bounds__(NB) void k_narrow_scatter(const void *__restrict__ 
                               });
 }
 
+hipError_t launch_narrow_scan(uint32_t *cmat, uint32_t rows, uint32_t ncols, uint32_t *tot, hipStream_t st) {
+  if (!rows || rows > NARROW_ROWS || !ncols || ncols > NARROW_COLS) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(k_narrow_scan, dim3((ncols + SCAN_COLS - 1) / SCAN_COLS), dim3(1024), 0, st, cmat, rows, ncols,
+                     tot);
+  return hipGetLastError();
+}
+
 namespace {
 
 template <typename K, int HK>
@@ -134,8 +141,8 @@ hipError_t launch_narrow_t(const LaunchNarrow &p, hipStream_t st) {
     hipLaunchKernelGGL((k_narrow_hist<uint32_t, HK>), dim3(p.rows), dim3(NB), 0, st, (const uint32_t *)p.keys, g, p.cmat);
   else
     hipLaunchKernelGGL((k_narrow_hist<K, HK>), dim3(p.rows), dim3(NB), 0, st, (const K *)p.keys, g, p.cmat);
-  hipLaunchKernelGGL(k_narrow_scan, dim3((g.ncols + SCAN_COLS - 1) / SCAN_COLS), dim3(1024), 0, st, p.cmat, p.rows,
-                     g.ncols, p.tot);
+  const hipError_t e = launch_narrow_scan(p.cmat, p.rows, g.ncols, p.tot, st);
+  if (e != hipSuccess) return e;
   auto kern = &k_narrow_scatter<K, HK, false>;
   if constexpr (sizeof(K) == 8 && HK == HK_MURMUR)
     if (p.pack) kern = &k_narrow_scatter<K, HK, true>;

@@ -294,3 +294,42 @@ def test_device_offsets_are_refused(dev):
     st = c.lib.hg_build_staged(c.bind_stream(), ctypes.byref(d), hg._hp(keys), ctypes.c_void_p(dout.data_ptr()),
                                hg._hp(csr), 4 * MiB)
     assert st == 1
+
+
+@pytest.mark.parametrize("kb,ob", [(4, 4), (8, 8)])
+def test_pinned_slabs_at_odd_places(kb, ob, dev):
+    """Pinned outputs that start one element off 16 bytes, many slabs and
+    chunks, a slab's worth of one key."""
+    import torch
+    import hashgraph_amd as hg
+    n, M = 700001, 650003
+    keys = wl.uniform_keys(17, n, kb)
+    keys[1000:30000] = keys[7]
+    csr = torch.empty(n + 1, dtype=torch.int32 if kb == 4 else torch.int64, pin_memory=True)[1:]
+    off = torch.empty(M + 2, dtype=torch.int32 if ob == 4 else torch.int64, pin_memory=True)[1:]
+    hg.build_staged(_host_keys(keys, True), M, offset_bytes=ob, device_budget=4 * MiB, device=0, out=(off, csr))
+    eoff, ecsr = o.build_csr(keys, M)
+    gcsr = _u(csr, kb).copy()
+    o.canon(eoff, gcsr)
+    o.canon(eoff, ecsr)
+    assert np.array_equal(_u(off, ob).astype(np.uint64), eoff) and np.array_equal(gcsr, ecsr)
+
+
+@pytest.mark.parametrize("kb,ob", [(4, 4), (8, 8)])
+def test_partitioned_pinned_many_slabs(kb, ob, dev):
+    """An empty partition and keys past the last split, in pinned memory."""
+    import hashgraph_amd as hg
+    n, M = 700001, 650003
+    keys = wl.uniform_keys(18, n, kb)
+    splits = [0, 100001, 100001, 400000, 640000]
+    off, csr, po = hg.build_partitioned_staged(_host_keys(keys, True), M, splits, ob, device_budget=4 * MiB, device=0)
+    bins = o.bins(keys, M).astype(np.int64)
+    goff, gcsr = _u(off, ob).astype(np.int64), _u(csr, kb)
+    for p in range(4):
+        lo, hi = splits[p], splits[p + 1]
+        own = (bins >= lo) & (bins < hi)
+        mine, mb = keys[own], bins[own] - lo
+        eo = np.concatenate([[0], np.cumsum(np.bincount(mb, minlength=hi - lo))])
+        assert np.array_equal(goff[lo + p:hi + p + 1], eo) and po[p + 1] - po[p] == len(mine)
+        got, gb = gcsr[po[p]:po[p + 1]], np.repeat(np.arange(hi - lo), np.diff(eo))
+        assert np.array_equal(got[np.lexsort((got, gb))], mine[np.lexsort((mine, mb))])
