@@ -29,7 +29,7 @@ static_assert(DEEP_ROWS % XCDS == 0 && DEEP_ROWS % (1024 / SUM_COLS) == 0 && DEE
 // Counts of the buckets over key range blockIdx.x (a row of fmat) and of the
 // groups (a row of cmat).  One workgroup a CU: its LDS holds a counter for
 // every bucket.
-template <typename K>
+template <typename K, int HK>
 __global__ __launch_bounds__(HB) void k_deep_hist(const K *__restrict__ keys, DeepGeom g, uint32_t *__restrict__ cmat,
                                                   uint32_t *__restrict__ fmat) {
   constexpr int U = sizeof(K) == 4 ? 16 : 8;
@@ -46,7 +46,7 @@ __global__ __launch_bounds__(HB) void k_deep_hist(const K *__restrict__ keys, De
     for (int j = 0; j < U; j++) kr[j] = buf_load<K>(rs, threadIdx.x * (uint32_t)sizeof(K), j * HB * (uint32_t)sizeof(K));
 #pragma unroll
     for (int j = 0; j < U; j++)
-      if (j * HB + threadIdx.x < cnt) atomicAdd(&s_cnt[divq(bin_of<K, HK_MURMUR>(kr[j], g.map) - g.bin_lo, g.fine)], 1u);
+      if (j * HB + threadIdx.x < cnt) atomicAdd(&s_cnt[divq(bin_of<K, HK>(kr[j], g.map) - g.bin_lo, g.fine)], 1u);
   }
   __syncthreads();
   for (uint32_t s = threadIdx.x >> 6; s < g.ngroups; s += HB / 64) {  // a wave a group
@@ -145,7 +145,7 @@ __global__ __launch_bounds__(1024) void k_deep_starts(const uint32_t *__restrict
 // second step, which writes 5 MB at a time; 2^28 uint32 keys).
 // The first workgroups also write the buckets' items and clear what the items'
 // kernels need.
-template <typename K, bool PACK>
+template <typename K, bool PACK, int HK>
 __global__ __launch_bounds__(SB) void k_deep_first(const void *__restrict__ keys, DeepGeom g, uint32_t chunk_keys,
                                                    uint32_t *__restrict__ gstart,
                                                    const uint32_t *__restrict__ fstart, K *__restrict__ out,
@@ -181,14 +181,14 @@ __global__ __launch_bounds__(SB) void k_deep_first(const void *__restrict__ keys
   const uint32_t n = (uint32_t)min((uint64_t)chunk_keys, end - k0);
   for (uint32_t base = 0; base < n; base += T)
     scatter_tile<K, SB, PACK>(keys, k0 + base, min(T, n - base), g.ngroups, s, out,
-                              [&](IN key) { return divq(bin_of<IN, HK_MURMUR>(key, g.map) - g.bin_lo, g.coarse); },
+                              [&](IN key) { return divq(bin_of<IN, HK>(key, g.map) - g.bin_lo, g.coarse); },
                               [&](uint32_t c) { return c ? atomicAdd(&gstart[x * g.ngroups + b], c) : 0u; });
 }
 
 // Second step: a chunk of one group into the group's buckets; every tile
 // reserves its places (fstart ends as the buckets' ends).  Consecutive chunks
 // run on one XCD, so the runs of a bucket meet in its L2.
-template <typename K>
+template <typename K, int HK>
 __global__ __launch_bounds__(SB) void k_deep_second(const K *__restrict__ keys, DeepGeom g,
                                                     const DeepChunk *__restrict__ chunks,
                                                     const uint32_t *__restrict__ nchunks, uint32_t *__restrict__ fstart,
@@ -203,7 +203,7 @@ __global__ __launch_bounds__(SB) void k_deep_second(const K *__restrict__ keys, 
   const uint32_t lo = g.bin_lo + f0 * g.fine.d;  // first bin of the group
   for (uint32_t base = 0; base < d.count; base += T)
     scatter_tile<K, SB, false>(keys, (uint64_t)d.start + base, min(T, d.count - base), ncols, s, out,
-                               [&](K key) { return divq(bin_of<K, HK_MURMUR>(key, g.map) - lo, g.fine); },
+                               [&](K key) { return divq(bin_of<K, HK>(key, g.map) - lo, g.fine); },
                                [&](uint32_t c) { return c ? atomicAdd(&fstart[f0 + threadIdx.x], c) : 0u; });
 }
 
@@ -216,27 +216,27 @@ uint32_t chunk_keys(uint64_t n, int key_bytes) {
   return (uint32_t)(t * std::min<uint64_t>(4, std::max<uint64_t>(1, n / (t * 3072))));
 }
 
-template <typename K>
+template <typename K, int HK>
 hipError_t launch_deep_t(const LaunchDeep &p, hipStream_t st) {
   const DeepGeom &g = p.geom;
   const uint32_t chunk = chunk_keys(g.n, p.key_bytes);
   const size_t hlds = (size_t)g.nfine * 4;
   if (p.pack)
-    hipLaunchKernelGGL(k_deep_hist<uint32_t>, dim3(p.rows), dim3(HB), hlds, st, (const uint32_t *)p.keys, g, p.cmat,
+    hipLaunchKernelGGL((k_deep_hist<uint32_t, HK>), dim3(p.rows), dim3(HB), hlds, st, (const uint32_t *)p.keys, g, p.cmat,
                        p.fmat);
   else
-    hipLaunchKernelGGL(k_deep_hist<K>, dim3(p.rows), dim3(HB), hlds, st, (const K *)p.keys, g, p.cmat, p.fmat);
+    hipLaunchKernelGGL((k_deep_hist<K, HK>), dim3(p.rows), dim3(HB), hlds, st, (const K *)p.keys, g, p.cmat, p.fmat);
   hipLaunchKernelGGL(k_deep_sum, dim3((g.nfine + SUM_COLS - 1) / SUM_COLS + (g.ngroups + SUM_COLS - 1) / SUM_COLS),
                      dim3(1024), 0, st, p.cmat, p.rows, g.ngroups, p.fmat, g.nfine, p.ftot);
   hipLaunchKernelGGL(k_deep_starts, dim3(1), dim3(1024), ((size_t)g.nfine + 1) * 4, st, (const uint32_t *)p.ftot, g,
                      p.rows, (const uint32_t *)p.cmat, chunk, p.fstart, p.gstart, p.chunks, p.nchunks);
-  auto first = &k_deep_first<K, false>;
-  if constexpr (sizeof(K) == 8)
-    if (p.pack) first = &k_deep_first<K, true>;
+  auto first = &k_deep_first<K, false, HK>;
+  if constexpr (sizeof(K) == 8 && HK == HK_MURMUR)
+    if (p.pack) first = &k_deep_first<K, true, HK>;
   const uint64_t share = std::min<uint64_t>((uint64_t)XROWS * g.per, g.n);
   hipLaunchKernelGGL(first, dim3((uint32_t)((share + chunk - 1) / chunk) * XCDS), dim3(SB), 0, st, p.keys, g, chunk,
                      p.gstart, (const uint32_t *)p.fstart, (K *)p.mid, p.items, p.maps, p.zero, p.nzero, p.zero_col);
-  hipLaunchKernelGGL(k_deep_second<K>, dim3(deep_max_chunks(g, p.key_bytes)), dim3(SB), 0, st, (const K *)p.mid, g,
+  hipLaunchKernelGGL((k_deep_second<K, HK>), dim3(deep_max_chunks(g, p.key_bytes)), dim3(SB), 0, st, (const K *)p.mid, g,
                      (const DeepChunk *)p.chunks, (const uint32_t *)p.nchunks, p.fstart, (K *)p.out);
   return hipGetLastError();
 }
@@ -253,9 +253,11 @@ hipError_t launch_deep(const LaunchDeep &p, hipStream_t st) {
       !g.ngroups || g.ngroups > DEEP_GROUPS || (uint64_t)g.ngroups * g.group < g.nfine ||
       (uint64_t)(g.ngroups - 1) * g.group >= g.nfine || !p.rows || p.rows > DEEP_ROWS ||
       (uint64_t)p.rows * g.per < g.n || (uint64_t)(p.rows - 1) * g.per >= g.n || p.nzero > (uint32_t)SB ||
-      g.map.kind != 0 || (uint64_t)g.nfine * g.fine.d < g.nbins || (p.pack && p.key_bytes != 8))
+      g.map.kind > 1 || (uint64_t)g.nfine * g.fine.d < g.nbins || (p.pack && (p.key_bytes != 8 || g.map.kind != 0)))
     return hipErrorInvalidValue;
-  return p.key_bytes == 4 ? launch_deep_t<uint32_t>(p, st) : launch_deep_t<uint64_t>(p, st);
+  if (p.key_bytes == 4)
+    return g.map.kind == 0 ? launch_deep_t<uint32_t, HK_MURMUR>(p, st) : launch_deep_t<uint32_t, HK_RMI>(p, st);
+  return g.map.kind == 0 ? launch_deep_t<uint64_t, HK_MURMUR>(p, st) : launch_deep_t<uint64_t, HK_RMI>(p, st);
 }
 
 hipError_t set_deep_kernel_attributes() {
@@ -263,7 +265,8 @@ hipError_t set_deep_kernel_attributes() {
     return hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (DEEP_FINE + 1) * 4);
   };
   hipError_t e = hipSuccess;
-  for (hipError_t x : {lds((const void *)&k_deep_hist<uint32_t>), lds((const void *)&k_deep_hist<uint64_t>),
+  for (hipError_t x : {lds((const void *)&k_deep_hist<uint32_t, HK_MURMUR>), lds((const void *)&k_deep_hist<uint64_t, HK_MURMUR>),
+                       lds((const void *)&k_deep_hist<uint32_t, HK_RMI>), lds((const void *)&k_deep_hist<uint64_t, HK_RMI>),
                        lds((const void *)&k_deep_starts)})
     if (x != hipSuccess) e = x;
   return e;

@@ -753,7 +753,11 @@ uint32_t deep_probe(uint64_t nb, uint64_t na, uint64_t M, int kb, uint32_t &W, u
 
 // Bucket class and width of a build's two-step partition; -1: none (the wide
 // pass).  Buckets of 8 K keys first: the final stage takes three of them to a
-// CU (2^28 uint32 keys: 0.57 ms against 0.90 with 32 K).
+// CU (2^28 uint32 keys: 0.57 ms against 0.90 with 32 K); 4 K and 16 K keys
+// measure within 3% for uint32, 16 K 8% slower for uint64 builds and 16-20%
+// slower for probes.  The line to the narrow pass lies where that one ends:
+// builds of 14.7 M uint32 keys take 129 us there and 136 us here (4 M: 53 and
+// 76), 25 M keys 208 us here.
 int deep_class(uint64_t n, uint64_t R, uint32_t &W) {
   for (int cls = 1; cls < FINAL_CLASSES; cls++) {
     if (0.875 * final_class_keys(cls) * (double)R < (double)n) continue;  // less than a bin a bucket
@@ -886,7 +890,7 @@ hg_status build_range(hg_ctx c, const BinMap &map, int kb, int ob, uint64_t n, u
   uint32_t Wn;
   if (const int cls = narrow_class(n, R, Wn); cls >= 0)
     return build_narrow(c, map, kb, ob, n, lo, R, cls, Wn, d_keys, d_off, d_csr, d_csr_index, pack_in);
-  if (const int cls = map.kind == 0 && n < (1ull << 32) ? deep_class(n, R, Wn) : -1; cls >= 0)
+  if (const int cls = n < (1ull << 32) ? deep_class(n, R, Wn) : -1; cls >= 0)
     return build_deep(c, map, kb, ob, n, lo, R, cls, Wn, d_keys, d_off, d_csr, d_csr_index, pack_in);
   const uint32_t W = choose_width(n, R, kb, build_fill());
   const uint64_t F = (R + W - 1) / W;
@@ -1238,7 +1242,7 @@ static hg_status probe_wide(hg_ctx c, const BinMap &map, int kb, uint64_t n_keys
 static hg_status probe_deep(hg_ctx c, const BinMap &map, int kb, uint64_t n_keys, uint64_t M, const void *d_probe,
                             uint64_t n_probe, uint64_t done, LaunchProbe &pr, bool &taken) {
   uint32_t W, lds = 0;
-  const uint32_t one = map.kind == 0 ? deep_probe(n_probe, n_keys, M, kb, W, lds) : 0;
+  const uint32_t one = deep_probe(n_probe, n_keys, M, kb, W, lds);
   if (!one) return HG_OK;
   const uint64_t F = (M + W - 1) / W;
   Plan P0, Px;

@@ -15,6 +15,7 @@
 #include "hg_device.hpp"
 #include "hg_final.hpp"
 #include "hg_kernels.hpp"
+#include "hg_scatter.hpp"
 
 namespace hg {
 
@@ -348,6 +349,35 @@ __global__ __launch_bounds__(BLOCK) void k_part_scatter(const K *__restrict__ ke
     for (uint32_t b = threadIdx.x; b < ncols; b += BLOCK) s_adj[b] += b + 1 < ncols ? s_cnt[b + 1] : tot;
     __syncthreads();
   }
+}
+
+// The same for range segments of at most FEW_COLS columns: tiles of 8 K (64-bit
+// keys: 4 K) keys on 512 threads, three workgroups a CU, one's loads and
+// stores under another's LDS phases (the kernel above holds one a CU).  1024
+// tables of 2^8..2^20 keys, build and counts: 3.31 ms with it, 3.61 without.
+constexpr uint32_t FEW_COLS = 512;
+template <typename K, int HK, bool PACK>
+__global__ __launch_bounds__(FEW_COLS) void k_part_scatter_few(const K *__restrict__ keys,
+                                                               const TileDesc *__restrict__ tiles,
+                                                               const SegDesc *__restrict__ segs,
+                                                               const uint32_t *__restrict__ cpos,
+                                                               K *__restrict__ out) {
+  constexpr uint32_t T = scatter_tile_keys<K>(FEW_COLS);
+  using IN = typename std::conditional<PACK, uint32_t, K>::type;
+  __shared__ ScatterLds<K, FEW_COLS> s;
+  const uint32_t tile = xcd_tile(blockIdx.x, gridDim.x);
+  const TileDesc td = tiles[tile];
+  const SegDesc sd = segs[td.seg];
+  const uint32_t ncols = sd.ncols, b = threadIdx.x;
+  uint32_t next = b < ncols ? cpos[sd.row_base + (uint64_t)(tile - sd.tile_begin) * ncols + b] : 0u;
+  for (uint32_t base = 0; base < td.count; base += T)
+    scatter_tile<K, FEW_COLS, PACK>(keys, td.key_start + base, min(T, td.count - base), ncols, s, out,
+                                    [&](IN key) { return bucket_of<IN, HK, SK_RANGE>(key, sd, nullptr); },
+                                    [&](uint32_t c) {
+                                      const uint32_t at = next;
+                                      next += c;
+                                      return at;
+                                    });
 }
 
 
@@ -2733,6 +2763,17 @@ static hipError_t launch_part_scatter_t(const LaunchPart &lp, hipStream_t st) {
   const size_t lds = 2 * cnt_bytes + (size_t)lp.stage_cap * (sizeof(K) + 2);
   return dispatch_part(lp.hk, lp.sk, [&](auto h, auto b) {
     constexpr int H = decltype(h)::value, S = decltype(b)::value;
+    if constexpr (S == SK_RANGE) {
+      if (lp.max_cols <= FEW_COLS) {
+        auto few = &k_part_scatter_few<K, H, false>;
+        if constexpr (sizeof(K) == 8 && H == HK_MURMUR) {
+          if (lp.pack) few = &k_part_scatter_few<K, H, true>;
+        }
+        hipLaunchKernelGGL(few, dim3(lp.ntiles), dim3(FEW_COLS), 0, st, (const K *)lp.keys, lp.tiles, lp.segs, lp.cmat,
+                           (K *)lp.out);
+        return hipGetLastError();
+      }
+    }
     // the packing instance exists for murmur3 levels of 8-byte records only
     // (launch_part_scatter checks)
     auto kern = &k_part_scatter<K, 1024, SCATTER_KPT, H, S>;

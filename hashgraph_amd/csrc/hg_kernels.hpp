@@ -160,7 +160,7 @@ struct DeepGeom {
   uint64_t n, nbins;
   uint32_t per, nfine, group, ngroups, bin_lo;
   Div32 fine, coarse;
-  BinMap map;  // murmur3
+  BinMap map;
 };
 struct DeepChunk {
   uint32_t start, count, group, pad;

@@ -273,12 +273,12 @@ def test_batch_of_many_tables_skewed(kb, dev):
     assert counts.cpu().numpy().tolist() == exp and total == sum(exp)
 
 
-def _csr_matches(hg, dk, off, csr, M):
+def _csr_matches(hg, dk, off, csr, M, **kw):
     """Table of dk on the device: degrees, bins in order, the same keys."""
     import torch
-    deg = torch.bincount(hg.table_bins(dk, M).to(torch.int64) & 0xFFFFFFFF, minlength=M)
+    deg = torch.bincount(hg.table_bins(dk, M, **kw).to(torch.int64) & 0xFFFFFFFF, minlength=M)
     assert int(off[0]) == 0 and torch.equal(off[1:].to(torch.int64) & 0xFFFFFFFF, torch.cumsum(deg, 0))
-    assert torch.equal(hg.table_bins(csr, M).to(torch.int64) & 0xFFFFFFFF,
+    assert torch.equal(hg.table_bins(csr, M, **kw).to(torch.int64) & 0xFFFFFFFF,
                        torch.repeat_interleave(torch.arange(M, device=dk.device), deg))
     assert torch.equal(torch.sort(csr).values, torch.sort(dk).values)
 
@@ -322,3 +322,36 @@ def test_two_step_build_in_place_and_indexed(kb, dev):
     off = torch.empty(M + 1, dtype=torch.int32, device=dev)
     hg.build(dk, M, out=(off, dk))
     _csr_matches(hg, keep, off, dk, M)
+
+
+def test_two_step_learned(dev):
+    """Skewed keys under a learned hash: the same matches as under murmur3."""
+    import torch
+    import hashgraph_amd as hg
+    n, M = 15000013, 15000001
+    A = wl.lognormal_keys(61, n, device=dev)
+    B = wl.mixed_probe(A, wl.lognormal_keys(62, n, device=dev), 63, 0.5)
+    model, _ = hg.rmi_train(A, M, seed=2)
+    kw = {"hash_kind": hg.HG_HASH_RMI, "rmi_model": model}
+    off, csr = hg.build(A, M, **kw)
+    _csr_matches(hg, A, off, csr, M, **kw)
+    cnt, out = hg.probe(off, csr, M, B, **kw)
+    ecnt, eout = hg.probe(*hg.build(A, M), M, B)
+    assert cnt == ecnt and torch.equal(torch.sort(out).values, torch.sort(eout).values)
+
+
+@pytest.mark.parametrize("kb,n", [(4, 28000001), (4, 30500003), (8, 28000001)])
+def test_partitions_around_the_few_column_scatter(kb, n, dev):
+    """Second partition levels just below and above its 512 columns."""
+    import torch
+    import hashgraph_amd as hg
+    M = n
+    dk = wl.uniform_keys(71, n, kb, device=dev)
+    off, csr, po = hg.build_partitioned(dk, M, [0, M // 2, M])
+    whole = hg.build(dk, M)[0].to(torch.int64)
+    for p, (lo, hi) in enumerate(((0, M // 2), (M // 2, M))):
+        assert torch.equal(off[lo + p:hi + p + 1].to(torch.int64), whole[lo:hi + 1] - whole[lo])
+    deg = whole[1:] - whole[:-1]
+    assert torch.equal(hg.table_bins(csr[:po[2]], M).to(torch.int64) & 0xFFFFFFFF,
+                       torch.repeat_interleave(torch.arange(M, device=dev), deg))
+    assert torch.equal(torch.sort(csr[:po[2]]).values, torch.sort(dk).values)
