@@ -832,6 +832,108 @@ __global__ __launch_bounds__(BLOCK) void k_join(const OFF *__restrict__ offA, co
     }
   }
   __syncthreads();
+  // Both sides in LDS and room behind one of them for a 16-bit bin number per
+  // key of B: a thread a key of B, which compares the keys of A in its bin (a
+  // thread a bin compares all pairs of its bin, and a wave waits for its
+  // longest product; its matches' places came from one LDS counter, one at a
+  // time).  A wave's matches take their places together.  @JOINFIG@
+  uint16_t *s_bin = pairs ? (uint16_t *)(s_ia + sa) : (uint16_t *)(s_b + sb);
+  const size_t spare = pairs ? (size_t)(key_cap - sa) * 8 : (size_t)(key_cap - sb) * sizeof(K);
+  if (a_lds && b_lds && 2 * (size_t)sb <= spare) {
+    for (uint32_t l = threadIdx.x; l < n; l += BLOCK) {
+      const uint32_t la = (uint32_t)(s_oa[l + 1] - s_oa[l]), lb = (uint32_t)(s_ob[l + 1] - s_ob[l]);
+      const bool heavy = la * lb > JOIN_PAIR_LIMIT;  // both below 2^16
+      if (heavy) {
+        const uint32_t i = atomicAdd(hlist_n, 1u);  // k_join_heavy answers this bin
+        if (i < hlist_cap) hlist[i] = (uint32_t)(b0 + l);
+      }
+      const uint32_t q0 = (uint32_t)(s_ob[l] - x0);
+      for (uint32_t q = q0; q < q0 + lb; q++) s_bin[q] = heavy ? (uint16_t)0xFFFF : (uint16_t)l;
+    }
+    __syncthreads();
+    // emit(place, slot of B, first and last slot of A, matches) per key with matches
+    auto walk = [&](auto emit) {
+      for (uint32_t base = 0; base < sb; base += BLOCK) {
+        const uint32_t q = base + threadIdx.x;
+        uint32_t m = 0, i0 = 0, i1 = 0;
+        if (q < sb) {
+          const uint32_t l = s_bin[q];
+          if (l != 0xFFFFu) {
+            i0 = (uint32_t)(s_oa[l] - a0);
+            i1 = (uint32_t)(s_oa[l + 1] - a0);
+          }
+          const K x = s_b[q];
+          for (uint32_t i = i0; i < i1; i++) m += s_a[i] == x;
+        }
+        if constexpr (emitting) {
+          const uint32_t inc = wave_inclusive_sum<uint32_t>(m);
+          uint32_t at = 0;
+          if ((threadIdx.x & 63) == 63 && inc) at = atomicAdd(&s_mn, inc);
+          at = __shfl(at, 63, 64) + inc - m;
+          if (m) emit(at, q, i0, i1, m);
+        } else {
+          emit(0u, q, i0, i1, m);
+        }
+      }
+    };
+    if constexpr (!emitting) {
+      __shared__ unsigned long long s_t64[BLOCK / 64 + 1];
+      unsigned long long mine = 0;
+      walk([&](uint32_t, uint32_t, uint32_t, uint32_t, uint32_t m) { mine += m; });
+      const unsigned long long t = block_sum<BLOCK, unsigned long long>(mine, s_t64);
+      if (threadIdx.x == 0 && t) atomicAdd(cursor, t);
+    } else {
+      walk([&](uint32_t at, uint32_t q, uint32_t i0, uint32_t i1, uint32_t m) {
+        if constexpr (pairs) {
+          for (uint32_t i = i0; i < i1; i++)
+            if (s_a[i] == s_b[q]) {
+              if (at < EBUF) s_m[at] = (i << 16) | q;
+              at++;
+            }
+        } else {
+          for (uint32_t r = 0; r < m; r++)
+            if (at + r < EBUF) s_m16[at + r] = (uint16_t)q;
+        }
+      });
+      __syncthreads();
+      const uint32_t nm = s_mn;
+      if (threadIdx.x == 0) s_base = nm ? atomicAdd(cursor, (unsigned long long)nm) : 0ull;
+      __syncthreads();
+      const unsigned long long w0 = s_base;
+      if (nm <= EBUF) {  // contiguous stores of the buffered matches
+        for (uint32_t q = threadIdx.x; q < nm; q += BLOCK) {
+          if (w0 + q >= capacity) break;
+          if (pairs) {
+            const uint32_t v = s_m[q];
+            pa[w0 + q] = s_ia[v >> 16];
+            pb[w0 + q] = s_ib[v & 0xFFFFu];
+          } else {
+            out[w0 + q] = s_b[s_m16[q]];
+          }
+        }
+        return;
+      }
+      if (threadIdx.x == 0) s_mn = 0;
+      __syncthreads();
+      walk([&](uint32_t at, uint32_t q, uint32_t i0, uint32_t i1, uint32_t m) {
+        unsigned long long w = w0 + at;
+        if constexpr (pairs) {
+          for (uint32_t i = i0; i < i1; i++)
+            if (s_a[i] == s_b[q]) {
+              if (w < capacity) {
+                pa[w] = s_ia[i];
+                pb[w] = s_ib[q];
+              }
+              w++;
+            }
+        } else {
+          for (uint32_t r = 0; r < m; r++, w++)
+            if (w < capacity) out[w] = s_b[q];
+        }
+      });
+    }
+    return;
+  }
   // an emitting join with both sides in LDS: every match appends its two LDS
   // slots (below key_cap < 2^16) to s_m during the counting walk
   const bool buffered = emitting && a_lds && b_lds;

@@ -355,3 +355,28 @@ def test_partitions_around_the_few_column_scatter(kb, n, dev):
     assert torch.equal(hg.table_bins(csr[:po[2]], M).to(torch.int64) & 0xFFFFFFFF,
                        torch.repeat_interleave(torch.arange(M, device=dev), deg))
     assert torch.equal(torch.sort(csr[:po[2]]).values, torch.sort(dk).values)
+
+
+# keys a bin around what the join stages: a bin number per key of B fits behind
+# the keys, then only the keys do, then not even they
+@pytest.mark.parametrize("kb,ob", [(4, 4), (8, 8)])
+@pytest.mark.parametrize("per", [0.3, 1.0, 1.4, 2.2, 2.6, 3.3, 5.0])
+def test_join_keys_per_bin(per, kb, ob, dev):
+    import hashgraph_amd as hg
+    M = 6145
+    n = int(per * M)
+    A = wl.uniform_keys(81, n, kb)
+    A[: n // 3] = A[n // 3: 2 * (n // 3)]   # every second match twice
+    A[5:140] = A[5]                         # a bin beyond the pair limit
+    B = wl.probe_keys(A, 82, n + 77, 0.9, kb)
+    B[300:400] = A[5]
+    ta, tb = (hg.build_indexed(_to_dev(x, dev), M, offset_bytes=ob) for x in (A, B))
+    eo, ek = o.build_csr(A, M)
+    bo, bk = o.build_csr(B, M)
+    ecnt, elst = o.intersect(eo, ek, bo, bk)
+    assert hg.intersect(ta[0], ta[1], tb[0], tb[1], M, emit=False)[0] == ecnt
+    cnt, out = hg.intersect(ta[0], ta[1], tb[0], tb[1], M)
+    assert cnt == ecnt and np.array_equal(np.sort(out.cpu().numpy().view(A.dtype)), np.sort(elst))
+    cnt, pa, pb = hg.intersect_indexed(*ta, *tb, M)
+    pa, pb = pa.cpu().numpy(), pb.cpu().numpy()
+    assert cnt == ecnt and np.array_equal(A[pa], B[pb]) and len(np.unique((pa << 32) | pb)) == cnt
