@@ -140,9 +140,9 @@ __global__ __launch_bounds__(1024) void k_deep_starts(const uint32_t *__restrict
 
 // First step: chunks of the keys into the groups; a tile reserves its places.
 // XCD x takes the x-th eighth of the keys in order and writes one part of each
-// group, so the tiles in flight on an XCD write next to each other (with a
-// contiguous key range for each workgroup instead: 747 against 519 us for the
-// second step, which writes 5 MB at a time; 2^28 uint32 keys).
+// group, so the tiles in flight on an XCD write next to each other: 2^28 uint32
+// keys in 515 us (747 with a contiguous key range for each workgroup; a plain
+// copy takes 410).
 // The first workgroups also write the buckets' items and clear what the items'
 // kernels need.
 template <typename K, bool PACK, int HK>
@@ -217,19 +217,22 @@ uint32_t chunk_keys(uint64_t n, int key_bytes) {
 }
 
 template <typename K, int HK>
-hipError_t launch_deep_t(const LaunchDeep &p, hipStream_t st) {
+hipError_t launch_deep_t(const LaunchDeep &p, bool scatter, hipStream_t st) {
   const DeepGeom &g = p.geom;
   const uint32_t chunk = chunk_keys(g.n, p.key_bytes);
-  const size_t hlds = (size_t)g.nfine * 4;
-  if (p.pack)
-    hipLaunchKernelGGL((k_deep_hist<uint32_t, HK>), dim3(p.rows), dim3(HB), hlds, st, (const uint32_t *)p.keys, g, p.cmat,
-                       p.fmat);
-  else
-    hipLaunchKernelGGL((k_deep_hist<K, HK>), dim3(p.rows), dim3(HB), hlds, st, (const K *)p.keys, g, p.cmat, p.fmat);
-  hipLaunchKernelGGL(k_deep_sum, dim3((g.nfine + SUM_COLS - 1) / SUM_COLS + (g.ngroups + SUM_COLS - 1) / SUM_COLS),
-                     dim3(1024), 0, st, p.cmat, p.rows, g.ngroups, p.fmat, g.nfine, p.ftot);
-  hipLaunchKernelGGL(k_deep_starts, dim3(1), dim3(1024), ((size_t)g.nfine + 1) * 4, st, (const uint32_t *)p.ftot, g,
-                     p.rows, (const uint32_t *)p.cmat, chunk, p.fstart, p.gstart, p.chunks, p.nchunks);
+  if (!scatter) {
+    const size_t hlds = (size_t)g.nfine * 4;
+    if (p.pack)
+      hipLaunchKernelGGL((k_deep_hist<uint32_t, HK>), dim3(p.rows), dim3(HB), hlds, st, (const uint32_t *)p.keys, g, p.cmat,
+                         p.fmat);
+    else
+      hipLaunchKernelGGL((k_deep_hist<K, HK>), dim3(p.rows), dim3(HB), hlds, st, (const K *)p.keys, g, p.cmat, p.fmat);
+    hipLaunchKernelGGL(k_deep_sum, dim3((g.nfine + SUM_COLS - 1) / SUM_COLS + (g.ngroups + SUM_COLS - 1) / SUM_COLS),
+                       dim3(1024), 0, st, p.cmat, p.rows, g.ngroups, p.fmat, g.nfine, p.ftot);
+    hipLaunchKernelGGL(k_deep_starts, dim3(1), dim3(1024), ((size_t)g.nfine + 1) * 4, st, (const uint32_t *)p.ftot, g,
+                       p.rows, (const uint32_t *)p.cmat, chunk, p.fstart, p.gstart, p.chunks, p.nchunks);
+    return hipGetLastError();
+  }
   auto first = &k_deep_first<K, false, HK>;
   if constexpr (sizeof(K) == 8 && HK == HK_MURMUR)
     if (p.pack) first = &k_deep_first<K, true, HK>;
@@ -247,7 +250,7 @@ uint32_t deep_max_chunks(const DeepGeom &g, int key_bytes) {
   return (uint32_t)(g.n / chunk_keys(g.n, key_bytes) + g.ngroups);
 }
 
-hipError_t launch_deep(const LaunchDeep &p, hipStream_t st) {
+static hipError_t launch_deep(const LaunchDeep &p, bool scatter, hipStream_t st) {
   const DeepGeom &g = p.geom;
   if (!g.n || g.n >= (1ull << 32) || !g.nfine || g.nfine > DEEP_FINE || !g.group || g.group > (uint32_t)SB ||
       !g.ngroups || g.ngroups > DEEP_GROUPS || (uint64_t)g.ngroups * g.group < g.nfine ||
@@ -256,17 +259,24 @@ hipError_t launch_deep(const LaunchDeep &p, hipStream_t st) {
       g.map.kind > 1 || (uint64_t)g.nfine * g.fine.d < g.nbins || (p.pack && (p.key_bytes != 8 || g.map.kind != 0)))
     return hipErrorInvalidValue;
   if (p.key_bytes == 4)
-    return g.map.kind == 0 ? launch_deep_t<uint32_t, HK_MURMUR>(p, st) : launch_deep_t<uint32_t, HK_RMI>(p, st);
-  return g.map.kind == 0 ? launch_deep_t<uint64_t, HK_MURMUR>(p, st) : launch_deep_t<uint64_t, HK_RMI>(p, st);
+    return g.map.kind == 0 ? launch_deep_t<uint32_t, HK_MURMUR>(p, scatter, st)
+                           : launch_deep_t<uint32_t, HK_RMI>(p, scatter, st);
+  return g.map.kind == 0 ? launch_deep_t<uint64_t, HK_MURMUR>(p, scatter, st)
+                         : launch_deep_t<uint64_t, HK_RMI>(p, scatter, st);
 }
+
+hipError_t launch_deep_count(const LaunchDeep &p, hipStream_t st) { return launch_deep(p, false, st); }
+hipError_t launch_deep_scatter(const LaunchDeep &p, hipStream_t st) { return launch_deep(p, true, st); }
 
 hipError_t set_deep_kernel_attributes() {
   const auto lds = [](const void *f) {
     return hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (DEEP_FINE + 1) * 4);
   };
   hipError_t e = hipSuccess;
-  for (hipError_t x : {lds((const void *)&k_deep_hist<uint32_t, HK_MURMUR>), lds((const void *)&k_deep_hist<uint64_t, HK_MURMUR>),
-                       lds((const void *)&k_deep_hist<uint32_t, HK_RMI>), lds((const void *)&k_deep_hist<uint64_t, HK_RMI>),
+  for (hipError_t x : {lds((const void *)&k_deep_hist<uint32_t, HK_MURMUR>),
+                       lds((const void *)&k_deep_hist<uint64_t, HK_MURMUR>),
+                       lds((const void *)&k_deep_hist<uint32_t, HK_RMI>),
+                       lds((const void *)&k_deep_hist<uint64_t, HK_RMI>),
                        lds((const void *)&k_deep_starts)})
     if (x != hipSuccess) e = x;
   return e;

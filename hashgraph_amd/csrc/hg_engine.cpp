@@ -837,8 +837,12 @@ hg_status build_deep(hg_ctx c, const BinMap &map, int kb, int ob, uint64_t n, ui
   p.zero = (unsigned long long *)rest;
   p.nzero = BIG_CTL_ZERO;
   {
+    Prof pf(c, "part_hist");
+    HG_HIP(launch_deep_count(p, c->stream));
+  }
+  {
     Prof pf(c, "part_scatter");
-    HG_HIP(launch_deep(p, c->stream));
+    HG_HIP(launch_deep_scatter(p, c->stream));
   }
   (void)i_cnt;
   LaunchFinal f{};
@@ -1268,8 +1272,12 @@ static hg_status probe_deep(hg_ctx c, const BinMap &map, int kb, uint64_t n_keys
   p.nzero = 2 + BIG_CTL_ZERO;
   p.zero_col = pr.hmark;
   {
+    Prof pf(c, "part_hist");
+    HG_HIP(launch_deep_count(p, c->stream));
+  }
+  {
     Prof pf(c, "part_scatter");
-    HG_HIP(launch_deep(p, c->stream));
+    HG_HIP(launch_deep_scatter(p, c->stream));
   }
   if (done) HG_HIP(launch_fill_u64(pr.cursor, done, 1, c->stream));
   pr.hk = (int)map.kind;

@@ -184,7 +184,9 @@ struct LaunchDeep {
   unsigned int *zero_col;      // nfine more (or null)
 };
 uint32_t deep_max_chunks(const DeepGeom &g, int key_bytes);
-hipError_t launch_deep(const LaunchDeep &p, hipStream_t st);
+// the histogram and the places, then both scatter steps
+hipError_t launch_deep_count(const LaunchDeep &p, hipStream_t st);
+hipError_t launch_deep_scatter(const LaunchDeep &p, hipStream_t st);
 hipError_t set_deep_kernel_attributes();
 
 // Staged builds: a slab's place among the CSR keys; a

@@ -380,3 +380,21 @@ def test_join_keys_per_bin(per, kb, ob, dev):
     cnt, pa, pb = hg.intersect_indexed(*ta, *tb, M)
     pa, pb = pa.cpu().numpy(), pb.cpu().numpy()
     assert cnt == ecnt and np.array_equal(A[pa], B[pb]) and len(np.unique((pa << 32) | pb)) == cnt
+
+
+def test_two_step_larger_buckets(dev):
+    """More keys than 8 K-key buckets can be counted for: the next class."""
+    import torch
+    import hashgraph_amd as hg
+    n = M = 302000011
+    dk = wl.uniform_keys(91, n, 4, device=dev)
+    off, csr = hg.build(dk, M)
+    deg = torch.bincount(hg.table_bins(dk, M), minlength=M)
+    assert int(off[0]) == 0 and torch.equal(off[1:].to(torch.int64), torch.cumsum(deg, 0))
+    assert torch.equal(hg.table_bins(csr, M).to(torch.int64), torch.repeat_interleave(torch.arange(M, device=dev), deg))
+    assert torch.equal(torch.sort(csr).values, torch.sort(dk).values)
+    q = wl.probe_keys(dk, 92, n // 2, 0.3, 4, device=dev)
+    cnt, out = hg.probe(off, csr, M, q)
+    tq = hg.build(q, M)
+    assert (cnt, int(out.to(torch.int64).sum())) == (lambda c, o: (c, int(o.to(torch.int64).sum())))(
+        *hg.intersect(off, csr, *tq, M))
