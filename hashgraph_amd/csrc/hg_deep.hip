@@ -116,6 +116,7 @@ __global__ __launch_bounds__(1024) void k_deep_starts(const uint32_t *__restrict
   __syncthreads();
   for (uint32_t f = threadIdx.x; f <= g.nfine; f += 1024) fstart[f] = s_a[f];
   const uint32_t s = threadIdx.x;
+  static_assert(DEEP_GROUPS == 256, "the search below");
   uint32_t a = 0, e = 0;
   if (s < g.ngroups) {
     a = s_a[s * g.group];
@@ -128,13 +129,23 @@ __global__ __launch_bounds__(1024) void k_deep_starts(const uint32_t *__restrict
   uint32_t all;
   const uint32_t c0 = block_exclusive_sum<1024, uint32_t>(nc, s_tmp, all);
   if (threadIdx.x == 0) *nchunks = all;
-  for (uint32_t i = 0; i < nc; i++) {
+  // the chunks of all groups in turn, a thread a chunk (a hot key's group has
+  // most of them)
+  __shared__ uint32_t s_c0[DEEP_GROUPS + 1];
+  if (s < g.ngroups) s_c0[s] = c0;
+  if (s == 0) s_c0[g.ngroups] = all;
+  __syncthreads();
+  for (uint32_t i = s; i < all; i += 1024) {
+    uint32_t q = 0;  // last group whose first chunk is at most i
+    for (uint32_t step = 128; step; step >>= 1)
+      if (q + step < g.ngroups && s_c0[q + step] <= i) q += step;
+    const uint32_t ga = s_a[q * g.group], ge = s_a[min(g.nfine, (q + 1) * g.group)];
     DeepChunk d;
-    d.start = a + i * chunk_keys;
-    d.count = min(chunk_keys, e - d.start);
-    d.group = s;
+    d.start = ga + (i - s_c0[q]) * chunk_keys;
+    d.count = min(chunk_keys, ge - d.start);
+    d.group = q;
     d.pad = 0;
-    chunks[c0 + i] = d;
+    chunks[i] = d;
   }
 }
 
