@@ -23,6 +23,7 @@ constexpr int HB = 1024;        // threads of the histogram
 constexpr int SB = 512;         // threads of the scatter steps
 constexpr int SUM_COLS = 32;    // columns of a column-sum workgroup
 constexpr uint32_t XCDS = 8;
+constexpr uint32_t HOT_GRID = 768;  // three workgroups a CU
 constexpr uint32_t XROWS = DEEP_ROWS / XCDS;  // key ranges of an XCD
 static_assert(DEEP_ROWS % XCDS == 0 && DEEP_ROWS % (1024 / SUM_COLS) == 0 && DEEP_GROUPS <= SB, "two-step geometry");
 
@@ -116,7 +117,7 @@ __global__ __launch_bounds__(1024) void k_deep_starts(const uint32_t *__restrict
   __syncthreads();
   for (uint32_t f = threadIdx.x; f <= g.nfine; f += 1024) fstart[f] = s_a[f];
   const uint32_t s = threadIdx.x;
-  static_assert(DEEP_GROUPS == 256, "the search below");
+  static_assert((DEEP_GROUPS & (DEEP_GROUPS - 1)) == 0, "the search below");
   uint32_t a = 0, e = 0;
   if (s < g.ngroups) {
     a = s_a[s * g.group];
@@ -126,22 +127,27 @@ __global__ __launch_bounds__(1024) void k_deep_starts(const uint32_t *__restrict
     for (uint32_t x = 0; x < XCDS; x++)
       if (x * XROWS < rows) gstart[x * g.ngroups + s] = a + cmat[(uint64_t)x * XROWS * g.ngroups + s];
   const uint32_t nc = (uint32_t)(((uint64_t)(e - a) + chunk_keys - 1) / chunk_keys);
-  uint32_t all;
-  const uint32_t c0 = block_exclusive_sum<1024, uint32_t>(nc, s_tmp, all);
-  if (threadIdx.x == 0) *nchunks = all;
-  // the chunks of all groups in turn, a thread a chunk (a hot key's group has
-  // most of them)
-  __shared__ uint32_t s_c0[DEEP_GROUPS + 1];
-  if (s < g.ngroups) s_c0[s] = c0;
-  if (s == 0) s_c0[g.ngroups] = all;
+  // ordinary groups' chunks, then the hot ones', a thread a chunk (a hot key's
+  // group may have most of them)
+  __shared__ uint32_t s_c0[2][DEEP_GROUPS];
+  const bool hot = e - a > g.n / g.ngroups * 2;
+  uint32_t all[2];
+  const uint32_t c0 = block_exclusive_sum<1024, uint32_t>(hot ? 0u : nc, s_tmp, all[0]);
+  const uint32_t c1 = block_exclusive_sum<1024, uint32_t>(hot ? nc : 0u, s_tmp, all[1]);
+  if (s < g.ngroups) {
+    s_c0[0][s] = c0;
+    s_c0[1][s] = c1;
+  }
+  if (s < 2) nchunks[s] = all[s];
   __syncthreads();
-  for (uint32_t i = s; i < all; i += 1024) {
-    uint32_t q = 0;  // last group whose first chunk is at most i
-    for (uint32_t step = 128; step; step >>= 1)
-      if (q + step < g.ngroups && s_c0[q + step] <= i) q += step;
+  for (uint32_t i = s; i < all[0] + all[1]; i += 1024) {
+    const uint32_t h = i >= all[0], ci = h ? i - all[0] : i;
+    uint32_t q = 0;  // last group whose first chunk is at most ci (groups without chunks precede it)
+    for (uint32_t step = DEEP_GROUPS / 2; step; step >>= 1)
+      if (q + step < g.ngroups && s_c0[h][q + step] <= ci) q += step;
     const uint32_t ga = s_a[q * g.group], ge = s_a[min(g.nfine, (q + 1) * g.group)];
     DeepChunk d;
-    d.start = ga + (i - s_c0[q]) * chunk_keys;
+    d.start = ga + (ci - s_c0[h][q]) * chunk_keys;
     d.count = min(chunk_keys, ge - d.start);
     d.group = q;
     d.pad = 0;
@@ -197,25 +203,46 @@ __global__ __launch_bounds__(SB) void k_deep_first(const void *__restrict__ keys
 }
 
 // Second step: a chunk of one group into the group's buckets; every tile
-// reserves its places (fstart ends as the buckets' ends).  Consecutive chunks
-// run on one XCD, so the runs of a bucket meet in its L2.
+// reserves its places (fstart ends as the buckets' ends).
+template <typename K, int HK, bool HOT>
+__device__ __forceinline__ void second_chunk(const K *__restrict__ keys, const DeepGeom &g, const DeepChunk &d,
+                                             ScatterLds<K, SB> &s, uint32_t *__restrict__ fstart,
+                                             K *__restrict__ out) {
+  constexpr uint32_t T = scatter_tile_keys<K>(SB);
+  const uint32_t f0 = d.group * g.group, ncols = min(g.group, g.nfine - f0);
+  const uint32_t lo = g.bin_lo + f0 * g.fine.d;  // first bin of the group
+  for (uint32_t base = 0; base < d.count; base += T)
+    scatter_tile<K, SB, false, HOT>(keys, (uint64_t)d.start + base, min(T, d.count - base), ncols, s, out,
+                                    [&](K key) { return divq(bin_of<K, HK>(key, g.map) - lo, g.fine); },
+                                    [&](uint32_t c) { return c ? atomicAdd(&fstart[f0 + threadIdx.x], c) : 0u; });
+}
+
+// Consecutive chunks run on one XCD, so the runs of a bucket meet in its L2.
 template <typename K, int HK>
 __global__ __launch_bounds__(SB) void k_deep_second(const K *__restrict__ keys, DeepGeom g,
                                                     const DeepChunk *__restrict__ chunks,
                                                     const uint32_t *__restrict__ nchunks, uint32_t *__restrict__ fstart,
                                                     K *__restrict__ out) {
-  constexpr uint32_t T = scatter_tile_keys<K>(SB);
   __shared__ ScatterLds<K, SB> s;
-  const uint32_t nc = *nchunks;
+  const uint32_t nc = nchunks[0];
   if (blockIdx.x >= nc) return;
   const uint32_t q = nc >> 3, r = nc & 7, x = blockIdx.x & 7;
-  const DeepChunk d = chunks[x * q + min(x, r) + (blockIdx.x >> 3)];
-  const uint32_t f0 = d.group * g.group, ncols = min(g.group, g.nfine - f0);
-  const uint32_t lo = g.bin_lo + f0 * g.fine.d;  // first bin of the group
-  for (uint32_t base = 0; base < d.count; base += T)
-    scatter_tile<K, SB, false>(keys, (uint64_t)d.start + base, min(T, d.count - base), ncols, s, out,
-                               [&](K key) { return divq(bin_of<K, HK>(key, g.map) - lo, g.fine); },
-                               [&](uint32_t c) { return c ? atomicAdd(&fstart[f0 + threadIdx.x], c) : 0u; });
+  second_chunk<K, HK, false>(keys, g, chunks[x * q + min(x, r) + (blockIdx.x >> 3)], s, fstart, out);
+}
+
+// The chunks of groups with more than twice their share of the keys: one value
+// fills most of them (a kernel of its own, since its registers would cost the
+// other one a workgroup a CU).  Builds of 2^27 uint32 keys: Zipf(1.1) 2.02 ms
+// without it, 1.88 with it, Zipf(1.3) 2.18 and 2.05; uniform keys pay a launch.
+template <typename K, int HK>
+__global__ __launch_bounds__(SB) void k_deep_hot(const K *__restrict__ keys, DeepGeom g,
+                                                 const DeepChunk *__restrict__ chunks,
+                                                 const uint32_t *__restrict__ nchunks, uint32_t *__restrict__ fstart,
+                                                 K *__restrict__ out) {
+  __shared__ ScatterLds<K, SB> s;
+  const uint32_t n0 = nchunks[0], n1 = nchunks[1];
+  for (uint32_t i = blockIdx.x; i < n1; i += gridDim.x)
+    second_chunk<K, HK, true>(keys, g, chunks[n0 + i], s, fstart, out);
 }
 
 namespace {
@@ -251,6 +278,8 @@ hipError_t launch_deep_t(const LaunchDeep &p, bool scatter, hipStream_t st) {
   hipLaunchKernelGGL(first, dim3((uint32_t)((share + chunk - 1) / chunk) * XCDS), dim3(SB), 0, st, p.keys, g, chunk,
                      p.gstart, (const uint32_t *)p.fstart, (K *)p.mid, p.items, p.maps, p.zero, p.nzero, p.zero_col);
   hipLaunchKernelGGL((k_deep_second<K, HK>), dim3(deep_max_chunks(g, p.key_bytes)), dim3(SB), 0, st, (const K *)p.mid, g,
+                     (const DeepChunk *)p.chunks, (const uint32_t *)p.nchunks, p.fstart, (K *)p.out);
+  hipLaunchKernelGGL((k_deep_hot<K, HK>), dim3(HOT_GRID), dim3(SB), 0, st, (const K *)p.mid, g,
                      (const DeepChunk *)p.chunks, (const uint32_t *)p.nchunks, p.fstart, (K *)p.out);
   return hipGetLastError();
 }

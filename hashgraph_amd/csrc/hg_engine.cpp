@@ -794,7 +794,7 @@ hg_status deep_launch(hg_ctx c, const BinMap &map, int kb, uint64_t n, uint64_t 
   const size_t i_cmat = P.add((size_t)DEEP_ROWS * g.ngroups * 4), i_fmat = P.add((size_t)DEEP_ROWS * g.nfine * 4),
                i_ftot = P.add(g.nfine * 4), i_fstart = P.add(((size_t)g.nfine + 1) * 4),
                i_gstart = P.add((size_t)8 * g.ngroups * 4),
-               i_chunks = P.add((size_t)deep_max_chunks(g, kb) * sizeof(DeepChunk)), i_nch = P.add(4),
+               i_chunks = P.add((size_t)deep_max_chunks(g, kb) * sizeof(DeepChunk)), i_nch = P.add(8),
                i_items = P.add((size_t)g.nfine * sizeof(FinItem)), i_maps = P.add(sizeof(BinMap)), i_rest = P.add(extra);
   HG_TRY(arena_ensure(c, 1, P.total()));
   Carve cv;

@@ -176,7 +176,7 @@ struct LaunchDeep {
   uint32_t *ftot, *fstart;     // nfine, nfine + 1
   uint32_t *gstart;            // 8 * ngroups
   DeepChunk *chunks;           // deep_max_chunks
-  uint32_t *nchunks;
+  uint32_t *nchunks;           // two
   FinItem *items;              // nfine
   BinMap *maps;                // one
   unsigned long long *zero;    // as in LaunchNarrow
