@@ -1448,7 +1448,12 @@ hg_status hg_scratch_bytes(const hg_table_desc *desc, int op, size_t *bytes) {
   const uint64_t F = std::min<uint64_t>((M + W - 1) / W, kFMax);
   const uint64_t tiles = (n + kTile - 1) / kTile + 1;
   (void)op;
-  *bytes = (size_t)n * kb * 2 + (size_t)(tiles * (F + 1) * 4) * 2 + (size_t)F * 64 + (size_t)tiles * 64 + (1 << 20);
+  // a probe's two-step partition holds two copies of its keys (as many as the
+  // table's here) in the half hg_ctx_reserve gives the first arena
+  uint32_t Wp, lds;
+  const bool two = n && !narrow_probe(n, n, M, kb, Wp, lds) && deep_probe(n, n, M, kb, Wp, lds);
+  *bytes = (size_t)n * kb * (two ? 4 : 2) + (size_t)(tiles * (F + 1) * 4) * 2 + (size_t)F * 64 + (size_t)tiles * 64 +
+           (1 << 20);
   return HG_OK;
 }
 

@@ -26,3 +26,15 @@ def test_library_exports_every_declared_symbol():
 def test_version_string():
     L = _lib.load()
     assert b"gfx950" in L.hg_version()
+
+
+def test_scratch_of_a_two_step_probe_holds_both_copies():
+    """hg_ctx_reserve halves the bytes; a large probe keeps two copies of its
+    keys in the first half."""
+    import ctypes
+    import hashgraph_amd as hg
+    L = _lib.load()
+    for kb, n in ((4, 1 << 28), (8, 1 << 27), (4, 1000)):
+        b = ctypes.c_size_t(0)
+        assert L.hg_scratch_bytes(ctypes.byref(hg._desc(n, n, kb, 4)), 1, ctypes.byref(b)) == 0
+        assert b.value // 2 >= (2 if n > 10 ** 7 else 1) * n * kb
