@@ -113,19 +113,30 @@ def _emit(call, guess: int, alloc, cnt, where: str):
     """Matches of a call whose caller named no capacity: one pass into buffers
     of `guess` matches instead of a counting pass before it (at 10^8 joined
     keys each pass takes about a millisecond).  More matches than that, or too
-    little memory for the guess, give buffers of the exact size and the pass
-    again.  call(bufs, capacity) -> status, alloc(n) -> list of n-match
+    little memory for the guess or for the library's scratch beside it, give
+    buffers of the exact size and the pass again.  call(bufs, capacity) -> status, alloc(n) -> list of n-match
     buffers; returns the buffers, exactly cnt long."""
+    torch = _torch()
     bufs = None
     if guess:
         try:
             bufs = alloc(guess)
-        except _torch().OutOfMemoryError:
+        except torch.OutOfMemoryError:
             pass
     st = call(bufs, guess if bufs else 0)
+    if st == _lib.HG_ERR_OOM and bufs:
+        # the library's scratch does not fit beside the guess, which the
+        # allocator would otherwise keep
+        bufs = None
+        torch.cuda.empty_cache()
+        st = call(None, 0)
     if st == _lib.HG_OK and bufs:
-        # the spare room goes back to the allocator
-        return bufs if cnt.value == guess else [b[: cnt.value].clone() for b in bufs]
+        if cnt.value == guess:
+            return bufs
+        try:  # the spare room goes back to the allocator
+            return [b[: cnt.value].clone() for b in bufs]
+        except torch.OutOfMemoryError:
+            return [b[: cnt.value] for b in bufs]
     if st != _lib.HG_OK and (st != _lib.HG_ERR_CAPACITY or not bufs):
         check(st, where)
     del bufs

@@ -14,6 +14,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(HERE, "lib", "libhashgraph_amd.so")
 
 HG_OK = 0
+HG_ERR_OOM = 2
 HG_ERR_CAPACITY = 4
 STATUS = {0: "HG_OK", 1: "HG_ERR_INVALID_ARG", 2: "HG_ERR_OOM", 3: "HG_ERR_DEVICE", 4: "HG_ERR_CAPACITY",
           5: "HG_ERR_MISMATCH", 6: "HG_ERR_UNSUPPORTED"}
