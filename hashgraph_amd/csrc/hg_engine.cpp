@@ -215,11 +215,31 @@ struct Prof {
   }
 };
 
-hg_status arena_ensure(hg_ctx c, int a, size_t bytes) {
+// Grows arena a to bytes.  The first `keep` bytes of its contents survive (and
+// the arena itself, when there is no memory); without any the old arena goes
+// before the new one is allocated.
+hg_status arena_ensure(hg_ctx c, int a, size_t bytes, size_t keep = 0) {
   if (bytes <= c->arena_cap[a]) return HG_OK;
   HG_HIP(hipStreamSynchronize(c->stream));
   size_t want = std::max(bytes, c->arena_cap[a] * 5 / 4);
   want = (want + (1 << 20) - 1) & ~(size_t)((1 << 20) - 1);
+  if (keep) {
+    char *p = nullptr;
+    if (hipMalloc(&p, want) != hipSuccess) {
+      (void)hipGetLastError();
+      return fail(HG_ERR_OOM, "scratch arena: cannot allocate " + std::to_string(want) + " bytes");
+    }
+    hipError_t e = hipMemcpyAsync(p, c->arena[a], keep, hipMemcpyDeviceToDevice, c->stream);
+    if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+    if (e != hipSuccess) {
+      (void)hipFree(p);
+      HG_HIP(e);
+    }
+    std::swap(p, c->arena[a]);
+    c->arena_cap[a] = want;
+    HG_HIP(hipFree(p));
+    return HG_OK;
+  }
   if (c->arena[a]) HG_HIP(hipFree(c->arena[a]));
   c->arena[a] = nullptr;
   c->arena_cap[a] = 0;
@@ -429,61 +449,79 @@ struct LevelDev {
   void *big_ctl;
 };
 
+// A level's descriptors in one host blob, and its pieces of arena 1.
+struct LevelBlob {
+  Blob b;
+  size_t tiles, segs, items, items2, psb, nch, maps, spl;
+  explicit LevelBlob(const Level &L) {
+    tiles = b.put(L.tiles);
+    segs = b.put(L.segs);
+    items = b.put(L.items);
+    items2 = b.put(L.items2);
+    psb = b.put(L.psum_base);
+    nch = b.put(L.nchunks);
+    maps = b.put(L.maps);
+    spl = b.put(L.splits);
+  }
+};
+struct LevelPlan {
+  Plan P;
+  uint64_t big_cap;
+  size_t blob, cmat, psum, coltot, bstart, fin, bslot, bctl, bcnt;
+  LevelPlan(const Level &L, size_t blob_bytes) {
+    const size_t cols = std::max<uint32_t>(L.ncols_total, 1);
+    blob = P.add(blob_bytes);
+    cmat = P.add(std::max<uint64_t>(L.cmat_elems, 1) * 4);
+    psum = P.add(std::max<uint64_t>(L.psum_elems, 1) * 4);
+    coltot = P.add(cols * 4);
+    bstart = P.add(cols * 4);
+    fin = P.add(cols * sizeof(FinItem));
+    // per-bin counters of the oversized buckets: 256 M counters at most (1 GB),
+    // fewer when the level has fewer bins
+    uint64_t nbins_total = 0;
+    for (const SegDesc &sd : L.segs) nbins_total += sd.seg_nbins;
+    big_cap = big_counters(nbins_total);
+    bslot = P.add(cols * 4);
+    bctl = P.add(final_big_ctl_bytes());
+    bcnt = P.add((size_t)big_cap * 4);
+  }
+  static uint64_t big_counters(uint64_t nbins) {
+    return std::max<uint64_t>(1, std::min<uint64_t>(nbins, 1ull << 28));
+  }
+};
+
 // Lays out a level in arena 1 (growing it if needed; the stream must be
 // idle of earlier users of arena 1, which holds because every level is
 // planned either at the start of an operation or after a read-back), patches
 // device pointers into the descriptors and uploads them.
 hg_status setup_level(hg_ctx c, Level &L, LevelDev &d) {
-  Blob b0;
-  const size_t o_tiles = b0.put(L.tiles), o_segs = b0.put(L.segs), o_items = b0.put(L.items), o_items2 = b0.put(L.items2),
-               o_psb = b0.put(L.psum_base), o_nch = b0.put(L.nchunks), o_maps = b0.put(L.maps), o_spl = b0.put(L.splits);
-  Plan P;
-  const size_t i_blob = P.add(b0.data.size());
-  const size_t i_cmat = P.add(std::max<uint64_t>(L.cmat_elems, 1) * 4);
-  const size_t i_psum = P.add(std::max<uint64_t>(L.psum_elems, 1) * 4);
-  const size_t i_coltot = P.add(std::max<uint32_t>(L.ncols_total, 1) * 4);
-  const size_t i_bstart = P.add(std::max<uint32_t>(L.ncols_total, 1) * 4);
-  const size_t i_fin = P.add((size_t)std::max<uint32_t>(L.ncols_total, 1) * sizeof(FinItem));
-  // per-bin counters of the oversized buckets: 256 M counters at most (1 GB),
-  // fewer when the level has fewer bins
-  uint64_t nbins_total = 0;
-  for (const SegDesc &sd : L.segs) nbins_total += sd.seg_nbins;
-  L.big_cap = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(nbins_total, 1ull << 28));
-  const size_t i_bslot = P.add((size_t)std::max<uint32_t>(L.ncols_total, 1) * 4);
-  const size_t i_bctl = P.add(final_big_ctl_bytes());
-  const size_t i_bcnt = P.add((size_t)L.big_cap * 4);
-  HG_TRY(arena_ensure(c, 1, P.total()));
+  const LevelBlob lb(L);
+  const LevelPlan q(L, lb.b.data.size());
+  L.big_cap = (uint32_t)q.big_cap;
+  HG_TRY(arena_ensure(c, 1, q.P.total()));
   Carve cv;
-  cv.init(c, 1, P);
-  char *blob = cv.get<char>(i_blob);
-  d.tiles = (TileDesc *)(blob + o_tiles);
-  d.segs = (SegDesc *)(blob + o_segs);
-  d.items = (ColItem *)(blob + o_items);
-  d.items2 = (ColItem *)(blob + o_items2);
-  d.psum_base = (uint64_t *)(blob + o_psb);
-  d.nchunks = (uint32_t *)(blob + o_nch);
-  d.maps = (BinMap *)(blob + o_maps);
-  d.splits = (int64_t *)(blob + o_spl);
-  d.cmat = cv.get<uint32_t>(i_cmat);
-  d.psum = cv.get<uint32_t>(i_psum);
-  d.coltot = cv.get<uint32_t>(i_coltot);
-  d.bstart = cv.get<uint32_t>(i_bstart);
-  d.fin = cv.get<FinItem>(i_fin);
-  d.big_slot = cv.get<uint32_t>(i_bslot);
-  d.big_ctl = cv.get<void>(i_bctl);
-  d.big_cnt = cv.get<uint32_t>(i_bcnt);
+  cv.init(c, 1, q.P);
+  char *blob = cv.get<char>(q.blob);
+  d.tiles = (TileDesc *)(blob + lb.tiles);
+  d.segs = (SegDesc *)(blob + lb.segs);
+  d.items = (ColItem *)(blob + lb.items);
+  d.items2 = (ColItem *)(blob + lb.items2);
+  d.psum_base = (uint64_t *)(blob + lb.psb);
+  d.nchunks = (uint32_t *)(blob + lb.nch);
+  d.maps = (BinMap *)(blob + lb.maps);
+  d.splits = (int64_t *)(blob + lb.spl);
+  d.cmat = cv.get<uint32_t>(q.cmat);
+  d.psum = cv.get<uint32_t>(q.psum);
+  d.coltot = cv.get<uint32_t>(q.coltot);
+  d.bstart = cv.get<uint32_t>(q.bstart);
+  d.fin = cv.get<FinItem>(q.fin);
+  d.big_slot = cv.get<uint32_t>(q.bslot);
+  d.big_ctl = cv.get<void>(q.bctl);
+  d.big_cnt = cv.get<uint32_t>(q.bcnt);
   for (SegDesc &sd : L.segs)
     if (sd.kind == 1) sd.splits = d.splits;
-  Blob b1;
-  b1.put(L.tiles);
-  b1.put(L.segs);
-  b1.put(L.items);
-  b1.put(L.items2);
-  b1.put(L.psum_base);
-  b1.put(L.nchunks);
-  b1.put(L.maps);
-  b1.put(L.splits);
-  return upload(c, blob, b1.data.data(), b1.data.size());
+  const LevelBlob patched(L);
+  return upload(c, blob, patched.b.data.data(), patched.b.data.size());
 }
 
 // scatter = false stops after the column scan (bucket sizes only).
@@ -665,29 +703,51 @@ LaunchNarrow narrow_launch(const BinMap &map, int kb, uint64_t n, uint64_t lo, u
   return p;
 }
 
+// Arena 1 of a narrow pass; extra bytes of the caller's behind it.
+struct NarrowPlan {
+  Plan P;
+  size_t cmat, tot, items, maps, slot, rest;
+  NarrowPlan(uint32_t rows, uint32_t ncols, size_t extra) {
+    cmat = P.add((size_t)rows * ncols * 4);
+    tot = P.add((size_t)ncols * 4);
+    items = P.add((size_t)ncols * sizeof(FinItem));
+    maps = P.add(sizeof(BinMap));
+    slot = P.add((size_t)ncols * 4);
+    rest = P.add(extra);
+  }
+  void carve(hg_ctx c, LaunchNarrow &p, uint32_t *&big_slot, char *&r) const {
+    Carve c1;
+    c1.init(c, 1, P);
+    p.cmat = c1.get<uint32_t>(cmat);
+    p.tot = c1.get<uint32_t>(tot);
+    p.items = c1.get<FinItem>(items);
+    p.maps = c1.get<BinMap>(maps);
+    big_slot = c1.get<uint32_t>(slot);
+    r = c1.get<char>(rest);
+  }
+};
+// What a build's final stage keeps there: the list of oversized buckets and
+// their per-bin counters (at *cnt of the rest).
+size_t final_rest(uint64_t R, size_t &cnt) {
+  cnt = (final_big_ctl_bytes() + 255) & ~(size_t)255;
+  return cnt + LevelPlan::big_counters(R) * 4;
+}
+
 hg_status build_narrow(hg_ctx c, const BinMap &map, int kb, int ob, uint64_t n, uint64_t lo, uint64_t R, int cls,
                        uint32_t W, const void *d_keys, void *d_off, void *d_csr, uint64_t *d_csr_index, bool pack_in) {
   LaunchNarrow p = narrow_launch(map, kb, n, lo, R, W);
   const NarrowGeom &g = p.geom;
   p.pack = pack_in;
-  const uint64_t big_cap = std::max<uint64_t>(1, std::min<uint64_t>(R, 1ull << 28));
-  Plan P0, P1;
-  const size_t i_part = P0.add(n * kb);
-  const size_t i_cmat = P1.add((size_t)p.rows * g.ncols * 4), i_tot = P1.add(g.ncols * 4),
-               i_items = P1.add(g.ncols * sizeof(FinItem)), i_maps = P1.add(sizeof(BinMap)),
-               i_slot = P1.add(g.ncols * 4), i_ctl = P1.add(final_big_ctl_bytes()), i_cnt = P1.add(big_cap * 4);
-  HG_TRY(arena_ensure(c, 0, P0.total()));
-  HG_TRY(arena_ensure(c, 1, P1.total()));
-  Carve c0, c1;
-  c0.init(c, 0, P0);
-  c1.init(c, 1, P1);
+  size_t o_cnt;
+  const NarrowPlan q(p.rows, g.ncols, final_rest(R, o_cnt));
+  HG_TRY(arena_ensure(c, 0, n * kb));
+  HG_TRY(arena_ensure(c, 1, q.P.total()));
+  uint32_t *big_slot;
+  char *rest;
+  q.carve(c, p, big_slot, rest);
   p.keys = d_keys;
-  p.out = c0.get<void>(i_part);
-  p.cmat = c1.get<uint32_t>(i_cmat);
-  p.tot = c1.get<uint32_t>(i_tot);
-  p.items = c1.get<FinItem>(i_items);
-  p.maps = c1.get<BinMap>(i_maps);
-  p.zero = c1.get<unsigned long long>(i_ctl);
+  p.out = c->arena[0];
+  p.zero = (unsigned long long *)rest;
   p.nzero = BIG_CTL_ZERO;
   {
     Prof pf(c, "part_scatter");
@@ -706,10 +766,10 @@ hg_status build_narrow(hg_ctx c, const BinMap &map, int kb, int ob, uint64_t n, 
   f.off = d_off;
   f.items = p.items;
   f.maps = p.maps;
-  f.big_slot = c1.get<uint32_t>(i_slot);
-  f.big_ctl = p.zero;
-  f.big_cnt = c1.get<uint32_t>(i_cnt);
-  f.big_cap = (uint32_t)big_cap;
+  f.big_slot = big_slot;
+  f.big_ctl = rest;
+  f.big_cnt = (uint32_t *)(rest + o_cnt);
+  f.big_cap = (uint32_t)LevelPlan::big_counters(R);
   f.csr_index = d_csr_index;
   Prof pf(c, "final");
   HG_HIP(launch_final(f, c->stream));
@@ -772,12 +832,8 @@ int deep_class(uint64_t n, uint64_t R, uint32_t &W) {
   return -1;
 }
 
-// Geometry of a two-step partition, its scratch in arena 1 (extra bytes of the
-// caller's behind it, at *rest) and its pointers, but for the keys' own.
-hg_status deep_launch(hg_ctx c, const BinMap &map, int kb, uint64_t n, uint64_t lo, uint64_t R, uint32_t W,
-                      size_t extra, LaunchDeep &p, char *&rest) {
-  p = LaunchDeep{};
-  DeepGeom &g = p.geom;
+DeepGeom deep_geom(const BinMap &map, uint64_t n, uint64_t lo, uint64_t R, uint32_t W) {
+  DeepGeom g{};
   g.n = n;
   g.nbins = R;
   g.per = (uint32_t)(((n + DEEP_ROWS - 1) / DEEP_ROWS + 1023) & ~1023ull);
@@ -788,27 +844,48 @@ hg_status deep_launch(hg_ctx c, const BinMap &map, int kb, uint64_t n, uint64_t 
   g.fine = make_div(W);
   g.coarse = make_div(W * g.group);
   g.map = map;
-  p.key_bytes = kb;
-  p.rows = (uint32_t)((n + g.per - 1) / g.per);
+  return g;
+}
+
+// Arena 1 of a two-step partition; extra bytes of the caller's behind it.
+struct DeepPlan {
   Plan P;
-  const size_t i_cmat = P.add((size_t)DEEP_ROWS * g.ngroups * 4), i_fmat = P.add((size_t)DEEP_ROWS * g.nfine * 4),
-               i_ftot = P.add(g.nfine * 4), i_fstart = P.add(((size_t)g.nfine + 1) * 4),
-               i_gstart = P.add((size_t)8 * g.ngroups * 4),
-               i_chunks = P.add((size_t)deep_max_chunks(g, kb) * sizeof(DeepChunk)), i_nch = P.add(8),
-               i_items = P.add((size_t)g.nfine * sizeof(FinItem)), i_maps = P.add(sizeof(BinMap)), i_rest = P.add(extra);
-  HG_TRY(arena_ensure(c, 1, P.total()));
+  size_t cmat, fmat, ftot, fstart, gstart, chunks, nch, items, maps, rest;
+  DeepPlan(const DeepGeom &g, int kb, size_t extra) {
+    cmat = P.add((size_t)DEEP_ROWS * g.ngroups * 4);
+    fmat = P.add((size_t)DEEP_ROWS * g.nfine * 4);
+    ftot = P.add(g.nfine * 4);
+    fstart = P.add(((size_t)g.nfine + 1) * 4);
+    gstart = P.add((size_t)8 * g.ngroups * 4);
+    chunks = P.add((size_t)deep_max_chunks(g, kb) * sizeof(DeepChunk));
+    nch = P.add(8);
+    items = P.add((size_t)g.nfine * sizeof(FinItem));
+    maps = P.add(sizeof(BinMap));
+    rest = P.add(extra);
+  }
+};
+
+// A two-step partition's launch, its scratch in arena 1 and its pointers, but
+// for the keys' own.
+hg_status deep_launch(hg_ctx c, const DeepGeom &g, int kb, size_t extra, LaunchDeep &p, char *&rest) {
+  p = LaunchDeep{};
+  p.geom = g;
+  p.key_bytes = kb;
+  p.rows = (uint32_t)((g.n + g.per - 1) / g.per);
+  const DeepPlan q(g, kb, extra);
+  HG_TRY(arena_ensure(c, 1, q.P.total()));
   Carve cv;
-  cv.init(c, 1, P);
-  p.cmat = cv.get<uint32_t>(i_cmat);
-  p.fmat = cv.get<uint32_t>(i_fmat);
-  p.ftot = cv.get<uint32_t>(i_ftot);
-  p.fstart = cv.get<uint32_t>(i_fstart);
-  p.gstart = cv.get<uint32_t>(i_gstart);
-  p.chunks = cv.get<DeepChunk>(i_chunks);
-  p.nchunks = cv.get<uint32_t>(i_nch);
-  p.items = cv.get<FinItem>(i_items);
-  p.maps = cv.get<BinMap>(i_maps);
-  rest = cv.get<char>(i_rest);
+  cv.init(c, 1, q.P);
+  p.cmat = cv.get<uint32_t>(q.cmat);
+  p.fmat = cv.get<uint32_t>(q.fmat);
+  p.ftot = cv.get<uint32_t>(q.ftot);
+  p.fstart = cv.get<uint32_t>(q.fstart);
+  p.gstart = cv.get<uint32_t>(q.gstart);
+  p.chunks = cv.get<DeepChunk>(q.chunks);
+  p.nchunks = cv.get<uint32_t>(q.nch);
+  p.items = cv.get<FinItem>(q.items);
+  p.maps = cv.get<BinMap>(q.maps);
+  rest = cv.get<char>(q.rest);
   return HG_OK;
 }
 
@@ -819,12 +896,12 @@ bool overlap(const void *a, uint64_t na, const void *b, uint64_t nb) {
 
 hg_status build_deep(hg_ctx c, const BinMap &map, int kb, int ob, uint64_t n, uint64_t lo, uint64_t R, int cls,
                      uint32_t W, const void *d_keys, void *d_off, void *d_csr, uint64_t *d_csr_index, bool pack_in) {
-  const uint64_t F = (R + W - 1) / W, big_cap = std::max<uint64_t>(1, std::min<uint64_t>(R, 1ull << 28));
-  Plan Px;
-  const size_t i_ctl = Px.add(final_big_ctl_bytes()), i_slot = Px.add(F * 4), i_cnt = Px.add(big_cap * 4);
+  const DeepGeom g = deep_geom(map, n, lo, R, W);
+  size_t o_cnt;
+  const size_t o_slot = final_rest(R, o_cnt);
   LaunchDeep p;
   char *rest;
-  HG_TRY(deep_launch(c, map, kb, n, lo, R, W, Px.total(), p, rest));
+  HG_TRY(deep_launch(c, g, kb, o_slot + (size_t)g.nfine * 4, p, rest));
   // the grouped keys pass through the CSR, which only the final stage writes
   // otherwise, unless the caller builds over the keys themselves
   void *mid = d_csr_index ? (void *)d_csr_index : d_csr;
@@ -838,7 +915,6 @@ hg_status build_deep(hg_ctx c, const BinMap &map, int kb, int ob, uint64_t n, ui
   p.keys = d_keys;
   p.mid = own ? c0.get<void>(i_mid) : mid;
   p.out = c0.get<void>(i_part);
-  const size_t o_slot = Px.sizes[i_ctl], o_cnt = o_slot + Px.sizes[i_slot];
   p.zero = (unsigned long long *)rest;
   p.nzero = BIG_CTL_ZERO;
   {
@@ -849,12 +925,11 @@ hg_status build_deep(hg_ctx c, const BinMap &map, int kb, int ob, uint64_t n, ui
     Prof pf(c, "part_scatter");
     HG_HIP(launch_deep_scatter(p, c->stream));
   }
-  (void)i_cnt;
   LaunchFinal f{};
   f.key_bytes = kb;
   f.off_bytes = ob;
   f.hk = (int)map.kind;
-  f.nitems = p.geom.nfine;
+  f.nitems = g.nfine;
   f.cls = cls;
   f.many = true;  // so many buckets that a few thousand keys too many are a throughput matter
   f.lds_bytes = std::max<uint32_t>((W + 1) / 2 * 4, std::min<uint32_t>(final_class_keys(cls) * (uint32_t)kb, 64 * 1024));
@@ -867,7 +942,7 @@ hg_status build_deep(hg_ctx c, const BinMap &map, int kb, int ob, uint64_t n, ui
   f.big_ctl = rest;
   f.big_slot = (uint32_t *)(rest + o_slot);
   f.big_cnt = (uint32_t *)(rest + o_cnt);
-  f.big_cap = (uint32_t)big_cap;
+  f.big_cap = (uint32_t)LevelPlan::big_counters(R);
   f.csr_index = d_csr_index;
   Prof pf(c, "final");
   HG_HIP(launch_final(f, c->stream));
@@ -1159,10 +1234,25 @@ std::vector<LaunchRmiBatch> rmi_launches(std::vector<RmiBatchItem> &items, int k
 // ===========================================================================
 // Wide pass of hg_probe: the probe keys partitioned by buckets of the table's
 // bins (one or two levels) and pr's items, their state and the one-pass
-// kernel's class filled in.
+// kernel's class filled in.  The probe keys are d_probe, or (null) the list the
+// direct probe left in the first `list` bytes of arena 0.
+struct WideProbePlan {
+  Plan P;
+  size_t list, part, part2, small, mark;
+  WideProbePlan(uint64_t n_probe, int kb, uint64_t F, bool two, size_t list_bytes) {
+    list = P.add(list_bytes);
+    part = P.add(n_probe * kb);
+    part2 = P.add(two ? n_probe * kb : 1);
+    small = P.add(256);
+    mark = P.add((size_t)(F + kFMax + 1) * 4);  // >= the buckets of the last level
+  }
+};
+static uint32_t probe_width(uint64_t n_probe, uint64_t n_keys, uint64_t M, int kb) {
+  return choose_width(std::max<uint64_t>(n_probe, n_keys), M, kb, probe_fill(kb));
+}
 static hg_status probe_wide(hg_ctx c, const BinMap &map, int kb, uint64_t n_keys, uint64_t M, const void *d_probe,
-                     uint64_t n_probe, uint64_t done, LaunchProbe &pr) {
-  const uint32_t W = choose_width(std::max<uint64_t>(n_probe, n_keys), M, kb, probe_fill(kb));
+                            uint64_t n_probe, size_t list, uint64_t done, LaunchProbe &pr) {
+  const uint32_t W = probe_width(n_probe, n_keys, M, kb);
   const uint64_t F = (M + W - 1) / W;
   // Beyond kFMax buckets, B is partitioned twice: into super-buckets of k
   // buckets, whose sizes are read back, then each super-bucket into its
@@ -1170,17 +1260,14 @@ static hg_status probe_wide(hg_ctx c, const BinMap &map, int kb, uint64_t n_keys
   const uint64_t k = level1_group(F);
   const bool two = k > 1;
   if ((uint64_t)W * k >= (1ull << 32)) return fail(HG_ERR_UNSUPPORTED, "probe geometry too large");
-  Plan P0;
-  const size_t i_part = P0.add(n_probe * kb);
-  const size_t i_part2 = P0.add(two ? n_probe * kb : 1);
-  const size_t i_small = P0.add(256);
-  const size_t i_mark = P0.add((size_t)(F + kFMax + 1) * 4);  // >= the buckets of the last level
-  HG_TRY(arena_ensure(c, 0, P0.total()));
+  const WideProbePlan q(n_probe, kb, F, two, list);
+  HG_TRY(arena_ensure(c, 0, q.P.total(), list));
   Carve cv0;
-  cv0.init(c, 0, P0);
-  void *part = cv0.get<void>(i_part);
-  unsigned long long *small = cv0.get<unsigned long long>(i_small);
-  unsigned int *hmark = cv0.get<unsigned int>(i_mark);
+  cv0.init(c, 0, q.P);
+  if (!d_probe) d_probe = cv0.get<void>(q.list);
+  void *part = cv0.get<void>(q.part);
+  unsigned long long *small = cv0.get<unsigned long long>(q.small);
+  unsigned int *hmark = cv0.get<unsigned int>(q.mark);
   Level L;
   LevelDev d;
   if (!two) {
@@ -1219,7 +1306,7 @@ static hg_status probe_wide(hg_ctx c, const BinMap &map, int kb, uint64_t n_keys
     L.auto_tile(n_probe);
     L.prepare();
     HG_TRY(setup_level(c, L, d));
-    void *part2 = cv0.get<void>(i_part2);
+    void *part2 = cv0.get<void>(q.part2);
     HG_TRY(run_level(c, L, d, kb, part, part2));
     part = part2;
   }
@@ -1245,34 +1332,48 @@ static hg_status probe_wide(hg_ctx c, const BinMap &map, int kb, uint64_t n_keys
   return HG_OK;
 }
 
+// What a narrow probe keeps behind its partition's scratch: the buckets' marks,
+// the cursor with the gates and the list of oversized buckets.
+static size_t narrow_probe_rest() { return NARROW_COLS * 4 + 256 + final_big_ctl_bytes(); }
+
 // Two-step partition of hg_probe's keys and pr's items and state; taken stays
 // false when its geometry or the memory for its second copy of the keys does
 // not allow it.
+struct DeepProbePlan {
+  Plan P0, rest;  // arena 0; what follows the partition's scratch in arena 1
+  size_t list, part, mid, slot, mark, ctl;
+  DeepProbePlan(uint64_t n_probe, int kb, uint64_t F, size_t list_bytes) {
+    list = P0.add(list_bytes);
+    part = P0.add(n_probe * kb);
+    mid = P0.add(n_probe * kb);
+    slot = rest.add(F * 4);
+    mark = rest.add(F * 4);
+    ctl = rest.add(256 + final_big_ctl_bytes());
+  }
+};
 static hg_status probe_deep(hg_ctx c, const BinMap &map, int kb, uint64_t n_keys, uint64_t M, const void *d_probe,
-                            uint64_t n_probe, uint64_t done, LaunchProbe &pr, bool &taken) {
+                            uint64_t n_probe, size_t list, uint64_t done, LaunchProbe &pr, bool &taken) {
   uint32_t W, lds = 0;
   const uint32_t one = deep_probe(n_probe, n_keys, M, kb, W, lds);
   if (!one) return HG_OK;
-  const uint64_t F = (M + W - 1) / W;
-  Plan P0, Px;
-  const size_t i_part = P0.add(n_probe * kb), i_mid = P0.add(n_probe * kb);
-  if (arena_ensure(c, 0, P0.total()) != HG_OK) return HG_OK;
-  const size_t i_slot = Px.add(F * 4), i_mark = Px.add(F * 4), i_ctl = Px.add(256 + final_big_ctl_bytes());
+  const DeepGeom g = deep_geom(map, n_probe, 0, M, W);
+  const DeepProbePlan q(n_probe, kb, g.nfine, list);
   LaunchDeep p;
   char *rest;
-  HG_TRY(deep_launch(c, map, kb, n_probe, 0, M, W, Px.total(), p, rest));
+  if (arena_ensure(c, 0, q.P0.total(), list) != HG_OK) return HG_OK;
+  HG_TRY(deep_launch(c, g, kb, q.rest.total(), p, rest));
   Carve c0;
-  c0.init(c, 0, P0);
+  c0.init(c, 0, q.P0);
+  if (!d_probe) d_probe = c0.get<void>(q.list);
   // the cursor and the gates end where the list of oversized buckets begins
   pr.big_slot = (uint32_t *)rest;
-  pr.hmark = (unsigned int *)(rest + Px.sizes[i_slot]);
-  pr.big_ctl = rest + Px.sizes[i_slot] + Px.sizes[i_mark] + 256;
+  pr.hmark = (unsigned int *)(rest + q.rest.sizes[q.slot]);
+  pr.big_ctl = rest + q.rest.sizes[q.slot] + q.rest.sizes[q.mark] + 256;
   pr.cursor = (unsigned long long *)pr.big_ctl - 2;
   pr.gate = (unsigned int *)(pr.cursor + 1);
-  (void)i_ctl;
   p.keys = d_probe;
-  p.mid = c0.get<void>(i_mid);
-  p.out = c0.get<void>(i_part);
+  p.mid = c0.get<void>(q.mid);
+  p.out = c0.get<void>(q.part);
   p.zero = pr.cursor;
   p.nzero = 2 + BIG_CTL_ZERO;
   p.zero_col = pr.hmark;
@@ -1305,18 +1406,100 @@ static hg_status probe_deep(hg_ctx c, const BinMap &map, int kb, uint64_t n_keys
 // way).  Tables of long bins go to the partitioned probe at once.
 constexpr uint64_t kDirectProbe = 1ull << 21, kDirectProbeShare = 32;       // where the other way is the wide pass
 constexpr uint64_t kDirectNarrow4 = 1ull << 20, kDirectNarrow8 = 5ull << 18;  // where it is the narrow one
-static bool probe_direct_takes(const hg_table_desc *A, const void *d_probe, uint64_t n_probe, const void *d_out,
-                        uint64_t capacity) {
+static bool probe_direct_size(const hg_table_desc *A, uint64_t n_probe) {
   if (A->n_keys > 8 * A->n_bins) return false;
   uint32_t W, lds;
   const bool narrow = narrow_probe(n_probe, A->n_keys, A->n_bins, (int)A->key_bytes, W, lds) != 0;
   const uint64_t most = !narrow ? std::max(kDirectProbe, A->n_keys / kDirectProbeShare)
                                 : A->key_bytes == 4 ? kDirectNarrow4 : kDirectNarrow8;
-  if (n_probe > most) return false;
+  return n_probe <= most;
+}
+static bool probe_direct_takes(const hg_table_desc *A, const void *d_probe, uint64_t n_probe, const void *d_out,
+                               uint64_t capacity) {
+  if (!probe_direct_size(A, n_probe)) return false;
   // matches are written while other workgroups still read the probe keys
   const uintptr_t o = (uintptr_t)d_out, q = (uintptr_t)d_probe;
   const uint64_t room = std::min<uint64_t>(capacity, 1ull << 40) * A->key_bytes;
   return !d_out || o + room <= q || q + n_probe * A->key_bytes <= o;
+}
+
+// Bytes of arenas 0 and 1 that a build, and a probe with as many keys, of a
+// description take (the pieces are those of the calls' own plans).
+struct ScratchNeed {
+  size_t a0 = 0, a1 = 0;
+  void add(size_t x0, size_t x1) {
+    a0 = std::max(a0, x0);
+    a1 = std::max(a1, x1);
+  }
+};
+
+// One level over F buckets of W bins or, with k > 1, a level over groups of k
+// buckets and one over each group's buckets (its keys shared evenly).
+static size_t need_levels(uint64_t n, uint64_t R, const BinMap &map, uint32_t W, uint64_t k) {
+  Level L;
+  L.segs.push_back(range_seg(0, n, 0, R, (uint32_t)std::min<uint64_t>((uint64_t)W * k, 0xFFFFFFFFull), map));
+  L.maps.push_back(map);
+  L.auto_tile(n);
+  L.prepare();
+  size_t need = LevelPlan(L, LevelBlob(L).b.data.size()).P.total();
+  if (k > 1) {
+    const uint64_t W1 = (uint64_t)W * k, G = L.ncols_total;
+    Level L2;
+    for (uint64_t g = 0; g < G; g++)
+      L2.segs.push_back(range_seg(n * g / G, n * (g + 1) / G, g * W1, std::min<uint64_t>(W1, R - g * W1), W, map));
+    L2.maps.push_back(map);
+    L2.auto_tile(n);
+    L2.prepare();
+    need = std::max(need, LevelPlan(L2, LevelBlob(L2).b.data.size()).P.total());
+  }
+  return need;
+}
+
+static void need_build(const hg_table_desc *d, ScratchNeed &need) {
+  const uint64_t n = d->n_keys, R = d->n_bins;
+  const int kb = (int)d->key_bytes;
+  const BinMap map = make_map(R, 0, nullptr);
+  uint32_t W;
+  size_t o_cnt;
+  if (build_one_takes(n, R, kb)) return;
+  if (narrow_class(n, R, W) >= 0) {
+    const LaunchNarrow p = narrow_launch(map, kb, n, 0, R, W);
+    return need.add(n * kb, NarrowPlan(p.rows, p.geom.ncols, final_rest(R, o_cnt)).P.total());
+  }
+  if (deep_class(n, R, W) >= 0) {  // in place: two copies of the keys
+    const DeepGeom g = deep_geom(map, n, 0, R, W);
+    return need.add(2 * ((n * kb + 255) & ~255ull), DeepPlan(g, kb, final_rest(R, o_cnt) + (size_t)g.nfine * 4).P.total());
+  }
+  W = choose_width(n, R, kb, build_fill());
+  const uint64_t k = level1_group((R + W - 1) / W);
+  need.add((k > 1 ? 2 : 1) * ((n * kb + 255) & ~255ull), need_levels(n, R, map, W, k));
+}
+
+static void need_probe(const hg_table_desc *d, ScratchNeed &need) {
+  const uint64_t n = d->n_keys, M = d->n_bins;
+  const int kb = (int)d->key_bytes;
+  const BinMap map = make_map(M, 0, nullptr);
+  // the direct probe may leave any number of its keys to the partitioned one,
+  // and fewer keys may take another of its ways
+  const bool direct = probe_direct_size(d, n);
+  const size_t list = direct ? n * kb : 0;
+  uint32_t W, lds = 0;
+  if (narrow_probe(n, n, M, kb, W, lds) || direct) {
+    Plan P0;
+    P0.add(list);
+    P0.add(n * kb);
+    need.add(P0.total(), NarrowPlan(NARROW_ROWS, NARROW_COLS, narrow_probe_rest()).P.total());
+    if (!direct) return;
+  }
+  if (deep_probe(n, n, M, kb, W, lds)) {
+    const DeepGeom g = deep_geom(map, n, 0, M, W);
+    const DeepProbePlan q(n, kb, g.nfine, list);
+    need.add(q.P0.total(), DeepPlan(g, kb, q.rest.total()).P.total() + (128 << 10));  // fewer keys: shorter chunks
+    if (!direct) return;
+  }
+  W = probe_width(n, n, M, kb);
+  const uint64_t F = (M + W - 1) / W, k = level1_group(F);
+  need.add(WideProbePlan(n, kb, F, k > 1, list).P.total(), need_levels(n, M, map, W, k));
 }
 
 extern "C" {
@@ -1439,21 +1622,18 @@ hg_status hg_ctx_reserve(hg_ctx c, size_t bytes) {
   return arena_ensure(c, 1, bytes - bytes / 2);
 }
 
+// hg_ctx_reserve halves its bytes between both arenas, so this is twice the
+// larger need.
 hg_status hg_scratch_bytes(const hg_table_desc *desc, int op, size_t *bytes) {
   HG_TRY(check_desc(desc));
   if (!bytes) return fail(HG_ERR_INVALID_ARG, "null bytes");
-  const uint64_t n = desc->n_keys, M = desc->n_bins;
-  const int kb = (int)desc->key_bytes;
-  const uint32_t W = choose_width(n, M, kb);
-  const uint64_t F = std::min<uint64_t>((M + W - 1) / W, kFMax);
-  const uint64_t tiles = (n + kTile - 1) / kTile + 1;
-  (void)op;
-  // a probe's two-step partition holds two copies of its keys (as many as the
-  // table's here) in the half hg_ctx_reserve gives the first arena
-  uint32_t Wp, lds;
-  const bool two = n && !narrow_probe(n, n, M, kb, Wp, lds) && deep_probe(n, n, M, kb, Wp, lds);
-  *bytes = (size_t)n * kb * (two ? 4 : 2) + (size_t)(tiles * (F + 1) * 4) * 2 + (size_t)F * 64 + (size_t)tiles * 64 +
-           (1 << 20);
+  (void)op;  // the larger of both
+  ScratchNeed need;
+  if (desc->n_keys) {
+    need_build(desc, need);
+    need_probe(desc, need);
+  }
+  *bytes = 2 * std::max(need.a0, need.a1) + (1 << 20);
   return HG_OK;
 }
 
@@ -1793,8 +1973,9 @@ hg_status hg_probe(hg_ctx c, const hg_table_desc *descA, const void *d_offA, con
   const BinMap map = make_map(M, descA->hash_kind, descA->d_rmi_model);
   uint64_t done = 0;  // matches already counted (and emitted) by the direct probe
   bool done_direct = false;
+  size_t list = 0;
   if (probe_direct_takes(descA, d_probe, n_probe, d_out, capacity)) {
-    HG_TRY(arena_ensure(c, 2, n_probe * kb));
+    HG_TRY(arena_ensure(c, 0, n_probe * kb));
     LaunchProbeDirect p{};
     p.key_bytes = kb;
     p.off_bytes = ob;
@@ -1805,7 +1986,7 @@ hg_status hg_probe(hg_ctx c, const hg_table_desc *descA, const void *d_offA, con
     p.n = (uint32_t)n_probe;
     p.out = d_out;
     p.capacity = d_out ? capacity : 0;
-    p.heavy = c->arena[2];
+    p.heavy = c->arena[0];
     p.state = c->direct_state;
     p.res = c->h_direct;
     {
@@ -1815,7 +1996,6 @@ hg_status hg_probe(hg_ctx c, const hg_table_desc *descA, const void *d_offA, con
     HG_HIP(hipStreamSynchronize(c->stream));
     done = c->h_direct[0];
     n_probe = c->h_direct[1];
-    d_probe = c->arena[2];
     if (n_probe == 0) {
       *h_count = done;
       if (d_out && done > capacity) return fail(HG_ERR_CAPACITY, "output capacity smaller than the match count");
@@ -1823,35 +2003,30 @@ hg_status hg_probe(hg_ctx c, const hg_table_desc *descA, const void *d_offA, con
     }
     done_direct = true;
     // the keys of long bins go through the partitioned probe, whose value
-    // tables answer them
+    // tables answer them; their list keeps the front of arena 0
+    d_probe = nullptr;
+    list = n_probe * kb;
   }
   LaunchProbe pr{};
   uint32_t Wn, lds = 0;
   if (const uint32_t one = narrow_probe(n_probe, descA->n_keys, M, kb, Wn, lds); one) {
     LaunchNarrow p = narrow_launch(map, kb, n_probe, 0, M, Wn);
-    Plan P0, P1;
-    const size_t i_part = P0.add(n_probe * kb);
-    const size_t i_cmat = P1.add((size_t)p.rows * p.geom.ncols * 4), i_tot = P1.add(NARROW_COLS * 4),
-                 i_items = P1.add(NARROW_COLS * sizeof(FinItem)), i_maps = P1.add(sizeof(BinMap)),
-                 i_slot = P1.add(NARROW_COLS * 4), i_mark = P1.add(NARROW_COLS * 4),
-                 i_small = P1.add(256 + final_big_ctl_bytes());
-    HG_TRY(arena_ensure(c, 0, P0.total()));
-    HG_TRY(arena_ensure(c, 1, P1.total()));
-    Carve c0, c1;
+    Plan P0;
+    const size_t i_list = P0.add(list), i_part = P0.add(n_probe * kb);
+    const NarrowPlan q(p.rows, p.geom.ncols, narrow_probe_rest());
+    HG_TRY(arena_ensure(c, 0, P0.total(), list));
+    HG_TRY(arena_ensure(c, 1, q.P.total()));
+    Carve c0;
     c0.init(c, 0, P0);
-    c1.init(c, 1, P1);
+    char *rest;
+    q.carve(c, p, pr.big_slot, rest);
     // the cursor and the gates end where the list of oversized buckets begins
-    pr.big_ctl = c1.get<char>(i_small) + 256;
+    pr.hmark = (unsigned int *)rest;
+    pr.big_ctl = rest + NARROW_COLS * 4 + 256;
     pr.cursor = (unsigned long long *)pr.big_ctl - 2;
     pr.gate = (unsigned int *)(pr.cursor + 1);
-    pr.hmark = c1.get<unsigned int>(i_mark);
-    pr.big_slot = c1.get<uint32_t>(i_slot);
-    p.keys = d_probe;
+    p.keys = d_probe ? d_probe : c0.get<void>(i_list);
     p.out = c0.get<void>(i_part);
-    p.cmat = c1.get<uint32_t>(i_cmat);
-    p.tot = c1.get<uint32_t>(i_tot);
-    p.items = c1.get<FinItem>(i_items);
-    p.maps = c1.get<BinMap>(i_maps);
     p.zero = pr.cursor;
     p.nzero = 2 + BIG_CTL_ZERO;
     p.zero_col = pr.hmark;
@@ -1869,8 +2044,8 @@ hg_status hg_probe(hg_ctx c, const hg_table_desc *descA, const void *d_offA, con
     pr.one_lds = lds;
   } else {
     bool two = false;
-    HG_TRY(probe_deep(c, map, kb, descA->n_keys, M, d_probe, n_probe, done, pr, two));
-    if (!two) HG_TRY(probe_wide(c, map, kb, descA->n_keys, M, d_probe, n_probe, done, pr));
+    HG_TRY(probe_deep(c, map, kb, descA->n_keys, M, d_probe, n_probe, list, done, pr, two));
+    if (!two) HG_TRY(probe_wide(c, map, kb, descA->n_keys, M, d_probe, n_probe, list, done, pr));
   }
   pr.key_bytes = kb;
   pr.off_bytes = ob;

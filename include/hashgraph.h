@@ -70,7 +70,8 @@ hg_status hg_ctx_set_stream(hg_ctx ctx, void *stream);
 /* Grow the scratch arena to at least bytes now (no allocation later for
  * calls whose scratch fits). */
 hg_status hg_ctx_reserve(hg_ctx ctx, size_t bytes);
-/* Device bytes of scratch a build / probe of this description needs. */
+/* Device bytes of scratch a build / probe of this description needs (as many
+ * probe keys as table keys). */
 hg_status hg_scratch_bytes(const hg_table_desc *desc, int op, size_t *bytes);
 const char *hg_last_error(void);
 const char *hg_version(void);

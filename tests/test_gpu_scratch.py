@@ -1,0 +1,93 @@
+"""Scratch memory of builds and probes: what hg_scratch_bytes states, what
+hg_ctx_reserve covers, and what happens when there is no more."""
+import ctypes
+
+import pytest
+import torch
+
+import hashgraph_amd as hg
+from hashgraph_amd import _lib
+from hashgraph_amd import workloads as wl
+
+P = hg._p
+
+
+def _scratch(n, M, kb, ob=4):
+    b = ctypes.c_size_t(0)
+    assert _lib.load().hg_scratch_bytes(ctypes.byref(hg._desc(n, M, kb, ob)), 0, ctypes.byref(b)) == 0
+    return b.value
+
+
+@pytest.mark.parametrize("kb", [4, 8])
+@pytest.mark.parametrize("n,M", [(1000, 1000), (1 << 16, 1 << 16), (1 << 20, 1 << 20), (1 << 20, 1 << 25)])
+def test_stated_scratch_holds_a_direct_probe(kb, n, M):
+    """Half of it (hg_ctx_reserve's share of each arena) holds the listed keys
+    and their partitioned copy, and a build's per-bin counters."""
+    assert _scratch(n, M, kb) // 2 >= 2 * n * kb
+    if n > 16384:
+        assert _scratch(n, M, kb) // 2 >= 4 * M
+
+
+def _keys(kind, n, kb):
+    if kind == "uniform":
+        return wl.uniform_keys(1, n, kb, device="cuda")
+    k = wl.zipf_keys(1, n, 1.1, device="cuda")
+    return k if kb == 8 else k.to(torch.int32)
+
+
+def _build_probe(c, A, B, M, off, csr):
+    d = hg._desc(A.numel(), M, A.element_size(), 4)
+    cnt = ctypes.c_uint64(0)
+    hg.check(c.lib.hg_build(c.bind_stream(), ctypes.byref(d), P(A), P(off), P(csr)), "hg_build")
+    hg.check(c.lib.hg_probe(c.bind_stream(), ctypes.byref(d), P(off), P(csr), P(B), B.numel(), None, 0,
+                            ctypes.byref(cnt)), "hg_probe")
+    return cnt.value
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["uniform", "zipf"])
+@pytest.mark.parametrize("kb", [4, 8])
+@pytest.mark.parametrize("n,M", [(1 << 20, 1 << 20), (1 << 22, 1 << 22), (3000001, 1 << 20), (1 << 25, 1 << 25),
+                                 (1 << 22, 1 << 17)])
+def test_reserved_context_allocates_nothing(kind, kb, n, M):
+    A, B = _keys(kind, n, kb), _keys(kind, n, kb).flip(0).contiguous()
+    fewer = B[: n // 3].clone()
+    off = torch.empty(M + 1, dtype=torch.int32, device="cuda")
+    csr = torch.empty_like(A)
+    want = _build_probe(hg.context(), A, B, M, off, csr)  # the kernels are loaded
+    c = hg.Context(0)
+    try:
+        c.reserve(_scratch(n, M, kb))
+        torch.cuda.synchronize()
+        free = torch.cuda.mem_get_info()[0]
+        assert _build_probe(c, A, B, M, off, csr) == want
+        assert _build_probe(c, A, fewer, M, off, csr) <= want
+        torch.cuda.synchronize()
+        assert torch.cuda.mem_get_info()[0] == free
+    finally:
+        c.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kb", [4, 8])
+def test_keys_listed_by_a_direct_probe_survive_a_growing_arena(kb):
+    """Every probe key is listed (long bins only), so the partitioned probe
+    that follows needs more of the arena than the list did."""
+    n, M = 1 << 19, 1 << 17
+    A = _keys("uniform", n, kb)[: n // 64].repeat(64)
+    B = A.flip(0).contiguous()
+    off = torch.empty(M + 1, dtype=torch.int32, device="cuda")
+    csr = torch.empty_like(A)
+    c = hg.Context(0)
+    try:
+        d = hg._desc(n, M, kb, 4)
+        hg.check(hg.context().lib.hg_build(hg.context().bind_stream(), ctypes.byref(d), P(A), P(off), P(csr)), "hg_build")
+        torch.cuda.synchronize()
+        cnt = ctypes.c_uint64(0)
+        out = torch.empty(n * 64, dtype=A.dtype, device="cuda")
+        hg.check(c.lib.hg_probe(c.bind_stream(), ctypes.byref(d), P(off), P(csr), P(B), n, P(out), n * 64,
+                                ctypes.byref(cnt)), "hg_probe")
+        assert cnt.value == n * 64
+        assert torch.equal(out.sort().values, B.repeat_interleave(64).sort().values)
+    finally:
+        c.close()
