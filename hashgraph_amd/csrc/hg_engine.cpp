@@ -251,6 +251,14 @@ hg_status arena_ensure(hg_ctx c, int a, size_t bytes, size_t keep = 0) {
   return HG_OK;
 }
 
+hg_status arena_release(hg_ctx c, int a) {
+  HG_HIP(hipStreamSynchronize(c->stream));
+  if (c->arena[a]) HG_HIP(hipFree(c->arena[a]));
+  c->arena[a] = nullptr;
+  c->arena_cap[a] = 0;
+  return HG_OK;
+}
+
 // Sizes of the arena pieces of one call, carved in order.
 struct Plan {
   std::vector<size_t> sizes;
@@ -894,21 +902,27 @@ bool overlap(const void *a, uint64_t na, const void *b, uint64_t nb) {
   return x < y + nb && y < x + na;
 }
 
+// taken stays false when the scratch does not fit (in place it is two copies
+// of the keys, one for the wide pass).
 hg_status build_deep(hg_ctx c, const BinMap &map, int kb, int ob, uint64_t n, uint64_t lo, uint64_t R, int cls,
-                     uint32_t W, const void *d_keys, void *d_off, void *d_csr, uint64_t *d_csr_index, bool pack_in) {
+                     uint32_t W, const void *d_keys, void *d_off, void *d_csr, uint64_t *d_csr_index, bool pack_in,
+                     bool &taken) {
+  taken = false;
   const DeepGeom g = deep_geom(map, n, lo, R, W);
   size_t o_cnt;
   const size_t o_slot = final_rest(R, o_cnt);
   LaunchDeep p;
   char *rest;
-  HG_TRY(deep_launch(c, g, kb, o_slot + (size_t)g.nfine * 4, p, rest));
+  if (const hg_status st = deep_launch(c, g, kb, o_slot + (size_t)g.nfine * 4, p, rest); st != HG_OK)
+    return st == HG_ERR_OOM ? HG_OK : st;
   // the grouped keys pass through the CSR, which only the final stage writes
   // otherwise, unless the caller builds over the keys themselves
   void *mid = d_csr_index ? (void *)d_csr_index : d_csr;
   const bool own = overlap(mid, n * kb, d_keys, n * (pack_in ? 4 : kb));
   Plan P0;
   const size_t i_part = P0.add(n * kb), i_mid = P0.add(own ? n * kb : 1);
-  HG_TRY(arena_ensure(c, 0, P0.total()));
+  if (const hg_status st = arena_ensure(c, 0, P0.total()); st != HG_OK) return st == HG_ERR_OOM ? HG_OK : st;
+  taken = true;
   Carve c0;
   c0.init(c, 0, P0);
   p.pack = pack_in;
@@ -974,8 +988,11 @@ hg_status build_range(hg_ctx c, const BinMap &map, int kb, int ob, uint64_t n, u
   uint32_t Wn;
   if (const int cls = narrow_class(n, R, Wn); cls >= 0)
     return build_narrow(c, map, kb, ob, n, lo, R, cls, Wn, d_keys, d_off, d_csr, d_csr_index, pack_in);
-  if (const int cls = n < (1ull << 32) ? deep_class(n, R, Wn) : -1; cls >= 0)
-    return build_deep(c, map, kb, ob, n, lo, R, cls, Wn, d_keys, d_off, d_csr, d_csr_index, pack_in);
+  if (const int cls = n < (1ull << 32) ? deep_class(n, R, Wn) : -1; cls >= 0) {
+    bool taken;
+    HG_TRY(build_deep(c, map, kb, ob, n, lo, R, cls, Wn, d_keys, d_off, d_csr, d_csr_index, pack_in, taken));
+    if (taken) return HG_OK;
+  }
   const uint32_t W = choose_width(n, R, kb, build_fill());
   const uint64_t F = (R + W - 1) / W;
   const uint64_t k = level1_group(F);
@@ -1360,8 +1377,12 @@ static hg_status probe_deep(hg_ctx c, const BinMap &map, int kb, uint64_t n_keys
   const DeepProbePlan q(n_probe, kb, g.nfine, list);
   LaunchDeep p;
   char *rest;
-  if (arena_ensure(c, 0, q.P0.total(), list) != HG_OK) return HG_OK;
-  HG_TRY(deep_launch(c, g, kb, q.rest.total(), p, rest));
+  if (const hg_status st = arena_ensure(c, 0, q.P0.total(), list); st != HG_OK) return st == HG_ERR_OOM ? HG_OK : st;
+  if (const hg_status st = deep_launch(c, g, kb, q.rest.total(), p, rest); st != HG_OK) {
+    if (st != HG_ERR_OOM) return st;
+    if (!list) HG_TRY(arena_release(c, 0));
+    return HG_OK;
+  }
   Carve c0;
   c0.init(c, 0, q.P0);
   if (!d_probe) d_probe = c0.get<void>(q.list);

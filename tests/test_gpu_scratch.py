@@ -91,3 +91,68 @@ def test_keys_listed_by_a_direct_probe_survive_a_growing_arena(kb):
         assert torch.equal(out.sort().values, B.repeat_interleave(64).sort().values)
     finally:
         c.close()
+
+
+class Room:
+    """While entered, holds the device's memory but for `nbytes`."""
+
+    def __init__(self, nbytes):
+        self.nbytes = nbytes
+
+    def __enter__(self):
+        torch.cuda.empty_cache()
+        torch.cuda.synchronize()
+        block = 64 << 20
+        self.held = [torch.empty(torch.cuda.mem_get_info()[0] - self.nbytes, dtype=torch.uint8, device="cuda")]
+        spare = []
+        try:  # what is free beyond the stated bytes, and inside cached segments (the first blocks), too
+            while len(spare) < 1024:
+                spare.append(torch.empty(block, dtype=torch.uint8, device="cuda"))
+        except torch.OutOfMemoryError:
+            pass
+        self.held += spare[: -(self.nbytes // block)]
+        del spare
+        torch.cuda.empty_cache()
+
+    def __exit__(self, *exc):
+        self.held.clear()
+        torch.cuda.empty_cache()
+
+
+@pytest.mark.gpu
+def test_build_in_place_without_memory_takes_one_copy():
+    """2^26 uint32 keys: 256 MiB a copy, as much again for the bins' counters.
+    The two-step partition needs two copies in place, the wide pass one."""
+    n = 1 << 26
+    keys = wl.uniform_keys(1, n, 4, device="cuda")
+    off, csr = hg.build(keys, n, 4)
+    off2 = torch.empty_like(off)
+    c = hg.Context(0)
+    try:
+        with Room(640 << 20):
+            hg.check(c.lib.hg_build(c.bind_stream(), ctypes.byref(hg._desc(n, n, 4, 4)), P(keys), P(off2), P(keys)),
+                     "hg_build")
+            torch.cuda.synchronize()
+    finally:
+        c.close()
+    assert torch.equal(off, off2)
+    bins = torch.repeat_interleave(torch.arange(n, dtype=torch.int32, device="cuda"), off.diff())
+    assert torch.equal(hg.hash_bins(keys, n), bins)
+    assert torch.equal(keys.sort().values, csr.sort().values)
+
+
+@pytest.mark.gpu
+def test_probe_without_memory_takes_one_copy():
+    """2^26 uint64 keys, 512 MiB a copy."""
+    n = 1 << 26
+    A = wl.uniform_keys(1, n, 8, device="cuda")
+    off, csr = hg.build(A, n, 4)
+    cnt = ctypes.c_uint64(0)
+    c = hg.Context(0)
+    try:
+        with Room(900 << 20):
+            hg.check(c.lib.hg_probe(c.bind_stream(), ctypes.byref(hg._desc(n, n, 8, 4)), P(off), P(csr), P(A), n, None,
+                                    0, ctypes.byref(cnt)), "hg_probe")
+    finally:
+        c.close()
+    assert cnt.value == hg.probe(off, csr, n, A, emit=False)[0] >= n
