@@ -1073,6 +1073,10 @@ constexpr uint64_t kPairCompareLimit = 1ull << 36;
 // Padded records of the run-length join's single pass (record + heavy-list
 // bytes) beyond which the two-pass form is used.
 constexpr uint64_t kRleOnePassBytes = 4ull << 30;
+// Room for them taken from the tables' sizes alone (a record per key of the
+// smaller table), which can be far more than the chunks' bounds add up to; a
+// larger call reads those back first, about 20 us of its milliseconds.
+constexpr uint64_t kRleBoundBytes = 256ull << 20;
 constexpr uint64_t kOvfChunk = 1ull << 16;
 
 hg_status rle_value_rich(hg_ctx c, const LaunchRle &r, const uint32_t *d_list, uint32_t n) {
@@ -2358,7 +2362,7 @@ hg_status hg_intersect_rle(hg_ctx c, const hg_table_desc *descA, const void *d_o
     sc.out32 = phbase;
     HG_HIP(launch_rle_scan(sc, status, c->stream));
     // the chunks' bounds add up to at most one record per key of the smaller
-    // side; only when that is too much are the sums themselves read back
+    // side; the sums are read back where that is too much
     const auto fits = [&] {
       return (double)s_rec * (descA->key_bytes + 16) + (double)s_heavy * 4 <= (double)kRleOnePassBytes;
     };
@@ -2373,7 +2377,8 @@ hg_status hg_intersect_rle(hg_ctx c, const hg_table_desc *descA, const void *d_o
     };
     s_rec = std::min(descA->n_keys, descB->n_keys);
     s_heavy = heavy_cap;
-    one_pass = fits() && arena_ensure(c, 0, layout()) == HG_OK;
+    const size_t bound = layout();
+    one_pass = fits() && (bound <= c->arena_cap[0] || (bound <= kRleBoundBytes && arena_ensure(c, 0, bound) == HG_OK));
     if (!one_pass) {
       unsigned long long sr = 0;
       uint32_t sh = 0;

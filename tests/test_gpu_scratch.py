@@ -156,3 +156,32 @@ def test_probe_without_memory_takes_one_copy():
     finally:
         c.close()
     assert cnt.value == hg.probe(off, csr, n, A, emit=False)[0] >= n
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kb", [4, 8])
+def test_run_length_join_keeps_to_its_bounds(kb):
+    """Tables of 2^24 keys without a common bin: no record, so no room for one
+    per key (335 MiB for uint32 keys, 403 for uint64)."""
+    n = M = 1 << 24
+    keys = wl.uniform_keys(1, 3 * n, kb, device="cuda")
+    low = hg.hash_bins(keys, M) < M // 2
+    ta, tb = (hg.build(k[:n].clone(), M, 4) for k in (keys[low], keys[~low]))
+    rk, ca, cb = (torch.empty(n, dtype=d, device="cuda") for d in (keys.dtype, torch.int64, torch.int64))
+    cnt, nrec = ctypes.c_uint64(1), ctypes.c_uint64(1)
+
+    def join(c):
+        d = hg._desc(n, M, kb, 4)
+        hg.check(c.lib.hg_intersect_rle(c.bind_stream(), ctypes.byref(d), P(ta[0]), P(ta[1]), ctypes.byref(d), P(tb[0]),
+                                        P(tb[1]), P(rk), P(ca), P(cb), n, ctypes.byref(nrec), ctypes.byref(cnt)), "rle")
+        assert (cnt.value, nrec.value) == (0, 0)
+        torch.cuda.synchronize()
+
+    join(hg.context())  # the kernels are loaded
+    c = hg.Context(0)
+    try:
+        free = torch.cuda.mem_get_info()[0]
+        join(c)
+        assert free - torch.cuda.mem_get_info()[0] < 200 << 20
+    finally:
+        c.close()
