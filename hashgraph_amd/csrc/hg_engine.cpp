@@ -76,7 +76,11 @@ Div32 make_div(uint32_t d) {
 
 uint32_t final_cap(int kb) { return std::min<uint32_t>(1024u * (uint32_t)final_kpt(kb), 65535u); }
 
-// Bucket fill of the build (HG_BUILD_FILL overrides it for tuning: above 1
+// HG_BUILD_FILL, HG_L1_FANOUT and HG_TILE_ROUNDS tune the wide pass, so with
+// one of them set every build and probe takes it, whatever its size.
+bool wide_only() { return getenv("HG_BUILD_FILL") || getenv("HG_L1_FANOUT") || getenv("HG_TILE_ROUNDS"); }
+
+// Bucket fill of the wide build (HG_BUILD_FILL overrides it for tuning: above 1
 // buckets exceed the final stage's VGPR capacity and take the oversized-bucket
 // kernels).
 double build_fill() {
@@ -970,7 +974,8 @@ hg_status build_range(hg_ctx c, const BinMap &map, int kb, int ob, uint64_t n, u
                       const void *d_keys, void *d_off, void *d_csr, uint64_t *d_csr_index = nullptr,
                       bool pack_in = false) {
   if (n == 0) return fill_offsets(c, d_off, ob, R + 1, 0);
-  if (!pack_in && !d_csr_index && build_one_takes(n, R, kb)) {
+  const bool wide = wide_only();
+  if (!wide && !pack_in && !d_csr_index && build_one_takes(n, R, kb)) {
     LaunchBuildOne b{};
     b.key_bytes = kb;
     b.off_bytes = ob;
@@ -986,9 +991,9 @@ hg_status build_range(hg_ctx c, const BinMap &map, int kb, int ob, uint64_t n, u
     return HG_OK;
   }
   uint32_t Wn;
-  if (const int cls = narrow_class(n, R, Wn); cls >= 0)
+  if (const int cls = wide ? -1 : narrow_class(n, R, Wn); cls >= 0)
     return build_narrow(c, map, kb, ob, n, lo, R, cls, Wn, d_keys, d_off, d_csr, d_csr_index, pack_in);
-  if (const int cls = n < (1ull << 32) ? deep_class(n, R, Wn) : -1; cls >= 0) {
+  if (const int cls = !wide && n < (1ull << 32) ? deep_class(n, R, Wn) : -1; cls >= 0) {
     bool taken;
     HG_TRY(build_deep(c, map, kb, ob, n, lo, R, cls, Wn, d_keys, d_off, d_csr, d_csr_index, pack_in, taken));
     if (taken) return HG_OK;
@@ -1486,12 +1491,13 @@ static void need_build(const hg_table_desc *d, ScratchNeed &need) {
   const BinMap map = make_map(R, 0, nullptr);
   uint32_t W;
   size_t o_cnt;
-  if (build_one_takes(n, R, kb)) return;
-  if (narrow_class(n, R, W) >= 0) {
+  const bool wide = wide_only();
+  if (!wide && build_one_takes(n, R, kb)) return;
+  if (!wide && narrow_class(n, R, W) >= 0) {
     const LaunchNarrow p = narrow_launch(map, kb, n, 0, R, W);
     return need.add(n * kb, NarrowPlan(p.rows, p.geom.ncols, final_rest(R, o_cnt)).P.total());
   }
-  if (deep_class(n, R, W) >= 0) {  // in place: two copies of the keys
+  if (!wide && deep_class(n, R, W) >= 0) {  // in place: two copies of the keys
     const DeepGeom g = deep_geom(map, n, 0, R, W);
     return need.add(2 * ((n * kb + 255) & ~255ull), DeepPlan(g, kb, final_rest(R, o_cnt) + (size_t)g.nfine * 4).P.total());
   }
@@ -1506,17 +1512,17 @@ static void need_probe(const hg_table_desc *d, ScratchNeed &need) {
   const BinMap map = make_map(M, 0, nullptr);
   // the direct probe may leave any number of its keys to the partitioned one,
   // and fewer keys may take another of its ways
-  const bool direct = probe_direct_size(d, n);
+  const bool wide = wide_only(), direct = !wide && probe_direct_size(d, n);
   const size_t list = direct ? n * kb : 0;
   uint32_t W, lds = 0;
-  if (narrow_probe(n, n, M, kb, W, lds) || direct) {
+  if (direct || (!wide && narrow_probe(n, n, M, kb, W, lds))) {
     Plan P0;
     P0.add(list);
     P0.add(n * kb);
     need.add(P0.total(), NarrowPlan(NARROW_ROWS, NARROW_COLS, narrow_probe_rest()).P.total());
     if (!direct) return;
   }
-  if (deep_probe(n, n, M, kb, W, lds)) {
+  if (!wide && deep_probe(n, n, M, kb, W, lds)) {
     const DeepGeom g = deep_geom(map, n, 0, M, W);
     const DeepProbePlan q(n, kb, g.nfine, list);
     need.add(q.P0.total(), DeepPlan(g, kb, q.rest.total()).P.total() + (128 << 10));  // fewer keys: shorter chunks
@@ -1999,7 +2005,8 @@ hg_status hg_probe(hg_ctx c, const hg_table_desc *descA, const void *d_offA, con
   uint64_t done = 0;  // matches already counted (and emitted) by the direct probe
   bool done_direct = false;
   size_t list = 0;
-  if (probe_direct_takes(descA, d_probe, n_probe, d_out, capacity)) {
+  const bool wide = wide_only();
+  if (!wide && probe_direct_takes(descA, d_probe, n_probe, d_out, capacity)) {
     HG_TRY(arena_ensure(c, 0, n_probe * kb));
     LaunchProbeDirect p{};
     p.key_bytes = kb;
@@ -2034,7 +2041,7 @@ hg_status hg_probe(hg_ctx c, const hg_table_desc *descA, const void *d_offA, con
   }
   LaunchProbe pr{};
   uint32_t Wn, lds = 0;
-  if (const uint32_t one = narrow_probe(n_probe, descA->n_keys, M, kb, Wn, lds); one) {
+  if (const uint32_t one = wide ? 0 : narrow_probe(n_probe, descA->n_keys, M, kb, Wn, lds); one) {
     LaunchNarrow p = narrow_launch(map, kb, n_probe, 0, M, Wn);
     Plan P0;
     const size_t i_list = P0.add(list), i_part = P0.add(n_probe * kb);
@@ -2069,7 +2076,7 @@ hg_status hg_probe(hg_ctx c, const hg_table_desc *descA, const void *d_offA, con
     pr.one_lds = lds;
   } else {
     bool two = false;
-    HG_TRY(probe_deep(c, map, kb, descA->n_keys, M, d_probe, n_probe, list, done, pr, two));
+    if (!wide) HG_TRY(probe_deep(c, map, kb, descA->n_keys, M, d_probe, n_probe, list, done, pr, two));
     if (!two) HG_TRY(probe_wide(c, map, kb, descA->n_keys, M, d_probe, n_probe, list, done, pr));
   }
   pr.key_bytes = kb;
