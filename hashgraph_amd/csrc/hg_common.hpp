@@ -8,6 +8,11 @@ namespace hg {
 // LDS by the partition kernels).
 constexpr uint32_t MAX_SPLITS = 4096;
 
+// Whether the bytes from p on lie in the size bytes from start on.
+constexpr bool covers(uint64_t start, uint64_t size, uint64_t p, uint64_t bytes) {
+  return p >= start && bytes <= size && p - start <= size - bytes;
+}
+
 // Division of a 32-bit value by an invariant d (1 <= d < 2^32) with one
 // 32-bit multiply-high (Granlund & Montgomery, "Division by invariant
 // integers using multiplication", PLDI 1994), l = floor(log2 d):

@@ -2833,20 +2833,25 @@ bool device_only(const void *p) {
 }
 
 // Device address of a range of pinned host memory that kernels can write, else
-// null (pageable, managed or device memory, a range beyond its allocation,
-// elements of kb bytes off their alignment).
+// null (pageable, managed or device memory, elements of kb bytes off their
+// alignment, a range that is not one allocation's or registration's: both its
+// ends may be pinned with something else between them).
 void *mapped_host(const void *p, size_t bytes, int kb) {
-  hipPointerAttribute_t a{}, e{};
+  hipPointerAttribute_t a{};
+  void *start = nullptr;
+  size_t size = 0;
   if ((uintptr_t)p % (size_t)kb) return nullptr;
-  if (hipPointerGetAttributes(&a, p) != hipSuccess ||
-      hipPointerGetAttributes(&e, (const char *)p + bytes - 1) != hipSuccess) {
+  if (hipPointerGetAttributes(&a, p) != hipSuccess || a.type != hipMemoryTypeHost || !a.devicePointer ||
+      hipPointerGetAttribute(&start, HIP_POINTER_ATTRIBUTE_RANGE_START_ADDR, (hipDeviceptr_t)p) != hipSuccess ||
+      hipPointerGetAttribute(&size, HIP_POINTER_ATTRIBUTE_RANGE_SIZE, (hipDeviceptr_t)p) != hipSuccess) {
     (void)hipGetLastError();
     return nullptr;
   }
-  if (a.type != hipMemoryTypeHost || e.type != hipMemoryTypeHost || !a.devicePointer ||
-      (char *)a.devicePointer + bytes - 1 != (char *)e.devicePointer)
-    return nullptr;
-  return a.devicePointer;
+  // the range's start may be stated as the host's or the device's address
+  return covers((uintptr_t)start, size, (uintptr_t)p, bytes) ||
+                 covers((uintptr_t)start, size, (uintptr_t)a.devicePointer, bytes)
+             ? a.devicePointer
+             : nullptr;
 }
 
 hg_status stage_streams(hg_ctx c, StageStreams &s) {
