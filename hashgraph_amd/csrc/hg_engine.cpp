@@ -788,33 +788,43 @@ hg_status build_narrow(hg_ctx c, const BinMap &map, int kb, int ob, uint64_t n, 
   return HG_OK;
 }
 
-// Geometry of a narrow probe: keys of B per workgroup and its LDS, the
-// smallest class whose buckets (W bins) are at most NARROW_COLS.  A bucket
-// should fill at most 0.8 of the class, and its keys of A with its offsets the
-// class's share of a CU's LDS, eight standard deviations above the mean (what
-// exceeds it takes k_probe).  Returns 0 when no class does: the wide pass.
-// Narrow against wide, as many uint32 probe keys as table keys: 60 against
-// 113 us at 2^21, 80 against 121 us at 2^22, 153 against 200 us at 12 M.
+// Most bins, up to w, whose 16-bit offsets and keys of A (r a bin, and eight
+// standard deviations above that mean) fit `room` bytes of LDS; lds: what they
+// take.  Below 1: not even one bin does.
+double probe_bins(double w, double r, int kb, uint32_t room, uint32_t &lds) {
+  for (; w >= 1; w *= 0.97) {
+    const double mean = w * r;
+    lds = probe_one_lds((uint32_t)w, (uint64_t)(mean + 8 * std::sqrt(mean) + 64), kb);
+    if (lds <= room) break;
+  }
+  return w;
+}
+// LDS of a one-pass probe's workgroup of the bucket classes (keys of B a
+// workgroup): three of them to a CU at 4 K, two at 8 K and 16 K, then one.
+uint32_t probe_room(int cls) { return cls == 0 ? 52 * 1024 : cls < 3 ? 78 * 1024 : PROBE1_LDS; }
+
+// Geometry of a probe's partition: keys of B per workgroup and its LDS, the
+// smallest class from `first` on whose buckets (W bins) are at most cols.  A
+// bucket should fill at most `fill` of the class; what exceeds its LDS takes
+// k_probe.  Returns 0 when no class does.
 uint32_t probe_geometry(uint64_t nb, uint64_t na, uint64_t M, int kb, int first, double fill, uint32_t cols, uint32_t &W,
                         uint32_t &lds) {
   const double r = (double)na / (double)M;
   for (int cls = first; cls < 4; cls++) {
     // the last two classes: 16 K keys with the whole LDS, then what the wide probe holds
     const uint32_t keys = cls < 3 ? 4096u << cls : probe_one_keys(kb);
-    const uint32_t room = cls == 0 ? 52 * 1024 : cls < 3 ? 78 * 1024 : PROBE1_LDS;
     double w = std::min(fill * keys * (double)M / (double)nb, 65535.0);
     w = std::min(w, std::max(2.0 * keys, std::ceil((double)M / cols)));
-    for (; w >= 1; w *= 0.97) {
-      const double mean = w * r;
-      lds = probe_one_lds((uint32_t)w, (uint64_t)(mean + 8 * std::sqrt(mean) + 64), kb);
-      if (lds <= room) break;
-    }
+    w = probe_bins(w, r, kb, probe_room(cls), lds);
     if (w < 1) continue;
     W = (uint32_t)w;
     if ((M + W - 1) / W <= cols) return keys;
   }
   return 0;
 }
+// The narrow partition of a probe; 0: the two-step or wide one.  Narrow against
+// wide, as many uint32 probe keys as table keys: 60 against 113 us at 2^21, 80
+// against 121 us at 2^22, 153 against 200 us at 12 M.
 uint32_t narrow_probe(uint64_t nb, uint64_t na, uint64_t M, int kb, uint32_t &W, uint32_t &lds) {
   return probe_geometry(nb, na, M, kb, 0, 0.8, NARROW_COLS, W, lds);
 }
@@ -3405,6 +3415,8 @@ BinMap batch_map(const hg_batch_desc *bd, uint32_t t) {
   return make_map(bd->h_n_bins[t], k, m);
 }
 
+// LDS of a batch's one-pass probe at its smaller class: 3 (uint64: 2) workgroups a CU.
+constexpr uint32_t batch_probe_room(int kb) { return kb == 4 ? 52 * 1024 : 78 * 1024; }
 // Buckets of one table beyond which a batch keeps to the largest bucket class.
 constexpr uint64_t kBatchCols = 1024;
 constexpr int kBatchCls = 1;  // the smaller class a plan tries: 8192 keys
@@ -3441,7 +3453,13 @@ hg_status batch_prepare(hg_ctx c, const hg_batch_desc *bd, const uint64_t *probe
     const uint64_t n = ko[t + 1] - ko[t], np = src[t + 1] - src[t], M = bd->h_n_bins[t];
     const uint64_t k = probe_off ? std::max(n, np) : n;
     if (cls == FINAL_CLASSES - 1) return choose_width(k, M, kb, probe_off ? std::min(cfg.fill, probe_fill(kb)) : cfg.fill);
-    return class_width(k, M, cls, probe_off ? 0.72 : cfg.fill, kBatchCols);
+    const uint32_t w = class_width(k, M, cls, probe_off ? 0.72 : cfg.fill, kBatchCols);
+    if (!probe_off) return w;
+    // sparse tables (more than about two bins a key): the offsets of so many
+    // bins leave the keys no room
+    uint32_t lds;
+    const double fit = probe_bins(w, (double)n / (double)M, kb, batch_probe_room(kb), lds);
+    return fit < 1 ? w : (uint32_t)fit;
   };
   S.L.cls = cfg.cls;
   for (uint32_t t = 0; t < bd->n_tables && S.L.cls != FINAL_CLASSES - 1; t++)
@@ -3503,9 +3521,9 @@ hg_status batch_launch_probe(hg_ctx c, const hg_batch_desc *bd, BatchSide &S, co
   if (S.L.cls == FINAL_CLASSES - 1) {
     pr.one_keys = probe_one_keys(pr.key_bytes);
     pr.one_lds = PROBE1_LDS;
-  } else {  // 0.72 of a class's keys with their offsets fit with 10% to spare; 3 (uint64: 2) workgroups a CU
+  } else {
     pr.one_keys = final_class_keys(S.L.cls);
-    pr.one_lds = pr.key_bytes == 4 ? 52 * 1024 : 78 * 1024;
+    pr.one_lds = batch_probe_room(pr.key_bytes);
   }
   pr.bpart = S.part;
   pr.items = S.d.fin;

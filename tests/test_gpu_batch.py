@@ -291,3 +291,32 @@ def test_plan_trains_models_in_graph(dev):
         assert plan.counts.cpu().numpy().tolist() == _expected_counts(keys, ko, probe, po)
     print(f"learned on {sum(use)} of {T} tables", flush=True)
     plan.close()
+
+
+@pytest.mark.parametrize("kb", [4, 8])
+@pytest.mark.parametrize("bins_per_key", [1.9, 2.2, 2.5, 2.9, 3.3, 5.0, 40.0])
+def test_sparse_tables(dev, kb, bins_per_key):
+    """Tables of more bins than keys: a bucket's offsets take as much of the
+    probe's LDS as its keys."""
+    import torch
+    import hashgraph_amd as hg
+    T, n = 6, 40000
+    ko = [0]
+    for t in range(T):
+        ko.append(ko[-1] + n + 1000 * t)
+    keys = wl.uniform_keys(41, ko[-1], kb)
+    probe = np.concatenate([wl.probe_keys(keys[ko[t]:ko[t + 1]], 43 + t, ko[t + 1] - ko[t], 0.5, kb) for t in range(T)])
+    for t in range(T):  # a bin beyond the walk limit in every table
+        keys[ko[t]:ko[t] + 50] = keys[ko[t]]
+    M = [int((ko[t + 1] - ko[t]) * bins_per_key) for t in range(T)]
+    print(f"sparse batch kb={kb} bins a key={bins_per_key}", flush=True)
+    dk, dp = _to_dev(keys, dev), _to_dev(probe, dev)
+    plan = hg.BatchPlan(dk, ko, M, dp, ko)
+    exp = _expected_counts(keys, ko, probe, ko)
+    for _ in range(3):
+        plan.run()
+        torch.cuda.synchronize()
+        assert plan.counts.cpu().numpy().tolist() == exp
+    for t in range(T):
+        off = hg.build(dk[ko[t]:ko[t + 1]].clone(), M[t])[0]
+        assert torch.equal(plan.offsets[plan.off_off[t]: plan.off_off[t] + M[t] + 1], off)
