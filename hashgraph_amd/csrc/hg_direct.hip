@@ -125,7 +125,7 @@ __global__ __launch_bounds__(BLOCK) void k_probe_direct(const K *__restrict__ pr
     for (int j = 0; j < U; j++)
       if ((hm >> j) & 1u) heavy[w++] = kr[j];
   }
-  if (out != nullptr && mine) {
+  if (out != nullptr && mine && s_base < capacity) {
     unsigned long long w = s_base + (ex & 0x3FFFFu);
 #pragma unroll
     for (int j = 0; j < U; j++)
