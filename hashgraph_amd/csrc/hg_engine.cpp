@@ -818,7 +818,14 @@ uint32_t probe_geometry(uint64_t nb, uint64_t na, uint64_t M, int kb, int first,
     w = probe_bins(w, r, kb, probe_room(cls), lds);
     if (w < 1) continue;
     W = (uint32_t)w;
-    if ((M + W - 1) / W <= cols) return keys;
+    if ((M + W - 1) / W > cols) continue;
+    // all the LDS that as many workgroups a CU leave each other: room for the
+    // buckets of duplicates, which spread wider than that, and for a learned
+    // model's leaves (4 M uint64 keys, 4096 leaves: 169 us with what the mean
+    // bucket needs, 98 with it; 8 M keys of 16 copies: 129 us a call of k_probe saved)
+    const uint32_t threads = cls < 2 ? 256u << cls : 1024;
+    lds = PROBE1_LDS / std::min(PROBE1_LDS / lds, 2048 / threads) & ~255u;
+    return keys;
   }
   return 0;
 }
