@@ -1631,7 +1631,9 @@ __device__ __forceinline__ void vt_fold(const K *__restrict__ keys, uint64_t a0,
 // largest find one.  On a partition of 2 M + 1 M Zipf(1.1) keys one workgroup's
 // longest bin took 78 us when only GIANT_MIN counted, and chunks of 64 K keys
 // 27 us a side; with GIANT_MID and 16 K chunks the whole pass over 16
-// partitions went from 6.79 to 5.34 ms (2^30 keys: 41.7 to 42.8 ms).
+// partitions went from 6.79 to 5.34 ms (2^30 keys: 41.7 to 42.8 ms, and to 39.1
+// once k_giant_prefix and k_sum_add were no longer one thread's and one
+// workgroup's work).
 constexpr uint32_t GIANT_MIN = 1u << 18, GIANT_MID = 1u << 15;
 constexpr uint32_t GIANT_CAP = 384, GIANT_MID_CAP = 128;
 constexpr uint32_t GIANT_CHUNK = 1u << 14;
@@ -1691,26 +1693,37 @@ __global__ __launch_bounds__(64) void k_giant_prefix(const OFF *__restrict__ off
                                                     const unsigned long long *__restrict__ nsmall,
                                                     unsigned long long *__restrict__ cursor,
                                                     unsigned long long *__restrict__ heavy_seen) {
-  if (threadIdx.x != 0) return;
-  *cursor = *nsmall;  // the heavy bins' records follow the small bins'
-  *heavy_seen = *heavy_n;
-  const uint32_t n = min(ctl->n, GIANT_CAP);
-  uint32_t a = 0, b = 0;
-  for (uint32_t s = 0; s < n; s++) {
-    const uint64_t bin = heavy[ctl->hidx[s]];
-    ctl->chA[s] = a;
-    ctl->chB[s] = b;
-    a += (uint32_t)(((uint64_t)(offA[bin + 1] - offA[bin]) + GIANT_CHUNK - 1) / GIANT_CHUNK);
-    b += (uint32_t)(((uint64_t)(offB[bin + 1] - offB[bin]) + GIANT_CHUNK - 1) / GIANT_CHUNK);
-    ctl->eA[s] = 0;
-    ctl->eB[s] = 0;
-    ctl->bad[s] = 0;
+  // a lane a bin: one thread that walked them all took 133 us for 384
+  const uint32_t lane = threadIdx.x, n = min(ctl->n, GIANT_CAP);
+  uint32_t a = 0, b = 0;  // chunks of the bins before s0
+  for (uint32_t s0 = 0; s0 < n; s0 += 64) {
+    const uint32_t s = s0 + lane;
+    uint32_t ca = 0, cb = 0;
+    if (s < n) {
+      const uint64_t bin = heavy[ctl->hidx[s]];
+      ca = (uint32_t)(((uint64_t)(offA[bin + 1] - offA[bin]) + GIANT_CHUNK - 1) / GIANT_CHUNK);
+      cb = (uint32_t)(((uint64_t)(offB[bin + 1] - offB[bin]) + GIANT_CHUNK - 1) / GIANT_CHUNK);
+      ctl->eA[s] = 0;
+      ctl->eB[s] = 0;
+      ctl->bad[s] = 0;
+    }
+    const uint32_t ia = wave_inclusive_sum<uint32_t>(ca), ib = wave_inclusive_sum<uint32_t>(cb);
+    if (s < n) {
+      ctl->chA[s] = a + ia - ca;
+      ctl->chB[s] = b + ib - cb;
+    }
+    a += __shfl(ia, 63, 64);
+    b += __shfl(ib, 63, 64);
   }
-  ctl->chA[n] = a;
-  ctl->chB[n] = b;
-  ctl->totalA = a;
-  ctl->totalB = b;
-  ctl->n = n;
+  if (lane == 0) {
+    *cursor = *nsmall;  // the heavy bins' records follow the small bins'
+    *heavy_seen = *heavy_n;
+    ctl->chA[n] = a;
+    ctl->chB[n] = b;
+    ctl->totalA = a;
+    ctl->totalB = b;
+    ctl->n = n;
+  }
 }
 
 template <typename K>
@@ -2187,12 +2200,12 @@ __global__ __launch_bounds__(1024) void k_rle_finish(const uint32_t *__restrict_
   if (threadIdx.x == 0) *cursor += tot;
 }
 
-// acc += sum of in[0..n) (one workgroup)
+// *acc += sum of in[0..n)
 __global__ __launch_bounds__(1024) void k_sum_add(const unsigned long long *__restrict__ in, uint64_t n,
                                                   unsigned long long *__restrict__ acc) {
   __shared__ unsigned long long s_t64[1024 / 64 + 1];
   unsigned long long s = 0;
-  for (uint64_t i = threadIdx.x; i < n; i += 1024) s += in[i];
+  for (uint64_t i = (uint64_t)blockIdx.x * 1024 + threadIdx.x; i < n; i += (uint64_t)gridDim.x * 1024) s += in[i];
   s = block_sum<1024, unsigned long long>(s, s_t64);
   if (threadIdx.x == 0 && s) atomicAdd(acc, s);
 }
@@ -3272,27 +3285,30 @@ __global__ void k_rle_caps(const OFF *__restrict__ offA, const OFF *__restrict__
   }
 }
 
-// One workgroup per chunk (grid-stride): its records and heavy bins from the
+// One wave per chunk (grid-stride): its records and heavy bins from the
 // padded places to the compact ones; records at or beyond capacity are
-// dropped, as when written directly.
+// dropped, as when written directly.  A chunk has a few dozen records, so the
+// time is the latency of its bounds, then its records (2^27 bins: 95 us,
+// 210 with a workgroup a chunk).
 template <typename K>
 __global__ __launch_bounds__(256) void k_rle_gather(LaunchRleGather g) {
   const K *srk = (const K *)g.srk;
   K *rk = (K *)g.rk;
-  for (uint32_t j = blockIdx.x; j < g.nch; j += gridDim.x) {
+  const uint32_t lane = threadIdx.x & 63;
+  for (uint32_t j = blockIdx.x * 4 + (threadIdx.x >> 6); j < g.nch; j += gridDim.x * 4) {
     const uint64_t s = g.pbase[j], n = g.cnt[j], d = g.cbase[j];
     const uint32_t hs = g.phbase[j], hn = g.hcnt[j], hd = g.hbase[j];
-    if (n > g.pbase[j + 1] - s || hn > g.phbase[j + 1] - hs) {  // uniform
-      if (threadIdx.x == 0) atomicOr(g.bad, 1u);
+    if (n > g.pbase[j + 1] - s || hn > g.phbase[j + 1] - hs) {  // uniform over the wave
+      if (lane == 0) atomicOr(g.bad, 1u);
       continue;
     }
-    for (uint64_t i = threadIdx.x; i < n; i += 256)
+    for (uint64_t i = lane; i < n; i += 64)
       if (d + i < g.capacity) {
         rk[d + i] = srk[s + i];
         g.rca[d + i] = g.srca[s + i];
         g.rcb[d + i] = g.srcb[s + i];
       }
-    for (uint32_t i = threadIdx.x; i < hn; i += 256)
+    for (uint32_t i = lane; i < hn; i += 64)
       if ((uint64_t)hd + i < g.heavy_cap) g.heavy[hd + i] = g.sheavy[hs + i];
   }
 }
@@ -3308,7 +3324,8 @@ hipError_t launch_rle_scan(const LaunchRleScan &p, void *status, hipStream_t st)
   if (e == hipSuccess) e = launch_scan(p.in32, p.out32, p.n, 4, status, st);
   if (e == hipSuccess && p.nzero) e = launch_fill_u32(p.zero, 0u, p.nzero, st);
   if (e == hipSuccess && p.add) {
-    hipLaunchKernelGGL(k_sum_add, dim3(1), dim3(1024), 0, st, p.add, p.n, p.acc);
+    hipLaunchKernelGGL(k_sum_add, dim3((uint32_t)std::min<uint64_t>((p.n + 8191) / 8192, 256)), dim3(1024), 0, st, p.add,
+                       p.n, p.acc);
     e = hipGetLastError();
   }
   return e;
@@ -3330,7 +3347,7 @@ hipError_t launch_rle_caps(const void *offA, const void *offB, int off_bytes, ui
 
 hipError_t launch_rle_gather(const LaunchRleGather &g, hipStream_t st) {
   if (!g.nch) return hipSuccess;
-  const uint32_t grid = std::min<uint32_t>(g.nch, 8192);
+  const uint32_t grid = std::min<uint32_t>((g.nch + 3) / 4, 8192);
   if (g.key_bytes == 4)
     hipLaunchKernelGGL(k_rle_gather<uint32_t>, dim3(grid), dim3(256), 0, st, g);
   else
