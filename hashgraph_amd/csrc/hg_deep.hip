@@ -9,6 +9,7 @@
 // counts to the groups', so the second step needs no histogram: a tile of it
 // reserves its places in the buckets.  The buckets can then be small ones
 // (8 K keys), which the final stage and the probe take several of to a CU.
+// A hot value's bucket skips the groups: the histogram tells before any key moves.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 #include <algorithm>
@@ -23,7 +24,7 @@ constexpr int HB = 1024;        // threads of the histogram
 constexpr int SB = 512;         // threads of the scatter steps
 constexpr int SUM_COLS = 32;    // columns of a column-sum workgroup
 constexpr uint32_t XCDS = 8;
-constexpr uint32_t HOT_GRID = 768;  // three workgroups a CU
+static_assert(2 * DEEP_GROUPS <= SB, "a column a group and one for its hot bucket");
 constexpr uint32_t XROWS = DEEP_ROWS / XCDS;  // key ranges of an XCD
 static_assert(DEEP_ROWS % XCDS == 0 && DEEP_ROWS % (1024 / SUM_COLS) == 0 && DEEP_GROUPS <= SB, "two-step geometry");
 
@@ -117,52 +118,85 @@ __global__ __launch_bounds__(1024) void k_deep_sum(uint32_t *__restrict__ cmat, 
 }
 
 // Starts of the buckets (fstart, nfine + 1), each XCD's first places in the
-// groups (gstart) and the second step's chunks, group by group.  One workgroup.
+// groups and in the hot buckets (gstart, hstart) and the second step's chunks,
+// group by group.  One workgroup.
+// A group's largest bucket is hot when it has more keys than a group's share:
+// hot holds its index in the group (NO_HOT: none).  Its keys never enter the
+// group, so they are taken off the group's counts.
+constexpr uint32_t NO_HOT = 255;
+static_assert(DEEP_FINE <= (NO_HOT - 1) * (NO_HOT - 1), "a bucket's index in its group");
 __global__ __launch_bounds__(1024) void k_deep_starts(const uint32_t *__restrict__ ftot, DeepGeom g, uint32_t rows,
-                                                      const uint32_t *__restrict__ cmat, uint32_t chunk_keys,
+                                                      const uint32_t *__restrict__ cmat,
+                                                      const uint32_t *__restrict__ fmat, uint32_t chunk_keys,
                                                       uint32_t *__restrict__ fstart, uint32_t *__restrict__ gstart,
+                                                      uint32_t *__restrict__ hot, uint32_t *__restrict__ hstart,
                                                       DeepChunk *__restrict__ chunks, uint32_t *__restrict__ nchunks) {
   extern __shared__ __align__(16) uint32_t s_a[];  // nfine + 1
   __shared__ uint32_t s_tmp[1024 / 64 + 1];
+  __shared__ unsigned long long s_hot[DEEP_GROUPS];  // keys of the group's hot bucket << 32 | its index
+  __shared__ uint32_t s_nhot;
+  const uint32_t t = threadIdx.x;
+  if (t < DEEP_GROUPS) s_hot[t] = 0;
+  if (t == 0) s_nhot = 0;
   lds_fill<uint32_t, 1024, 8>(s_a, ftot, g.nfine);
   __syncthreads();
   const uint32_t tot = lds_exclusive_scan<1024>(s_a, g.nfine, s_tmp);
-  if (threadIdx.x == 0) s_a[g.nfine] = tot;
+  if (t == 0) s_a[g.nfine] = tot;
   __syncthreads();
-  for (uint32_t f = threadIdx.x; f <= g.nfine; f += 1024) fstart[f] = s_a[f];
-  const uint32_t s = threadIdx.x;
-  static_assert((DEEP_GROUPS & (DEEP_GROUPS - 1)) == 0, "the search below");
-  uint32_t a = 0, e = 0;
-  if (s < g.ngroups) {
-    a = s_a[s * g.group];
-    e = s_a[min(g.nfine, (s + 1) * g.group)];
+  const uint32_t share = (uint32_t)(g.n / g.ngroups);
+  for (uint32_t f = t; f <= g.nfine; f += 1024) {
+    const uint32_t at = s_a[f];
+    fstart[f] = at;
+    if (f < g.nfine && s_a[f + 1] - at > share)
+      atomicMax(&s_hot[f / g.group], ((unsigned long long)(s_a[f + 1] - at) << 32) | (f % g.group));
   }
-  if (s < g.ngroups)
+  __syncthreads();
+  // a wave a group: the hot bucket's keys in each XCD's eighth of the rows
+  for (uint32_t s = t / 64; s < g.ngroups; s += 1024 / 64) {
+    const uint32_t lane = t & 63, c = (uint32_t)(s_hot[s] >> 32), b = c ? (uint32_t)s_hot[s] : NO_HOT;
+    if (lane == 0) hot[s] = b;
+    if (!c) continue;
+    if (lane == 0) atomicAdd(&s_nhot, 1u);
+    const uint32_t f = s * g.group + b;
+    uint32_t before = 0;
+    for (uint32_t x = 0; x < XCDS; x += 64 / XROWS) {
+      const uint32_t r = x * XROWS + lane;
+      uint32_t v = r < rows ? fmat[(uint64_t)r * g.nfine + f] : 0u;
+      for (uint32_t d = XROWS / 2; d; d >>= 1) v += __shfl_xor(v, d, 64);
+      for (uint32_t y = 0; y < 64 / XROWS; y++) {
+        if (lane == 0) hstart[(x + y) * g.ngroups + s] = s_a[f] + before;
+        before += __shfl(v, y * XROWS, 64);
+      }
+    }
+  }
+  __syncthreads();
+  static_assert((DEEP_GROUPS & (DEEP_GROUPS - 1)) == 0 && 64 % XROWS == 0, "the search below, the sums above");
+  __shared__ uint32_t s_n[DEEP_GROUPS], s_c0[DEEP_GROUPS];  // keys of a group without its hot bucket, its first chunk
+  uint32_t nc = 0;
+  if (t < g.ngroups) {
+    const uint32_t a = s_a[t * g.group], e = s_a[min(g.nfine, (t + 1) * g.group)], c = (uint32_t)(s_hot[t] >> 32);
     for (uint32_t x = 0; x < XCDS; x++)
-      if (x * XROWS < rows) gstart[x * g.ngroups + s] = a + cmat[(uint64_t)x * XROWS * g.ngroups + s];
-  const uint32_t nc = (uint32_t)(((uint64_t)(e - a) + chunk_keys - 1) / chunk_keys);
-  // ordinary groups' chunks, then the hot ones', a thread a chunk (a hot key's
-  // group may have most of them)
-  __shared__ uint32_t s_c0[2][DEEP_GROUPS];
-  const bool hot = e - a > g.n / g.ngroups * 2;
-  uint32_t all[2];
-  const uint32_t c0 = block_exclusive_sum<1024, uint32_t>(hot ? 0u : nc, s_tmp, all[0]);
-  const uint32_t c1 = block_exclusive_sum<1024, uint32_t>(hot ? nc : 0u, s_tmp, all[1]);
-  if (s < g.ngroups) {
-    s_c0[0][s] = c0;
-    s_c0[1][s] = c1;
+      if (x * XROWS < rows)
+        gstart[x * g.ngroups + t] = a + cmat[(uint64_t)x * XROWS * g.ngroups + t] -
+                                    (c ? hstart[x * g.ngroups + t] - hstart[t] : 0u);
+    s_n[t] = e - a - c;
+    nc = (uint32_t)(((uint64_t)s_n[t] + chunk_keys - 1) / chunk_keys);
   }
-  if (s < 2) nchunks[s] = all[s];
+  uint32_t all;
+  const uint32_t c0 = block_exclusive_sum<1024, uint32_t>(nc, s_tmp, all);
+  if (t < g.ngroups) s_c0[t] = c0;
+  if (t == 0) {
+    nchunks[0] = all;
+    nchunks[1] = s_nhot;
+  }
   __syncthreads();
-  for (uint32_t i = s; i < all[0] + all[1]; i += 1024) {
-    const uint32_t h = i >= all[0], ci = h ? i - all[0] : i;
-    uint32_t q = 0;  // last group whose first chunk is at most ci (groups without chunks precede it)
+  for (uint32_t i = t; i < all; i += 1024) {  // a thread a chunk
+    uint32_t q = 0;  // last group whose first chunk is at most i (groups without chunks precede it)
     for (uint32_t step = DEEP_GROUPS / 2; step; step >>= 1)
-      if (q + step < g.ngroups && s_c0[h][q + step] <= ci) q += step;
-    const uint32_t ga = s_a[q * g.group], ge = s_a[min(g.nfine, (q + 1) * g.group)];
+      if (q + step < g.ngroups && s_c0[q + step] <= i) q += step;
     DeepChunk d;
-    d.start = ga + (ci - s_c0[h][q]) * chunk_keys;
-    d.count = min(chunk_keys, ge - d.start);
+    d.start = s_a[q * g.group] + (i - s_c0[q]) * chunk_keys;
+    d.count = min(chunk_keys, s_n[q] - (i - s_c0[q]) * chunk_keys);
     d.group = q;
     d.pad = 0;
     chunks[i] = d;
@@ -174,18 +208,26 @@ __global__ __launch_bounds__(1024) void k_deep_starts(const uint32_t *__restrict
 // group, so the tiles in flight on an XCD write next to each other: 2^28 uint32
 // keys in 515 us (747 with a contiguous key range for each workgroup; a plain
 // copy takes 410).
+// A group's hot bucket is a column of its own, whose keys go to their places in
+// out at once and so are moved once instead of twice: 2^27 uint64 keys of
+// Zipf(1.3) are built in 2.22 ms (2.60 with both steps for all of them, 2.35
+// through the wide pass), half of them one value 1.83 (2.21, 2.05); uniform keys
+// take the same 1.65.  Six waves a SIMD (80 registers): with four, 915 us of
+// 2^27 uniform uint32 keys became 951.
 // The first workgroups also write the buckets' items and clear what the items'
 // kernels need.
 template <typename K, bool PACK, int HK>
-__global__ __launch_bounds__(SB) void k_deep_first(const void *__restrict__ keys, DeepGeom g, uint32_t chunk_keys,
-                                                   uint32_t *__restrict__ gstart,
-                                                   const uint32_t *__restrict__ fstart, K *__restrict__ out,
-                                                   FinItem *__restrict__ items, BinMap *__restrict__ maps,
-                                                   unsigned long long *__restrict__ zero, uint32_t nzero,
-                                                   unsigned int *__restrict__ zero_col) {
+__global__ __launch_bounds__(SB, 6) void k_deep_first(const void *__restrict__ keys, DeepGeom g, uint32_t chunk_keys,
+                                                   const uint32_t *__restrict__ nhot, const uint32_t *__restrict__ hot,
+                                                   uint32_t *__restrict__ hstart, uint32_t *__restrict__ gstart,
+                                                   const uint32_t *__restrict__ fstart, K *__restrict__ mid,
+                                                   K *__restrict__ out, FinItem *__restrict__ items,
+                                                   BinMap *__restrict__ maps, unsigned long long *__restrict__ zero,
+                                                   uint32_t nzero, unsigned int *__restrict__ zero_col) {
   constexpr uint32_t T = scatter_tile_keys<K>(SB);
   using IN = typename std::conditional<PACK, uint32_t, K>::type;
   __shared__ ScatterLds<K, SB> s;
+  __shared__ uint8_t s_hot[DEEP_GROUPS];  // (in bytes it leaves room for three workgroups a CU)
   const uint32_t b = threadIdx.x;
   for (uint32_t f = blockIdx.x * SB + b; f < g.nfine; f += gridDim.x * SB) {
     FinItem it;
@@ -210,53 +252,49 @@ __global__ __launch_bounds__(SB) void k_deep_first(const void *__restrict__ keys
   const uint64_t k0 = x * share + (uint64_t)(blockIdx.x / XCDS) * chunk_keys;
   if (k0 >= end) return;
   const uint32_t n = (uint32_t)min((uint64_t)chunk_keys, end - k0);
+  if (*nhot == 0) {
+    for (uint32_t base = 0; base < n; base += T)
+      scatter_tile<K, SB, PACK>(keys, k0 + base, min(T, n - base), g.ngroups, s, [&](uint32_t) { return mid; },
+                                [&](IN key) { return divq(bin_of<IN, HK>(key, g.map) - g.bin_lo, g.coarse); },
+                                [&](uint32_t c) { return c ? atomicAdd(&gstart[x * g.ngroups + b], c) : 0u; });
+    return;
+  }
+  if (b < g.ngroups) s_hot[b] = (uint8_t)hot[b];
+  __syncthreads();
+  const auto column = [&](IN key) {
+    const uint32_t rel = bin_of<IN, HK>(key, g.map) - g.bin_lo, c = divq(rel, g.coarse);
+    // a bucket of index NO_HOT lies in another group (past the tile's end: key
+    // 0, whose bin may lie outside)
+    return rel - (c * g.group + s_hot[min(c, DEEP_GROUPS - 1)]) * g.fine.d < g.fine.d ? c + g.ngroups : c;
+  };
+  uint32_t *const at = (b < g.ngroups ? gstart + b : hstart + (b - g.ngroups)) + x * g.ngroups;
   for (uint32_t base = 0; base < n; base += T)
-    scatter_tile<K, SB, PACK>(keys, k0 + base, min(T, n - base), g.ngroups, s, out,
-                              [&](IN key) { return divq(bin_of<IN, HK>(key, g.map) - g.bin_lo, g.coarse); },
-                              [&](uint32_t c) { return c ? atomicAdd(&gstart[x * g.ngroups + b], c) : 0u; });
+    scatter_tile<K, SB, PACK>(keys, k0 + base, min(T, n - base), 2 * g.ngroups, s,
+                              [&](uint32_t c) { return c < g.ngroups ? mid : out; }, column,
+                              [&](uint32_t c) { return c ? atomicAdd(at, c) : 0u; });
 }
 
 // Second step: a chunk of one group into the group's buckets; every tile
-// reserves its places (fstart ends as the buckets' ends).
-template <typename K, int HK, bool HOT>
-__device__ __forceinline__ void second_chunk(const K *__restrict__ keys, const DeepGeom &g, const DeepChunk &d,
-                                             ScatterLds<K, SB> &s, uint32_t *__restrict__ fstart,
-                                             K *__restrict__ out) {
-  constexpr uint32_t T = scatter_tile_keys<K>(SB);
-  const uint32_t f0 = d.group * g.group, ncols = min(g.group, g.nfine - f0);
-  const uint32_t lo = g.bin_lo + f0 * g.fine.d;  // first bin of the group
-  for (uint32_t base = 0; base < d.count; base += T)
-    scatter_tile<K, SB, false, HOT>(keys, (uint64_t)d.start + base, min(T, d.count - base), ncols, s, out,
-                                    [&](K key) { return divq(bin_of<K, HK>(key, g.map) - lo, g.fine); },
-                                    [&](uint32_t c) { return c ? atomicAdd(&fstart[f0 + threadIdx.x], c) : 0u; });
-}
-
-// Consecutive chunks run on one XCD, so the runs of a bucket meet in its L2.
+// reserves its places (fstart ends as the buckets' ends).  Consecutive chunks
+// run on one XCD, so the runs of a bucket meet in its L2.
 template <typename K, int HK>
 __global__ __launch_bounds__(SB) void k_deep_second(const K *__restrict__ keys, DeepGeom g,
                                                     const DeepChunk *__restrict__ chunks,
                                                     const uint32_t *__restrict__ nchunks, uint32_t *__restrict__ fstart,
                                                     K *__restrict__ out) {
+  constexpr uint32_t T = scatter_tile_keys<K>(SB);
   __shared__ ScatterLds<K, SB> s;
   const uint32_t nc = nchunks[0];
   if (blockIdx.x >= nc) return;
   const uint32_t q = nc >> 3, r = nc & 7, x = blockIdx.x & 7;
-  second_chunk<K, HK, false>(keys, g, chunks[x * q + min(x, r) + (blockIdx.x >> 3)], s, fstart, out);
-}
-
-// The chunks of groups with more than twice their share of the keys: one value
-// fills most of them (a kernel of its own, since its registers would cost the
-// other one a workgroup a CU).  Builds of 2^27 uint32 keys: Zipf(1.1) 2.02 ms
-// without it, 1.88 with it, Zipf(1.3) 2.18 and 2.05; uniform keys pay a launch.
-template <typename K, int HK>
-__global__ __launch_bounds__(SB) void k_deep_hot(const K *__restrict__ keys, DeepGeom g,
-                                                 const DeepChunk *__restrict__ chunks,
-                                                 const uint32_t *__restrict__ nchunks, uint32_t *__restrict__ fstart,
-                                                 K *__restrict__ out) {
-  __shared__ ScatterLds<K, SB> s;
-  const uint32_t n0 = nchunks[0], n1 = nchunks[1];
-  for (uint32_t i = blockIdx.x; i < n1; i += gridDim.x)
-    second_chunk<K, HK, true>(keys, g, chunks[n0 + i], s, fstart, out);
+  const DeepChunk d = chunks[x * q + min(x, r) + (blockIdx.x >> 3)];
+  const uint32_t f0 = d.group * g.group, ncols = min(g.group, g.nfine - f0);
+  const uint32_t lo = g.bin_lo + f0 * g.fine.d;  // first bin of the group
+  for (uint32_t base = 0; base < d.count; base += T)
+    scatter_tile<K, SB, false>(keys, (uint64_t)d.start + base, min(T, d.count - base), ncols, s,
+                               [&](uint32_t) { return out; },
+                               [&](K key) { return divq(bin_of<K, HK>(key, g.map) - lo, g.fine); },
+                               [&](uint32_t c) { return c ? atomicAdd(&fstart[f0 + threadIdx.x], c) : 0u; });
 }
 
 namespace {
@@ -286,18 +324,18 @@ hipError_t launch_deep_t(const LaunchDeep &p, bool scatter, hipStream_t st) {
     hipLaunchKernelGGL(k_deep_sum, dim3((g.nfine + SUM_COLS - 1) / SUM_COLS + (g.ngroups + SUM_COLS - 1) / SUM_COLS),
                        dim3(1024), 0, st, p.cmat, p.rows, g.ngroups, p.fmat, g.nfine, p.ftot);
     hipLaunchKernelGGL(k_deep_starts, dim3(1), dim3(1024), ((size_t)g.nfine + 1) * 4, st, (const uint32_t *)p.ftot, g,
-                       p.rows, (const uint32_t *)p.cmat, chunk, p.fstart, p.gstart, p.chunks, p.nchunks);
+                       p.rows, (const uint32_t *)p.cmat, (const uint32_t *)p.fmat, chunk, p.fstart, p.gstart, p.hot,
+                       p.hstart, p.chunks, p.nchunks);
     return hipGetLastError();
   }
+  const uint64_t share = std::min<uint64_t>((uint64_t)XROWS * g.per, g.n);
   auto first = &k_deep_first<K, false, HK>;
   if constexpr (sizeof(K) == 8 && HK == HK_MURMUR)
     if (p.pack) first = &k_deep_first<K, true, HK>;
-  const uint64_t share = std::min<uint64_t>((uint64_t)XROWS * g.per, g.n);
   hipLaunchKernelGGL(first, dim3((uint32_t)((share + chunk - 1) / chunk) * XCDS), dim3(SB), 0, st, p.keys, g, chunk,
-                     p.gstart, (const uint32_t *)p.fstart, (K *)p.mid, p.items, p.maps, p.zero, p.nzero, p.zero_col);
+                     (const uint32_t *)(p.nchunks + 1), (const uint32_t *)p.hot, p.hstart, p.gstart,
+                     (const uint32_t *)p.fstart, (K *)p.mid, (K *)p.out, p.items, p.maps, p.zero, p.nzero, p.zero_col);
   hipLaunchKernelGGL((k_deep_second<K, HK>), dim3(deep_max_chunks(g, p.key_bytes)), dim3(SB), 0, st, (const K *)p.mid, g,
-                     (const DeepChunk *)p.chunks, (const uint32_t *)p.nchunks, p.fstart, (K *)p.out);
-  hipLaunchKernelGGL((k_deep_hot<K, HK>), dim3(HOT_GRID), dim3(SB), 0, st, (const K *)p.mid, g,
                      (const DeepChunk *)p.chunks, (const uint32_t *)p.nchunks, p.fstart, (K *)p.out);
   return hipGetLastError();
 }

@@ -879,13 +879,15 @@ DeepGeom deep_geom(const BinMap &map, uint64_t n, uint64_t lo, uint64_t R, uint3
 // Arena 1 of a two-step partition; extra bytes of the caller's behind it.
 struct DeepPlan {
   Plan P;
-  size_t cmat, fmat, ftot, fstart, gstart, chunks, nch, items, maps, rest;
+  size_t cmat, fmat, ftot, fstart, gstart, hot, hstart, chunks, nch, items, maps, rest;
   DeepPlan(const DeepGeom &g, int kb, size_t extra) {
     cmat = P.add((size_t)DEEP_ROWS * g.ngroups * 4);
     fmat = P.add((size_t)DEEP_ROWS * g.nfine * 4);
     ftot = P.add(g.nfine * 4);
     fstart = P.add(((size_t)g.nfine + 1) * 4);
     gstart = P.add((size_t)8 * g.ngroups * 4);
+    hot = P.add((size_t)g.ngroups * 4);
+    hstart = P.add((size_t)8 * g.ngroups * 4);
     chunks = P.add((size_t)deep_max_chunks(g, kb) * sizeof(DeepChunk));
     nch = P.add(8);
     items = P.add((size_t)g.nfine * sizeof(FinItem));
@@ -910,6 +912,8 @@ hg_status deep_launch(hg_ctx c, const DeepGeom &g, int kb, size_t extra, LaunchD
   p.ftot = cv.get<uint32_t>(q.ftot);
   p.fstart = cv.get<uint32_t>(q.fstart);
   p.gstart = cv.get<uint32_t>(q.gstart);
+  p.hot = cv.get<uint32_t>(q.hot);
+  p.hstart = cv.get<uint32_t>(q.hstart);
   p.chunks = cv.get<DeepChunk>(q.chunks);
   p.nchunks = cv.get<uint32_t>(q.nch);
   p.items = cv.get<FinItem>(q.items);

@@ -371,7 +371,7 @@ __global__ __launch_bounds__(FEW_COLS) void k_part_scatter_few(const K *__restri
   const uint32_t ncols = sd.ncols, b = threadIdx.x;
   uint32_t next = b < ncols ? cpos[sd.row_base + (uint64_t)(tile - sd.tile_begin) * ncols + b] : 0u;
   for (uint32_t base = 0; base < td.count; base += T)
-    scatter_tile<K, FEW_COLS, PACK>(keys, td.key_start + base, min(T, td.count - base), ncols, s, out,
+    scatter_tile<K, FEW_COLS, PACK>(keys, td.key_start + base, min(T, td.count - base), ncols, s, [&](uint32_t) { return out; },
                                     [&](IN key) { return bucket_of<IN, HK, SK_RANGE>(key, sd, nullptr); },
                                     [&](uint32_t c) {
                                       const uint32_t at = next;

@@ -152,7 +152,8 @@ struct LaunchNarrow {
 
 // Two-step partition: keys whose bins lie in [bin_lo, bin_lo + nbins) into
 // nfine buckets of fine.d bins, by way of ngroups groups of `group` buckets;
-// key range r of per keys is counted in row r.
+// key range r of per keys is counted in row r.  A group's largest bucket, when
+// it has more keys than a group's share of them, is hot: its keys skip the groups.
 constexpr uint32_t DEEP_ROWS = 256;     // a histogram workgroup on every CU
 constexpr uint32_t DEEP_GROUPS = 256;
 constexpr uint32_t DEEP_FINE = 39424;   // a counter each in the histogram's LDS
@@ -175,8 +176,9 @@ struct LaunchDeep {
   uint32_t *cmat, *fmat;       // DEEP_ROWS * ngroups, DEEP_ROWS * nfine
   uint32_t *ftot, *fstart;     // nfine, nfine + 1
   uint32_t *gstart;            // 8 * ngroups
+  uint32_t *hot, *hstart;      // ngroups, 8 * ngroups
   DeepChunk *chunks;           // deep_max_chunks
-  uint32_t *nchunks;           // two
+  uint32_t *nchunks;           // two: chunks, hot buckets
   FinItem *items;              // nfine
   BinMap *maps;                // one
   unsigned long long *zero;    // as in LaunchNarrow

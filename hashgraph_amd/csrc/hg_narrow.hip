@@ -116,7 +116,7 @@ __global__ __launch_bounds__(NB) void k_narrow_scatter(const void *__restrict__ 
   const uint64_t k0 = (uint64_t)blockIdx.x * g.per;
   const uint32_t n = (uint32_t)min((uint64_t)g.per, g.n - k0);
   for (uint32_t base = 0; base < n; base += T)
-    scatter_tile<K, NB, PACK>(keys, k0 + base, min(T, n - base), g.ncols, s, out,
+    scatter_tile<K, NB, PACK>(keys, k0 + base, min(T, n - base), g.ncols, s, [&](uint32_t) { return out; },
                               [&](IN key) { return divq(bin_of<IN, HK>(key, g.map) - g.bin_lo, g.div); },
                               [&](uint32_t c) {
                                 const uint32_t at = next;

@@ -28,12 +28,11 @@ struct ScatterLds {
 // take(c) gives thread b the place of bucket b's run of c keys (called by
 // threads b < ncols, its result used only after the staging, so that a
 // global reservation's latency is hidden).
+// dst(b) is the array that bucket b's places count in.
 // PACK: the keys are 32-bit and the output 8-byte records (position << 32 | key).
-// HOT: most keys share a bucket; a wave counts the keys of its first lane's
-// bucket with one LDS atomic (64 to one address take their turns).
-template <typename K, int BLOCK, bool PACK, bool HOT = false, typename BUCKET, typename TAKE>
+template <typename K, int BLOCK, bool PACK, typename DST, typename BUCKET, typename TAKE>
 __device__ __forceinline__ void scatter_tile(const void *__restrict__ keys, uint64_t k0, uint32_t cnt, uint32_t ncols,
-                                             ScatterLds<K, BLOCK> &s, K *__restrict__ out, BUCKET bucket, TAKE take) {
+                                             ScatterLds<K, BLOCK> &s, DST dst, BUCKET bucket, TAKE take) {
   constexpr int KPT = scatter_tile_keys<K>(BLOCK) / BLOCK;
   using IN = typename std::conditional<PACK, uint32_t, K>::type;
   const uint32_t b = threadIdx.x;
@@ -51,18 +50,7 @@ __device__ __forceinline__ void scatter_tile(const void *__restrict__ keys, uint
 #pragma unroll
   for (int j = 0; j < KPT; j++) {
     const bool valid = j * BLOCK + threadIdx.x < cnt;
-    if constexpr (HOT) {
-      const uint32_t lane = threadIdx.x & 63;
-      const bool in = valid && pk[j] == __builtin_amdgcn_readfirstlane(pk[j]);  // lane 0 too, if any lane is valid
-      const unsigned long long m = __ballot(in);
-      uint32_t r = 0;
-      if (valid && (lane == 0 || !in)) r = atomicAdd(&s.cnt[pk[j]], lane == 0 ? (uint32_t)__popcll(m) : 1u);
-      const uint32_t r0 = __builtin_amdgcn_readfirstlane(r);
-      if (in) r = r0 + (uint32_t)__popcll(m & ((1ull << lane) - 1));
-      if (valid) pk[j] = (pk[j] << 16) | r;
-    } else if (valid) {
-      pk[j] = (pk[j] << 16) | atomicAdd(&s.cnt[pk[j]], 1u);
-    }
+    if (valid) pk[j] = (pk[j] << 16) | atomicAdd(&s.cnt[pk[j]], 1u);
   }
   __syncthreads();
   const uint32_t c = col ? s.cnt[b] : 0u;
@@ -87,7 +75,10 @@ __device__ __forceinline__ void scatter_tile(const void *__restrict__ keys, uint
 #pragma unroll
   for (int j = 0; j < KPT; j++) {
     const uint32_t q = j * BLOCK + threadIdx.x;
-    if (q < cnt) out[s.adj[s.bkt[q]] + q] = s.key[q];
+    if (q < cnt) {
+      const uint32_t c = s.bkt[q];
+      dst(c)[s.adj[c] + q] = s.key[q];
+    }
   }
   __syncthreads();
 }

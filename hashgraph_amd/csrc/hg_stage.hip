@@ -85,7 +85,7 @@ __global__ __launch_bounds__(PB) void k_stage_scatter(LaunchStagePart p, uint32_
   uint32_t next = b <= ns ? start + p.cmat[(uint64_t)blockIdx.x * (ns + 1) + b] : 0u;
   const uint32_t k0 = blockIdx.x * per, n = min(per, p.n - k0);
   for (uint32_t base = 0; base < n; base += T)
-    scatter_tile<K, PB, false>(p.keys, k0 + base, min(T, n - base), ns + 1, s, (K *)p.out,
+    scatter_tile<K, PB, false>(p.keys, k0 + base, min(T, n - base), ns + 1, s, [&](uint32_t) { return (K *)p.out; },
                                [&](K key) { return slab_of(bin_of<K, HK>(key, p.map), s_bound, ns); },
                                [&](uint32_t c) {
                                  const uint32_t at = next;
