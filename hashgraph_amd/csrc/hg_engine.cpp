@@ -684,17 +684,24 @@ hg_status finish_two_level(hg_ctx c, const std::vector<Coarse> &cs, const BinMap
 // NARROW_COLS buckets (W bins each).  Returns the class, -1 when none does
 // (from about 14.7 M keys on at one key a bin, or more bins than the buckets
 // can count): the wide pass then.  Narrow against wide, uint32 keys: 28
-// against 91 us at 2^16, 35 against 78 us at 2^20, 51 against 92 us at 2^22,
+// against 91 us at 2^16, 35 against 78 us at 2^20, 49 against 92 us at 2^22,
 // 124 against 153 us at 14 M.
 int narrow_class(uint64_t n, uint64_t R, uint32_t &W) {
   for (int cls = 0; cls < FINAL_CLASSES; cls++) {
-    const double w = std::floor(0.875 * final_class_keys(cls) * (double)R / (double)n);
+    const double fit = final_class_keys(cls) * (double)R / (double)n;  // bins whose mean keys fill a bucket
+    const uint32_t least = (uint32_t)((R + NARROW_COLS - 1) / NARROW_COLS);
+    const double w = std::floor(0.875 * fit);
     if (w < 1) continue;
     W = (uint32_t)std::min(w, 65535.0);
     // sparse tables: more buckets of fewer bins, since a bucket's time then
     // goes to its bins (10^5 keys over 10^6 bins: 32 us, 56 with the class's full width)
-    W = std::min<uint32_t>(W, std::max<uint32_t>(2 * final_class_keys(cls), (uint32_t)((R + NARROW_COLS - 1) / NARROW_COLS)));
-    if ((R + W - 1) / W <= NARROW_COLS) return cls;
+    W = std::min<uint32_t>(W, std::max<uint32_t>(2 * final_class_keys(cls), least));
+    if ((R + W - 1) / W > NARROW_COLS) continue;
+    // columns to spare leave the buckets room for duplicates, which spread wide
+    // (4 M uint64 keys, 64 copies each: 124 us full to 7/8, 75 half full; 79
+    // and 75 without copies)
+    W = std::min(W, std::max(least, (uint32_t)std::max(1.0, std::min(0.5 * fit, 65535.0))));
+    return cls;
   }
   return -1;
 }

@@ -127,3 +127,26 @@ def test_hot_slabs_of_a_staged_build(dev):
     off, csr = off.to(dev), csr.to(dev)
     _check_table(off, csr, keys, _bins(keys, M), M)
     assert torch.equal(_bins(csr, M), torch.repeat_interleave(torch.arange(M, device=dev), off.diff().to(torch.int64)))
+
+
+@pytest.mark.parametrize("kb,ob", [(4, 4), (8, 8)])
+@pytest.mark.parametrize("copies", [1, 64, 300])
+@pytest.mark.parametrize("n,M", [(40000, 40000), (1 << 18, 1 << 18), (3 << 20, 3 << 20), (4194305, 1 << 22),
+                                 (14600000, 14600000), (1 << 20, 1 << 25), (1 << 21, 1 << 13)])
+def test_narrow_builds_of_copies(n, M, copies, kb, ob, dev):
+    """The narrow pass's widths, from the fewest buckets of a class to all of
+    its columns; copies of the keys fill the buckets unevenly."""
+    import torch
+    import hashgraph_amd as hg
+    print(f"narrow n={n} M={M} copies={copies} kb={kb} ob={ob}", flush=True)
+    keys = wl.uniform_keys(29, n, kb, device=dev)
+    if copies > 1:
+        keys = keys % (n // copies)
+    bins = _bins(keys, M)
+    off, csr = hg.build(keys, M, offset_bytes=ob)
+    _check_table(off, csr, keys, bins, M)
+    order = torch.repeat_interleave(torch.arange(M, device=dev), off.diff().to(torch.int64))
+    assert torch.equal(_bins(csr, M), order)
+    off2, ck, ind = hg.build_indexed(keys, M, offset_bytes=ob)
+    assert torch.equal(off2, off) and torch.equal(torch.sort(ind).values, torch.arange(n, device=dev))
+    assert torch.equal(ck, keys[ind]) and torch.equal(bins[ind], order)
