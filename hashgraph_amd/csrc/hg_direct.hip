@@ -201,13 +201,12 @@ hipError_t direct_lds() {
 
 }  // namespace
 
-bool build_one_takes(uint64_t n, uint64_t nbins, int key_bytes) {
-  (void)key_bytes;
+bool build_one_takes(uint64_t n, uint64_t nbins) {
   return n && n <= BUILD_ONE_KEYS && nbins <= 65535;
 }
 
 hipError_t launch_build_one(const LaunchBuildOne &b, hipStream_t st) {
-  if (!build_one_takes(b.n, b.nbins, b.key_bytes) || b.map.kind > 1) return hipErrorInvalidValue;
+  if (!build_one_takes(b.n, b.nbins) || b.map.kind > 1) return hipErrorInvalidValue;
   if (b.key_bytes == 4)
     return b.off_bytes == 4 ? launch_one_hk<uint32_t, uint32_t>(b, st) : launch_one_hk<uint32_t, uint64_t>(b, st);
   return b.off_bytes == 4 ? launch_one_hk<uint64_t, uint32_t>(b, st) : launch_one_hk<uint64_t, uint64_t>(b, st);

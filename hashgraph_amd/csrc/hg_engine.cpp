@@ -1003,7 +1003,7 @@ hg_status build_range(hg_ctx c, const BinMap &map, int kb, int ob, uint64_t n, u
                       bool pack_in = false) {
   if (n == 0) return fill_offsets(c, d_off, ob, R + 1, 0);
   const bool wide = wide_only();
-  if (!wide && !pack_in && !d_csr_index && build_one_takes(n, R, kb)) {
+  if (!wide && !pack_in && !d_csr_index && build_one_takes(n, R)) {
     LaunchBuildOne b{};
     b.key_bytes = kb;
     b.off_bytes = ob;
@@ -1520,7 +1520,7 @@ static void need_build(const hg_table_desc *d, ScratchNeed &need) {
   uint32_t W;
   size_t o_cnt;
   const bool wide = wide_only();
-  if (!wide && build_one_takes(n, R, kb)) return;
+  if (!wide && build_one_takes(n, R)) return;
   if (!wide && narrow_class(n, R, W) >= 0) {
     const LaunchNarrow p = narrow_launch(map, kb, n, 0, R, W);
     return need.add(n * kb, NarrowPlan(p.rows, p.geom.ncols, final_rest(R, o_cnt)).P.total());

@@ -1464,10 +1464,10 @@ __device__ __forceinline__ void vt_add_existing(const K *s_key, C *s_cnt, K v, u
 // ---------------------------------------------------------------------------
 // Value table of the probe's and the join's long bins: HT_SLOTS values of A
 // with u32 copy counts in LDS; keys equal to the all-ones sentinel are
-// counted apart.  A bin of A is folded in rounds: before each chunk of BLOCK
-// keys a table more than half full is answered (the probe keys look their
-// values up) and cleared, so a chunk's inserts (at most BLOCK new values)
-// always find a free slot.  Copies of one value folded in different rounds
+// counted apart.  A bin of A is folded in rounds: before each step of up to
+// HT_SLOTS / 2 keys a table more than half full is answered (the probe keys
+// look their values up) and cleared, so a step's inserts always find a free
+// slot.  A step may leave the table full, so a lookup ends after HT_SLOTS slots.  Copies of one value folded in different rounds
 // are answered in each round; their counts and emitted copies add up, so the
 // result equals one answer over the whole bin.
 // ---------------------------------------------------------------------------
@@ -1549,11 +1549,11 @@ __device__ void vt_answer(const K *s_key, const uint32_t *s_cnt, uint32_t ecnt, 
 }
 
 // Folds the sequence key_at(0..n) into the table.  The keys are loaded
-// FOLD_U * BLOCK at a time (all loads in flight together) and inserted
-// BLOCK at a time; before each insert step a table more than half full is
-// answered and cleared, so a step's inserts (at most BLOCK new values) always
-// find a free slot.  Must start after a barrier; ends with one.  pending:
-// values folded since the last answer.
+// FOLD_U * BLOCK at a time (all loads in flight together) and inserted in one
+// step where that many fit half the table (512 threads), else BLOCK at a time;
+// before each step a table more than half full is answered and cleared.  Must
+// start after a barrier; ends with one.  pending: values folded since the last
+// answer.
 constexpr int FOLD_U = 4;
 template <typename K, int BLOCK, typename AT, typename ANSWER>
 __device__ __forceinline__ void vt_fold_seq(uint64_t n, AT &&key_at, K *s_key, uint32_t *s_cnt, uint32_t *s_fill,
@@ -2840,6 +2840,10 @@ __global__ __launch_bounds__(BLOCK) void k_join_heavy(const OFF *__restrict__ of
 template <int V> using IC = std::integral_constant<int, V>;
 
 // Calls f(IC<hash kind>) for the specialisation of hash kind hk.
+// Mixed hash kinds (HK_ANY) occur in batches only, whose offsets are 4 bytes
+// and whose buckets are of class 1 or the largest: the final stage and the
+// one-pass probe have no other instances of it.
+template <typename OFF, int HK> constexpr bool mixed_off = HK != HK_ANY || sizeof(OFF) == 4;
 template <typename F> static hipError_t dispatch_hk(int hk, F &&f) {
   if (hk == HK_MURMUR) return f(IC<HK_MURMUR>{});
   if (hk == HK_RMI) return f(IC<HK_RMI>{});
@@ -2949,21 +2953,27 @@ static hipError_t launch_final_t(const LaunchFinal &lf, hipStream_t st) {
     constexpr int H = decltype(h)::value;
     // the split store exists for murmur3 tables only (launch_final checks)
     constexpr bool S = SPLIT && H == HK_MURMUR;
+    hipError_t r = hipErrorInvalidValue;
     auto go = [&](auto kern, uint32_t block) {
       hipLaunchKernelGGL(kern, dim3(lf.nitems), dim3(block), lf.lds_bytes, st, (const K *)lf.part, (K *)lf.csr,
                          (OFF *)lf.off, lf.items, lf.maps, lf.lds_bytes, ctl, lf.big_slot, lf.big_cnt, lf.big_cap,
                          lf.csr_index, lf.many);
-      return hipGetLastError();
+      r = hipGetLastError();
     };
-    if (lf.cls == FINAL_CLASSES - 1) return go(&k_final<K, OFF, 1024, KPT, H, S>, 1024);
-    hipError_t r = lf.cls == 0   ? go(&k_final<K, OFF, 256, 16, H, S>, 256)
-                   : lf.cls == 1 ? go(&k_final<K, OFF, 512, 16, H, S>, 512)
-                                 : go(&k_final<K, OFF, 1024, 16, H, S>, 1024);
-    if (r != hipSuccess || !lf.many) return r;
-    const uint32_t lds = std::max(lf.lds_bytes, 128u * 1024);
-    hipLaunchKernelGGL((k_final_mid<K, OFF, 1024, KPT, H, S>), dim3(256), dim3(1024), lds, st, (const K *)lf.part,
-                       (K *)lf.csr, (OFF *)lf.off, lf.items, lf.maps, lds, (const BigCtl *)ctl, lf.csr_index);
-    return hipGetLastError();
+    if constexpr (mixed_off<OFF, H>) {
+      if (lf.cls == FINAL_CLASSES - 1) go(&k_final<K, OFF, 1024, KPT, H, S>, 1024);
+      if (lf.cls == 1) go(&k_final<K, OFF, 512, 16, H, S>, 512);
+      if constexpr (H != HK_ANY) {
+        if (lf.cls == 0) go(&k_final<K, OFF, 256, 16, H, S>, 256);
+        if (lf.cls == 2) go(&k_final<K, OFF, 1024, 16, H, S>, 1024);
+      }
+      if (r != hipSuccess || !lf.many || lf.cls == FINAL_CLASSES - 1) return r;
+      const uint32_t lds = std::max(lf.lds_bytes, 128u * 1024);
+      hipLaunchKernelGGL((k_final_mid<K, OFF, 1024, KPT, H, S>), dim3(256), dim3(1024), lds, st, (const K *)lf.part,
+                         (K *)lf.csr, (OFF *)lf.off, lf.items, lf.maps, lds, (const BigCtl *)ctl, lf.csr_index);
+      r = hipGetLastError();
+    }
+    return r;
   });
   if (e != hipSuccess) return e;
   // three kernels that return at once when no item was oversized: two
@@ -3013,17 +3023,25 @@ static hipError_t launch_probe_one_t(const LaunchProbe &p, hipStream_t st) {
   constexpr int KPT = sizeof(K) == 4 ? KPT_U32 : 32;
   return dispatch_hk(p.hk, [&](auto h) {
     constexpr int H = decltype(h)::value;
+    hipError_t r = hipErrorInvalidValue;
     auto go = [&](auto kern, uint32_t block) {
       hipLaunchKernelGGL(kern, dim3(p.nitems), dim3(block), (size_t)p.one_lds, st, (const K *)p.bpart, p.items, p.maps,
                          (const OFF *)p.offA, (const K *)p.keysA, (K *)p.out, p.capacity, p.cursor, p.one_lds, p.hmark,
                          p.gate, p.out_off, std::min(1024u * KPT, 65535u), (BigCtl *)p.big_ctl, p.big_slot);
-      return hipGetLastError();
+      r = hipGetLastError();
     };
-    if (p.one_keys == 4096) return go(&k_probe1<K, OFF, 256, 16, H>, 256);
-    if (p.one_keys == 8192) return go(&k_probe1<K, OFF, 512, 16, H>, 512);
-    if (p.one_keys == 16384) return go(&k_probe1<K, OFF, 1024, 16, H>, 1024);
-    if (p.one_keys != probe_one_keys((int)sizeof(K))) return hipErrorInvalidValue;
-    return go(&k_probe1<K, OFF, 1024, probe1_kpt<K>(), H>, 1024);
+    if constexpr (mixed_off<OFF, H>) {
+      if (p.one_keys == probe_one_keys((int)sizeof(K))) {
+        go(&k_probe1<K, OFF, 1024, probe1_kpt<K>(), H>, 1024);
+        return r;
+      }
+      if (p.one_keys == 8192) go(&k_probe1<K, OFF, 512, 16, H>, 512);
+      if constexpr (H != HK_ANY) {
+        if (p.one_keys == 4096) go(&k_probe1<K, OFF, 256, 16, H>, 256);
+        if (p.one_keys == 16384) go(&k_probe1<K, OFF, 1024, 16, H>, 1024);
+      }
+    }
+    return r;
   });
 }
 
@@ -3034,10 +3052,15 @@ static hipError_t launch_probe_rest_t(const LaunchProbe &p, hipStream_t st) {
   if (p.akey_cap < PROBE_BIN_LIMIT) return hipErrorInvalidValue;  // a walkable bin must fit in LDS
   const size_t lds = ((SUB + 2) * sizeof(OFF) + 15) / 16 * 16 + (size_t)p.akey_cap * sizeof(K);
   const hipError_t e = dispatch_hk(p.hk, [&](auto h) {
-    hipLaunchKernelGGL((k_probe<K, OFF, 1024, KPT, SUB, decltype(h)::value>), dim3(p.nitems), dim3(1024), lds, st,
-                       (const K *)p.bpart, p.items, p.maps, (const OFF *)p.offA, (const K *)p.keysA, (K *)p.out,
-                       p.capacity, p.cursor, p.akey_cap, p.hmark, p.one_keys, p.one_lds, p.gate, p.out_off);
-    return hipGetLastError();
+    constexpr int H = decltype(h)::value;
+    if constexpr (mixed_off<OFF, H>) {
+      hipLaunchKernelGGL((k_probe<K, OFF, 1024, KPT, SUB, H>), dim3(p.nitems), dim3(1024), lds, st,
+                         (const K *)p.bpart, p.items, p.maps, (const OFF *)p.offA, (const K *)p.keysA, (K *)p.out,
+                         p.capacity, p.cursor, p.akey_cap, p.hmark, p.one_keys, p.one_lds, p.gate, p.out_off);
+      return hipGetLastError();
+    } else {
+      return hipErrorInvalidValue;
+    }
   });
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL((k_probe_big<K, OFF, 1024>), dim3(PROBE_BIG_GRID), dim3(1024), 0, st, (const K *)p.bpart,
@@ -3481,18 +3504,32 @@ static hipError_t join_set_lds() {
 
 template <typename K, typename OFF, int H, bool S>
 static hipError_t set_final_classes() {
-  hipError_t r = set_lds(&k_final<K, OFF, 256, 16, H, S>);
+  hipError_t r = set_lds(&k_final<K, OFF, 1024, sizeof(K) == 4 ? KPT_U32 : 32, H, S>);
   if (r == hipSuccess) r = set_lds(&k_final<K, OFF, 512, 16, H, S>);
-  if (r == hipSuccess) r = set_lds(&k_final<K, OFF, 1024, 16, H, S>);
-  if (r == hipSuccess) r = set_lds(&k_final_mid<K, OFF, 1024, 32, H, S>);
+  if (r == hipSuccess) r = set_lds(&k_final_mid<K, OFF, 1024, sizeof(K) == 4 ? KPT_U32 : 32, H, S>);
+  if constexpr (H != HK_ANY) {
+    if (r == hipSuccess) r = set_lds(&k_final<K, OFF, 256, 16, H, S>);
+    if (r == hipSuccess) r = set_lds(&k_final<K, OFF, 1024, 16, H, S>);
+  }
   return r;
 }
 
+// The final stage's and the probe's kernels of one hash kind.
 template <typename K, typename OFF, int H>
-static hipError_t set_probe_classes() {
-  hipError_t r = set_lds(&k_probe1<K, OFF, 256, 16, H>);
-  if (r == hipSuccess) r = set_lds(&k_probe1<K, OFF, 512, 16, H>);
-  if (r == hipSuccess) r = set_lds(&k_probe1<K, OFF, 1024, 16, H>);
+static hipError_t set_bucket_kernels() {
+  hipError_t r = hipSuccess;
+  if constexpr (mixed_off<OFF, H>) {
+    r = set_final_classes<K, OFF, H, false>();
+    if (r == hipSuccess) r = set_lds(&k_probe<K, OFF, 1024, sizeof(K) == 4 ? KPT_U32 : 32, probe_sub<OFF>(), H>);
+    if constexpr (sizeof(K) == 8 && H == HK_MURMUR)
+      if (r == hipSuccess) r = set_final_classes<K, OFF, H, true>();
+    if (r == hipSuccess) r = set_lds(&k_probe1<K, OFF, 1024, probe1_kpt<K>(), H>);
+    if (r == hipSuccess) r = set_lds(&k_probe1<K, OFF, 512, 16, H>);
+    if constexpr (H != HK_ANY) {
+      if (r == hipSuccess) r = set_lds(&k_probe1<K, OFF, 256, 16, H>);
+      if (r == hipSuccess) r = set_lds(&k_probe1<K, OFF, 1024, 16, H>);
+    }
+  }
   return r;
 }
 
@@ -3517,32 +3554,10 @@ hipError_t set_kernel_attributes() {
   for (int hk = 0; hk < 3; hk++)
     HG_SET_D(dispatch_hk(hk, [&](auto h) {
       constexpr int H = decltype(h)::value;
-      hipError_t r = set_lds(&k_final<uint32_t, uint32_t, 1024, KPT_U32, H>);
-      if (r == hipSuccess) r = set_lds(&k_final<uint32_t, uint64_t, 1024, KPT_U32, H>);
-      if (r == hipSuccess) r = set_lds(&k_final<uint64_t, uint32_t, 1024, 32, H>);
-      if (r == hipSuccess) r = set_lds(&k_final<uint64_t, uint64_t, 1024, 32, H>);
-      if constexpr (H == HK_MURMUR) {
-        if (r == hipSuccess) r = set_lds(&k_final<uint64_t, uint32_t, 1024, 32, H, true>);
-        if (r == hipSuccess) r = set_lds(&k_final<uint64_t, uint64_t, 1024, 32, H, true>);
-        if (r == hipSuccess) r = set_final_classes<uint64_t, uint32_t, H, true>();
-        if (r == hipSuccess) r = set_final_classes<uint64_t, uint64_t, H, true>();
-      }
-      if (r == hipSuccess) r = set_final_classes<uint32_t, uint32_t, H, false>();
-      if (r == hipSuccess) r = set_final_classes<uint32_t, uint64_t, H, false>();
-      if (r == hipSuccess) r = set_final_classes<uint64_t, uint32_t, H, false>();
-      if (r == hipSuccess) r = set_final_classes<uint64_t, uint64_t, H, false>();
-      if (r == hipSuccess) r = set_lds(&k_probe1<uint32_t, uint32_t, 1024, probe1_kpt<uint32_t>(), H>);
-      if (r == hipSuccess) r = set_lds(&k_probe1<uint32_t, uint64_t, 1024, probe1_kpt<uint32_t>(), H>);
-      if (r == hipSuccess) r = set_lds(&k_probe1<uint64_t, uint32_t, 1024, probe1_kpt<uint64_t>(), H>);
-      if (r == hipSuccess) r = set_lds(&k_probe1<uint64_t, uint64_t, 1024, probe1_kpt<uint64_t>(), H>);
-      if (r == hipSuccess) r = set_probe_classes<uint32_t, uint32_t, H>();
-      if (r == hipSuccess) r = set_probe_classes<uint32_t, uint64_t, H>();
-      if (r == hipSuccess) r = set_probe_classes<uint64_t, uint32_t, H>();
-      if (r == hipSuccess) r = set_probe_classes<uint64_t, uint64_t, H>();
-      if (r == hipSuccess) r = set_lds(&k_probe<uint32_t, uint32_t, 1024, KPT_U32, probe_sub<uint32_t>(), H>);
-      if (r == hipSuccess) r = set_lds(&k_probe<uint32_t, uint64_t, 1024, KPT_U32, probe_sub<uint64_t>(), H>);
-      if (r == hipSuccess) r = set_lds(&k_probe<uint64_t, uint32_t, 1024, 32, probe_sub<uint32_t>(), H>);
-      if (r == hipSuccess) r = set_lds(&k_probe<uint64_t, uint64_t, 1024, 32, probe_sub<uint64_t>(), H>);
+      hipError_t r = set_bucket_kernels<uint32_t, uint32_t, H>();
+      if (r == hipSuccess) r = set_bucket_kernels<uint32_t, uint64_t, H>();
+      if (r == hipSuccess) r = set_bucket_kernels<uint64_t, uint32_t, H>();
+      if (r == hipSuccess) r = set_bucket_kernels<uint64_t, uint64_t, H>();
       return r;
     }));
   HG_SET_D(join_set_lds<JOIN_COUNT>());

@@ -405,7 +405,7 @@ hipError_t set_direct_kernel_attributes();
 // Keys up to which a table is built by one workgroup (16-bit counters: at
 // most 65535 bins): 14 us at 16384 uint32 keys against 87 us partitioned.
 constexpr uint32_t BUILD_ONE_KEYS = 16384;
-bool build_one_takes(uint64_t n, uint64_t nbins, int key_bytes);
+bool build_one_takes(uint64_t n, uint64_t nbins);
 hipError_t launch_build_one(const LaunchBuildOne &b, hipStream_t st);
 hipError_t launch_probe_direct(const LaunchProbeDirect &p, hipStream_t st);
 // maps[t].kind and each segment's map kind from use[] (learned when set)
