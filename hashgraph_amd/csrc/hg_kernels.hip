@@ -2788,15 +2788,24 @@ __global__ __launch_bounds__(BLOCK, BLOCK == 512 && sizeof(K) == 4 ? 6 : 4) void
       if (threadIdx.x < nh) s_hx[threadIdx.x] = lx;
       if (threadIdx.x == 0) s_hx[nh] = tot;
       __syncthreads();
-      // key i of the sequence: bin j with s_hx[j] <= i < s_hx[j + 1]
-      auto key_at = [&](uint64_t i) {
-        uint32_t lo = 0, hi = nh;  // s_hx[lo] <= i < s_hx[hi]
-        while (hi - lo > 1) {
-          const uint32_t mid = (lo + hi) >> 1;
-          if (s_hx[mid] <= i) lo = mid;
-          else hi = mid;
+      // key i of the sequence: bin j with s_hx[j] <= i < s_hx[j + 1].  A thread
+      // keeps its last bin: most of the sequence is one hot value's bin (2^25
+      // Zipf(1.1) uint64 keys, 2^24 probes: 5.25 -> 4.74 ms).
+      uint32_t j0 = 0, j1 = 0, js = 0;
+      auto key_at = [&](uint64_t q) {
+        const uint32_t i = (uint32_t)q;
+        if (i - j0 >= j1 - j0) {
+          uint32_t lo = 0, hi = nh;  // s_hx[lo] <= i < s_hx[hi]
+          while (hi - lo > 1) {
+            const uint32_t mid = (lo + hi) >> 1;
+            if (s_hx[mid] <= i) lo = mid;
+            else hi = mid;
+          }
+          j0 = s_hx[lo];
+          j1 = s_hx[lo + 1];
+          js = s_hs[lo];
         }
-        return ka[s_hs[lo] + (i - s_hx[lo])];
+        return ka[js + (i - j0)];
       };
       vt_fold_seq<K, BLOCK>(tot, key_at, s_key, s_cnt, &s_fill, &s_ecnt, answer, pending);
     }
