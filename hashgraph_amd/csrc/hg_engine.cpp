@@ -155,9 +155,10 @@ struct hg_ctx_s {
   bool hev_used[kSlots] = {false, false, false, false};
   int next_slot = 0;
   unsigned long long *h_small = nullptr;  // pinned read-back area
-  // direct probe: device counters (zero between calls) and the pinned words
-  // its last workgroup stores them to
+  // direct probe: device counters (cleared before its first call, zero between
+  // calls) and the pinned words its last workgroup stores them to
   void *direct_state = nullptr;
+  bool direct_ready = false;
   unsigned long long *h_direct = nullptr;
   // staged tables: upload and copy-back streams and their events
   hipStream_t st_in = nullptr, st_out = nullptr;
@@ -1585,8 +1586,7 @@ hg_status hg_ctx_create(int device, hg_ctx *out) {
     return fail(HG_ERR_DEVICE, "hipHostMalloc failed");
   }
   if (hipHostMalloc((void **)&c->h_direct, 64, hipHostMallocCoherent) != hipSuccess ||
-      hipMalloc(&c->direct_state, DIRECT_STATE_BYTES) != hipSuccess ||
-      hipMemset(c->direct_state, 0, DIRECT_STATE_BYTES) != hipSuccess || hipDeviceSynchronize() != hipSuccess) {
+      hipMalloc(&c->direct_state, DIRECT_STATE_BYTES) != hipSuccess) {
     hg_ctx_destroy(c);
     return fail(HG_ERR_DEVICE, "context counters: allocation failed");
   }
@@ -2036,6 +2036,10 @@ hg_status hg_probe(hg_ctx c, const hg_table_desc *descA, const void *d_offA, con
   const bool wide = wide_only();
   if (!wide && probe_direct_takes(descA, d_probe, n_probe, d_out, capacity)) {
     HG_TRY(arena_ensure(c, 0, n_probe * kb));
+    if (!c->direct_ready) {
+      HG_HIP(launch_fill_u64((unsigned long long *)c->direct_state, 0ull, DIRECT_STATE_BYTES / 8, c->stream));
+      c->direct_ready = true;
+    }
     LaunchProbeDirect p{};
     p.key_bytes = kb;
     p.off_bytes = ob;

@@ -185,3 +185,39 @@ def test_run_length_join_keeps_to_its_bounds(kb):
         assert free - torch.cuda.mem_get_info()[0] < 200 << 20
     finally:
         c.close()
+
+
+@pytest.mark.gpu
+def test_context_created_while_a_stream_captures():
+    """A context made by one thread neither waits for another thread's capture
+    nor spoils it."""
+    import threading
+    x = torch.zeros(1000, device="cuda")
+    made, g = [], torch.cuda.CUDAGraph()
+
+    def make():
+        try:
+            made.append(hg.Context(0))
+        except hg.HGError as e:
+            made.append(e)
+
+    with torch.cuda.graph(g, stream=torch.cuda.Stream(), capture_error_mode="thread_local"):
+        x += 1
+        t = threading.Thread(target=make)
+        t.start()
+        t.join()
+        x += 1
+    assert isinstance(made[0], hg.Context), made[0]
+    for i in range(3):
+        g.replay()
+        torch.cuda.synchronize()
+        assert bool((x == 2 * (i + 1)).all())
+    keys = torch.arange(1000, dtype=torch.int32, device="cuda")
+    off, csr = hg.build(keys, 1000)
+    cnt = ctypes.c_uint64(0)
+    c = made[0]
+    for _ in range(3):
+        hg.check(c.lib.hg_probe(c.bind_stream(), ctypes.byref(hg._desc(1000, 1000, 4)), P(off), P(csr), P(keys), 1000,
+                                None, 0, ctypes.byref(cnt)), "hg_probe")
+        assert cnt.value == 1000
+    c.close()
