@@ -827,6 +827,14 @@ uint32_t probe_geometry(uint64_t nb, uint64_t na, uint64_t M, int kb, int first,
     if (w < 1) continue;
     W = (uint32_t)w;
     if ((M + W - 1) / W > cols) continue;
+    if (first == 0) {
+      // the narrow pass's columns to spare, down to buckets half as wide: where
+      // the keys of A set the width, full buckets leave CUs idle (5 M uint64
+      // keys, 50 to a bin, a third as many probes: 881 us, 441 spread; one to a
+      // bin: 82 and 79)
+      const uint32_t least = (uint32_t)((M + cols - 1) / cols);
+      W = (uint32_t)probe_bins(std::min(W, std::max(least, (W + 1) / 2)), r, kb, probe_room(cls), lds);
+    }
     // all the LDS that as many workgroups a CU leave each other: room for the
     // buckets of duplicates, which spread wider than that, and for a learned
     // model's leaves (4 M uint64 keys, 4096 leaves: 169 us with what the mean
@@ -843,8 +851,14 @@ uint32_t probe_geometry(uint64_t nb, uint64_t na, uint64_t M, int kb, int first,
 uint32_t narrow_probe(uint64_t nb, uint64_t na, uint64_t M, int kb, uint32_t &W, uint32_t &lds) {
   return probe_geometry(nb, na, M, kb, 0, 0.8, NARROW_COLS, W, lds);
 }
-// The same for a probe's two-step partition (8 K-key buckets first).
+// The same for a probe's two-step partition (8 K-key buckets first).  Not for
+// tables of about 17.5 to 25 keys a bin: there nearly every bucket has a few
+// bins beyond the walk limit and so is gone through a second time, and the wide
+// pass has two thirds of the buckets (2^26 uint64 keys, a third as many probes:
+// 629 us here and 678 wide at 16 keys a bin, 1162 and 878 at 20, 1699 and 2022
+// at 28).
 uint32_t deep_probe(uint64_t nb, uint64_t na, uint64_t M, int kb, uint32_t &W, uint32_t &lds) {
+  if (2 * na > 35 * M && na < 25 * M) return 0;
   return probe_geometry(nb, na, M, kb, 1, 0.875, DEEP_FINE, W, lds);
 }
 

@@ -150,3 +150,22 @@ def test_narrow_builds_of_copies(n, M, copies, kb, ob, dev):
     off2, ck, ind = hg.build_indexed(keys, M, offset_bytes=ob)
     assert torch.equal(off2, off) and torch.equal(torch.sort(ind).values, torch.arange(n, device=dev))
     assert torch.equal(ck, keys[ind]) and torch.equal(bins[ind], order)
+
+
+@pytest.mark.parametrize("kb", [4, 8])
+@pytest.mark.parametrize("per", [0.1, 1, 4, 16, 17.5, 18, 24.9, 25, 40, 300])
+@pytest.mark.parametrize("n", [2500000, 12582912, 20000003])
+def test_dense_probes(n, per, kb, dev):
+    """Keys of A a bin on both sides of the lines between the probe's ways."""
+    import torch
+    import hashgraph_amd as hg
+    M = int(n / per)
+    print(f"dense probe n={n} M={M} kb={kb}", flush=True)
+    A = wl.uniform_keys(31, n, kb, device=dev)
+    B = wl.probe_keys(A, 32, n // 2, 0.4, kb, device=dev)
+    off, csr = hg.build(A, M)
+    ua, ca = torch.unique(A, return_counts=True)
+    pos = torch.searchsorted(ua, B).clamp(max=ua.numel() - 1)
+    want = torch.repeat_interleave(B, torch.where(ua[pos] == B, ca[pos], 0))
+    cnt, out = hg.probe(off, csr, M, B)
+    assert cnt == want.numel() and torch.equal(torch.sort(out).values, torch.sort(want).values)
