@@ -224,8 +224,9 @@ hg_status hg_intersect_indexed(hg_ctx ctx, const hg_table_desc *descA, const voi
  *                 stay in the context's scratch until hg_ctx_destroy.
  *  n_keys may reach 2^32 and beyond (offset_bytes 8).  A build slab of k keys
  *  and r bins takes about k (6 key_bytes + 1) + r (2 offset_bytes + 4) bytes
- *  of 0.9 of the budget; a join slab up to budget / (4 key_bytes) keys of A
- *  and B together.  A run of bins with more keys than one slab holds is
+ *  of 0.9 of the budget; a join slab takes up to 0.35 of it for the keys and
+ *  offsets of A and B together, and no bin of more than budget / (4 key_bytes)
+ *  keys of both.  A run of bins with more keys than one slab holds is
  *  refused with HG_ERR_UNSUPPORTED, as is a single bin with more matches than
  *  budget / (8 key_bytes).  Offsets buffers must be host-accessible (device-
  *  only memory is HG_ERR_INVALID_ARG).  The call returns after its last copy.
@@ -331,14 +332,14 @@ hg_status hg_batch_probe_emit(hg_ctx ctx, const hg_batch_desc *bd, const uint32_
  * a hipGraph; hg_batch_plan_run replays it, ordered after the work already
  * queued on the context's stream and before work queued later.  With
  * autotune & HG_PLAN_AUTOTUNE the plan times candidate tile sizes (8 K, 32 K, 128 K keys per
- * partition workgroup) and bucket fills (bins per final-stage workgroup) by replaying
- * each candidate's graph, and keeps the fastest.  Buffers passed here must
+ * partition workgroup) and bucket sizes (8 K or 32 K keys per final-stage workgroup)
+ * by replaying each candidate's graph, and keeps the fastest.  Buffers passed here must
  * stay valid for the plan's life.  A plan has its own stream and scratch;
  * destroy it before its context. */
 typedef struct hg_batch_plan_s *hg_batch_plan;
 typedef struct {
   uint32_t tile_keys;   /* keys per partition tile */
-  float fill;           /* bucket fill target of the final stage */
+  float fill;           /* bucket fill target of the final stage, of 32 K keys */
   uint32_t candidates;  /* configurations timed */
   float tuned_ms;       /* replay time of the chosen one (-1 without tuning) */
   uint32_t learned_tables; /* tables on their learned model (with HG_PLAN_TRAIN: after the last replay) */
