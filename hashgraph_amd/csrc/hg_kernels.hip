@@ -1467,9 +1467,10 @@ __device__ __forceinline__ void vt_add_existing(const K *s_key, C *s_cnt, K v, u
 // counted apart.  A bin of A is folded in rounds: before each step of up to
 // HT_SLOTS / 2 keys a table more than half full is answered (the probe keys
 // look their values up) and cleared, so a step's inserts always find a free
-// slot.  A step may leave the table full, so a lookup ends after HT_SLOTS slots.  Copies of one value folded in different rounds
-// are answered in each round; their counts and emitted copies add up, so the
-// result equals one answer over the whole bin.
+// slot.  A step may leave the table full, so a lookup ends after HT_SLOTS
+// slots.  Copies of one value folded in different rounds are answered in each
+// round; their counts and emitted copies add up, so the result equals one
+// answer over the whole bin.
 // ---------------------------------------------------------------------------
 template <typename K, int BLOCK>
 __device__ __forceinline__ void vt_clear(K *s_key, uint32_t *s_cnt, uint32_t *s_fill, uint32_t *s_ecnt) {
